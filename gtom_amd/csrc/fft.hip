@@ -24,7 +24,8 @@
 namespace gx {
 
 // ---------------------------------------------------------------------------
-// Column transforms along a strided axis, in place. Workgroup = TX adjacent
+// Column transforms along a strided axis, from src into data (which may be
+// src: a workgroup reads its columns before it writes them). Workgroup = TX adjacent
 // columns (contiguous in memory) x R2 threads per column. Plane p selects the
 // base offset (p / P1) * S1 + (p % P1) * S0.
 // ---------------------------------------------------------------------------
@@ -35,7 +36,7 @@ template <int N> constexpr int fft_col_tx() { return (N == 128 || N == 256) ? 32
 
 template <int N, int DIR>
 __global__ __launch_bounds__(fft_col_tx<N>() * ColShape<N>::R2, (N == 512 ? 2 : 1)) void k_cols(
-    float2* __restrict__ data, int width, long long axis_stride, long long nplanes, long long P1,
+    const float2* src, float2* data, int width, long long axis_stride, long long nplanes, long long P1,
     long long S0, long long S1, const float2* __restrict__ tw) {
   constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = fft_col_tx<N>();
   __shared__ float2 xch[R2 > 1 ? TX * N : 1];
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(fft_col_tx<N>() * ColShape<N>::R2, (N == 512 ? 2 : 
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1; ++m)
-      v[m] = valid ? data[base + (long long)(j + R2 * m) * axis_stride] : make_float2(0.f, 0.f);
+      v[m] = valid ? src[base + (long long)(j + R2 * m) * axis_stride] : make_float2(0.f, 0.f);
     __syncthreads();
     if constexpr (LDS_TW)
       fft_two_step<N, R1, R2, DIR>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; },
@@ -663,11 +664,11 @@ __global__ __launch_bounds__(256) void k_zero_outside_band(float2* __restrict__ 
 namespace {
 
 template <int DIR>
-int launch_cols_n(int n, float2* data, int width, long long axis_stride, long long nplanes,
+int launch_cols_n(int n, const float2* src, float2* data, int width, long long axis_stride, long long nplanes,
                   long long P1, long long S0, long long S1, const float2* tw, hipStream_t s) {
   auto go = [&](auto kernel, int TX, int R2) -> int {
     dim3 grid((width + TX - 1) / TX, (unsigned)std::min<long long>(nplanes, 65535));
-    hipLaunchKernelGGL(kernel, grid, dim3(TX * R2), 0, s, data, width, axis_stride, nplanes, P1, S0, S1, tw);
+    hipLaunchKernelGGL(kernel, grid, dim3(TX * R2), 0, s, src, data, width, axis_stride, nplanes, P1, S0, S1, tw);
     GX_LAUNCHED("k_cols");
     return GTOMX_OK;
   };
@@ -768,15 +769,15 @@ int launch_lines(int n, const float2* src, float2* dst, const LineMap& p, const 
   }
 }
 
-// One strided axis of length L in place; above 256 through `scratch`, which
-// mirrors data's extent.
+// One strided axis of length L from src into data (src may be data); above 256
+// through `scratch`, which mirrors data's extent.
 template <int DIR>
-int cols_axis(int L, float2* data, float2* scratch, int width, long long as, long long nplanes, long long P1,
+int cols_axis(int L, const float2* src, float2* data, float2* scratch, int width, long long as, long long nplanes, long long P1,
               long long S0, long long S1, const float2* tw, hipStream_t s, int band = 0) {
   // one pass up to 256 and at 512 (the exchange of 16 columns fits LDS), two otherwise or
   // with a band
   if (L <= 256 || (L == 512 && band == 0))
-    return launch_cols_n<DIR>(L, data, width, as, nplanes, P1, S0, S1, tw, s);
+    return launch_cols_n<DIR>(L, src, data, width, as, nplanes, P1, S0, S1, tw, s);
   int L1, L2;
   if (!split_len(L, &L1, &L2) || !scratch) return fail(GTOMX_ERR_INTERNAL, "axis length not split");
   if ((long long)L * as >= (1LL << 31)) return fail(GTOMX_ERR_UNSUPPORTED, "axis span of 2^31 elements or more");
@@ -784,7 +785,7 @@ int cols_axis(int L, float2* data, float2* scratch, int width, long long as, lon
   a.P1 = P1, a.S0s = a.S0d = S0, a.S1s = a.S1d = S1, a.Cs = a.Cd = 1;
   a.G = L2, a.Gs = a.Gd = as, a.Ms = a.Md = L2 * as, a.nplanes = nplanes * L2, a.width = width;
   a.L = L, a.TG = 1, a.TC = 0, a.scale = 1.f, a.band = band;
-  GX_TRY(launch_lines<DIR>(L1, data, scratch, a, tw, s));
+  GX_TRY(launch_lines<DIR>(L1, src, scratch, a, tw, s));
   LineMap b = a;
   b.G = L1, b.Gs = L2 * as, b.Gd = as, b.Ms = as, b.Md = L1 * as, b.nplanes = nplanes * L1, b.L = 0, b.band = 0;
   return launch_lines<DIR>(L2, scratch, data, b, tw, s);
@@ -826,46 +827,28 @@ int launch_rows_long(int n, const void* in, void* out, long long nrows, float sc
 }
 
 
-// Stream-ordered scratch for the two-pass axes: taken from the stream's pool
-// and given back on the same stream, so no synchronisation is needed.
-struct StreamScratch {
-  float2* p = nullptr;
-  hipStream_t s = nullptr;
-  int take(size_t n, hipStream_t st) {
-    s = st;
-    void* q = nullptr;
-    hipError_t e = hipMallocAsync(&q, n * sizeof(float2), st);
-    if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(FFT scratch)");
-    p = static_cast<float2*>(q);
-    return GTOMX_OK;
-  }
-  ~StreamScratch() {
-    if (p) (void)hipFreeAsync(p, s);
-  }
-};
-
 // The y and z transforms of half spectra over their first `cols` columns
-// (cols = 0: all n/2 + 1).
-int yz_axes(float2* data, float2* scr, gtomx_int3 d, unsigned batch, int dir, const float2* tw, hipStream_t s,
-            int cols = 0) {
+// (cols = 0: all n/2 + 1), from src into data (which may be src; both axes 1: nothing is done).
+int yz_axes(const float2* src, float2* data, float2* scr, gtomx_int3 d, unsigned batch, int dir, const float2* tw,
+            hipStream_t s, int cols = 0) {
   const long long nh = d.x / 2 + 1;
   const int w = cols > 0 ? cols : (int)nh;
-  auto zax = [&](auto DIRC) {
-    return cols_axis<decltype(DIRC)::value>(d.z, data, scr, w, nh * d.y, (long long)d.y * batch, d.y, nh,
+  auto zax = [&](auto DIRC, const float2* from) {
+    return cols_axis<decltype(DIRC)::value>(d.z, from, data, scr, w, nh * d.y, (long long)d.y * batch, d.y, nh,
                                             nh * d.y * d.z, tw, s);
   };
-  auto yax = [&](auto DIRC) {
-    return cols_axis<decltype(DIRC)::value>(d.y, data, scr, w, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0,
+  auto yax = [&](auto DIRC, const float2* from) {
+    return cols_axis<decltype(DIRC)::value>(d.y, from, data, scr, w, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0,
                                             tw, s);
   };
   using F = std::integral_constant<int, -1>;
   using B = std::integral_constant<int, 1>;
   if (dir < 0) {
-    if (d.y > 1) GX_TRY(yax(F{}));
-    if (d.z > 1) GX_TRY(zax(F{}));
+    if (d.y > 1) GX_TRY(yax(F{}, src));
+    if (d.z > 1) GX_TRY(zax(F{}, d.y > 1 ? data : src));
   } else {
-    if (d.z > 1) GX_TRY(zax(B{}));
-    if (d.y > 1) GX_TRY(yax(B{}));
+    if (d.z > 1) GX_TRY(zax(B{}, src));
+    if (d.y > 1) GX_TRY(yax(B{}, d.z > 1 ? data : src));
   }
   return GTOMX_OK;
 }
@@ -873,18 +856,34 @@ int yz_axes(float2* data, float2* scr, gtomx_int3 d, unsigned batch, int dir, co
 int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s);
 int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s);
 
+// Items of a batch that go through the two-pass axes together (0: no axis needs
+// them): scratch of about 128 MB, which the 256 MB last-level cache holds beside
+// what one pass reads or writes, and which bounds what a call keeps.
+unsigned two_pass_items(gtomx_int3 d, unsigned batch) {
+  auto two = [](int L) { return L > 256 && L != 512; };
+  if (!two(d.y) && !two(d.z)) return 0;
+  return (unsigned)std::max<size_t>(1, std::min<size_t>(batch, (128u << 20) / (elements_ft(d) * sizeof(float2))));
+}
+
 int fft_r2c(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s) {
   if (!dims_native(d)) return fft_r2c_any(in, out, d, batch, s);
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
-  const long long rows = (long long)d.y * d.z * batch;
   StreamScratch scr;
-  if (d.y > 256 || d.z > 256) GX_TRY(scr.take(elements_ft(d) * batch, s));
-  if (d.x > 256)
-    GX_TRY(launch_rows_long<true>(d.x, in, out, rows, 1.f, tw, s));
-  else
-    GX_TRY(launch_rows_r2c(d.x, in, out, rows, tw, s));
-  return yz_axes(out, scr.p, d, batch, -1, tw, s);
+  const unsigned per = two_pass_items(d, batch);
+  if (per) GX_TRY(scr.take(elements_ft(d) * per, s));
+  for (unsigned b = 0; b < batch; b += per ? per : batch) {
+    const unsigned nb = per ? std::min(per, batch - b) : batch;
+    const long long rows = (long long)d.y * d.z * nb;
+    const float* ib = in + b * elements(d);
+    float2* ob = out + b * elements_ft(d);
+    if (d.x > 256)
+      GX_TRY(launch_rows_long<true>(d.x, ib, ob, rows, 1.f, tw, s));
+    else
+      GX_TRY(launch_rows_r2c(d.x, ib, ob, rows, tw, s));
+    GX_TRY(yz_axes(ob, ob, scr.p, d, nb, -1, tw, s));
+  }
+  return GTOMX_OK;
 }
 
 int fft_c2r(const float2* in, float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s,
@@ -893,14 +892,33 @@ int fft_c2r(const float2* in, float2* work, float* out, gtomx_int3 d, unsigned b
   GX_TRY(twiddles(&tw));
   const size_t H = elements_ft(d) * batch;
   if (cols < 0 || cols > d.x / 2 + 1) return fail(GTOMX_ERR_INTERNAL, "column count outside the half spectrum");
-  if (work != in) GX_HIP(hipMemcpyAsync(work, in, H * sizeof(float2), hipMemcpyDeviceToDevice, s));
-  if (!dims_native(d)) return fft_c2r_any(work, out, d, batch, scale, s);
+  if (!dims_native(d)) {
+    if (work != in) GX_HIP(hipMemcpyAsync(work, in, H * sizeof(float2), hipMemcpyDeviceToDevice, s));
+    return fft_c2r_any(work, out, d, batch, scale, s);
+  }
+  const bool axes = d.y > 1 || d.z > 1;
+  // with a column limit the first axis leaves the other columns as they are
+  if (work != in && axes && cols > 0) {
+    GX_HIP(hipMemcpyAsync(work, in, H * sizeof(float2), hipMemcpyDeviceToDevice, s));
+    in = work;
+  }
   StreamScratch scr;
-  if (d.y > 256 || d.z > 256) GX_TRY(scr.take(H, s));
-  GX_TRY(yz_axes(work, scr.p, d, batch, 1, tw, s, cols));
-  const long long rows = (long long)d.y * d.z * batch;
-  if (d.x > 256) return launch_rows_long<false>(d.x, work, out, rows, scale, tw, s);
-  return launch_rows_c2r(d.x, work, out, rows, scale, tw, s);
+  const unsigned per = two_pass_items(d, batch);
+  if (per) GX_TRY(scr.take(elements_ft(d) * per, s));
+  for (unsigned b = 0; b < batch; b += per ? per : batch) {
+    const unsigned nb = per ? std::min(per, batch - b) : batch;
+    const float2* ib = in + b * elements_ft(d);
+    float2* wb = work + b * elements_ft(d);
+    float* ob = out + b * elements(d);
+    GX_TRY(yz_axes(ib, wb, scr.p, d, nb, 1, tw, s, cols));
+    const float2* from = axes ? wb : ib;
+    const long long rows = (long long)d.y * d.z * nb;
+    if (d.x > 256)
+      GX_TRY(launch_rows_long<false>(d.x, from, ob, rows, scale, tw, s));
+    else
+      GX_TRY(launch_rows_c2r(d.x, from, ob, rows, scale, tw, s));
+  }
+  return GTOMX_OK;
 }
 
 
@@ -971,7 +989,7 @@ int image_c2r_banded(float2* work, float* out, int n, unsigned nb, int cols, int
   const long long nh = n / 2 + 1;
   StreamScratch scr;
   GX_TRY(scr.take((size_t)nh * n * nb, s));
-  GX_TRY(cols_axis<1>(n, work, scr.p, cols, nh, (long long)nb, 1LL << 62, nh * n, 0, tw, s));
+  GX_TRY(cols_axis<1>(n, work, work, scr.p, cols, nh, (long long)nb, 1LL << 62, nh * n, 0, tw, s));
   return launch_rows_long<false>(n, work, out, (long long)nb * 2 * band, scale, tw, s, n, band);
 }
 
@@ -985,7 +1003,7 @@ int image_r2c_banded(const float* in, float2* out, int n, unsigned nb, int band,
   GX_TRY(launch_rows_long<true>(n, in, out, (long long)nb * 2 * band, 1.f, tw, s, n, band));
   StreamScratch scr;
   GX_TRY(scr.take((size_t)nh * n * nb, s));
-  return cols_axis<-1>(n, out, scr.p, (int)nh, nh, (long long)nb, 1LL << 62, nh * n, 0, tw, s, band);
+  return cols_axis<-1>(n, out, out, scr.p, (int)nh, nh, (long long)nb, 1LL << 62, nh * n, 0, tw, s, band);
 }
 
 int rows_per_workgroup(int n) {
@@ -1005,7 +1023,7 @@ int volume_c2r_banded(float2* work, float* out, gtomx_int3 d, unsigned nb, int c
   GX_TRY(twiddles(&tw));
   if (d.x > 256 || d.y > 256 || d.z > 256 || by <= 0 || 2 * by > d.y || bz < 0 || 2 * bz > d.z)
     return fail(GTOMX_ERR_INTERNAL, "banded C2R outside its range");
-  GX_TRY(yz_axes(work, nullptr, d, nb, 1, tw, s, cols));
+  GX_TRY(yz_axes(work, work, nullptr, d, nb, 1, tw, s, cols));
   RowBand rb;
   rb.ny = d.y, rb.by = by, rb.nz = d.z, rb.bz = bz;
   const long long rows = (long long)nb * (bz ? 2 * bz : d.z) * 2 * by;
@@ -1027,15 +1045,15 @@ int volume_r2c_banded(const float* in, float2* out, gtomx_int3 d, unsigned nb, i
   if (d.y > 1) {  // planes outside the z band are zero: their y transform is skipped
     if (bz > 0) {
       const long long pl = nh * d.y;
-      GX_TRY(launch_cols_n<-1>(d.y, out, (int)nh, nh, (long long)nb * bz, bz, pl, pl * d.z, tw, s));
-      GX_TRY(launch_cols_n<-1>(d.y, out + (d.z - bz) * pl, (int)nh, nh, (long long)nb * bz, bz, pl, pl * d.z, tw,
-                               s));
+      GX_TRY(launch_cols_n<-1>(d.y, out, out, (int)nh, nh, (long long)nb * bz, bz, pl, pl * d.z, tw, s));
+      GX_TRY(launch_cols_n<-1>(d.y, out + (d.z - bz) * pl, out + (d.z - bz) * pl, (int)nh, nh, (long long)nb * bz,
+                               bz, pl, pl * d.z, tw, s));
     } else {
-      GX_TRY(launch_cols_n<-1>(d.y, out, (int)nh, nh, (long long)d.z * nb, 1LL << 62, nh * d.y, 0, tw, s));
+      GX_TRY(launch_cols_n<-1>(d.y, out, out, (int)nh, nh, (long long)d.z * nb, 1LL << 62, nh * d.y, 0, tw, s));
     }
   }
   if (d.z > 1)
-    GX_TRY(launch_cols_n<-1>(d.z, out, (int)nh, nh * d.y, (long long)d.y * nb, d.y, nh, nh * d.y * d.z, tw, s));
+    GX_TRY(launch_cols_n<-1>(d.z, out, out, (int)nh, nh * d.y, (long long)d.y * nb, d.y, nh, nh * d.y * d.z, tw, s));
   return GTOMX_OK;
 }
 
@@ -1043,8 +1061,13 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   StreamScratch scr;
-  if (d.y > 256 || d.z > 256) GX_TRY(scr.take(elements_ft(d) * batch, s));
-  return yz_axes(data, scr.p, d, batch, 1, tw, s);
+  const unsigned per = two_pass_items(d, batch);
+  if (per) GX_TRY(scr.take(elements_ft(d) * per, s));
+  for (unsigned b = 0; b < batch; b += per ? per : batch) {
+    float2* db = data + b * elements_ft(d);
+    GX_TRY(yz_axes(db, db, scr.p, d, per ? std::min(per, batch - b) : batch, 1, tw, s));
+  }
+  return GTOMX_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1308,11 +1331,11 @@ int blue_axis(const void* src, AxisLines as, void* dst, AxisLines ad, long long 
                          l0, nl, L, nh, M, t.chirp, W.p);
       GX_LAUNCHED("k_blue_load_rows");
     }
-    GX_TRY(cols_axis<-1>(M, W.p, W2.p, nl, nl, 1, 1LL << 62, (long long)M * nl, 0, tw, s));
+    GX_TRY(cols_axis<-1>(M, W.p, W.p, W2.p, nl, nl, 1, 1LL << 62, (long long)M * nl, 0, tw, s));
     hipLaunchKernelGGL(k_blue_mul, dim3(blue_grid((long long)M * nl)), dim3(256), 0, s, W.p, nl, M,
                        DIR < 0 ? t.bf : t.bi);
     GX_LAUNCHED("k_blue_mul");
-    GX_TRY(cols_axis<1>(M, W.p, W2.p, nl, nl, 1, 1LL << 62, (long long)M * nl, 0, tw, s));
+    GX_TRY(cols_axis<1>(M, W.p, W.p, W2.p, nl, nl, 1, 1LL << 62, (long long)M * nl, 0, tw, s));
     if constexpr (OUT == 0) {
       hipLaunchKernelGGL((k_blue_store<OUT, DIR>), dim3(blue_grid((long long)nout * nl)), dim3(256), 0, s, W.p, ad,
                          l0, nl, nout, t.chirp, dst, scale);
@@ -1338,14 +1361,14 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
   auto yax = [&](auto DIRC) -> int {
     constexpr int D = decltype(DIRC)::value;
     if (fft_len_ok_any(d.y))
-      return cols_axis<D>(d.y, data, scr.p, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, tw, s);
+      return cols_axis<D>(d.y, data, data, scr.p, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, tw, s);
     const AxisLines a{nh, 1, nh * d.y, nh};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.z * batch, d.y, 0, 1.f, s);
   };
   auto zax = [&](auto DIRC) -> int {
     constexpr int D = decltype(DIRC)::value;
     if (fft_len_ok_any(d.z))
-      return cols_axis<D>(d.z, data, scr.p, (int)nh, nh * d.y, (long long)d.y * batch, d.y, nh, nh * d.y * d.z, tw,
+      return cols_axis<D>(d.z, data, data, scr.p, (int)nh, nh * d.y, (long long)d.y * batch, d.y, nh, nh * d.y * d.z, tw,
                           s);
     const AxisLines a{nh * d.y, 1, nh * d.y * d.z, nh * d.y};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.y * batch, d.z, 0, 1.f, s);
@@ -1421,12 +1444,11 @@ extern "C" int gtomx_ifft_c2r(const gtomx_complex* d_input, float* d_output, int
   GX_TRY(check_fft_dims_any(ndims, dims));
   if (!d_input || !d_output) return fail(GTOMX_ERR_INVALID_ARGUMENT, "NULL buffer");
   if (batch == 0) return fail(GTOMX_ERR_INVALID_ARGUMENT, "batch must be positive");
-  DevBuf work;
-  GX_TRY(work.alloc(elements_ft(dims) * batch * sizeof(float2)));
   hipStream_t s = as_stream(stream);
+  StreamScratch work;
+  GX_TRY(work.take(elements_ft(dims) * batch, s, true));
   float scale = renormalize ? (float)(1.0 / (double)elements(dims)) : 1.0f;
-  GX_TRY(fft_c2r(reinterpret_cast<const float2*>(d_input), work.as<float2>(), d_output, dims, batch, scale, s));
-  // The workspace is released when this call returns; wait for its last use.
+  GX_TRY(fft_c2r(reinterpret_cast<const float2*>(d_input), work.p, d_output, dims, batch, scale, s));
   GX_HIP(hipStreamSynchronize(s));
   return GTOMX_OK;
 }

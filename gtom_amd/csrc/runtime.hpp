@@ -138,6 +138,23 @@ struct DevBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Stream-ordered scratch of one call: taken on stream s, given back on s when
+// the object goes away, so the caller does not synchronise. Blocks are kept
+// for the next call of any thread or stream (scratch_take in runtime.cpp).
+struct StreamScratch {
+  float2* p = nullptr;
+  StreamScratch() = default;
+  StreamScratch(const StreamScratch&) = delete;
+  StreamScratch& operator=(const StreamScratch&) = delete;
+  ~StreamScratch();
+  // n complex values; counted: an allocation for the fault-injection hook
+  int take(size_t n, hipStream_t st, bool counted = false);
+
+ private:
+  hipStream_t s = nullptr;
+  int block = -1;  // index in the pool, or -1 for a hipMallocAsync allocation
+};
+
 // ---- internal host API shared between translation units ----
 // Batched 3D/2D transforms (dims with dims.z == 1 for 2D). `work` must hold
 // elements_ft(dims) * batch complex values for c2r (the input is copied
@@ -148,8 +165,8 @@ int fft_r2c(const float* in, float2* out, gtomx_int3 dims, unsigned batch, hipSt
 // and z inverses skip them (the result is the same).
 int fft_c2r(const float2* in, float2* work, float* out, gtomx_int3 dims, unsigned batch,
             float scale, hipStream_t s, int cols = 0);
-// Axes above 256 go through two passes with a scratch copy of the data, taken
-// from the stream's memory pool (hipMallocAsync) and returned on the stream.
+// Axes above 256 go through two passes with a scratch copy of the data
+// (StreamScratch).
 // L = L1 * L2 as the two-pass transforms split it (L above 256).
 int fft_len_split(int L, int* L1, int* L2);
 // Pass 2 of the inverse y transform of nb n x n half spectra (n above 256),

@@ -1,0 +1,72 @@
+"""The transforms' kept scratch (StreamScratch): results do not depend on what earlier calls, streams
+or threads left in the blocks, and a C2R leaves its input as it was. Transforms of every size class that
+takes scratch are compared bit for bit with the first call's result."""
+import threading
+
+import numpy as np
+import pytest
+
+from tests._util import to_np
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2, (3, 512, 640)), (2, (5, 768, 1024)), (3, (2, 40, 384, 75)), (2, (1, 1000, 96)), (3, (1, 512, 32, 48))]
+
+
+def _round(gx, x, ndims):
+    X = gx.d_FFTR2C(x, ndims=ndims)
+    return X, gx.d_IFFTC2R(X, x.shape[-1], ndims=ndims)
+
+
+def test_scratch_across_sizes_and_streams(gx, cuda):
+    import torch
+    rng = np.random.default_rng(5)
+    data = [(nd, torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(cuda)) for nd, s in SHAPES]
+    want = []
+    for nd, x in data:
+        X, y = _round(gx, x, nd)
+        ref = np.fft.rfftn(to_np(x).astype(np.float64), axes=tuple(range(-nd, 0)))
+        # single-precision transforms of these lengths stay below 1e-6 normwise
+        assert np.linalg.norm(to_np(X) - ref) <= 1e-6 * np.linalg.norm(ref)
+        assert np.linalg.norm(to_np(y) - to_np(x)) <= 2e-6 * np.linalg.norm(to_np(x))
+        want.append((to_np(X), to_np(y)))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for k in range(6):
+        got = []
+        for i, (nd, x) in enumerate(data):
+            with torch.cuda.stream(streams[(i + k) % 3]):
+                X = gx.d_FFTR2C(x, ndims=nd)
+                keep = X.clone()
+                got.append((X, keep, gx.d_IFFTC2R(X, x.shape[-1], ndims=nd)))
+        torch.cuda.synchronize()
+        for (X, keep, y), (wX, wy) in zip(got, want):
+            assert torch.equal(torch.view_as_real(X), torch.view_as_real(keep))
+            assert np.array_equal(to_np(X), wX) and np.array_equal(to_np(y), wy)
+
+
+def test_scratch_from_threads(gx, cuda):
+    import torch
+    rng = np.random.default_rng(6)
+    data = [(nd, torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(cuda)) for nd, s in SHAPES]
+    want = [tuple(map(to_np, _round(gx, x, nd))) for nd, x in data]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for i in range(8):
+                nd, x = data[(i + k) % len(data)]
+                X, y = _round(gx, x, nd)
+                s.synchronize()
+                w = want[(i + k) % len(data)]
+                if not (np.array_equal(to_np(X), w[0]) and np.array_equal(to_np(y), w[1])):
+                    bad.append((k, i))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
