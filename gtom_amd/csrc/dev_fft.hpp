@@ -266,6 +266,28 @@ __device__ __forceinline__ float2 twiddle_from(const float2* tw, int m, TwiddleL
   return DIR > 0 ? make_float2(w.x, -w.y) : w;
 }
 
+// Or an LDS copy of the table of length 2N (the rows' half-length transforms share the columns' table).
+struct TwiddleLDSHalf {};
+template <int DIR, int N>
+__device__ __forceinline__ float2 twiddle_from(const float2* tw, int m, TwiddleLDSHalf) {
+  const float2 w = tw[(2 * m) % (2 * N)];
+  return DIR > 0 ? make_float2(w.x, -w.y) : w;
+}
+
+// What separates the writes of the exchange from its reads: the workgroup's
+// barrier, or, where the R2 threads of a transform are lanes of one wave and
+// nobody else touches their exchange area, the wave's own order (LDS accesses
+// of a wave complete in order; the fence keeps the compiler from moving them).
+struct SyncGroup {
+  __device__ __forceinline__ void operator()() const { __syncthreads(); }
+};
+struct SyncWave {
+  __device__ __forceinline__ void operator()() const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+
 // Or twiddles the thread holds in registers: w[k1] = exp(DIR 2 pi i j k1 / N)
 // for its j (w[0] unused), loaded once by load_two_step_twiddles.
 template <int R1> struct TwiddleRegs {
@@ -286,9 +308,9 @@ __device__ __forceinline__ float2 stage_twiddle(const float2*, int, int k1, Twid
   return src.w[k1];
 }
 
-template <int N, int R1, int R2, int DIR, class Xch, class Src = TwiddleGlobal>
+template <int N, int R1, int R2, int DIR, class Xch, class Src = TwiddleGlobal, class Sync = SyncGroup>
 __device__ __forceinline__ void fft_two_step(float2 (&v)[R1], int j, const float2* __restrict__ tw, Xch xch,
-                                             Src src = Src{}) {
+                                             Src src = Src{}, Sync sync = Sync{}) {
   static_assert(R1 * R2 == N, "bad factorisation");
   dft<R1, DIR>(v);
   if constexpr (R2 > 1) {
@@ -297,7 +319,7 @@ __device__ __forceinline__ void fft_two_step(float2 (&v)[R1], int j, const float
     for (int k1 = 1; k1 < R1; ++k1) v[k1] = cmul(v[k1], stage_twiddle<DIR, N>(tw, j, k1, src));
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) *xch(k1, j) = v[k1];
-    __syncthreads();
+    sync();
 #pragma unroll
     for (int u = 0; u < R1 / R2; ++u) {
       float2 z[R2];

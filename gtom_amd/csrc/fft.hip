@@ -1079,10 +1079,312 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
 // done with the native M-point column transforms: load a[j] = x[j] c[j]
 // (zero for j >= L), forward M-point DFT, times B[k] / M with B the DFT of
 // b[m] = conj(c[m]) (m in (-L, L), wrapped), inverse M-point DFT, times c[k].
-// The inverse DFT uses conj(c) for c and c for b. The lines of one axis are
-// gathered into an M x (lines) block (line index fastest, the layout the
+// The inverse DFT uses conj(c) for c and c for b. Lengths up to 512 run the whole
+// convolution of a line inside one kernel (below); above, the lines of one axis
+// are gathered into an M x (lines) block (line index fastest, the layout the
 // column kernels take), in chunks that keep the block within 2^31 elements
 // and 256 MB.
+
+// ---------------------------------------------------------------------------
+// Lengths up to 512: load, both M-point transforms and the store in one kernel,
+// one pass over memory instead of five over a block 2 to 4 times as long (a 200^3
+// search spent 64% of its time in the column transforms and k_blue_mul of that
+// block). R2 threads hold a line; thread j the points j + R2 m. L <= M/2, so only
+// m < R1/2 hold input and only those are wanted back: the compiler drops the
+// rest of the first and last stages. The transform ends with every k2 of a k1 in
+// one thread (k = k1 + R1 k2), which is where the inverse can start, so the
+// product with B needs no exchange of its own: two exchanges in all, the second
+// through the addresses a thread read itself.
+// ---------------------------------------------------------------------------
+template <int M> struct BlueShape;
+template <> struct BlueShape<16>   { static constexpr int R1 = 4,  R2 = 4,  TX = 64; };
+template <> struct BlueShape<24>   { static constexpr int R1 = 12, R2 = 2,  TX = 64; };
+template <> struct BlueShape<32>   { static constexpr int R1 = 8,  R2 = 4,  TX = 64; };
+template <> struct BlueShape<48>   { static constexpr int R1 = 12, R2 = 4,  TX = 64; };
+template <> struct BlueShape<64>   { static constexpr int R1 = 8,  R2 = 8,  TX = 32; };
+template <> struct BlueShape<96>   { static constexpr int R1 = 24, R2 = 4,  TX = 32; };
+template <> struct BlueShape<128>  { static constexpr int R1 = 16, R2 = 8,  TX = 32; };
+template <> struct BlueShape<192>  { static constexpr int R1 = 24, R2 = 8,  TX = 16; };
+template <> struct BlueShape<256>  { static constexpr int R1 = 16, R2 = 16, TX = 16; };
+template <> struct BlueShape<512>  { static constexpr int R1 = 32, R2 = 16, TX = 16; };
+template <> struct BlueShape<1024> { static constexpr int R1 = 32, R2 = 32, TX = 16; };
+#define GX_FOR_BLUE(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512) X(1024)
+constexpr int BLUE_FUSED_MAX = 512;  // longest L of the fused form
+
+// The circular convolution of one line with the kernel whose spectrum is B (LDS,
+// M values with the 1/M in them). v[m] in and out: point j + R2 m, zero for
+// m >= R1/2 on entry, meaningful for m < R1/2 on exit.
+template <int M, class Xch, class Sync>
+__device__ __forceinline__ void blue_convolve(float2 (&v)[BlueShape<M>::R1], int j, const float2* twl,
+                                              const float2* B, Xch xch, Sync sync) {
+  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2;
+  dft<R1, -1>(v);
+#pragma unroll
+  for (int k1 = 1; k1 < R1; ++k1) v[k1] = cmul(v[k1], twl[j * k1]);
+#pragma unroll
+  for (int k1 = 0; k1 < R1; ++k1) *xch(k1, j) = v[k1];
+  sync();
+#pragma unroll
+  for (int u = 0; u < R1 / R2; ++u) {
+    const int k1 = j * (R1 / R2) + u;
+    float2 z[R2];
+#pragma unroll
+    for (int jj = 0; jj < R2; ++jj) z[jj] = *xch(k1, jj);
+    dft<R2, -1>(z);
+#pragma unroll
+    for (int k2 = 0; k2 < R2; ++k2) z[k2] = cmul(z[k2], B[k1 + R1 * k2]);
+    dft<R2, 1>(z);
+#pragma unroll
+    for (int jj = 0; jj < R2; ++jj) *xch(k1, jj) = jj == 0 ? z[jj] : cmulc(z[jj], twl[jj * k1]);
+  }
+  sync();
+#pragma unroll
+  for (int k1 = 0; k1 < R1; ++k1) v[k1] = *xch(k1, j);
+  dft<R1, 1>(v);
+}
+
+// The tables of a workgroup: twiddles of M, the kernel spectrum, the chirp as the
+// direction multiplies by it.
+template <int M, int DIR>
+__device__ __forceinline__ void blue_stage(int t, int nt, int L, const float2* __restrict__ tw,
+                                           const float2* __restrict__ B, const float2* __restrict__ chirp, float2* twl,
+                                           float2* bl, float2* cl) {
+  for (int i = t; i < M; i += nt) {
+    twl[i] = twiddle<-1, M>(tw, i);
+    bl[i] = B[i];
+  }
+  for (int i = t; i < M / 2; i += nt) {
+    const float2 c = i < L ? chirp[i] : make_float2(0.f, 0.f);
+    cl[i] = DIR < 0 ? c : cconj(c);
+  }
+}
+
+// A strided axis, from src into dst (which may be src), addressed as k_cols.
+template <int M, int DIR>
+__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols(
+    const float2* src, float2* dst, int width, long long axis_stride, long long nplanes, long long P1, long long S0,
+    long long S1, int L, const float2* __restrict__ chirp, const float2* __restrict__ B,
+    const float2* __restrict__ tw) {
+  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
+  __shared__ float2 xch[TX * M];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  blue_stage<M, DIR>(t, NT, L, tw, B, chirp, twl, bl, cl);
+  const int col = blockIdx.x * TX + c;
+  const bool valid = col < width;
+  for (long long pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
+    const long long base = (pl / P1) * S1 + (pl % P1) * S0 + col;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      v[m] = valid && p < L ? src[base + (long long)p * axis_stride] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();  // the tables are staged, the last plane's exchange is read
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      if (valid && p < L) dst[base + (long long)p * axis_stride] = cmul(v[m], cl[p]);
+    }
+  }
+}
+
+// Rows, two to a transform: one as the real, one as the imaginary part. A pair's
+// R2 threads are lanes of one wave, so the exchanges need no barrier. Pairs per
+// workgroup of 256 threads, and their LDS area (R1 values of padding spread the
+// reads of a k1 over the banks).
+template <int M> struct BlueRows {
+  static constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2;
+  static constexpr int TP = 256 / R2, AREA = M + R1;
+};
+
+// z[p] = A[p] + i B[p] of two half-spectrum rows completed as X[L - q] = conj X[q],
+// without the imaginary parts of X[0] and X[L/2] (the real part of the inverse).
+__device__ __forceinline__ float2 row_pair_bin(const float2* __restrict__ a, const float2* __restrict__ b, bool va,
+                                               bool vb, int p, int L) {
+  const int nh = L / 2 + 1;
+  const bool mirror = p >= nh;
+  const int q = mirror ? L - p : p;
+  float2 x = va ? a[q] : make_float2(0.f, 0.f), y = vb ? b[q] : make_float2(0.f, 0.f);
+  if (q == 0 || 2 * q == L) x.y = y.y = 0.f;
+  return mirror ? make_float2(x.x + y.y, y.x - x.y) : make_float2(x.x - y.y, x.y + y.x);
+}
+
+template <int M>
+__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_c2r(const float2* __restrict__ in, float* __restrict__ out,
+                                                       long long nrows, int L, float scale,
+                                                       const float2* __restrict__ chirp,
+                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
+  using S = BlueRows<M>;
+  constexpr int R1 = S::R1, R2 = S::R2;
+  __shared__ float2 area[S::TP * S::AREA];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, j = t % R2;
+  float2* xch = area + (t / R2) * S::AREA;
+  blue_stage<M, 1>(t, 256, L, tw, B, chirp, twl, bl, cl);
+  __syncthreads();
+  const long long step = 2LL * S::TP * gridDim.x;
+  for (long long row = 2 * ((long long)blockIdx.x * S::TP + t / R2); row < nrows; row += step) {
+    const int nh = L / 2 + 1;
+    const bool two = row + 1 < nrows;
+    const float2* a = in + row * nh;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      v[m] = row_pair_bin(a, a + nh, p < L, p < L && two, p < L ? p : 0, L);
+    }
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    SyncWave{}();
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      if (p >= L) continue;
+      const float2 r = cmul(v[m], cl[p]);
+      out[row * L + p] = r.x * scale;
+      if (two) out[(row + 1) * L + p] = r.y * scale;
+    }
+  }
+}
+
+// A[k] = (Z[k] + conj Z[L - k]) / 2, B[k] = (Z[k] - conj Z[L - k]) / 2i of Z = DFT(a + i b).
+template <int M>
+__global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
+                                                       long long nrows, int L, const float2* __restrict__ chirp,
+                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
+  using S = BlueRows<M>;
+  constexpr int R1 = S::R1, R2 = S::R2;
+  __shared__ float2 area[S::TP * S::AREA];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, j = t % R2;
+  float2* xch = area + (t / R2) * S::AREA;
+  blue_stage<M, -1>(t, 256, L, tw, B, chirp, twl, bl, cl);
+  __syncthreads();
+  const long long step = 2LL * S::TP * gridDim.x;
+  for (long long row = 2 * ((long long)blockIdx.x * S::TP + t / R2); row < nrows; row += step) {
+    const int nh = L / 2 + 1;
+    const bool two = row + 1 < nrows;
+    const float* a = in + row * L;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      v[m] = make_float2(p < L ? a[p] : 0.f, p < L && two ? a[L + p] : 0.f);
+    }
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    SyncWave{}();
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) xch[j + R2 * m] = cmul(v[m], cl[j + R2 * m]);
+    SyncWave{}();
+    for (int k = j; k < nh; k += R2) {
+      const float2 z = xch[k], w = cconj(xch[k == 0 ? 0 : L - k]);
+      const float2 s = cadd(z, w), d = csub(z, w);
+      out[row * nh + k] = make_float2(0.5f * s.x, 0.5f * s.y);
+      if (two) out[(row + 1) * nh + k] = make_float2(0.5f * d.y, -0.5f * d.x);
+    }
+    SyncWave{}();
+  }
+}
+
+// The generic search's row pass: the C2R of every row of the orientations
+// o in group blockIdx.y (og of them), times scale[o], folded into a running
+// maximum in registers (strict >, increasing o). FRESH as in k_pick_x_max.
+template <int M, bool FRESH>
+__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(const float2* __restrict__ G, long long H, int nb, int n,
+                                                       int nrows, int angle0, const float* __restrict__ scale,
+                                                       float* __restrict__ best, int32_t* __restrict__ bidx, int og,
+                                                       const float2* __restrict__ chirp,
+                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
+  using S = BlueRows<M>;
+  constexpr int R1 = S::R1, R2 = S::R2, HP = R1 / 2;
+  __shared__ float2 area[S::TP * S::AREA];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, j = t % R2;
+  float2* xch = area + (t / R2) * S::AREA;
+  blue_stage<M, 1>(t, 256, n, tw, B, chirp, twl, bl, cl);
+  __syncthreads();
+  const int row = 2 * (blockIdx.x * S::TP + t / R2);
+  if (row >= nrows) return;  // no barrier below
+  const bool two = row + 1 < nrows;
+  int o0 = 0, o1 = nb;
+  if (FRESH) {
+    o0 = og * (int)blockIdx.y;
+    o1 = min(nb, o0 + og);
+    best += (size_t)blockIdx.y * nrows * n;
+    bidx += (size_t)blockIdx.y * nrows * n;
+  }
+  const int nh = n / 2 + 1;
+  float bv[2][HP];
+  int32_t bi[2][HP];
+#pragma unroll
+  for (int m = 0; m < HP; ++m) {
+    const int p = j + R2 * m;
+    const size_t i = (size_t)row * n + p;
+    const bool in = !FRESH && p < n;
+    bv[0][m] = in ? best[i] : -__builtin_inff();
+    bi[0][m] = in ? bidx[i] : 0;
+    bv[1][m] = in && two ? best[i + n] : -__builtin_inff();
+    bi[1][m] = in && two ? bidx[i + n] : 0;
+  }
+  for (int o = o0; o < o1; ++o) {
+    const float2* a = G + o * H + (long long)row * nh;
+    const float sc = scale[o];
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < HP; ++m) {
+      const int p = j + R2 * m;
+      v[m] = row_pair_bin(a, a + nh, p < n, p < n && two, p < n ? p : 0, n);
+    }
+#pragma unroll
+    for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+    for (int m = HP; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    SyncWave{}();
+#pragma unroll
+    for (int m = 0; m < HP; ++m) {
+      const float2 r = cmul(v[m], cl[j + R2 * m]);
+      const float c0 = r.x * sc, c1 = r.y * sc;
+      if (c0 > bv[0][m]) {
+        bv[0][m] = c0;
+        bi[0][m] = angle0 + o;
+      }
+      if (c1 > bv[1][m]) {
+        bv[1][m] = c1;
+        bi[1][m] = angle0 + o;
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < HP; ++m) {
+    const int p = j + R2 * m;
+    if (p >= n) continue;
+    const size_t i = (size_t)row * n + p;
+    best[i] = bv[0][m];
+    bidx[i] = bi[0][m];
+    if (two) {
+      best[i + n] = bv[1][m];
+      bidx[i + n] = bi[1][m];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Lengths above 512.
+// ---------------------------------------------------------------------------
 
 // Line l of an axis: its first point at (l / P) * S1 + (l % P) * S0, its
 // points es apart.
@@ -1233,6 +1535,14 @@ struct BlueTables {
 std::mutex g_blue_mu;
 std::map<std::pair<int, int>, BlueTables> g_blue;
 
+int blue_fused_len(int L) {
+#define GX_CASE(M) \
+  if (M >= 2 * L - 1) return M;
+  GX_FOR_BLUE(GX_CASE)
+#undef GX_CASE
+  return 0;
+}
+
 int blue_tables(int L, BlueTables* out) {
   int dev = 0;
   GX_HIP(hipGetDevice(&dev));
@@ -1245,7 +1555,12 @@ int blue_tables(int L, BlueTables* out) {
   // the shortest native length (2^a or 3 * 2^a, at least 8) that holds the linear convolution
   if (L > 2048) return fail(GTOMX_ERR_UNSUPPORTED, "lengths without a native transform must be at most 2048");
   int M = 8;
-  while (M < 2 * L - 1 || !fft_len_ok_any(M)) ++M;
+  if (L <= BLUE_FUSED_MAX) {
+    // the shortest the fused form has (384 and 768 points need three steps there)
+    M = blue_fused_len(L);
+  } else {
+    while (M < 2 * L - 1 || !fft_len_ok_any(M)) ++M;
+  }
   const long double pi = 3.141592653589793238462643383279502884L;
   std::vector<std::complex<long double>> c(L), bf(M), bi(M);
   for (int j = 0; j < L; ++j) {
@@ -1298,6 +1613,107 @@ int blue_tables(int L, BlueTables* out) {
 }
 
 unsigned blue_grid(long long n) { return (unsigned)std::max<long long>(1, std::min<long long>((n + 255) / 256, 65536)); }
+
+// f(integral_constant M) for the fused form's length M.
+template <class F> int with_blue_len(int M, F f) {
+  switch (M) {
+#define GX_CASE(N) \
+  case N:          \
+    return f(std::integral_constant<int, N>{});
+    GX_FOR_BLUE(GX_CASE)
+#undef GX_CASE
+    default: return fail(GTOMX_ERR_INTERNAL, "chirp-z length not instantiated");
+  }
+}
+
+// The fused form on a strided axis, from src into dst (which may be src).
+template <int DIR>
+int blue_cols(int L, const float2* src, float2* dst, int width, long long as, long long nplanes, long long P1,
+              long long S0, long long S1, hipStream_t s) {
+  const float2* tw = nullptr;
+  GX_TRY(twiddles(&tw));
+  BlueTables t;
+  GX_TRY(blue_tables(L, &t));
+  return with_blue_len(t.M, [&](auto MC) -> int {
+    constexpr int M = decltype(MC)::value;
+    using S = BlueShape<M>;
+    const int gx = (width + S::TX - 1) / S::TX;
+    // enough workgroups to fill the device several times over, and several planes each to share the staged tables
+    const long long gy = std::min<long long>(nplanes, std::max<long long>(1, 8192 / gx));
+    hipLaunchKernelGGL((k_blue_cols<M, DIR>), dim3(gx, (unsigned)gy), dim3(S::TX * S::R2), 0, s, src, dst, width, as,
+                       nplanes, P1, S0, S1, L, t.chirp, DIR < 0 ? t.bf : t.bi, tw);
+    GX_LAUNCHED("k_blue_cols");
+    return GTOMX_OK;
+  });
+}
+
+// The fused form on nrows contiguous rows of L reals / L/2 + 1 bins.
+int blue_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s) {
+  const float2* tw = nullptr;
+  GX_TRY(twiddles(&tw));
+  BlueTables t;
+  GX_TRY(blue_tables(L, &t));
+  return with_blue_len(t.M, [&](auto MC) -> int {
+    constexpr int M = decltype(MC)::value;
+    const long long wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
+    hipLaunchKernelGGL(k_blue_rows_r2c<M>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), 0, s, in, out,
+                       nrows, L, t.chirp, t.bf, tw);
+    GX_LAUNCHED("k_blue_rows_r2c");
+    return GTOMX_OK;
+  });
+}
+int blue_rows_c2r(int L, const float2* in, float* out, long long nrows, float scale, hipStream_t s) {
+  const float2* tw = nullptr;
+  GX_TRY(twiddles(&tw));
+  BlueTables t;
+  GX_TRY(blue_tables(L, &t));
+  return with_blue_len(t.M, [&](auto MC) -> int {
+    constexpr int M = decltype(MC)::value;
+    const long long wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
+    hipLaunchKernelGGL(k_blue_rows_c2r<M>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), 0, s, in, out,
+                       nrows, L, scale, t.chirp, t.bi, tw);
+    GX_LAUNCHED("k_blue_rows_c2r");
+    return GTOMX_OK;
+  });
+}
+
+bool rows_max_any_fused(int n) { return n <= BLUE_FUSED_MAX; }
+
+int rows_max_any_groups(int n, unsigned batch, int cus) {
+  const int M = blue_fused_len(n);
+  int wgs = 0, per_cu = 1;
+  const int st = with_blue_len(M, [&](auto MC) -> int {
+    constexpr int N = decltype(MC)::value;
+    wgs = (n * n + 2 * BlueRows<N>::TP - 1) / (2 * BlueRows<N>::TP);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_blue_rows_max<N, true>, 256, 0) != hipSuccess ||
+        per_cu < 1)
+      per_cu = 1;
+    return GTOMX_OK;
+  });
+  if (st != GTOMX_OK || wgs < 1) return 1;
+  return std::max(1, std::min((int)batch, per_cu * cus / wgs));
+}
+
+int rows_max_any(int n, const float2* G, long long H, int nb, int angle0, const float* scale, float* best,
+                 int32_t* idx, int og, hipStream_t s) {
+  const float2* tw = nullptr;
+  GX_TRY(twiddles(&tw));
+  BlueTables t;
+  GX_TRY(blue_tables(n, &t));
+  return with_blue_len(t.M, [&](auto MC) -> int {
+    constexpr int M = decltype(MC)::value;
+    const int nrows = n * n, wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
+    const int groups = og > 0 ? (nb + og - 1) / og : 1;
+    if (groups == 1)
+      hipLaunchKernelGGL((k_blue_rows_max<M, false>), dim3(wgs, 1), dim3(256), 0, s, G, H, nb, n, nrows, angle0, scale,
+                         best, idx, og, t.chirp, t.bi, tw);
+    else
+      hipLaunchKernelGGL((k_blue_rows_max<M, true>), dim3(wgs, groups), dim3(256), 0, s, G, H, nb, n, nrows, angle0,
+                         scale, best, idx, og, t.chirp, t.bi, tw);
+    GX_LAUNCHED("k_blue_rows_max");
+    return GTOMX_OK;
+  });
+}
 
 // One axis of nlines lines of length L by the chirp-z form: IN / OUT are the
 // load and store modes above, src / dst laid out by as / ad (they may be the
@@ -1362,6 +1778,8 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
     constexpr int D = decltype(DIRC)::value;
     if (fft_len_ok_any(d.y))
       return cols_axis<D>(d.y, data, data, scr.p, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, tw, s);
+    if (d.y <= BLUE_FUSED_MAX)
+      return blue_cols<D>(d.y, data, data, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, s);
     const AxisLines a{nh, 1, nh * d.y, nh};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.z * batch, d.y, 0, 1.f, s);
   };
@@ -1370,6 +1788,8 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
     if (fft_len_ok_any(d.z))
       return cols_axis<D>(d.z, data, data, scr.p, (int)nh, nh * d.y, (long long)d.y * batch, d.y, nh, nh * d.y * d.z, tw,
                           s);
+    if (d.z <= BLUE_FUSED_MAX && nh * d.y < (1LL << 30))  // the columns of a volume are one contiguous row
+      return blue_cols<D>(d.z, data, data, (int)(nh * d.y), nh * d.y, batch, 1LL << 62, nh * d.y * d.z, 0, s);
     const AxisLines a{nh * d.y, 1, nh * d.y * d.z, nh * d.y};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.y * batch, d.z, 0, 1.f, s);
   };
@@ -1399,6 +1819,8 @@ int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipS
       GX_TRY(launch_rows_long<true>(d.x, in, out, rows, 1.f, tw, s));
     else
       GX_TRY(launch_rows_r2c(d.x, in, out, rows, tw, s));
+  } else if (d.x <= BLUE_FUSED_MAX) {
+    GX_TRY(blue_rows_r2c(d.x, in, out, rows, s));
   } else {
     GX_TRY((blue_axis<1, 1, -1>(in, AxisLines{1LL << 62, d.x, 0, 1}, out, AxisLines{1LL << 62, nh, 0, 1}, rows, d.x,
                                 (int)nh, 1.f, s)));
@@ -1416,6 +1838,7 @@ int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float sc
     if (d.x > 256) return launch_rows_long<false>(d.x, work, out, rows, scale, tw, s);
     return launch_rows_c2r(d.x, work, out, rows, scale, tw, s);
   }
+  if (d.x <= BLUE_FUSED_MAX) return blue_rows_c2r(d.x, work, out, rows, scale, s);
   return blue_axis<2, 2, 1>(work, AxisLines{1LL << 62, nh, 0, 1}, out, AxisLines{1LL << 62, d.x, 0, 1}, rows, d.x,
                             (int)nh, scale, s);
 }

@@ -207,6 +207,14 @@ int yz_axes_any(float2* data, gtomx_int3 dims, unsigned batch, int dir, hipStrea
 // spectrum o fills the first n^3 floats of its slot (every row is read before
 // the rows it overwrites are written). n at most 2048.
 int rows_c2r_any_inplace(float2* G, int n, int nb, long long H, hipStream_t s);
+// The generic search's row pass on sides up to 512 (rows_max_any_fused): the C2R
+// of the n * n rows of nb half spectra H apart in G, times scale[o], folded into
+// best / idx in orientation order from angle0 (strict >). og > 0 and below nb:
+// group g of og orientations starts afresh and writes at g * n^3 of best / idx.
+bool rows_max_any_fused(int n);
+int rows_max_any_groups(int n, unsigned batch, int cus);  // groups of a batch that fill the device
+int rows_max_any(int n, const float2* G, long long H, int nb, int angle0, const float* scale, float* best,
+                 int32_t* idx, int og, hipStream_t s);
 
 // Fourier-space resizing (resize.hip): op is one of the GTOMX_FFT_* values.
 constexpr int FFT_CROP = GTOMX_FFT_CROP, FFT_PAD = GTOMX_FFT_PAD, FFT_FULL_CROP = GTOMX_FFT_FULL_CROP,

@@ -105,3 +105,21 @@ def test_local_std_any_extent_matches_oracle(gx, orc, cuda, shape, r):
     print(f"local std {shape}: {err:.2e}")
     assert err < 1e-5
     assert rel_linf(to_np(mean).reshape(rmean.shape), rmean) < 1e-5
+
+
+# Lengths at the edges of the fused form's convolution lengths (16, 24, 32, 48, ... 512, 1024: the longest
+# line of each and the shortest of the next), odd row counts (the last row of a pair alone), and 513, the
+# first above it. As above, single-precision transforms: 4e-6 normwise.
+EDGES = [5, 7, 9, 11, 13, 15, 17, 23, 25, 31, 33, 47, 49, 63, 65, 95, 97, 127, 129, 191, 193, 255, 257, 511, 513]
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_fft_any_edges_of_the_fused_lengths(gx, cuda, n):
+    import torch
+    rng = np.random.default_rng(n)
+    for shape in ((3, 5, n), (3, n, 6), (n, 3, 10)):  # the length along x, y and z
+        x = rng.standard_normal(shape).astype(np.float32)
+        X = gx.d_FFTR2C(torch.from_numpy(x[None]).to(cuda))
+        assert rel_linf(to_np(X)[0], np.fft.rfftn(x.astype(np.float64))) < TOL, shape
+        back = gx.d_IFFTC2R(X, shape[2])
+        assert rel_linf(to_np(back)[0], x) < TOL, shape
