@@ -118,7 +118,7 @@ int slot_loop(SizeSlot& sl, unsigned nangles, hipStream_t s) {
   const size_t V = (size_t)sl.n * sl.n;
   GX_TRY(fill_f32(sl.best, V, -1e30f, s));  // d_ValueFill (SubTomograms.cu:41-42)
   GX_TRY(fill_i32(sl.idx, V, 0, s));
-  return launch_update_batches(sl.plan, sl.P, sl.centred ? &sl.C : nullptr, sl.plan->mats, nangles, sl.E, sl.ctf,
+  return launch_update_batches(sl.plan, sl.P, sl.centred ? &sl.C : nullptr, sl.plan->mats, nangles, 1, sl.E, sl.ctf, 0,
                                sl.best, sl.idx, 0, s);
 }
 
@@ -297,7 +297,7 @@ int gtomx_mpick_tune(int p, int n, const gtomx_complex* d_projectorft, const uns
     int st = upload_matrices(plan, h_angles, nangles, oversample, s);
     const bool centred = st == GTOMX_OK && setup_projector(plan, d_projectorft, oversample, s, &P, &C, &st);
     auto loop = [&]() {
-      return launch_update_batches(plan, P, centred ? &C : nullptr, plan->mats, nangles, E.as<float2>(), nullptr,
+      return launch_update_batches(plan, P, centred ? &C : nullptr, plan->mats, nangles, 1, E.as<float2>(), nullptr, 0,
                                    best.as<float>(), idx.as<int32_t>(), 0, s);
     };
     if (st == GTOMX_OK) st = loop();  // warm-up

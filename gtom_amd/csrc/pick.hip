@@ -8,9 +8,8 @@
 //     Q = E_v * conj(R) with DC = 0            (src/Correlation/SubTomograms.cu:127-136)
 //     and the partial sums of |R|^2; inverse DFT along z, written to the
 //     batch buffer G[o].
-//  k_pick_herm_norm: the correction of those sums on the x = 0 plane (the
-//     x = n/2 plane meets the sphere only at its centre bin), so that together
-//     they are sum |R'|^2 for R' = Herm(R) with DC
+//  k_pick_herm_norm: the correction of those sums on the x = 0 plane and the
+//     one bin of the x = n/2 plane inside the sphere, so that together they are sum |R'|^2 for R' = Herm(R) with DC
 //     zeroed: the Fourier form of C2R -> mean0/std1 -> R2C -> /RMS
 //     (src/Correlation/SubTomograms.cu:66-70, src/ImageManipulation/Norm.cu:242-284, 476-509).
 //  pass 2 (k_pick_y): inverse DFT along y in place; one workgroup per
@@ -19,6 +18,7 @@
 //     inverse), times the scale, then the running max/argmax with strict '>'
 //     in increasing orientation index (src/Correlation/SubTomograms.cu:138-158)
 //     for all B orientations, best/argmax held in registers.
+// Sides up to 128 run passes 2 and 3 as one kernel per z plane (k_pick_plane_max).
 // After the last orientation, pick_finish divides by the local standard
 // deviation of C2R(E_v) (src/Correlation/SubTomograms.cu:103-118).
 #include <algorithm>
@@ -35,54 +35,45 @@
 namespace gx {
 
 // Layout of the batch buffer G (one block of STRIDE complex values per
-// orientation). When n/2 is a multiple of the column-tile width TX ("split"),
-// the x < n/2 columns form rows of exactly PITCH = n/2 values, so every tile
-// row is a whole number of 128-byte lines, and the x = n/2 (Nyquist) column is
-// stored after them as a compact [z][y] array. Otherwise rows hold all n/2+1
-// columns padded to whole tiles (PITCH), and the padding is never read.
+// orientation): rows (z, y) of the columns x < n/2, padded to whole column
+// tiles (PITCH; no padding where n/2 is a multiple of the tile width, so that
+// every tile row is a whole number of 128-byte lines); the padding is never
+// read. The column x = n/2 is not stored: the sphere |k| <= n/2 meets it only at
+// (n/2, 0, 0), so its z and y transforms are that bin's value at every row, of
+// which the C2R takes the real part. The kernels that hold the row transform
+// get it as one float per orientation (sn[o].y, beside the scale), and no pass carries the column
+// (1/129 of the traffic at n = 256, and of a 2D image's pass 1 one tile in nine
+// that held 16 of its 4,096 bins).
 template <int N> struct GLayout {
   static constexpr int TX = ColShape<N>::TX;
-  static constexpr bool SPLIT = (N / 2) % TX == 0;
-  static constexpr int PITCH = SPLIT ? N / 2 : (N / 2 + 1 + TX - 1) / TX * TX;
-  static constexpr size_t MAIN = (size_t)PITCH * N * N;
-  static constexpr size_t STRIDE = MAIN + (SPLIT ? (size_t)N * N : 0);
+  static constexpr int FT = (N / 2 + TX - 1) / TX;  // column tiles of a row
+  static constexpr int PITCH = FT * TX;
+  // the spectra of a batch start 8,448 bytes past a power of two apart: at 256^3 pass 2 takes 2.91 ms
+  // per 128 orientations with the padding and 3.03 without
+  static constexpr size_t STRIDE = (size_t)PITCH * N * N + 1056;
   static constexpr int ROWS = N * N;  // rows (z, y) of the x transform
 };
 
-// The 2D branch (n x n images): per orientation, n rows (y) of all n/2+1
-// columns, padded to whole column tiles.
+// The 2D branch (n x n images): per orientation, n rows (y).
 template <int N> struct GLayout2 {
   static constexpr int TX = ColShape<N>::TX;
-  static constexpr bool SPLIT = false;
-  static constexpr int FT = (N / 2 + 1 + TX - 1) / TX;  // column tiles
+  static constexpr int FT = (N / 2 + TX - 1) / TX;
   static constexpr int PITCH = FT * TX;
-  static constexpr size_t MAIN = (size_t)PITCH * N;
-  static constexpr size_t STRIDE = MAIN;
+  static constexpr size_t STRIDE = (size_t)PITCH * N;
   static constexpr int ROWS = N;
 };
 
-// Workgroup layout of the column passes (1 and 2). In the split layout the
-// first NQ workgroups take the Nyquist column of TX rows at once, one row per
-// lane (their strided accesses are slower, so they start first), and the
-// remaining FT*N workgroups take TX full columns of one row each. Otherwise
-// every row has FT tiles and lanes past x = n/2 idle.
+// Workgroups of the column passes (1 and 2): w takes TX columns of one row; row
+// is y in pass 1 and z in pass 2. Lanes past x = n/2 - 1 idle.
 template <int N, int TXW = ColShape<N>::TX> struct ColMap {
   static constexpr int TX = TXW;
-  static_assert(TXW == ColShape<N>::TX || (GLayout<N>::SPLIT && (N / 2) % TXW == 0),
-                "a tile width other than the layout's needs the split layout");
-  static constexpr bool SPLIT = GLayout<N>::SPLIT;
-  static constexpr int FT = SPLIT ? (N / 2) / TX : (N / 2 + TX) / TX;
-  static constexpr int NQ = SPLIT ? N / TX : 0;
-  static constexpr int NWG = FT * N + NQ;
-  // (workgroup w, lane column c) -> (x, row); row is y in pass 1 and z in pass 2.
+  static_assert(GLayout<N>::PITCH % TXW == 0, "tiles are whole within the layout's rows");
+  static constexpr int FT = GLayout<N>::PITCH / TX;
+  static constexpr int NWG = FT * N;
+  // (workgroup w, lane column c) -> (x, row)
   __device__ static void map(int w, int c, int& x, int& row) {
-    if (w < NQ) {
-      x = N / 2;
-      row = w * TX + c;
-    } else {
-      x = ((w - NQ) % FT) * TX + c;
-      row = (w - NQ) / FT;
-    }
+    x = (w % FT) * TX + c;
+    row = w / FT;
   }
 };
 
@@ -201,9 +192,8 @@ k_pick_project_z(
     const int w = tiles[ti];
     int ix, iy;
     ColMap<N>::map(w, c, ix, iy);
-    const bool nyq_wg = w < ColMap<N>::NQ;
     const int y = signed_freq(iy, N);
-    const bool valid = ix < NH && column_in_disc<N>(ix, y);
+    const bool valid = ix < HALF && column_in_disc<N>(ix, y);
 
     // E_v and the CTF at this thread's bins of the tile (element (x, y, z) at
     // (z*N + y)*NH + x; the z part is the constant m*R2*N*NH).
@@ -220,9 +210,8 @@ k_pick_project_z(
     // Output of this thread's first bin (z = j*(R1/R2)) and the step between its outputs.
     const int zrow0 = j * (R1 / R2);
     // Lanes of columns outside the disc store nothing (out-of-range offset).
-    const int gbase8 = !valid ? OUT_OF_RANGE
-                              : (nyq_wg ? (int)L::MAIN + zrow0 * N + iy : (zrow0 * N + iy) * L::PITCH + ix) * 8;
-    const int gstep = nyq_wg ? N : N * L::PITCH;  // per unit of output z
+    const int gbase8 = !valid ? OUT_OF_RANGE : ((zrow0 * N + iy) * L::PITCH + ix) * 8;
+    constexpr int gstep = N * L::PITCH;  // per unit of output z
 
     for (int o = o0; o < o1; ++o) {
       float M[9];
@@ -289,47 +278,35 @@ template <int N> std::vector<int> disc_tiles() {
   using CM = ColMap<N>;
   std::vector<int> out;
   for (int w = 0; w < CM::NWG; ++w) {
-    bool in;
-    if (w < CM::NQ) {
-      in = w == 0;  // the Nyquist column (n/2, y) meets the disc only at y = 0
-    } else {
-      const int x0 = ((w - CM::NQ) % CM::FT) * CM::TX, row = (w - CM::NQ) / CM::FT;
-      const int y = row <= N / 2 ? row : row - N;
-      in = x0 * x0 + y * y <= (N / 2) * (N / 2);
-    }
-    if (in) out.push_back(w);
+    const int x0 = (w % CM::FT) * CM::TX, row = w / CM::FT;
+    const int y = row <= N / 2 ? row : row - N;
+    if (x0 < N / 2 && x0 * x0 + y * y <= (N / 2) * (N / 2)) out.push_back(w);
   }
   return out;
 }
 
 // ---------------------------------------------------------------------------
-// Unit-RMS correction on the x = 0 and x = n/2 planes: for every bin k of the
-// two planes, |Herm R(k)|^2 - |R(k)|^2 with Herm R(k) = (R(k) + conj R(-k))/2
-// (R(-k) sampled at the mirrored stored bin) and Herm R(0) = 0. Added to the
-// pass-1 sums it gives sum |R'|^2 for R' = Herm(R) with DC zeroed, the
-// spectrum that C2R -> mean0/std1 -> R2C produces in the reference.
+// Unit-RMS correction: |Herm R(k)|^2 - |R(k)|^2 over the bins of the x = 0 plane,
+// with Herm R(k) = (R(k) + conj R(-k))/2 (R(-k) sampled at the mirrored stored
+// bin) and Herm R(0) = 0, and over the x = n/2 plane, which the sphere meets only
+// at its own mirror (n/2, 0, 0). Added to the pass-1 sums it gives sum |R'|^2 for
+// R' = Herm(R) with DC zeroed, the spectrum that C2R -> mean0/std1 -> R2C produces
+// in the reference. |Herm R| is the same at k and -k, so each pair is taken once.
 // ---------------------------------------------------------------------------
 constexpr int HERM_BLOCKS = 32;
 
-// NT = 0: the side is the run-time n.
-template <int NT>
-__global__ __launch_bounds__(256) void k_pick_herm_norm(Projector P, const float* __restrict__ mats,
-                                                        const float* __restrict__ ctf, float* __restrict__ corr,
-                                                        int n) {
-  const int N = NT ? NT : n;
-  const int NH = N / 2 + 1, HALF = N / 2, RMAX2 = HALF * HALF;
-  __shared__ float red[4];
-  const int o = blockIdx.y;
-  float M[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
-  const __amdgpu_buffer_rsrc_t rs = projector_rsrc(P);
+// The sum over the pairs of the x = 0 plane that thread `first` of `step` takes:
+// rows iz = 0 .. n/2 of the disc, of the rows that are their own mirrors (0, and
+// n/2 where n is even) half.
+__device__ __forceinline__ float herm_plane_sum(const Projector& P, __amdgpu_buffer_rsrc_t rs, const float* M,
+                                                const float* __restrict__ ctf, int N, int first, int step) {
+  const int NH = N / 2 + 1, RMAX2 = (N / 2) * (N / 2);
   float acc = 0.f;
-  // the x = 0 plane: bins of the disc y^2 + z^2 <= (n/2)^2 (R is 0 elsewhere), paired with -k
-  for (int b = blockIdx.x * 256 + threadIdx.x; b < N * N; b += gridDim.x * 256) {
+  for (int b = first; b < (N / 2 + 1) * N; b += step) {
     const int iy = b % N, iz = b / N;
-    const int y = signed_freq(iy, N), z = signed_freq(iz, N);
-    if (y * y + z * z > RMAX2) continue;
+    const int y = signed_freq(iy, N), z = iz;
+    const bool own_row = iz == 0 || 2 * iz == N;
+    if (y * y + z * z > RMAX2 || (own_row && 2 * iy > N)) continue;
     const int iyp = (N - iy) % N, izp = (N - iz) % N;
     const int yp = signed_freq(iyp, N), zp = signed_freq(izp, N);
     const float c = ctf ? ctf[((size_t)iz * N + iy) * NH] : 1.f;
@@ -340,17 +317,77 @@ __global__ __launch_bounds__(256) void k_pick_herm_norm(Projector P, const float
         project_at(rs, P.p, P.ph, M[1] * yp + M[2] * zp, M[4] * yp + M[5] * zp, M[7] * yp + M[8] * zp), cp);
     float2 h = make_float2(0.5f * (R.x + Rp.x), 0.5f * (R.y - Rp.y));
     if (b == 0) h = make_float2(0.f, 0.f);  // DC
-    acc += (h.x * h.x + h.y * h.y) - (R.x * R.x + R.y * R.y);
+    const float hh = h.x * h.x + h.y * h.y, rr = R.x * R.x + R.y * R.y;
+    acc += own_row && iyp == iy ? hh - rr : 2.f * hh - rr - (Rp.x * Rp.x + Rp.y * Rp.y);
   }
-  // the x = n/2 plane meets the sphere only at (n/2, 0, 0), its own mirror: Herm R = Re R (odd n have
-  // no such plane)
+  return acc;
+}
+
+// CTF times the sample at (n/2, 0, 0).
+__device__ __forceinline__ float2 nyquist_sample(const Projector& P, __amdgpu_buffer_rsrc_t rs, const float* M,
+                                                 const float* __restrict__ ctf, int N) {
+  const int HALF = N / 2;
+  return cscale(project_at(rs, P.p, P.ph, M[0] * HALF, M[3] * HALF, M[6] * HALF), ctf ? ctf[HALF] : 1.f);
+}
+
+// NT = 0: the side is the run-time n. With sn (the fused passes, whose pass 1
+// leaves the x = n/2 plane out) the bin's whole |Herm R|^2 = (Re R)^2 enters, and
+// sn[o].y receives Re(E conj(CTF R)) there.
+template <int NT>
+__global__ __launch_bounds__(256) void k_pick_herm_norm(Projector P, const float* __restrict__ mats,
+                                                        const float* __restrict__ ctf, float* __restrict__ corr,
+                                                        int n, const float2* __restrict__ E = nullptr,
+                                                        float2* __restrict__ sn = nullptr) {
+  const int N = NT ? NT : n;
+  __shared__ float red[4];
+  const int o = blockIdx.y;
+  float M[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
+  const __amdgpu_buffer_rsrc_t rs = projector_rsrc(P);
+  float acc = herm_plane_sum(P, rs, M, ctf, N, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256);
+  // (odd n have no x = n/2 plane)
   if ((N & 1) == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
-    const float c = ctf ? ctf[HALF] : 1.f;
-    const float2 R = cscale(project_at(rs, P.p, P.ph, M[0] * HALF, M[3] * HALF, M[6] * HALF), c);
-    acc -= R.y * R.y;
+    const float2 R = nyquist_sample(P, rs, M, ctf, N);
+    acc += sn ? R.x * R.x : -R.y * R.y;
+    if (sn) sn[o].y = cmulc(E[N / 2], R).x;
   }
   const float tot = block_sum(acc, red);
   if (threadIdx.x == 0) corr[(size_t)o * gridDim.x + blockIdx.x] = tot;
+}
+
+// The correction, the reduction of the pass-1 sums and the scale in one launch of
+// a workgroup per orientation, for the sides of k_pick_plane_max: their planes
+// are at most 128 x 65 pairs, and one launch less per batch counts (64^3, 196
+// orientations: 27 us for the 32-workgroup form above).
+template <int N>
+__global__ __launch_bounds__(512) void k_pick_norm(Projector P, const float* __restrict__ mats,
+                                                   const float2* __restrict__ E, const float* __restrict__ ctf,
+                                                   const float* __restrict__ partial, int nparts,
+                                                   float2* __restrict__ sn) {
+  __shared__ double red[8];
+  const int o = blockIdx.x, t = threadIdx.x;
+  float M[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
+  const __amdgpu_buffer_rsrc_t rs = projector_rsrc(P);
+  double sum = (double)herm_plane_sum(P, rs, M, ctf, N, t, 512);
+  if (t == 0) {
+    const float2 R = nyquist_sample(P, rs, M, ctf, N);
+    sum += (double)(R.x * R.x);
+    sn[o].y = cmulc(E[N / 2], R).x;
+  }
+  for (int i = t; i < nparts; i += 512) sum += (double)partial[(size_t)o * nparts + i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((t & 63) == 0) red[t >> 6] = sum;
+  __syncthreads();
+  if (t == 0) {
+    double s = 0;
+    for (int w = 0; w < 8; ++w) s += red[w];
+    constexpr double H = (double)(N / 2 + 1) * N * N;
+    sn[o].x = (float)(1.0 / fmax(sqrt(s / H), 1e-20));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -360,13 +397,13 @@ __global__ __launch_bounds__(256) void k_pick_herm_norm(Projector P, const float
 // layout): 32 columns (256-byte row segments) where the split layout allows,
 // which streams measurably better than 16.
 template <int N> struct Pass2Tile {
-  static constexpr int TX = (GLayout<N>::SPLIT && (N / 2) % 32 == 0) ? 32 : ColShape<N>::TX;
+  static constexpr int TX = GLayout<N>::PITCH % 32 == 0 && ColShape<N>::TX < 32 ? 32 : ColShape<N>::TX;
 };
 
 template <int N>
 __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
     float2* __restrict__ G, const float* __restrict__ partial, int ntiles, const float* __restrict__ corr,
-    float* __restrict__ scale, const float2* __restrict__ tw, const uint8_t* __restrict__ tmask) {
+    float2* __restrict__ sn, const float2* __restrict__ tw, const uint8_t* __restrict__ tmask) {
   using L = GLayout<N>;
   constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = Pass2Tile<N>::TX;
   using CM = ColMap<N, TX>;
@@ -382,14 +419,11 @@ __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
   int ix, z;
   CM::map(blockIdx.x, c, ix, z);
   const int o = blockIdx.y;
-  const bool nyq_wg = (int)blockIdx.x < CM::NQ;
-  // Column (x, z) along y: main rows (stride PITCH) or the compact Nyquist column (stride 1).
-  const int base = nyq_wg ? (int)L::MAIN + z * N : z * N * L::PITCH + ix;
-  const int ystep = nyq_wg ? 1 : L::PITCH;
+  const int base = z * N * L::PITCH + ix;  // column (x, z) along y
+  constexpr int ystep = L::PITCH;
   const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + (size_t)o * L::STRIDE, (unsigned)(L::STRIDE * 8));
-  // a whole workgroup's plane is skipped when its tile layer is empty (the Nyquist
-  // workgroups hold several planes and always run)
-  const bool skip = tmask && !nyq_wg && !layer_any<N>(tmask, z);
+  // a whole workgroup's plane is skipped when its tile layer is empty
+  const bool skip = tmask && !layer_any<N>(tmask, z);
   if (!skip) {
   float2 v[R1];
 #pragma unroll
@@ -411,7 +445,7 @@ __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
   for (int s = 0; s < R1; ++s) {
     const int u = s / R2, k2 = s % R2;  // output y = j*(R1/R2) + u + R1*k2
     const int y = j * (R1 / R2) + u + R1 * k2;
-    if (tmask && !nyq_wg && tmask[(z / 32) * (N / 32) + y / 32] == 0) continue;
+    if (tmask && tmask[(z / 32) * (N / 32) + y / 32] == 0) continue;
     const u32x2 vs = __builtin_bit_cast(u32x2, v[s]);
     __builtin_amdgcn_raw_buffer_store_b64(vs, rG, obase * 8, (u + R1 * k2) * ystep * 8, CPOL_NT);
   }
@@ -431,7 +465,7 @@ __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
     }
     if (t == 0) {
       double rms = sqrt(dred[0] / (double)H);
-      scale[o] = (float)(1.0 / fmax(rms, 1e-20));
+      sn[o].x = (float)(1.0 / fmax(rms, 1e-20));
     }
   }
 }
@@ -440,13 +474,14 @@ __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
 // pass 3
 // ---------------------------------------------------------------------------
 // L is the batch buffer's layout (GLayout for volumes, GLayout2 for images).
-// With FRESH the running maximum starts at -1e30 / 0 instead of the values in
+// With FRESH the running maximum starts at -infinity / 0 instead of the values in
 // best/bidx: orientation group blockIdx.y (og orientations from og*blockIdx.y)
-// then writes its own maximum to best/bidx + blockIdx.y * ROWS * N, and
-// k_pick_merge combines the groups in order.
+// of image blockIdx.z (whose nb spectra follow those of the images before it)
+// then writes its own maximum to best/bidx + (image * groups + group) * ROWS * N,
+// and k_pick_merge combines the groups in order.
 template <int N, class L = GLayout<N>, bool FRESH = false>
 __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G, int nb, int angle0,
-                                                    const float* __restrict__ scale, float* __restrict__ best,
+                                                    const float2* __restrict__ sn, float* __restrict__ best,
                                                     int32_t* __restrict__ bidx, const float2* __restrict__ tw,
                                                     int og = 0, const uint8_t* __restrict__ tmask = nullptr) {
   constexpr int NC = N / 2;
@@ -465,13 +500,13 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
   }
   const bool valid = row < L::ROWS && xbits != 0;
   if (FRESH) {
-    const int o0 = og * (int)blockIdx.y;
-    G += (size_t)o0 * L::STRIDE;
-    scale += o0;
+    const int o0 = og * (int)blockIdx.y, slot = nb * (int)blockIdx.z + o0;
+    G += (size_t)slot * L::STRIDE;
+    sn += slot;
     angle0 += o0;
     nb = min(og, nb - o0);
-    best += (size_t)blockIdx.y * L::ROWS * N;
-    bidx += (size_t)blockIdx.y * L::ROWS * N;
+    best += ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * L::ROWS * N;
+    bidx += ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * L::ROWS * N;
   }
 
   float bv[2 * R1];
@@ -481,15 +516,13 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
 #pragma unroll
   for (int s = 0; s < R1; ++s) {
     const int m = out_index<R1, R2>(j, s);
-    float2 b = valid && !FRESH ? bp[m] : make_float2(-1e30f, -1e30f);
+    float2 b = valid && !FRESH ? bp[m] : make_float2(-__builtin_inff(), -__builtin_inff());
     int2 a = valid && !FRESH ? ip[m] : make_int2(0, 0);
     bv[2 * s] = b.x;
     bv[2 * s + 1] = b.y;
     bi[2 * s] = a.x;
     bi[2 * s + 1] = a.y;
   }
-  // Row bins X[0..n/2-1] in the main rows, X[n/2] in the Nyquist column
-  // (split layout) or at the end of the row.
   // This thread's twiddles, the same for every orientation, held in
   // registers: exp(2 pi i k/N) for its pre-processing bins k = j + R2*m and
   // the stage twiddles of the half-length transform.
@@ -498,21 +531,22 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
   for (int m = 0; m < R1; ++m) twp[m] = twiddle<1, N>(tw, j + R2 * m);
   load_two_step_twiddles<NC, R1, 1>(twh, j, tw);
   const int xrow = valid ? row * L::PITCH : (int)L::STRIDE;  // invalid rows read nothing (0)
-  const int xnyq = valid ? (L::SPLIT ? (int)L::MAIN + row : row * L::PITCH + NC) : (int)L::STRIDE;
 
   for (int o = 0; o < nb; ++o) {
-    const float sc = scale[o];
+    const float sc = sn[o].x, xn = sn[o].y;
     const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + (size_t)o * L::STRIDE, (unsigned)(L::STRIDE * 8));
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1; ++m) {
       const int k = j + R2 * m;
-      // a = X[k]; b = X[n/2 - k], which is X[n/2] for k = 0
+      // a = X[k]; b = X[n/2 - k], for k = 0 X[n/2]: that lane loads nothing (0) and adds the value, which
+      // keeps the loads together (a select between a load and xn becomes a branch with a wait of its own:
+      // 2.35 against 2.05 ms per 128 orientations at 256^3)
       const float2 a = buf_load2(rG, (xrow + j) * 8, R2 * m * 8);
-      const float2 b = buf_load2(rG, (m == 0 && j == 0 ? xnyq : xrow + NC - k) * 8, 0);
+      const float2 b = buf_load2(rG, m == 0 && j == 0 ? OUT_OF_RANGE : (xrow + NC - k) * 8, 0);
       // the imaginary parts of X[0] and X[n/2] do not enter the real inverse
       const float2 a0 = k == 0 ? make_float2(a.x, 0.f) : a;
-      const float2 bc = k == 0 ? make_float2(b.x, 0.f) : cconj(b);
+      const float2 bc = make_float2(m == 0 ? b.x + (j == 0 ? xn : 0.f) : b.x, -b.y);
       v[m] = cadd(cadd(a0, bc), mul_pj<1>(cmul(twp[m], csub(a0, bc))));
     }
     __syncthreads();
@@ -544,6 +578,141 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
 }
 
 // ---------------------------------------------------------------------------
+// passes 2 and 3 in one, for sides whose z plane fits LDS beside others (16 to
+// 128): a workgroup takes PL planes z and a group of orientations, and for each
+// orientation reads the plane's columns once, runs the y inverse, turns the
+// plane to rows in LDS, runs the row C2R and folds the plane into a running
+// maximum in registers. Orientation group blockIdx.y writes its own maximum and
+// k_pick_merge combines the groups in order; one group updates best directly.
+//
+// Two passes moved the batch through memory three times (read, write, read) and
+// pass 3 had one workgroup per 256 / R2 rows, each with a serial chain of loads
+// over the whole batch: at 64^3 64 workgroups on 256 CUs, 5 us per orientation.
+// Here the spectra are read once, and the groups give the grid the workgroups
+// that the planes do not.
+// ---------------------------------------------------------------------------
+template <int N> struct PlaneShape {
+  static constexpr int NC = N / 2;
+  // y transform: R1 x R2 with R2 threads per column; row transform of NC points:
+  // R1 x (R2 / 2), so that both use the same NC * R2 = N * (R2 / 2) threads
+  static constexpr int R2 = N <= 24 ? 2 : (N == 64 || N == 128 ? 8 : 4);
+  static constexpr int R1 = N / R2, XR2 = R2 / 2;
+  static constexpr int T = NC * R2;
+  static constexpr int PL = T <= 32 ? 256 / 32 : (T <= 128 ? 256 / T : 1);  // planes per workgroup
+  // LDS row pitch: XR2 extra values put the 16 lanes that an 8-byte access
+  // serves at once on different banks, in the row reads (rows NCP apart, XR2
+  // lanes each) and in the row transform's exchange (XR2 slots of R1 + 1)
+  static constexpr int NCP = NC + XR2;
+  static_assert(N % PL == 0 && 64 % XR2 == 0, "whole planes, rows within a wave");
+};
+
+// MASKED (tile masks): planes of layers without a searched tile run no
+// orientation, and only voxels of searched tiles are updated.
+template <int N, bool FRESH, bool MASKED = false>
+__global__ __launch_bounds__(PlaneShape<N>::T * PlaneShape<N>::PL) void k_pick_plane_max(
+    const float2* __restrict__ G, int nb, int angle0, const float2* __restrict__ sn, float* __restrict__ best,
+    int32_t* __restrict__ bidx, const float2* __restrict__ tw, int og, const uint8_t* __restrict__ tmask = nullptr) {
+  using L = GLayout<N>;
+  using S = PlaneShape<N>;
+  constexpr int NC = S::NC, R1 = S::R1, R2 = S::R2, XR2 = S::XR2, T = S::T, NCP = S::NCP, NT = T * S::PL;
+  __shared__ float2 area[S::PL * N * NCP];
+  __shared__ float2 twl[N];
+  const int t = threadIdx.x;
+  for (int i = t; i < N; i += NT) twl[i] = twiddle<-1, N>(tw, i);
+  const int pl = t / T, tp = t % T;
+  float2* xch = area + pl * N * NCP;
+  const int z = blockIdx.x * S::PL + pl;
+  const int c = tp % NC, j = tp / NC;    // column c, thread j of its y transform
+  const int r = tp / XR2, jx = tp % XR2; // row r, thread jx of its row transform
+  int o0 = 0, o1 = nb;
+  size_t out0 = 0;
+  if (FRESH) {
+    o0 = og * (int)blockIdx.y;
+    o1 = min(nb, o0 + og);
+    out0 = (size_t)blockIdx.y * L::ROWS * N;
+  }
+  unsigned xbits = 0;  // tile bits of this row: bit k covers x in [32k, 32k + 32)
+  if constexpr (MASKED) {
+    static_assert(N % 32 == 0 && 32 % S::PL == 0, "a workgroup's planes lie in one tile layer");
+    xbits = tmask[(z / 32) * (N / 32) + r / 32];
+    if (!layer_any<N>(tmask, z)) o1 = o0;
+  }
+  float bv[2 * R1];
+  int32_t bi[2 * R1];
+  float2* bp = reinterpret_cast<float2*>(best + out0 + (size_t)(z * N + r) * N);
+  int2* ip = reinterpret_cast<int2*>(bidx + out0 + (size_t)(z * N + r) * N);
+#pragma unroll
+  for (int s = 0; s < R1; ++s) {
+    const int m = out_index<R1, XR2>(jx, s);
+    const float2 b = FRESH ? make_float2(-__builtin_inff(), -__builtin_inff()) : bp[m];
+    const int2 a = FRESH ? make_int2(0, 0) : ip[m];
+    bv[2 * s] = b.x;
+    bv[2 * s + 1] = b.y;
+    bi[2 * s] = a.x;
+    bi[2 * s + 1] = a.y;
+  }
+  const int gbase = ((z * N + j) * L::PITCH + c) * 8;
+  for (int o = o0; o < o1; ++o) {
+    const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + (size_t)o * L::STRIDE, (unsigned)(L::STRIDE * 8));
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1; ++m) {
+      // bins of columns outside the disc were not written by pass 1 and are zero
+      const int voff = column_in_disc<N>(c, signed_freq(j + R2 * m, N)) ? gbase : OUT_OF_RANGE;
+      v[m] = buf_load2(rG, voff, m * R2 * L::PITCH * 8);
+    }
+    const float sc = sn[o].x, xn = sn[o].y;
+    __syncthreads();  // the last orientation's rows are done (and, the first time, the twiddles staged)
+    fft_two_step<N, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * NC + c]; },
+                               TwiddleLDS{});
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < R1; ++s) xch[out_index<R1, R2>(j, s) * NCP + c] = v[s];
+    __syncthreads();
+    // row C2R as in k_pick_x_max; from here on a row belongs to XR2 lanes of one wave
+#pragma unroll
+    for (int m = 0; m < R1; ++m) {
+      const int k = jx + XR2 * m;
+      const float2 a = xch[r * NCP + k];
+      float2 b = xch[r * NCP + (m == 0 && jx == 0 ? 0 : NC - k)];
+      if (m == 0) {  // X[n/2] for k = 0, without a branch around the load
+        b.x = __builtin_unpredictable(jx == 0) ? xn : b.x;
+        b.y = __builtin_unpredictable(jx == 0) ? 0.f : b.y;
+      }
+      const float2 a0 = k == 0 ? make_float2(a.x, 0.f) : a;
+      const float2 bc = cconj(b);
+      v[m] = cadd(cadd(a0, bc), mul_pj<1>(cmul(cconj(twl[k]), csub(a0, bc))));
+    }
+    SyncWave{}();
+    fft_two_step<NC, R1, XR2, 1>(v, jx, twl, [&](int k1, int jj) { return &xch[r * NCP + jj * (R1 + 1) + k1]; },
+                                 TwiddleLDSHalf{}, SyncWave{});
+    const int32_t oi = angle0 + o;
+#pragma unroll
+    for (int s = 0; s < R1; ++s) {
+      const float c0 = v[s].x * sc, c1 = v[s].y * sc;
+      if (MASKED && !((xbits >> (out_index<R1, XR2>(jx, s) >> 4)) & 1u)) continue;  // x = 2m, 2m + 1
+      if (c0 > bv[2 * s]) {
+        bv[2 * s] = c0;
+        bi[2 * s] = oi;
+      }
+      if (c1 > bv[2 * s + 1]) {
+        bv[2 * s + 1] = c1;
+        bi[2 * s + 1] = oi;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < R1; ++s) {
+    const int m = out_index<R1, XR2>(jx, s);
+    bp[m] = make_float2(bv[2 * s], bv[2 * s + 1]);
+    ip[m] = make_int2(bi[2 * s], bi[2 * s + 1]);
+  }
+}
+
+// Sides that k_pick_plane_max takes (a 192 plane fills a CU's LDS, 256 does not fit).
+constexpr bool plane_side(int n) { return n >= 16 && n <= 128; }
+
+// ---------------------------------------------------------------------------
 // The centred projector layout (CentredProjector): element (cx, cy, cz) of a
 // PX x PY x PY array, PX = p/2 + 2, PY = p + 3, is the reference's projector
 // at linear index (iz*p + iy)*(p/2+1) + cx with iy = (cy - OFF) mod p,
@@ -564,82 +733,135 @@ __global__ __launch_bounds__(256) void k_centre_projector(const float2* __restri
 
 inline int centred_bytes(int p) { return (p / 2 + 2) * (p + 3) * (p + 3) * 8; }
 
-// Combines the per-group maxima of the 2D pass 3 in increasing group order with
-// strict '>', so the first maximum over all orientations wins.
+// Combines the per-group maxima in increasing group order with strict '>', so
+// that the first maximum over all orientations wins. A workgroup takes 64 voxels
+// of volume or image blockIdx.y; each of its 4 waves folds a quarter of the
+// groups, in order.
 __global__ __launch_bounds__(256) void k_pick_merge(const float* __restrict__ gbest, const int32_t* __restrict__ gidx,
                                                    int groups, size_t v, float* __restrict__ best,
                                                    int32_t* __restrict__ bidx) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < v; i += (size_t)gridDim.x * 256) {
-    float b = best[i];
-    int32_t k = bidx[i];
-    for (int g = 0; g < groups; ++g) {
-      const float c = gbest[(size_t)g * v + i];
+  __shared__ float sb[256];
+  __shared__ int32_t sk[256];
+  const int t = threadIdx.x, q = t >> 6;
+  const size_t i = (size_t)blockIdx.x * 64 + (t & 63);
+  const int g0 = groups * q / 4, g1 = groups * (q + 1) / 4;
+  gbest += (size_t)blockIdx.y * groups * v;
+  gidx += (size_t)blockIdx.y * groups * v;
+  best += (size_t)blockIdx.y * v;
+  bidx += (size_t)blockIdx.y * v;
+  float b = -__builtin_inff();
+  int g = -1;
+  if (i < v)
+    for (int k = g0; k < g1; ++k) {
+      const float c = gbest[(size_t)k * v + i];
       if (c > b) {
         b = c;
-        k = gidx[(size_t)g * v + i];
+        g = k;
       }
     }
-    best[i] = b;
-    bidx[i] = k;
+  sb[t] = b;
+  sk[t] = g;
+  __syncthreads();
+  if (t >= 64 || i >= v) return;
+  float top = best[i];
+  g = -1;
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+    if (sb[64 * w + t] > top) {
+      top = sb[64 * w + t];
+      g = sk[64 * w + t];
+    }
+  if (g >= 0) {
+    best[i] = top;
+    bidx[i] = gidx[(size_t)g * v + i];
   }
 }
 
 // ---------------------------------------------------------------------------
 // The 2D branch, pass 1: one workgroup per (column tile, orientation) projects
 // the central section M (x, y, 0) (Project3DArraytoNDKernel<2>) at its TX
-// columns and all y, applies the CTF, forms E * conj(R) with the DC zeroed and
-// inverse-transforms along y; per-workgroup sums of |R|^2 go to partial.
+// columns and all y once, and for each of vb images applies the image's CTF,
+// forms E * conj(R) with the DC zeroed and inverse-transforms along y into slot
+// v * nb + o; per-workgroup sums of |R|^2 go to partial. The samples do not
+// depend on the image, and they are most of the instructions: 16 images of
+// 256^2 x 1,000 orientations spent 4.7 of 11.4 ms sampling every image anew.
+// E and the CTFs of the images stay in L2 (264 KB a spectrum at 256^2).
 // ---------------------------------------------------------------------------
 template <int N, class PJ>
 __global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_pick2d_project_y(
-    PJ P, const float* __restrict__ mats, const float2* __restrict__ E, const float* __restrict__ ctf,
-    float2* __restrict__ G, float* __restrict__ partial, const float2* __restrict__ tw) {
+    PJ P, const float* __restrict__ mats, int vb, const float2* __restrict__ E, const float* __restrict__ ctf,
+    size_t ctf_stride, float2* __restrict__ G, float* __restrict__ partial, const float2* __restrict__ tw) {
   using L = GLayout2<N>;
   constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = ColShape<N>::TX;
   constexpr int NH = N / 2 + 1, HALF = N / 2, RMAX2 = HALF * HALF;
+  constexpr size_t H = (size_t)NH * N;
   constexpr int NT = TX * R2;
   __shared__ float2 xch[R2 > 1 ? TX * N : 1];
   __shared__ float red[(NT + 63) / 64];
   __shared__ float2 twl[N];
   const int t = threadIdx.x, c = t % TX, j = t / TX;
   for (int i = t; i < N; i += NT) twl[i] = twiddle<-1, N>(tw, i);
-  const int tile = blockIdx.x, o = blockIdx.y;
+  const int tile = blockIdx.x, o = blockIdx.y, nb = gridDim.y;
   const int ix = tile * TX + c;
-  const bool valid = ix < NH;
+  const bool valid = ix < HALF;
   float M[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
   const __amdgpu_buffer_rsrc_t rs = sampler_rsrc(P);
-  float acc = 0.f;
-  float2 v[R1];
+  float2 r[R1];
 #pragma unroll
   for (int m = 0; m < R1; ++m) {
-    const int iy = j + R2 * m, y = signed_freq(iy, N);
+    const int y = signed_freq(j + R2 * m, N);
     const bool ins = valid && ix * ix + y * y <= RMAX2;
-    const float2 e = valid ? E[iy * NH + ix] : make_float2(0.f, 0.f);
-    const float cf = valid ? (ctf ? ctf[iy * NH + ix] : 1.f) : 0.f;
-    const float2 r = cscale(sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins),
-                            cf);
-    acc += r.x * r.x + r.y * r.y;
-    v[m] = cmulc(e, r);
+    r[m] = sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins);
   }
-  if (ix == 0 && j == 0) v[0] = make_float2(0.f, 0.f);  // DC
-  __syncthreads();
-  fft_two_step<N, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; },
-                             TwiddleLDS{});
-  float2* g = G + (size_t)o * L::STRIDE;
+  const size_t bin = valid ? (size_t)j * NH + ix : 0;
+  for (int w = 0; w < vb; ++w) {
+    const float2* Ew = E + w * H + bin;
+    const float* cw = ctf ? ctf + w * ctf_stride + bin : nullptr;
+    float acc = 0.f;
+    float2 v[R1];
 #pragma unroll
-  for (int s = 0; s < R1; ++s) g[(size_t)out_index<R1, R2>(j, s) * L::PITCH + ix] = v[s];
-  const float tot = block_sum(acc, red);
-  if (t == 0) partial[(size_t)o * L::FT + tile] = tot;
+    for (int m = 0; m < R1; ++m) {
+      const float2 e = valid ? Ew[m * R2 * NH] : make_float2(0.f, 0.f);
+      const float cf = valid ? (cw ? cw[m * R2 * NH] : 1.f) : 0.f;
+      const float2 rc = cscale(r[m], cf);
+      acc += rc.x * rc.x + rc.y * rc.y;
+      v[m] = cmulc(e, rc);
+    }
+    if (ix == 0 && j == 0) v[0] = make_float2(0.f, 0.f);  // DC
+    __syncthreads();
+    fft_two_step<N, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; },
+                               TwiddleLDS{});
+    float2* g = G + (size_t)(w * nb + o) * L::STRIDE;
+#pragma unroll
+    for (int s = 0; s < R1; ++s) g[(size_t)out_index<R1, R2>(j, s) * L::PITCH + ix] = v[s];
+    const float tot = block_sum(acc, red);
+    if (t == 0) partial[(size_t)(w * nb + o) * L::FT + tile] = tot;
+  }
+}
+
+// |Herm R|^2 - |R|^2 at (0, y) of the section, iy = b.
+template <int N>
+__device__ __forceinline__ float herm_line_term(const Projector& P, __amdgpu_buffer_rsrc_t rs, const float* M,
+                                                const float* __restrict__ ctf, int b) {
+  constexpr int NH = N / 2 + 1;
+  const int iyp = (N - b) % N;
+  const int y = signed_freq(b, N), yp = signed_freq(iyp, N);
+  const float c = ctf ? ctf[b * NH] : 1.f;
+  const float cp = ctf ? ctf[iyp * NH] : 1.f;
+  const float2 R = cscale(project_at(rs, P.p, P.ph, M[1] * y, M[4] * y, M[7] * y), c);
+  const float2 Rp = cscale(project_at(rs, P.p, P.ph, M[1] * yp, M[4] * yp, M[7] * yp), cp);
+  float2 h = make_float2(0.5f * (R.x + Rp.x), 0.5f * (R.y - Rp.y));
+  if (b == 0) h = make_float2(0.f, 0.f);  // DC
+  return (h.x * h.x + h.y * h.y) - (R.x * R.x + R.y * R.y);
 }
 
 // The 2D unit-RMS correction: |Herm R|^2 - |R|^2 on the lines x = 0 and
-// x = n/2, Herm R(0, y) = (R(0, y) + conj R(0, -y))/2, DC removed.
+// x = n/2, Herm R(0, y) = (R(0, y) + conj R(0, -y))/2, DC removed (images above 256).
 template <int N>
 __global__ __launch_bounds__(256) void k_pick2d_herm_norm(Projector P, const float* __restrict__ mats,
                                                           const float* __restrict__ ctf, float* __restrict__ corr) {
-  constexpr int NH = N / 2 + 1, HALF = N / 2, RMAX2 = HALF * HALF;
   __shared__ float red[4];
   const int o = blockIdx.x;
   float M[9];
@@ -647,23 +869,48 @@ __global__ __launch_bounds__(256) void k_pick2d_herm_norm(Projector P, const flo
   for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
   const __amdgpu_buffer_rsrc_t rs = projector_rsrc(P);
   float acc = 0.f;
-  for (int b = threadIdx.x; b < 2 * N; b += 256) {
-    const int ix = b < N ? 0 : HALF;
-    const int iy = b % N, iyp = (N - iy) % N;
-    const int y = signed_freq(iy, N), yp = signed_freq(iyp, N);
-    const bool in = ix * ix + y * y <= RMAX2;
-    const float c = ctf ? ctf[iy * NH + ix] : 1.f;
-    const float cp = ctf ? ctf[iyp * NH + ix] : 1.f;
-    const float2 R = cscale(project_at(rs, P.p, P.ph, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y,
-                                       M[6] * ix + M[7] * y, in), c);
-    const float2 Rp = cscale(project_at(rs, P.p, P.ph, M[0] * ix + M[1] * yp, M[3] * ix + M[4] * yp,
-                                        M[6] * ix + M[7] * yp, in), cp);
-    float2 h = make_float2(0.5f * (R.x + Rp.x), 0.5f * (R.y - Rp.y));
-    if (b == 0) h = make_float2(0.f, 0.f);
-    acc += (h.x * h.x + h.y * h.y) - (R.x * R.x + R.y * R.y);
+  for (int b = threadIdx.x; b < N; b += 256) acc += herm_line_term<N>(P, rs, M, ctf, b);
+  if (threadIdx.x == 0) {  // the x = n/2 line meets the disc only at (n/2, 0), its own mirror
+    const float2 R = nyquist_sample(P, rs, M, ctf, N);
+    acc -= R.y * R.y;
   }
   const float tot = block_sum(acc, red);
   if (threadIdx.x == 0) corr[o] = tot;
+}
+
+// The same correction, the sum of the pass-1 sums and the scale of orientation
+// blockIdx.x on image blockIdx.y in one launch (the fused passes, whose pass 1
+// leaves the x = n/2 line out: its one bin in the disc enters as (Re R)^2, and
+// sn[].y receives Re(E conj(CTF R))).
+template <int N>
+__global__ __launch_bounds__(256) void k_pick2d_norm(Projector P, const float* __restrict__ mats,
+                                                     const float2* __restrict__ E, const float* __restrict__ ctf,
+                                                     size_t ctf_stride, const float* __restrict__ partial,
+                                                     float2* __restrict__ sn) {
+  constexpr int FT = GLayout2<N>::FT;
+  constexpr size_t H = (size_t)(N / 2 + 1) * N;
+  __shared__ double red[4];
+  const int o = blockIdx.x, w = blockIdx.y, t = threadIdx.x;
+  const size_t slot = (size_t)w * gridDim.x + o;
+  const float* cw = ctf ? ctf + w * ctf_stride : nullptr;
+  float M[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
+  const __amdgpu_buffer_rsrc_t rs = projector_rsrc(P);
+  float acc = 0.f;
+  for (int b = t; b < N; b += 256) acc += herm_line_term<N>(P, rs, M, cw, b);
+  double sum = (double)acc;
+  if (t == 0) {
+    const float2 R = nyquist_sample(P, rs, M, cw, N);
+    sum += (double)(R.x * R.x);
+    sn[slot].y = cmulc(E[w * H + N / 2], R).x;
+  }
+  for (int i = t; i < FT; i += 256) sum += (double)partial[slot * FT + i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((t & 63) == 0) red[t >> 6] = sum;
+  __syncthreads();
+  if (t == 0) sn[slot].x = (float)(1.0 / fmax(sqrt((red[0] + red[1] + red[2] + red[3]) / (double)H), 1e-20));
 }
 
 // scale[o] = 1/max(sqrt((sum of partial sums + corrections)/H), 1e-20) in double
@@ -818,6 +1065,10 @@ __global__ __launch_bounds__(256) void k_pick3d_project_any(PJ P, const float* _
 namespace gx {
 namespace {
 
+// Images of one launch of the fused 2D passes: with 4 the samples cost a quarter,
+// and the plan's 240 spectra still give 60 orientations to fill the device.
+constexpr int MAX_IMAGES2 = 4;
+
 void plan_release(gtomx_pick_plan* pl) {
   if (!pl) return;
   pl->fence.release();
@@ -826,6 +1077,7 @@ void plan_release(gtomx_pick_plan* pl) {
   dev_free(pl->tiles);
   dev_free(pl->corr);
   dev_free(pl->scale);
+  dev_free(pl->sn);
   dev_free(pl->mats);
   dev_free(pl->ls_mem);
   dev_free(pl->ebuf);
@@ -934,12 +1186,45 @@ template <class F> int timed(gtomx_pick_plan* pl, int stage, hipStream_t s, F la
   return GTOMX_OK;
 }
 
+// Workgroups of k_pick_plane_max that are resident at once on the whole device.
+template <int N> int resident_planes(int cus) {
+  int per_cu = 0;
+  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_plane_max<N, true>,
+                                                              PlaneShape<N>::T * PlaneShape<N>::PL, 0);
+  if (e != hipSuccess || per_cu < 1) per_cu = 1;
+  return per_cu * cus;
+}
+
+// Orientation groups of k_pick_plane_max for a full batch: as many as fill the
+// device once, none smaller than one orientation.
+template <int N> int plane_groups(unsigned batch, int cus) {
+  if constexpr (plane_side(N))
+    return std::max(1, std::min((int)batch, resident_planes<N>(cus) / (N / PlaneShape<N>::PL)));
+  return 0;
+}
+int plane_groups_for(int n, unsigned batch, int cus) {
+  switch (n) {
+#define GX_CASE(N) \
+  case N:          \
+    return plane_groups<N>(batch, cus);
+    GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+  }
+  return 0;
+}
+
+int merge_groups(gtomx_pick_plan* pl, int groups, float* best, int32_t* idx, hipStream_t s, unsigned items = 1) {
+  hipLaunchKernelGGL(k_pick_merge, dim3((unsigned)((pl->V + 63) / 64), items), dim3(256), 0, s, pl->gbest, pl->gidx, groups,
+                     pl->V, best, idx);
+  GX_LAUNCHED("k_pick_merge");
+  return GTOMX_OK;
+}
+
 template <int N, class PJ>
 int run_batch(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, const float2* E,
               const float* ctf, float* best, int32_t* idx, int angle0, const float2* tw, hipStream_t s,
               const uint8_t* tmask) {
   constexpr int TX = ColShape<N>::TX, R2 = ColShape<N>::R2;
-  constexpr int RW = 256 / RowShape<N / 2>::R2;
   GX_TRY(timed(pl, 0, s, [&]() -> int {
     const int g = pl->grid1[std::is_same<PJ, CentredProjector>::value ? 1 : 0];
     if (tmask)
@@ -951,22 +1236,49 @@ int run_batch(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float
     GX_LAUNCHED("k_pick_project_z");
     return GTOMX_OK;
   }));
-  // stage 1 of the timings: the plane correction and pass 2
-  GX_TRY(timed(pl, 1, s, [&]() -> int {
-    hipLaunchKernelGGL(k_pick_herm_norm<N>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, pl->corr, N);
-    GX_LAUNCHED("k_pick_herm_norm");
-    hipLaunchKernelGGL(k_pick_y<N>, dim3(ColMap<N, Pass2Tile<N>::TX>::NWG, nb), dim3(Pass2Tile<N>::TX * R2), 0, s,
-                       pl->G, pl->partial, pl->ntiles, pl->corr, pl->scale, tw, tmask);
-    GX_LAUNCHED("k_pick_y");
-    return GTOMX_OK;
-  }));
-  GX_TRY(timed(pl, 2, s, [&]() -> int {
-    hipLaunchKernelGGL(k_pick_x_max<N>, dim3((N * N + RW - 1) / RW), dim3(256), 0, s, pl->G, nb, angle0, pl->scale,
-                       best, idx, tw, 0, tmask);
-    GX_LAUNCHED("k_pick_x_max");
-    return GTOMX_OK;
-  }));
-  return GTOMX_OK;
+  if constexpr (plane_side(N)) {
+    using S = PlaneShape<N>;
+    GX_TRY(timed(pl, 1, s, [&]() -> int {
+      hipLaunchKernelGGL(k_pick_norm<N>, dim3(nb), dim3(512), 0, s, P, mats, E, ctf, pl->partial,
+                         pl->ntiles * pass1_waves<N>(), pl->sn);
+      GX_LAUNCHED("k_pick_norm");
+      return GTOMX_OK;
+    }));
+    return timed(pl, 2, s, [&]() -> int {
+      const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
+      const bool fresh = groups > 1;
+      auto go = [&](auto kernel) -> int {
+        hipLaunchKernelGGL(kernel, dim3(N / S::PL, groups), dim3(S::T * S::PL), 0, s, pl->G, nb, angle0, pl->sn,
+                           fresh ? pl->gbest : best, fresh ? pl->gidx : idx, tw, og, tmask);
+        GX_LAUNCHED("k_pick_plane_max");
+        return GTOMX_OK;
+      };
+      if constexpr (N % 32 == 0) {
+        if (tmask)
+          GX_TRY(fresh ? go(k_pick_plane_max<N, true, true>) : go(k_pick_plane_max<N, false, true>));
+      }
+      if (!tmask) GX_TRY(fresh ? go(k_pick_plane_max<N, true>) : go(k_pick_plane_max<N, false>));
+      return fresh ? merge_groups(pl, groups, best, idx, s) : GTOMX_OK;
+    });
+  } else {
+    // stage 1 of the timings: the plane correction and pass 2
+    GX_TRY(timed(pl, 1, s, [&]() -> int {
+      hipLaunchKernelGGL(k_pick_herm_norm<N>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, pl->corr, N, E,
+                         pl->sn);
+      GX_LAUNCHED("k_pick_herm_norm");
+      hipLaunchKernelGGL(k_pick_y<N>, dim3(ColMap<N, Pass2Tile<N>::TX>::NWG, nb), dim3(Pass2Tile<N>::TX * R2), 0, s,
+                         pl->G, pl->partial, pl->ntiles, pl->corr, pl->sn, tw, tmask);
+      GX_LAUNCHED("k_pick_y");
+      return GTOMX_OK;
+    }));
+    return timed(pl, 2, s, [&]() -> int {
+      constexpr int RW = 256 / RowShape<N / 2>::R2;
+      hipLaunchKernelGGL(k_pick_x_max<N>, dim3((N * N + RW - 1) / RW), dim3(256), 0, s, pl->G, nb, angle0, pl->sn, best,
+                         idx, tw, 0, tmask);
+      GX_LAUNCHED("k_pick_x_max");
+      return GTOMX_OK;
+    });
+  }
 }
 
 // Volumes above 256: pass 1 over the whole half spectrum, the plane correction
@@ -977,13 +1289,15 @@ int herm_norm3_any(int n, const Projector& P, const float* mats, const float* ct
   switch (n) {
 #define GX_CASE(N)                                                                                    \
   case N:                                                                                             \
-    hipLaunchKernelGGL(k_pick_herm_norm<N>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, corr, N); \
+    hipLaunchKernelGGL(k_pick_herm_norm<N>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, corr, N, \
+                       nullptr, nullptr);                                                             \
     GX_LAUNCHED("k_pick_herm_norm");                                                                  \
     return GTOMX_OK;
     GX_CASE(512) GX_CASE(768) GX_CASE(1024)
 #undef GX_CASE
   }
-  hipLaunchKernelGGL(k_pick_herm_norm<0>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, corr, n);
+  hipLaunchKernelGGL(k_pick_herm_norm<0>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, corr, n,
+                     nullptr, nullptr);
   GX_LAUNCHED("k_pick_herm_norm");
   return GTOMX_OK;
 }
@@ -1029,6 +1343,12 @@ int run_batch3d_any(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const
     return fft_c2r_cols_inplace(pl->G, gtomx_int3{n, n, n}, (unsigned)nb, s);
   }));
   return timed(pl, 2, s, [&]() -> int {
+    if (pl->gen3d && rows_max_any_fused(n)) {
+      const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
+      if (groups == 1) return rows_max_any(n, pl->G, H, nb, angle0, pl->scale, best, idx, nb, s);
+      GX_TRY(rows_max_any(n, pl->G, H, nb, angle0, pl->scale, pl->gbest, pl->gidx, og, s));
+      return merge_groups(pl, groups, best, idx, s);
+    }
     if (pl->gen3d) {
       // the rows' C2R into the first n^3 floats of each spectrum's slot, then the in-order update
       GX_TRY(rows_c2r_any_inplace(pl->G, n, nb, H, s));
@@ -1064,39 +1384,61 @@ int run_batch_n(gtomx_pick_plan* pl, const CentredProjector* C, const Projector&
   return fail(GTOMX_ERR_UNSUPPORTED, "volume side not supported");
 }
 
-// The 2D branch: pass 1 (projection + y transform), the line correction and
-// the scale, then pass 3 per orientation group and the in-order merge.
+// Workgroups of the 2D row pass that are resident at once on the whole device,
+// and its workgroups per image and group.
+template <int N> int resident_rows2(int cus) {
+  int per_cu = 0;
+  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_x_max<N, GLayout2<N>, true>, 256, 0);
+  if (e != hipSuccess || per_cu < 1) per_cu = 1;
+  return per_cu * cus;
+}
+template <int N> constexpr int row_blocks2() {
+  constexpr int RW = 256 / RowShape<N / 2>::R2;
+  return (N + RW - 1) / RW;
+}
+
+// Most (image, group) pairs of a launch: enough to fill the device once with the
+// row pass, at least one per image.
+int pairs2_for(int n, unsigned batch, int cus) {
+  switch (n) {
+#define GX_CASE(N) \
+  case N:          \
+    return std::max(MAX_IMAGES2, std::min((int)batch, resident_rows2<N>(cus) / row_blocks2<N>()));
+    GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+  }
+  return 0;
+}
+
+// The 2D branch on vb images (vb * nb at most the plan's batch): pass 1
+// (projection + y transform), the line correction and the scale, then pass 3 per
+// orientation group and the in-order merge.
 template <int N, class PJ>
-int run_batch2d(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, const float2* E,
-                const float* ctf, float* best, int32_t* idx, int angle0, const float2* tw, hipStream_t s) {
+int run_batch2d(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, unsigned vb,
+                const float2* E, const float* ctf, size_t ctf_stride, float* best, int32_t* idx, int angle0,
+                const float2* tw, hipStream_t s) {
   using L = GLayout2<N>;
   constexpr int TX = ColShape<N>::TX, R2 = ColShape<N>::R2;
-  constexpr int RW = 256 / RowShape<N / 2>::R2;
   GX_TRY(timed(pl, 0, s, [&]() -> int {
-    hipLaunchKernelGGL((k_pick2d_project_y<N, PJ>), dim3(L::FT, nb), dim3(TX * R2), 0, s, PS, mats, E, ctf, pl->G,
-                       pl->partial, tw);
+    hipLaunchKernelGGL((k_pick2d_project_y<N, PJ>), dim3(L::FT, nb), dim3(TX * R2), 0, s, PS, mats, (int)vb, E, ctf,
+                       ctf_stride, pl->G, pl->partial, tw);
     GX_LAUNCHED("k_pick2d_project_y");
     return GTOMX_OK;
   }));
-  hipLaunchKernelGGL(k_pick2d_herm_norm<N>, dim3(nb), dim3(256), 0, s, P, mats, ctf, pl->corr);
-  GX_LAUNCHED("k_pick2d_herm_norm");
   GX_TRY(timed(pl, 1, s, [&]() -> int {
-    hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, L::FT, pl->corr, 1, (double)pl->H,
-                       pl->scale);
-    GX_LAUNCHED("k_pick_scale");
+    hipLaunchKernelGGL(k_pick2d_norm<N>, dim3(nb, vb), dim3(256), 0, s, P, mats, E, ctf, ctf_stride, pl->partial,
+                       pl->sn);
+    GX_LAUNCHED("k_pick2d_norm");
     return GTOMX_OK;
   }));
-  const int groups = (nb + pl->og - 1) / pl->og;
-  GX_TRY(timed(pl, 2, s, [&]() -> int {
-    hipLaunchKernelGGL((k_pick_x_max<N, L, true>), dim3((N + RW - 1) / RW, groups), dim3(256), 0, s, pl->G, nb,
-                       angle0, pl->scale, pl->gbest, pl->gidx, tw, pl->og);
+  const int most = std::max(1, pl->pairs2 / (int)vb);
+  const int og = (nb + most - 1) / most, groups = (nb + og - 1) / og;
+  return timed(pl, 2, s, [&]() -> int {
+    hipLaunchKernelGGL((k_pick_x_max<N, L, true>), dim3(row_blocks2<N>(), groups, vb), dim3(256), 0, s, pl->G, nb,
+                       angle0, pl->sn, pl->gbest, pl->gidx, tw, og);
     GX_LAUNCHED("k_pick_x_max");
-    const unsigned grid = (unsigned)std::min<size_t>((pl->V + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_pick_merge, dim3(grid), dim3(256), 0, s, pl->gbest, pl->gidx, groups, pl->V, best, idx);
-    GX_LAUNCHED("k_pick_merge");
-    return GTOMX_OK;
-  }));
-  return GTOMX_OK;
+    return merge_groups(pl, groups, best, idx, s, vb);
+  });
 }
 
 // The 2D branch above 256: pass 1 fused with the first half of the y
@@ -1153,16 +1495,16 @@ int run_batch2d_any(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const
 }
 
 int run_batch2d_n(gtomx_pick_plan* pl, const CentredProjector* C, const Projector& P, const float* mats, int nb,
-                  const float2* E, const float* ctf, float* best, int32_t* idx, int angle0, const float2* tw,
-                  hipStream_t s) {
+                  unsigned vb, const float2* E, const float* ctf, size_t ctf_stride, float* best, int32_t* idx,
+                  int angle0, const float2* tw, hipStream_t s) {
   if (pl->n > 256)
     return C ? run_batch2d_any(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, tw, s)
              : run_batch2d_any(pl, P, P, mats, nb, E, ctf, best, idx, angle0, tw, s);
   switch (pl->n) {
-#define GX_CASE(N)                                                                         \
-  case N:                                                                                  \
-    return C ? run_batch2d<N>(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, tw, s)       \
-             : run_batch2d<N>(pl, P, P, mats, nb, E, ctf, best, idx, angle0, tw, s);
+#define GX_CASE(N)                                                                                       \
+  case N:                                                                                                \
+    return C ? run_batch2d<N>(pl, *C, P, mats, nb, vb, E, ctf, ctf_stride, best, idx, angle0, tw, s)     \
+             : run_batch2d<N>(pl, P, P, mats, nb, vb, E, ctf, ctf_stride, best, idx, angle0, tw, s);
     GX_FOR_SIZES(GX_CASE)
 #undef GX_CASE
   }
@@ -1278,17 +1620,37 @@ int check_update_args(const gtomx_pick_plan* plan, const gtomx_complex* d_projec
   return GTOMX_OK;
 }
 
+// Items per pass for `count` of them, at most `most`: as few passes as that
+// allows, of equal size (a short last pass leaves the device half idle: 588
+// orientations of 64^3 as 256 + 256 + 76 or 3 x 196). Results do not depend on it.
+unsigned even_batch(unsigned most, unsigned count) {
+  const unsigned passes = (count + most - 1) / most;
+  return (count + passes - 1) / passes;
+}
+
 int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const CentredProjector* C, const float* mats,
-                          unsigned nangles, const float2* E, const float* ctf, float* best, int32_t* idx,
-                          int angle0, hipStream_t s) {
+                          unsigned nangles, unsigned nvol, const float2* E, const float* ctf, size_t ctf_stride,
+                          float* best, int32_t* idx, int angle0, hipStream_t s) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
-  for (unsigned b0 = 0; b0 < nangles; b0 += pl->B) {
-    const int nb = (int)std::min<unsigned>(pl->B, nangles - b0);
-    if (pl->nz == 1)
-      GX_TRY(run_batch2d_n(pl, C, P, mats + 9 * (size_t)b0, nb, E, ctf, best, idx, angle0 + (int)b0, tw, s));
-    else
-      GX_TRY(run_batch_n(pl, C, P, mats + 9 * (size_t)b0, nb, E, ctf, best, idx, angle0 + (int)b0, tw, s));
+  if (nangles == 0) return GTOMX_OK;
+  // images of the fused 2D passes share the samples of an orientation
+  const unsigned images = pl->nz == 1 && pl->n <= 256 ? std::min({nvol, (unsigned)MAX_IMAGES2, pl->B}) : 1u;
+  for (unsigned v = 0; v < nvol; v += images) {
+    const unsigned vb = std::min(images, nvol - v);
+    const unsigned B = even_batch(pl->B / vb, nangles);
+    const float2* Ev = E + (size_t)v * pl->H;
+    const float* cv = ctf ? ctf + (size_t)v * ctf_stride : nullptr;
+    float* bv = best + (size_t)v * pl->V;
+    int32_t* iv = idx + (size_t)v * pl->V;
+    for (unsigned b0 = 0; b0 < nangles; b0 += B) {
+      const int nb = (int)std::min<unsigned>(B, nangles - b0);
+      const float* mb = mats + 9 * (size_t)b0;
+      if (pl->nz == 1)
+        GX_TRY(run_batch2d_n(pl, C, P, mb, nb, vb, Ev, cv, ctf_stride, bv, iv, angle0 + (int)b0, tw, s));
+      else
+        GX_TRY(run_batch_n(pl, C, P, mb, nb, Ev, cv, bv, iv, angle0 + (int)b0, tw, s));
+    }
   }
   return GTOMX_OK;
 }
@@ -1416,7 +1778,6 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   // orientations of 64^3 at 256 against 2.68 ms at 16)
   pl->B = batch ? batch : (is2d ? (big2d ? big_b : 240u) : (any3d ? big3_b : (dv.x >= 128 ? 128u : 256u)));
   pl->gen3d = gen3d;
-  pl->og = dv.x >= 128 ? 2 : 1;
   int L1 = 0, L2 = 0;
   if (big2d && fft_len_split(dv.x, &L1, &L2) != GTOMX_OK) {
     delete pl;
@@ -1432,15 +1793,26 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
     plan_release(pl);
     return hip_fail(he, "hipGetDevice");
   }
+  int cus = 0;
+  he = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device);
+  if (he != hipSuccess) {
+    plan_release(pl);
+    return hip_fail(he, "hipDeviceGetAttribute");
+  }
+  if (is2d && !big2d) pl->pairs2 = pairs2_for(pl->n, pl->B, cus);
+  if (!is2d && !any3d) pl->groups3 = plane_groups_for(pl->n, pl->B, cus);
+  if (gen3d && rows_max_any_fused(pl->n)) pl->groups3 = rows_max_any_groups(pl->n, pl->B, cus);
   void* d = nullptr;
   auto alloc = [&](void** dst, size_t bytes) {
     if (s != GTOMX_OK) return;
     s = dev_alloc(dst, bytes);
     if (s == GTOMX_OK) pl->device_bytes += bytes;
   };
-  // The batch buffer also serves as the C2R workspace in pick_finish (H elements).
-  const size_t gstride = (big2d || any3d) ? pl->H : (is2d ? g2_stride_for(pl->n) : g_stride_for(pl->n));
-  alloc(&d, std::max((size_t)pl->B * gstride, pl->H) * sizeof(float2));
+  // The batch buffer also serves as the C2R workspace in pick_finish (H elements)
+  // and holds whole half spectra in the split-precision search.
+  const size_t gstride =
+      std::max(pl->H, (big2d || any3d) ? pl->H : (is2d ? g2_stride_for(pl->n) : g_stride_for(pl->n)));
+  alloc(&d, (size_t)pl->B * gstride * sizeof(float2));
   pl->G = static_cast<float2*>(d);
   d = nullptr;
   // up to 4 pass-1 waves per tile; above 256, one sum per pass-1 workgroup
@@ -1456,6 +1828,9 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   alloc(&d, (size_t)pl->B * sizeof(float));
   pl->scale = static_cast<float*>(d);
   d = nullptr;
+  alloc(&d, (size_t)pl->B * sizeof(float2));
+  pl->sn = static_cast<float2*>(d);
+  d = nullptr;
   alloc(&pl->ls_mem, local_std_scratch_bytes(dv));
   alloc(&d, pl->V * sizeof(float));
   pl->ebuf = static_cast<float*>(d);
@@ -1466,8 +1841,8 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
     d = nullptr;
     alloc(&d, (size_t)pl->B * pl->H * sizeof(float2));
     pl->scr = static_cast<float2*>(d);
-  } else if (is2d) {
-    const size_t groups = (pl->B + pl->og - 1) / pl->og;
+  } else if (is2d || pl->groups3 > 1) {
+    const size_t groups = is2d ? (size_t)pl->pairs2 : (size_t)pl->groups3;
     d = nullptr;
     alloc(&d, groups * pl->V * sizeof(float));
     pl->gbest = static_cast<float*>(d);
@@ -1483,8 +1858,6 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   pl->ls = local_std_carve(pl->ls_mem, dv);
   he = hipMemcpy(pl->tiles, tiles.data(), std::min(tiles.size(), (size_t)pl->ntiles) * sizeof(int),
                  hipMemcpyHostToDevice);
-  int cus = 0;
-  if (he == hipSuccess) he = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device);
   if (he != hipSuccess) {
     plan_release(pl);
     return hip_fail(he, "plan set-up");
@@ -1589,8 +1962,6 @@ int gtomx_pick_update(gtomx_pick_plan* plan, const gtomx_complex* d_projectorft,
   if (!(oversample > 0.f) || !std::isfinite(oversample))
     return fail(GTOMX_ERR_INVALID_ARGUMENT, "projectoroversample must be positive");
   hipStream_t s = as_stream(stream);
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
   GX_TRY(plan->fence.enter(s));
   GX_TRY(upload_matrices(plan, h_angles, nangles, oversample, s));
   Projector P;
@@ -1598,21 +1969,9 @@ int gtomx_pick_update(gtomx_pick_plan* plan, const gtomx_complex* d_projectorft,
   int st = GTOMX_OK;
   const bool centred = setup_projector(plan, d_projectorft, oversample, s, &P, &C, &st);
   GX_TRY(st);
-  for (unsigned v = 0; v < nvolumes; ++v) {
-    const float2* Ev = reinterpret_cast<const float2*>(d_expft) + (size_t)v * plan->H;
-    const float* cv = d_ctf ? d_ctf + (size_t)v * ctf_volume_stride : nullptr;
-    float* bv = d_best + (size_t)v * plan->V;
-    int32_t* iv = d_idx + (size_t)v * plan->V;
-    for (unsigned b0 = 0; b0 < nangles; b0 += plan->B) {
-      int nb = (int)std::min<unsigned>(plan->B, nangles - b0);
-      if (plan->nz == 1)
-        GX_TRY(run_batch2d_n(plan, centred ? &C : nullptr, P, plan->mats + 9 * (size_t)b0, nb, Ev, cv, bv, iv,
-                             (int)(angle_offset + b0), tw, s));
-      else
-        GX_TRY(run_batch_n(plan, centred ? &C : nullptr, P, plan->mats + 9 * (size_t)b0, nb, Ev, cv, bv, iv,
-                           (int)(angle_offset + b0), tw, s));
-    }
-  }
+  GX_TRY(launch_update_batches(plan, P, centred ? &C : nullptr, plan->mats, nangles, nvolumes,
+                               reinterpret_cast<const float2*>(d_expft), d_ctf, ctf_volume_stride, d_best, d_idx,
+                               (int)angle_offset, s));
   return plan->fence.leave(s);
 }
 

@@ -25,6 +25,7 @@ struct gtomx_pick_plan {
   float* partial = nullptr;
   float* corr = nullptr;  // B x HERM_BLOCKS plane corrections of the unit-RMS sums
   float* scale = nullptr;
+  float2* sn = nullptr;   // B: (scale, the x = n/2 bin of the rows) of each orientation (fused passes)
   float* mats = nullptr;
   size_t mats_cap = 0;   // orientations
   float* h_mats = nullptr;  // pinned staging
@@ -35,9 +36,10 @@ struct gtomx_pick_plan {
   gx::LocalStdScratch ls{};
   float* ebuf = nullptr;
   float2* cproj = nullptr;  // centred projector layout
-  float* gbest = nullptr;   // 2D: per-orientation-group maxima (groups x V)
+  float* gbest = nullptr;   // per-orientation-group maxima (groups x V)
   int32_t* gidx = nullptr;
-  int og = 0;               // 2D: orientations per group
+  int pairs2 = 0;           // fused 2D passes: most (image, group) pairs of a launch
+  int groups3 = 0;          // 3D sides of k_pick_plane_max and k_blue_rows_max: most groups of a batch
   bool gen3d = false;       // 3D volumes whose side has no fused or long-row search: chirp-z transforms
   int nparts = 0;           // 2D above 256: pass-1 workgroups per orientation
   float2* scr = nullptr;    // 2D above 256: pass-1 output (B spectra)
@@ -83,11 +85,12 @@ int check_update_args(const gtomx_pick_plan* plan, const gtomx_complex* d_projec
                       gtomx_int3 dimsprojector, const gtomx_complex* d_expft, gtomx_int3 dimsvolume,
                       unsigned nvolumes, const float* d_best, const int32_t* d_idx);
 
-// The orientation loop of one volume or image: batches of pl->B orientations
-// of mats (nangles matrices already on the device) through the search's kernels
-// with indices angle0 + o. Kernel launches only (no host synchronisation, no
-// allocation), so it can be captured in a graph.
+// The orientation loop of nvol volumes or images (spectra H apart, CTFs
+// ctf_stride apart): batches of at most pl->B spectra over mats (nangles matrices
+// already on the device) through the search's kernels with indices angle0 + o.
+// Kernel launches only (no host synchronisation, no allocation), so it can be
+// captured in a graph.
 int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const CentredProjector* C, const float* mats,
-                          unsigned nangles, const float2* E, const float* ctf, float* best, int32_t* idx,
-                          int angle0, hipStream_t s);
+                          unsigned nangles, unsigned nvol, const float2* E, const float* ctf, size_t ctf_stride,
+                          float* best, int32_t* idx, int angle0, hipStream_t s);
 }  // namespace gx
