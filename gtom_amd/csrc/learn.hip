@@ -78,162 +78,300 @@ __device__ __forceinline__ bool tap_src(int t, int S, int z, int y, int x, int& 
 }
 
 // ---------------------------------------------------------------------------
-// Convolution (3^3, zero padding), forward or data gradient. One wave: 16
-// consecutive voxels of one tile x 16 output channels. out = (acc + bias),
-// ReLU if relu, zeroed where mask (a post-ReLU activation) is not positive.
-// wb: CIN = 16: [27][16 out][16 in] bf16; CIN = 1: [16 out][32 taps] bf16.
+// The first layer (1 -> 16 channels at 32^3) never keeps its activation, which is
+// 16 times its input and was most of a training pass's traffic (268 MB of the 256
+// tiles, written once and read three times): the forward pass pools it in the
+// kernel that makes it and leaves one bit per value, whether it is positive
+// (16 bits per voxel), and the weight gradient expands the pooled gradient from
+// those bits as it goes. 256 tiles: convolution 191 + pooling 56 us, expansion
+// 304 + gradient 331 us as separate passes.
+//
+// A workgroup stages input planes with a zero halo in LDS: rows of HX values, the
+// voxel (z, y, x) of the slab's first plane z0 at ((z - z0 + 1) * HY + y + 1) * HX + x + 1.
 // ---------------------------------------------------------------------------
-template <int S, int CIN>
+constexpr int HY = PT + 2, HX = PT + 2;
+
+__device__ __forceinline__ void stage_slab(const u16* __restrict__ tin, int z0, int planes, u16* slab) {
+  // planes z0 - 1 .. z0 + planes; two values at a time (rows of 32 start at odd places: 16-bit stores)
+  for (int k = threadIdx.x; k < (planes + 2) * HY * HX; k += 256) {
+    const int x = k % HX - 1, y = (k / HX) % HY - 1, z = z0 - 1 + k / (HY * HX);
+    const bool in = (unsigned)x < (unsigned)PT && (unsigned)y < (unsigned)PT && (unsigned)z < (unsigned)PT;
+    slab[k] = in ? tin[(z * PT + y) * PT + x] : (u16)0;
+  }
+}
+
+// conv1 + bias + ReLU (rounded to bf16), its positive bits, and the 2^3 average of
+// the rounded values. One workgroup per (tile, pooled plane); one wave per 16
+// voxels of the four rows under 8 pooled ones, which lie in one lane: D's rows are
+// 4 consecutive voxels.
+__global__ __launch_bounds__(256) void k_conv1_pool(const u16* __restrict__ in, const u16* __restrict__ wb,
+                                                    const float* __restrict__ bias, u16* __restrict__ bits,
+                                                    u16* __restrict__ out) {
+  constexpr int H = PT / 2, V = PT * PT * PT;
+  __shared__ u16 slab[4 * HY * HX];
+  const int tile = blockIdx.x / H, zp = blockIdx.x % H;
+  stage_slab(in + (size_t)tile * V, 2 * zp, 2, slab);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const u16x8 w = load8(wb + i * 32 + 8 * g);
+  const float bb = bias[i];
+  int off[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int t = 8 * g + e, tt = t < NTAP ? t : 0;  // taps past 26 have zero weights
+    off[e] = (tt / 9 * HY + (tt / 3) % 3) * HX + tt % 3;
+  }
+  for (int k = threadIdx.x >> 6; k < 2 * H; k += 4) {
+    const int yp = k >> 1, x0 = 16 * (k & 1);
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int dz = r >> 1, y = 2 * yp + (r & 1);
+      const u16* src = slab + (dz * HY + y) * HX + x0 + i;
+      u16x8 a;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] = src[off[e]];
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      acc = mfma(a, w, acc);
+      u16 mine = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u16 q = f2bf(fmaxf(acc[e] + bb, 0.f));
+        sum[e >> 1] += bf2f(q);
+        const unsigned long long pos = __ballot(bf_pos(q));
+        if (i == e) mine = (u16)(pos >> (16 * g));
+      }
+      if (i < 4) bits[(size_t)tile * V + ((2 * zp + dz) * PT + y) * PT + x0 + 4 * g + i] = mine;
+    }
+    const size_t o = (((size_t)tile * H + zp) * H + yp) * H + x0 / 2 + 2 * g;
+    out[o * PC + i] = f2bf(sum[0] * 0.125f);
+    out[(o + 1) * PC + i] = f2bf(sum[1] * 0.125f);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Convolution (3^3, zero padding) of 16 channels, forward or data gradient. One
+// wave: VG groups of 16 consecutive voxels of one tile x 16 output channels, with
+// each tap pair's weights loaded once for all. out = (acc + bias), ReLU if relu,
+// zeroed where mask (a post-ReLU activation) is not positive.
+// wb: [27][16 out][16 in] bf16.
+// ---------------------------------------------------------------------------
+constexpr int VG = 4;
+
+template <int S>
 __global__ __launch_bounds__(256) void k_conv(const u16* __restrict__ in, const u16* __restrict__ wb,
                                               const float* __restrict__ bias, const u16* __restrict__ mask,
                                               u16* __restrict__ out, int ntiles, int relu) {
-  constexpr int V = S * S * S, WPT = V / 16;
+  constexpr int V = S * S * S, WPT = V / (16 * VG);
   const int lane = threadIdx.x & 63;
   const long wave = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (wave >= (long)ntiles * WPT) return;
-  const int tile = (int)(wave / WPT), v0 = (int)(wave % WPT) * 16;
+  const int tile = (int)(wave / WPT), v0 = (int)(wave % WPT) * 16 * VG;
   const int i = lane & 15, g = lane >> 4;
-  const int v = v0 + i, x = v % S, y = (v / S) % S, z = v / (S * S);
-  const u16* tin = in + (size_t)tile * V * CIN;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (CIN == 1) {
-    u16x8 a;
+  const u16* tin = in + (size_t)tile * V * PC;
+  const int ci0 = 8 * (g & 1);
+  f32x4 acc[VG];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int t = 8 * g + e;
-      int src;
-      a[e] = (t < NTAP && tap_src(t, S, z, y, x, src)) ? tin[src] : (u16)0;
-    }
-    acc = mfma(a, load8(wb + i * 32 + 8 * g), acc);
-  } else {
-    const int ci0 = 8 * (g & 1);
+  for (int q = 0; q < VG; ++q) acc[q] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int p = 0; p < 14; ++p) {
-      const int t = 2 * p + (g >> 1);
-      u16x8 a = {0, 0, 0, 0, 0, 0, 0, 0}, b = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int p = 0; p < 14; ++p) {
+    const int t = 2 * p + (g >> 1);
+    u16x8 b = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (t < NTAP) b = load8(wb + (t * PC + i) * PC + ci0);
+#pragma unroll
+    for (int q = 0; q < VG; ++q) {
+      const int v = v0 + 16 * q + i, x = v % S, y = (v / S) % S, z = v / (S * S);
+      u16x8 a = {0, 0, 0, 0, 0, 0, 0, 0};
       int src;
-      if (t < NTAP) {
-        b = load8(wb + (t * PC + i) * PC + ci0);
-        if (tap_src(t, S, z, y, x, src)) a = load8(tin + (size_t)src * PC + ci0);
-      }
-      acc = mfma(a, b, acc);
+      if (t < NTAP && tap_src(t, S, z, y, x, src)) a = load8(tin + (size_t)src * PC + ci0);
+      acc[q] = mfma(a, b, acc[q]);
     }
   }
   const int co = i;
   const float bb = bias ? bias[co] : 0.f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const size_t o = ((size_t)tile * V + v0 + 4 * g + e) * PC + co;
-    float val = acc[e] + bb;
-    if (relu) val = fmaxf(val, 0.f);
-    if (mask && !bf_pos(mask[o])) val = 0.f;
-    out[o] = f2bf(val);
-  }
+  for (int q = 0; q < VG; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const size_t o = ((size_t)tile * V + v0 + 16 * q + 4 * g + e) * PC + co;
+      float val = acc[q][e] + bb;
+      if (relu) val = fmaxf(val, 0.f);
+      if (mask && !bf_pos(mask[o])) val = 0.f;
+      out[o] = f2bf(val);
+    }
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient partial sums over a chunk of voxels (all tiles' voxels in
-// one linear range): dW[t][co][ci] += dz[v][co] * in[v + off_t][ci], and the
-// bias gradient dz[v][co]. One wave per chunk of `steps` x 32 voxels; its
-// partials go to part[wave][...] (CIN = 16: 27*256 weights then 16 biases;
-// CIN = 1: [16 co][27] then 16 biases).
+// Weight gradients: dW[t][co][ci] = sum_v dz[v][co] * in[v + off_t][ci], and the
+// bias gradient sum_v dz[v][co]; M = co, N = ci (or taps), K = 32 voxels. A
+// workgroup sums its waves' results and writes one set of partials (27 * 256
+// weights, or [16 co][27], then 16 biases), which k_reduce_parts adds.
 // ---------------------------------------------------------------------------
 template <int CIN> constexpr int dw_part_len() { return CIN == 1 ? PC * NTAP + PC : NTAP * PC * PC + PC; }
 
-template <int S, int CIN>
-__global__ __launch_bounds__(256) void k_conv_dw(const u16* __restrict__ in, const u16* __restrict__ dz,
-                                                 float* __restrict__ part, long nvox, int steps, int nwaves) {
-  constexpr int V = S * S * S;
-  constexpr int NB = CIN == 1 ? 2 : NTAP;  // accumulators
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wave >= nwaves) return;
-  const int i = lane & 15, g = lane >> 4;
-  f32x4 acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = {0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  const long first = (long)wave * steps * 32;
-  for (int st = 0; st < steps; ++st) {
-    const long vb = first + (long)st * 32 + 8 * g;
-    if (first + (long)st * 32 >= nvox) break;
-    u16x8 a;
-    int tl[8], zz[8], yy[8], xx[8];
-    bool ok[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const long vv = vb + e;
-      ok[e] = vv < nvox;
-      const long vc = ok[e] ? vv : 0;
-      tl[e] = (int)(vc / V);
-      const int v = (int)(vc % V);
-      xx[e] = v % S;
-      yy[e] = (v / S) % S;
-      zz[e] = v / (S * S);
-      a[e] = ok[e] ? dz[vc * PC + i] : (u16)0;
-      bsum += bf2f(a[e]);
+// The input of a 16-channel weight gradient, channels first with a zero halo:
+// xt[tile][ci][S+2][S+2][S+2]. B's operand is 8 voxels along x of one channel at
+// each of 27 shifts: with this layout one 16-byte load without bounds checks, where
+// the channels-last one takes 8 checked 2-byte loads (571 us of 256 tiles at 16^3).
+template <int S>
+__global__ __launch_bounds__(256) void k_halo_channels(const u16* __restrict__ in, u16* __restrict__ xt, int ntiles) {
+  constexpr int P = S + 2, VP = P * P * P, V = S * S * S;
+  const long total = (long)ntiles * VP;
+  for (long id = blockIdx.x * 256L + threadIdx.x; id < total; id += (long)gridDim.x * 256) {
+    const int tile = (int)(id / VP), r = (int)(id % VP);
+    const int x = r % P - 1, y = (r / P) % P - 1, z = r / (P * P) - 1;
+    u16x8 lo = {0, 0, 0, 0, 0, 0, 0, 0}, hi = lo;
+    if ((unsigned)x < (unsigned)S && (unsigned)y < (unsigned)S && (unsigned)z < (unsigned)S) {
+      const u16* p = in + ((size_t)tile * V + (z * S + y) * S + x) * PC;
+      lo = load8(p);
+      hi = load8(p + 8);
     }
-    if constexpr (CIN == 1) {
+    u16* o = xt + (size_t)tile * PC * VP + r;
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        const int t = 16 * nb + i;
-        u16x8 b;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          int src;
-          b[e] = (ok[e] && t < NTAP && tap_src(t, S, zz[e], yy[e], xx[e], src)) ? in[(size_t)tl[e] * V + src]
-                                                                                 : (u16)0;
-        }
-        acc[nb] = mfma(a, b, acc[nb]);
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < NTAP; ++t) {
-        u16x8 b;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          int src;
-          b[e] = (ok[e] && tap_src(t, S, zz[e], yy[e], xx[e], src)) ? in[((size_t)tl[e] * V + src) * PC + i]
-                                                                   : (u16)0;
-        }
-        acc[t] = mfma(a, b, acc[t]);
-      }
+    for (int c = 0; c < 8; ++c) {
+      o[(size_t)c * VP] = lo[c];
+      o[(size_t)(c + 8) * VP] = hi[c];
     }
   }
-  // D: column = lane & 15 (ci, or tap), rows co = 4g + e
-  float* pw = part + (size_t)wave * dw_part_len<CIN>();
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int co = 4 * g + e;
-      if constexpr (CIN == 1) {
-        const int t = 16 * b + i;
-        if (t < NTAP) pw[co * NTAP + t] = acc[b][e];
-      } else {
-        pw[(b * PC + co) * PC + i] = acc[b][e];
-      }
-    }
-  // bias: lanes i, i+16, i+32, i+48 hold the four voxel groups of channel i
-  bsum += __shfl_xor(bsum, 16);
-  bsum += __shfl_xor(bsum, 32);
-  if (g == 0) pw[dw_part_len<CIN>() - PC + i] = bsum;
 }
 
-// grad[off + k] = sum over waves of part[w][k], k < len; one workgroup per k.
-__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int len, int nwaves,
-                                                      float* __restrict__ grad) {
-  __shared__ float red[256];
-  const int k = blockIdx.x;
-  float s = 0.f;
-  for (int w = threadIdx.x; w < nwaves; w += 256) s += part[(size_t)w * len + k];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+// 8 values at any 2-byte place.
+__device__ __forceinline__ u16x8 load8_any(const u16* p) {
+  u16x8 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+template <int S>
+__global__ __launch_bounds__(256) void k_conv_dw(const u16* __restrict__ xt, const u16* __restrict__ dz,
+                                                 float* __restrict__ part, int ntiles) {
+  constexpr int V = S * S * S, P = S + 2, VP = P * P * P, SPT = V / 32;  // steps of 32 voxels per tile
+  constexpr int LEN = dw_part_len<PC>();
+  __shared__ float sum[LEN];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = lane & 15, g = lane >> 4;
+  f32x4 acc[NTAP];
+#pragma unroll
+  for (int t = 0; t < NTAP; ++t) acc[t] = {0.f, 0.f, 0.f, 0.f};
+  float bsum = 0.f;
+  const long steps = (long)ntiles * SPT, waves = (long)gridDim.x * 4, me = (long)blockIdx.x * 4 + w;
+  for (long st = steps * me / waves; st < steps * (me + 1) / waves; ++st) {
+    const int tile = (int)(st / SPT), v = (int)(st % SPT) * 32 + 8 * g;  // 8 voxels of one row
+    const int x = v % S, y = (v / S) % S, z = v / (S * S);
+    const u16* d = dz + ((size_t)tile * V + v) * PC + i;
+    u16x8 a;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      a[e] = d[e * PC];
+      bsum += bf2f(a[e]);
+    }
+    const u16* src = xt + ((size_t)tile * PC + i) * VP + (z * P + y) * P + x;
+#pragma unroll
+    for (int t = 0; t < NTAP; ++t)
+      acc[t] = mfma(a, load8_any(src + (t / 9 * P + (t / 3) % 3) * P + t % 3), acc[t]);
+  }
+  bsum += __shfl_xor(bsum, 16);
+  bsum += __shfl_xor(bsum, 32);
+  // D: column = lane & 15 (ci), rows co = 4g + e; the waves add in turn
+  for (int k = 0; k < 4; ++k) {
+    if (w == k) {
+#pragma unroll
+      for (int t = 0; t < NTAP; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int q = (t * PC + 4 * g + e) * PC + i;
+          sum[q] = k == 0 ? acc[t][e] : sum[q] + acc[t][e];
+        }
+      if (g == 0) sum[LEN - PC + i] = k == 0 ? bsum : sum[LEN - PC + i] + bsum;
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) grad[k] = red[0];
+  float* pw = part + (size_t)blockIdx.x * LEN;
+  for (int k = threadIdx.x; k < LEN; k += 256) pw[k] = sum[k];
+}
+
+// The first layer's: dz[v][co] = the pooled gradient of v's parent / 8 where the
+// activation's bit is set. Items are slabs of 4 planes of a tile.
+__global__ __launch_bounds__(256) void k_conv1_dw(const u16* __restrict__ in, const u16* __restrict__ bits,
+                                                  const u16* __restrict__ dp, float* __restrict__ part, int ntiles) {
+  constexpr int H = PT / 2, V = PT * PT * PT, ZS = 4, SLABS = PT / ZS;
+  constexpr int LEN = dw_part_len<1>();
+  __shared__ u16 slab[(ZS + 2) * HY * HX];
+  __shared__ float sum[LEN];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = lane & 15, g = lane >> 4;
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  float bsum = 0.f;
+  int off[2];
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb) {
+    const int t = 16 * nb + i < NTAP ? 16 * nb + i : 0;  // columns past tap 26 are not kept
+    off[nb] = (t / 9 * HY + (t / 3) % 3) * HX + t % 3;
+  }
+  for (int item = blockIdx.x; item < ntiles * SLABS; item += gridDim.x) {
+    const int tile = item / SLABS, z0 = (item % SLABS) * ZS;
+    __syncthreads();
+    stage_slab(in + (size_t)tile * V, z0, ZS, slab);
+    __syncthreads();
+    for (int row = w; row < ZS * PT; row += 4) {  // one row of 32 voxels per step
+      const int dz = row / PT, y = row % PT, z = z0 + dz;
+      const size_t v = (size_t)tile * V + (z * PT + y) * PT + 8 * g;
+      const u16x8 m = load8(bits + v);
+      const u16* d = dp + ((((size_t)tile * H + z / 2) * H + y / 2) * H + 4 * g) * PC + i;
+      u16x8 a;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const u16 q = f2bf(bf2f(d[(e >> 1) * PC]) * 0.125f);
+        a[e] = (m[e] >> i) & 1 ? q : (u16)0;
+        bsum += bf2f(a[e]);
+      }
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        const u16* src = slab + (dz * HY + y) * HX + 8 * g + off[nb];
+        u16x8 b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = src[e];
+        acc[nb] = mfma(a, b, acc[nb]);
+      }
+    }
+  }
+  bsum += __shfl_xor(bsum, 16);
+  bsum += __shfl_xor(bsum, 32);
+  __syncthreads();
+  // D: column = lane & 15 (tap), rows co = 4g + e
+  for (int k = 0; k < 4; ++k) {
+    if (w == k) {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = 16 * nb + i, q = (4 * g + e) * NTAP + t;
+          if (t < NTAP) sum[q] = k == 0 ? acc[nb][e] : sum[q] + acc[nb][e];
+        }
+      if (g == 0) sum[LEN - PC + i] = k == 0 ? bsum : sum[LEN - PC + i] + bsum;
+    }
+    __syncthreads();
+  }
+  float* pw = part + (size_t)blockIdx.x * LEN;
+  for (int k = threadIdx.x; k < LEN; k += 256) pw[k] = sum[k];
+}
+
+// grad[k] = sum over p of part[p][k], k < len: a workgroup takes 16 values of k,
+// 16 threads each (the partials of a set are contiguous: 64-byte reads).
+__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int len, int nparts,
+                                                      float* __restrict__ grad) {
+  __shared__ float red[256];
+  const int t = threadIdx.x, k = blockIdx.x * 16 + (t & 15);
+  float s = 0.f;
+  if (k < len)
+    for (int p = t >> 4; p < nparts; p += 16) s += part[(size_t)p * len + k];
+  red[t] = s;
+  __syncthreads();
+  for (int h = 128; h >= 16; h >>= 1) {
+    if (t < h) red[t] += red[t + h];
+    __syncthreads();
+  }
+  if (t < 16 && k < len) grad[k] = red[t];
 }
 
 // ---------------------------------------------------------------------------
@@ -302,13 +440,23 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ A, long sa
   const int i = lane & 15, g = lane >> 4;
   const int m = mb * 16 + i, n = nb * 16 + i;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // an operand whose k runs contiguously at 16-byte places is loaded 8 values at a time
+  const bool va = sak == 1 && sam % 8 == 0 && K % 32 == 0 && ((size_t)A & 15) == 0;
+  const bool vb = sbk == 1 && sbn % 8 == 0 && K % 32 == 0 && ((size_t)B & 15) == 0;
   for (int k0 = 0; k0 < K; k0 += 32) {
-    u16x8 a, b;
+    u16x8 a = {0, 0, 0, 0, 0, 0, 0, 0}, b = a;
+    const int kk = k0 + 8 * g;
+    if (va) {
+      if (m < M) a = load8(A + m * sam + kk);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int k = k0 + 8 * g + e;
-      a[e] = (m < M && k < K) ? A[m * sam + k * sak] : (u16)0;
-      b[e] = (n < N && k < K) ? B[k * sbk + n * sbn] : (u16)0;
+      for (int e = 0; e < 8; ++e) a[e] = (m < M && kk + e < K) ? A[m * sam + (kk + e) * sak] : (u16)0;
+    }
+    if (vb) {
+      if (n < N) b = load8(B + n * sbn + kk);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) b[e] = (n < N && kk + e < K) ? B[(kk + e) * sbk + n * sbn] : (u16)0;
     }
     acc = mfma(a, b, acc);
   }
@@ -568,16 +716,16 @@ struct gtomx_pnet {
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // NPARAM each
   long step = 0;
   u16 *w1b = nullptr, *wcb = nullptr, *wct = nullptr, *wfb = nullptr;
-  u16 *x = nullptr, *a1 = nullptr, *p1 = nullptr, *a2 = nullptr, *p2 = nullptr, *a3 = nullptr, *a4 = nullptr,
+  u16* xt = nullptr;  // input of a 16-channel weight gradient, channels first with a halo (16^3 the largest)
+  u16 *x = nullptr, *bits1 = nullptr, *p1 = nullptr, *a2 = nullptr, *p2 = nullptr, *a3 = nullptr, *a4 = nullptr,
       *feat = nullptr;
   float* logits = nullptr;
   float* dlog = nullptr;
   u16* dlogb = nullptr;
   float* dfeat = nullptr;
   float* loss = nullptr;
-  u16 *dz4 = nullptr, *dz3 = nullptr, *dp2 = nullptr, *dz2 = nullptr, *dp1 = nullptr, *dz1 = nullptr;
+  u16 *dz4 = nullptr, *dz3 = nullptr, *dp2 = nullptr, *dz2 = nullptr, *dp1 = nullptr;
   float* part = nullptr;
-  size_t part_floats = 0;
   double* mom = nullptr;  // moments partials of k_moments
   unsigned nlast = 0;     // tiles of the last forward pass
   size_t device_bytes = 0;
@@ -593,10 +741,10 @@ void pnet_release(gtomx_pnet* nt) {
   if (!nt) return;
   nt->fence.release();
   for (void* q : {(void*)nt->p, (void*)nt->g, (void*)nt->m, (void*)nt->v, (void*)nt->w1b, (void*)nt->wcb,
-                  (void*)nt->wct, (void*)nt->wfb, (void*)nt->x, (void*)nt->a1, (void*)nt->p1, (void*)nt->a2,
+                  (void*)nt->wct, (void*)nt->wfb, (void*)nt->x, (void*)nt->xt, (void*)nt->bits1, (void*)nt->p1, (void*)nt->a2,
                   (void*)nt->p2, (void*)nt->a3, (void*)nt->a4, (void*)nt->feat, (void*)nt->logits, (void*)nt->dlog,
                   (void*)nt->dlogb, (void*)nt->dfeat, (void*)nt->loss, (void*)nt->dz4, (void*)nt->dz3,
-                  (void*)nt->dp2, (void*)nt->dz2, (void*)nt->dp1, (void*)nt->dz1, (void*)nt->part, (void*)nt->mom})
+                  (void*)nt->dp2, (void*)nt->dz2, (void*)nt->dp1, (void*)nt->part, (void*)nt->mom})
     dev_free(q);
   delete nt;
 }
@@ -616,33 +764,41 @@ int refresh(gtomx_pnet* nt, hipStream_t s) {
   return GTOMX_OK;
 }
 
-template <int S, int CIN>
+template <int S>
 int conv(const u16* in, const u16* wb, const float* bias, const u16* mask, u16* out, unsigned n, int relu,
          hipStream_t s) {
-  const long waves = (long)n * (S * S * S / 16);
-  hipLaunchKernelGGL((k_conv<S, CIN>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, in, wb, bias, mask, out,
-                     (int)n, relu);
+  const long waves = (long)n * (S * S * S / (16 * VG));
+  hipLaunchKernelGGL((k_conv<S>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, in, wb, bias, mask, out, (int)n,
+                     relu);
   GX_LAUNCHED("k_conv");
   return GTOMX_OK;
 }
 
-// Weight and bias gradient of one convolution into grad + woff (weights) and grad + boff (bias).
-template <int S, int CIN>
-int conv_dw(gtomx_pnet* nt, const u16* in, const u16* dz, unsigned n, float* wgrad, float* bgrad, hipStream_t s) {
-  const long nvox = (long)n * S * S * S;
-  const int len = dw_part_len<CIN>();
-  // about 2048 waves, each at least 4 steps of 32 voxels
-  int steps = (int)std::max<long>(4, (nvox + 2048L * 32 - 1) / (2048L * 32));
-  int nw = (int)((nvox + (long)steps * 32 - 1) / ((long)steps * 32));
-  if ((size_t)nw * len > nt->part_floats) return fail(GTOMX_ERR_INTERNAL, "gradient partials exceed the scratch");
-  hipLaunchKernelGGL((k_conv_dw<S, CIN>), dim3((nw + 3) / 4), dim3(256), 0, s, in, dz, nt->part, nvox, steps, nw);
-  GX_LAUNCHED("k_conv_dw");
-  const int wl = len - PC;
-  hipLaunchKernelGGL(k_reduce_parts, dim3(wl), dim3(256), 0, s, nt->part, len, nw, wgrad);
-  GX_LAUNCHED("k_reduce_parts");
-  hipLaunchKernelGGL(k_reduce_parts, dim3(PC), dim3(256), 0, s, nt->part + wl, len, nw, bgrad);
+constexpr int DW_PARTS = 512;  // workgroups (and sets of partials) of a weight gradient: two per CU
+
+int reduce_parts(gtomx_pnet* nt, int len, int nparts, float* grad, hipStream_t s) {
+  hipLaunchKernelGGL(k_reduce_parts, dim3((len + 15) / 16), dim3(256), 0, s, nt->part, len, nparts, grad);
   GX_LAUNCHED("k_reduce_parts");
   return GTOMX_OK;
+}
+
+// Weight and bias gradient of a 16-channel convolution into grad (weights, then bias).
+template <int S> int conv_dw(gtomx_pnet* nt, const u16* in, const u16* dz, unsigned n, float* grad, hipStream_t s) {
+  constexpr int VP = (S + 2) * (S + 2) * (S + 2);
+  hipLaunchKernelGGL((k_halo_channels<S>), dim3(grid_of((size_t)n * VP)), dim3(256), 0, s, in, nt->xt, (int)n);
+  GX_LAUNCHED("k_halo_channels");
+  const int nparts = (int)std::min<long>(DW_PARTS, ((long)n * (S * S * S / 32) + 3) / 4);
+  hipLaunchKernelGGL((k_conv_dw<S>), dim3(nparts), dim3(256), 0, s, nt->xt, dz, nt->part, (int)n);
+  GX_LAUNCHED("k_conv_dw");
+  return reduce_parts(nt, dw_part_len<PC>(), nparts, grad, s);
+}
+
+// The first layer's, from the pooled gradient.
+int conv1_dw(gtomx_pnet* nt, unsigned n, float* grad, hipStream_t s) {
+  const int nparts = (int)std::min<long>(2 * DW_PARTS, (long)n * 8);
+  hipLaunchKernelGGL(k_conv1_dw, dim3(nparts), dim3(256), 0, s, nt->x, nt->bits1, nt->dp1, nt->part, (int)n);
+  GX_LAUNCHED("k_conv1_dw");
+  return reduce_parts(nt, dw_part_len<1>(), nparts, grad, s);
 }
 
 int gemm(const u16* A, long sam, long sak, const u16* B, long sbk, long sbn, float* C, long scm, int M, int N, int K,
@@ -672,12 +828,13 @@ unsigned rows_of(unsigned n) { return (n + 15) / 16 * 16; }
 // Forward pass over n tiles already in nt->x.
 int forward(gtomx_pnet* nt, unsigned n, hipStream_t s) {
   const unsigned rows = rows_of(n);
-  GX_TRY((conv<32, 1>(nt->x, nt->w1b, nt->p + OFF_B1, nullptr, nt->a1, n, 1, s)));
-  GX_TRY(pool<32>(nt->a1, nt->p1, n, n, s));
-  GX_TRY((conv<16, 16>(nt->p1, nt->wcb, nt->p + OFF_B2, nullptr, nt->a2, n, 1, s)));
+  hipLaunchKernelGGL(k_conv1_pool, dim3(n * (PT / 2)), dim3(256), 0, s, nt->x, nt->w1b, nt->p + OFF_B1, nt->bits1,
+                     nt->p1);
+  GX_LAUNCHED("k_conv1_pool");
+  GX_TRY((conv<16>(nt->p1, nt->wcb, nt->p + OFF_B2, nullptr, nt->a2, n, 1, s)));
   GX_TRY(pool<16>(nt->a2, nt->p2, n, n, s));
-  GX_TRY((conv<8, 16>(nt->p2, nt->wcb + NTAP * PC * PC, nt->p + OFF_B3, nullptr, nt->a3, n, 1, s)));
-  GX_TRY((conv<8, 16>(nt->a3, nt->wcb + 2 * NTAP * PC * PC, nt->p + OFF_B4, nullptr, nt->a4, n, 1, s)));
+  GX_TRY((conv<8>(nt->p2, nt->wcb + NTAP * PC * PC, nt->p + OFF_B3, nullptr, nt->a3, n, 1, s)));
+  GX_TRY((conv<8>(nt->a3, nt->wcb + 2 * NTAP * PC * PC, nt->p + OFF_B4, nullptr, nt->a4, n, 1, s)));
   GX_TRY(pool<8>(nt->a4, nt->feat, n, rows, s));
   // logits[r][c] = feat[r] . Wf[c] + bf[c] for the 501 classes (columns 501..511 stay zero)
   GX_TRY(gemm(nt->feat, NFEAT, 1, nt->wfb, 1, NFEAT, nt->logits, CPAD, (int)rows, NCLS, NFEAT, nt->p + OFF_BF, s));
@@ -699,16 +856,14 @@ int backward(gtomx_pnet* nt, const int* d_labels, unsigned n, hipStream_t s) {
   // dfeat[r][f] = sum_c dlog[r][c] Wf[c][f]
   GX_TRY(gemm(nt->dlogb, CPAD, 1, nt->wfb, NFEAT, 1, nt->dfeat, NFEAT, (int)rows, NFEAT, CPAD, nullptr, s));
   GX_TRY((unpool<8, float>(nt->dfeat, nt->a4, nt->dz4, n, s)));
-  GX_TRY((conv_dw<8, 16>(nt, nt->a3, nt->dz4, n, nt->g + OFF_W4, nt->g + OFF_B4, s)));
-  GX_TRY((conv<8, 16>(nt->dz4, nt->wct + 2 * NTAP * PC * PC, nullptr, nt->a3, nt->dz3, n, 0, s)));
-  GX_TRY((conv_dw<8, 16>(nt, nt->p2, nt->dz3, n, nt->g + OFF_W3, nt->g + OFF_B3, s)));
-  GX_TRY((conv<8, 16>(nt->dz3, nt->wct + NTAP * PC * PC, nullptr, nullptr, nt->dp2, n, 0, s)));
+  GX_TRY(conv_dw<8>(nt, nt->a3, nt->dz4, n, nt->g + OFF_W4, s));
+  GX_TRY((conv<8>(nt->dz4, nt->wct + 2 * NTAP * PC * PC, nullptr, nt->a3, nt->dz3, n, 0, s)));
+  GX_TRY(conv_dw<8>(nt, nt->p2, nt->dz3, n, nt->g + OFF_W3, s));
+  GX_TRY((conv<8>(nt->dz3, nt->wct + NTAP * PC * PC, nullptr, nullptr, nt->dp2, n, 0, s)));
   GX_TRY((unpool<16, u16>(nt->dp2, nt->a2, nt->dz2, n, s)));
-  GX_TRY((conv_dw<16, 16>(nt, nt->p1, nt->dz2, n, nt->g + OFF_W2, nt->g + OFF_B2, s)));
-  GX_TRY((conv<16, 16>(nt->dz2, nt->wct, nullptr, nullptr, nt->dp1, n, 0, s)));
-  GX_TRY((unpool<32, u16>(nt->dp1, nt->a1, nt->dz1, n, s)));
-  GX_TRY((conv_dw<32, 1>(nt, nt->x, nt->dz1, n, nt->g + OFF_W1, nt->g + OFF_B1, s)));
-  return GTOMX_OK;
+  GX_TRY(conv_dw<16>(nt, nt->p1, nt->dz2, n, nt->g + OFF_W2, s));
+  GX_TRY((conv<16>(nt->dz2, nt->wct, nullptr, nullptr, nt->dp1, n, 0, s)));
+  return conv1_dw(nt, n, nt->g + OFF_W1, s);
 }
 
 }  // namespace
@@ -748,7 +903,8 @@ int gtomx_pnet_create(gtomx_pnet** out, unsigned max_tiles) {
   alloc(&nt->wct, 3 * NTAP * PC * PC * 2);
   alloc(&nt->wfb, (size_t)CPAD * NFEAT * 2);
   alloc(&nt->x, C * V1 * 2);
-  alloc(&nt->a1, C * V1 * PC * 2);
+  alloc(&nt->xt, C * PC * 18 * 18 * 18 * 2);
+  alloc(&nt->bits1, C * V1 * 2);
   alloc(&nt->p1, C * V2 * PC * 2);
   alloc(&nt->a2, C * V2 * PC * 2);
   alloc(&nt->p2, C * V3 * PC * 2);
@@ -765,9 +921,8 @@ int gtomx_pnet_create(gtomx_pnet** out, unsigned max_tiles) {
   alloc(&nt->dp2, C * V3 * PC * 2);
   alloc(&nt->dz2, C * V2 * PC * 2);
   alloc(&nt->dp1, C * V2 * PC * 2);
-  alloc(&nt->dz1, C * V1 * PC * 2);
-  nt->part_floats = (size_t)2100 * (NTAP * PC * PC + PC);
-  alloc(&nt->part, nt->part_floats * 4);
+  static_assert(2 * dw_part_len<1>() <= dw_part_len<PC>(), "the first layer's partials fit the others' scratch");
+  alloc(&nt->part, (size_t)DW_PARTS * dw_part_len<PC>() * 4);
   alloc(&nt->mom, (size_t)MOM_BLOCKS * 2 * sizeof(double));
   if (st != GTOMX_OK) {
     std::string msg = gtomx_last_error();
