@@ -18,7 +18,9 @@
 #include <vector>
 #include <type_traits>
 
+#include "dev_blue.hpp"
 #include "dev_fft.hpp"
+#include "dev_project.hpp"
 #include "runtime.hpp"
 
 namespace gx {
@@ -125,9 +127,21 @@ __global__ __launch_bounds__(256) void k_rows_c2r(const float2* __restrict__ in,
 // Row R2C: N reals -> N/2+1 bins. z[m] = x[2m] + i x[2m+1], Z = DFT_{N/2}(z),
 // X[k] = ((Z[k] + conj Z[N/2-k]) - i w^k (Z[k] - conj Z[N/2-k])) / 2, w = e^{-2 pi i/N}.
 // ---------------------------------------------------------------------------
-template <int N>
+// A line of n0 points in FFT order (origin first, c of them at non-negative
+// positions) inside a longer one: the index of the n-point line's point p in the
+// short one, -1 where the long line is zero. n0 = 0: the line itself.
+struct PadMap {
+  int n0 = 0, c = 0;
+  __device__ __forceinline__ int at(int p, int n) const {
+    return p < c ? p : (p >= n - (n0 - c) ? p - (n - n0) : -1);
+  }
+};
+
+// PAD: the rows hold pm.n0 reals, padded to N on load.
+template <int N, bool PAD = false>
 __global__ __launch_bounds__(256) void k_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                  long long nrows, const float2* __restrict__ tw, RowBand rb) {
+                                                  long long nrows, const float2* __restrict__ tw, RowBand rb,
+                                                  PadMap pm = PadMap{}) {
   constexpr int NC = N / 2, NH = N / 2 + 1;
   constexpr int R1 = RowShape<NC>::R1, R2 = RowShape<NC>::R2, RW = 256 / R2;
   constexpr int GS = R2 * (R1 + 1);
@@ -137,10 +151,19 @@ __global__ __launch_bounds__(256) void k_rows_r2c(const float* __restrict__ in, 
   const int t = threadIdx.x, r = t / R2, j = t % R2;
   const bool valid = (long long)blockIdx.x * RW + r < nrows;
   const long long row = band_row((long long)blockIdx.x * RW, rb) + r;
-  const float2* x = reinterpret_cast<const float2*>(in + row * N);
   float2 v[R1];
+  if constexpr (PAD) {
+    const float* x = in + row * pm.n0;
 #pragma unroll
-  for (int m = 0; m < R1; ++m) v[m] = valid ? x[j + R2 * m] : make_float2(0.f, 0.f);
+    for (int m = 0; m < R1; ++m) {
+      const int a = pm.at(2 * (j + R2 * m), N), b = pm.at(2 * (j + R2 * m) + 1, N);
+      v[m] = make_float2(valid && a >= 0 ? x[a] : 0.f, valid && b >= 0 ? x[b] : 0.f);
+    }
+  } else {
+    const float2* x = reinterpret_cast<const float2*>(in + row * N);
+#pragma unroll
+    for (int m = 0; m < R1; ++m) v[m] = valid ? x[j + R2 * m] : make_float2(0.f, 0.f);
+  }
   fft_two_step<NC, R1, R2, -1>(v, j, tw, [&](int k1, int jj) { return &xch[r * GS + jj * (R1 + 1) + k1]; });
 #pragma unroll
   for (int s = 0; s < R1; ++s) zrow[r * ZS + out_index<R1, R2>(j, s)] = v[s];
@@ -709,7 +732,7 @@ int launch_rows_r2c(int n, const float* in, float2* out, long long nrows, const 
   auto go = [&](auto kernel, int rw) -> int {
     if (rb.by % rw) return fail(GTOMX_ERR_INTERNAL, "row band not a multiple of the rows per workgroup");
     dim3 grid((unsigned)((nrows + rw - 1) / rw));
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, out, nrows, tw, rb);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, out, nrows, tw, rb, PadMap{});
     GX_LAUNCHED("k_rows_r2c");
     return GTOMX_OK;
   };
@@ -1096,75 +1119,14 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
 // product with B needs no exchange of its own: two exchanges in all, the second
 // through the addresses a thread read itself.
 // ---------------------------------------------------------------------------
-template <int M> struct BlueShape;
-template <> struct BlueShape<16>   { static constexpr int R1 = 4,  R2 = 4,  TX = 64; };
-template <> struct BlueShape<24>   { static constexpr int R1 = 12, R2 = 2,  TX = 64; };
-template <> struct BlueShape<32>   { static constexpr int R1 = 8,  R2 = 4,  TX = 64; };
-template <> struct BlueShape<48>   { static constexpr int R1 = 12, R2 = 4,  TX = 64; };
-template <> struct BlueShape<64>   { static constexpr int R1 = 8,  R2 = 8,  TX = 32; };
-template <> struct BlueShape<96>   { static constexpr int R1 = 24, R2 = 4,  TX = 32; };
-template <> struct BlueShape<128>  { static constexpr int R1 = 16, R2 = 8,  TX = 32; };
-template <> struct BlueShape<192>  { static constexpr int R1 = 24, R2 = 8,  TX = 16; };
-template <> struct BlueShape<256>  { static constexpr int R1 = 16, R2 = 16, TX = 16; };
-template <> struct BlueShape<512>  { static constexpr int R1 = 32, R2 = 16, TX = 16; };
-template <> struct BlueShape<1024> { static constexpr int R1 = 32, R2 = 32, TX = 16; };
-#define GX_FOR_BLUE(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512) X(1024)
-constexpr int BLUE_FUSED_MAX = 512;  // longest L of the fused form
-
-// The circular convolution of one line with the kernel whose spectrum is B (LDS,
-// M values with the 1/M in them). v[m] in and out: point j + R2 m, zero for
-// m >= R1/2 on entry, meaningful for m < R1/2 on exit.
-template <int M, class Xch, class Sync>
-__device__ __forceinline__ void blue_convolve(float2 (&v)[BlueShape<M>::R1], int j, const float2* twl,
-                                              const float2* B, Xch xch, Sync sync) {
-  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2;
-  dft<R1, -1>(v);
-#pragma unroll
-  for (int k1 = 1; k1 < R1; ++k1) v[k1] = cmul(v[k1], twl[j * k1]);
-#pragma unroll
-  for (int k1 = 0; k1 < R1; ++k1) *xch(k1, j) = v[k1];
-  sync();
-#pragma unroll
-  for (int u = 0; u < R1 / R2; ++u) {
-    const int k1 = j * (R1 / R2) + u;
-    float2 z[R2];
-#pragma unroll
-    for (int jj = 0; jj < R2; ++jj) z[jj] = *xch(k1, jj);
-    dft<R2, -1>(z);
-#pragma unroll
-    for (int k2 = 0; k2 < R2; ++k2) z[k2] = cmul(z[k2], B[k1 + R1 * k2]);
-    dft<R2, 1>(z);
-#pragma unroll
-    for (int jj = 0; jj < R2; ++jj) *xch(k1, jj) = jj == 0 ? z[jj] : cmulc(z[jj], twl[jj * k1]);
-  }
-  sync();
-#pragma unroll
-  for (int k1 = 0; k1 < R1; ++k1) v[k1] = *xch(k1, j);
-  dft<R1, 1>(v);
-}
-
-// The tables of a workgroup: twiddles of M, the kernel spectrum, the chirp as the
-// direction multiplies by it.
-template <int M, int DIR>
-__device__ __forceinline__ void blue_stage(int t, int nt, int L, const float2* __restrict__ tw,
-                                           const float2* __restrict__ B, const float2* __restrict__ chirp, float2* twl,
-                                           float2* bl, float2* cl) {
-  for (int i = t; i < M; i += nt) {
-    twl[i] = twiddle<-1, M>(tw, i);
-    bl[i] = B[i];
-  }
-  for (int i = t; i < M / 2; i += nt) {
-    const float2 c = i < L ? chirp[i] : make_float2(0.f, 0.f);
-    cl[i] = DIR < 0 ? c : cconj(c);
-  }
-}
-
-// A strided axis, from src into dst (which may be src), addressed as k_cols.
+// A strided axis, from src into dst (which may be src), addressed as k_cols. With
+// half > 0 the axis is y of a search's planes, whose entries outside the disc
+// x^2 + y^2 <= half^2 (x the column) were not written and read as zero.
 template <int M, int DIR>
 __global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols(
     const float2* src, float2* dst, int width, long long axis_stride, long long nplanes, long long P1, long long S0,
     long long S1, int L, const float2* __restrict__ chirp, const float2* __restrict__ B,
-    const float2* __restrict__ tw) {
+    const float2* __restrict__ tw, int half) {
   constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
   __shared__ float2 xch[TX * M];
   __shared__ float2 twl[M], bl[M], cl[M / 2];
@@ -1177,8 +1139,9 @@ __global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_co
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
-      v[m] = valid && p < L ? src[base + (long long)p * axis_stride] : make_float2(0.f, 0.f);
+      const int p = j + R2 * m, y = p <= L / 2 ? p : p - L;
+      const bool in = half == 0 || col * col + y * y <= half * half;
+      v[m] = valid && p < L && in ? src[base + (long long)p * axis_stride] : make_float2(0.f, 0.f);
     }
     __syncthreads();  // the tables are staged, the last plane's exchange is read
 #pragma unroll
@@ -1257,10 +1220,12 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_c2r(const
 }
 
 // A[k] = (Z[k] + conj Z[L - k]) / 2, B[k] = (Z[k] - conj Z[L - k]) / 2i of Z = DFT(a + i b).
+// With pm.n0 the rows hold that many reals, padded to L on load.
 template <int M>
 __global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
                                                        long long nrows, int L, const float2* __restrict__ chirp,
-                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
+                                                       const float2* __restrict__ B, const float2* __restrict__ tw,
+                                                       PadMap pm) {
   using S = BlueRows<M>;
   constexpr int R1 = S::R1, R2 = S::R2;
   __shared__ float2 area[S::TP * S::AREA];
@@ -1273,12 +1238,13 @@ __global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__
   for (long long row = 2 * ((long long)blockIdx.x * S::TP + t / R2); row < nrows; row += step) {
     const int nh = L / 2 + 1;
     const bool two = row + 1 < nrows;
-    const float* a = in + row * L;
+    const int len = pm.n0 ? pm.n0 : L;
+    const float* a = in + row * len;
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
-      v[m] = make_float2(p < L ? a[p] : 0.f, p < L && two ? a[L + p] : 0.f);
+      const int p = j + R2 * m, q = p >= L ? -1 : (pm.n0 ? pm.at(p, L) : p);
+      v[m] = make_float2(q >= 0 ? a[q] : 0.f, q >= 0 && two ? a[len + q] : 0.f);
     }
 #pragma unroll
     for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
@@ -1299,17 +1265,22 @@ __global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__
   }
 }
 
-// The generic search's row pass: the C2R of every row of the orientations
-// o in group blockIdx.y (og of them), times scale[o], folded into a running
-// maximum in registers (strict >, increasing o). FRESH as in k_pick_x_max.
-template <int M, bool FRESH>
-__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(const float2* __restrict__ G, long long H, int nb, int n,
-                                                       int nrows, int angle0, const float* __restrict__ scale,
-                                                       float* __restrict__ best, int32_t* __restrict__ bidx, int og,
-                                                       const float2* __restrict__ chirp,
-                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
+// A search's row pass: the C2R of every row of the orientations o in group
+// blockIdx.y (og of them), folded into a running maximum in registers (strict >,
+// increasing o). With FRESH the maximum starts at -infinity / -1 and goes to the
+// group's own nrows * n values. SEARCH: rows of (n + 1) / 2 bins without X[n/2],
+// which is sn[o].y, times sn[o].x; otherwise rows of n/2 + 1 bins, not scaled.
+// A pair of voxels keeps its two orientations as 16-bit offsets in the group in
+// one register (NONE: unchanged): with 32-bit indices the 512-point form spills
+// (200^3: 1.38 ms per 32 orientations).
+template <int M, bool FRESH, bool SEARCH>
+__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(
+    const float2* __restrict__ G, long long H, int nb, int n, int nrows, int angle0, const float2* __restrict__ sn,
+    float* __restrict__ best, int32_t* __restrict__ bidx, int og, const float2* __restrict__ chirp,
+    const float2* __restrict__ B, const float2* __restrict__ tw) {
   using S = BlueRows<M>;
   constexpr int R1 = S::R1, R2 = S::R2, HP = R1 / 2;
+  constexpr unsigned NONE = 0xffffu;
   __shared__ float2 area[S::TP * S::AREA];
   __shared__ float2 twl[M], bl[M], cl[M / 2];
   const int t = threadIdx.x, j = t % R2;
@@ -1326,45 +1297,59 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(const
     best += (size_t)blockIdx.y * nrows * n;
     bidx += (size_t)blockIdx.y * nrows * n;
   }
-  const int nh = n / 2 + 1;
+  const int pitch = SEARCH ? (n + 1) / 2 : n / 2 + 1;
   float bv[2][HP];
-  int32_t bi[2][HP];
+  unsigned bi[HP];
 #pragma unroll
   for (int m = 0; m < HP; ++m) {
     const int p = j + R2 * m;
     const size_t i = (size_t)row * n + p;
     const bool in = !FRESH && p < n;
     bv[0][m] = in ? best[i] : -__builtin_inff();
-    bi[0][m] = in ? bidx[i] : 0;
     bv[1][m] = in && two ? best[i + n] : -__builtin_inff();
-    bi[1][m] = in && two ? bidx[i + n] : 0;
+    bi[m] = NONE | NONE << 16;
   }
   for (int o = o0; o < o1; ++o) {
-    const float2* a = G + o * H + (long long)row * nh;
-    const float sc = scale[o];
+    const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + o * H, (unsigned)(H * 8));
+    const float2 so = SEARCH ? sn[o] : make_float2(1.f, 0.f);
+    // opaque per orientation: what follows from it alone (addresses, bounds) is recomputed rather than held
+    // in registers, which would spill
+    int jo = j;
+    asm volatile("" : "+v"(jo));
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < HP; ++m) {
-      const int p = j + R2 * m;
-      v[m] = row_pair_bin(a, a + nh, p < n, p < n && two, p < n ? p : 0, n);
+      // z[p] of row_pair_bin; a last row without a partner reads past the buffer's end, which gives 0
+      const int p = jo + R2 * m;
+      const bool mirror = p > n / 2, mid = 2 * p == n;
+      const int q = mirror ? n - p : p;
+      const int off = p < n && !(SEARCH && mid) ? (row * pitch + q) * 8 : OUT_OF_RANGE;
+      float2 x = buf_load2(rG, off, 0), y = buf_load2(rG, off, pitch * 8);
+      if (SEARCH) {
+        x.x += mid ? so.y : 0.f;
+        y.x += mid ? so.y : 0.f;
+      }
+      if (mid || p == 0) x.y = y.y = 0.f;
+      v[m] = mirror ? make_float2(x.x + y.y, y.x - x.y) : make_float2(x.x - y.y, x.y + y.x);
     }
 #pragma unroll
-    for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+    for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[jo + R2 * m]);
 #pragma unroll
     for (int m = HP; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    blue_convolve<M>(v, jo, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
     SyncWave{}();
+    const unsigned lo = (unsigned)(o - o0);
 #pragma unroll
     for (int m = 0; m < HP; ++m) {
-      const float2 r = cmul(v[m], cl[j + R2 * m]);
-      const float c0 = r.x * sc, c1 = r.y * sc;
+      const float2 r = cmul(v[m], cl[jo + R2 * m]);
+      const float c0 = r.x * so.x, c1 = r.y * so.x;
       if (c0 > bv[0][m]) {
         bv[0][m] = c0;
-        bi[0][m] = angle0 + o;
+        bi[m] = (bi[m] & 0xffff0000u) | lo;
       }
       if (c1 > bv[1][m]) {
         bv[1][m] = c1;
-        bi[1][m] = angle0 + o;
+        bi[m] = (bi[m] & NONE) | lo << 16;
       }
     }
   }
@@ -1373,11 +1358,277 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(const
     const int p = j + R2 * m;
     if (p >= n) continue;
     const size_t i = (size_t)row * n + p;
-    best[i] = bv[0][m];
-    bidx[i] = bi[0][m];
-    if (two) {
+    const unsigned a = bi[m] & NONE, b = bi[m] >> 16;
+    if (FRESH || a != NONE) {
+      best[i] = bv[0][m];
+      bidx[i] = a == NONE ? -1 : angle0 + o0 + (int)a;
+    }
+    if (two && (FRESH || b != NONE)) {
       best[i + n] = bv[1][m];
-      bidx[i + n] = bi[1][m];
+      bidx[i + n] = b == NONE ? -1 : angle0 + o0 + (int)b;
+    }
+  }
+}
+
+// The same, not scaled, on rows with a native transform.
+template <int N, bool FRESH>
+__global__ __launch_bounds__(256) void k_rows_max(const float2* __restrict__ G, long long H, int nb, int nrows,
+                                                  int angle0, float* __restrict__ best, int32_t* __restrict__ bidx,
+                                                  int og, const float2* __restrict__ tw) {
+  constexpr int NC = N / 2, NH = NC + 1;
+  constexpr int R1 = RowShape<NC>::R1, R2 = RowShape<NC>::R2, RW = 256 / R2;
+  constexpr int GS = R2 * (R1 + 1);
+  __shared__ float2 area[R2 > 1 ? RW * GS : 1];
+  __shared__ float2 twl[N];
+  const int t = threadIdx.x, r = t / R2, j = t % R2;
+  for (int i = t; i < N; i += 256) twl[i] = twiddle<-1, N>(tw, i);
+  __syncthreads();
+  const int row = blockIdx.x * RW + r;
+  if (row >= nrows) return;  // no barrier below: a row's R2 threads are lanes of one wave
+  int o0 = 0, o1 = nb;
+  if (FRESH) {
+    o0 = og * (int)blockIdx.y;
+    o1 = min(nb, o0 + og);
+    best += (size_t)blockIdx.y * nrows * N;
+    bidx += (size_t)blockIdx.y * nrows * N;
+  }
+  float2* bp = reinterpret_cast<float2*>(best + (size_t)row * N);
+  int2* ip = reinterpret_cast<int2*>(bidx + (size_t)row * N);
+  float bv[2 * R1];
+  int32_t bi[2 * R1];
+#pragma unroll
+  for (int q = 0; q < R1; ++q) {
+    const int m = out_index<R1, R2>(j, q);
+    const float2 b = FRESH ? make_float2(-__builtin_inff(), -__builtin_inff()) : bp[m];
+    const int2 a = FRESH ? make_int2(-1, -1) : ip[m];
+    bv[2 * q] = b.x;
+    bv[2 * q + 1] = b.y;
+    bi[2 * q] = a.x;
+    bi[2 * q + 1] = a.y;
+  }
+  for (int o = o0; o < o1; ++o) {
+    const float2* X = G + o * H + (long long)row * NH;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1; ++m) {
+      const int k = j + R2 * m;
+      float2 a = X[k], b = X[NC - k];
+      if (k == 0) a.y = b.y = 0.f;
+      const float2 bc = cconj(b);
+      v[m] = cadd(cadd(a, bc), mul_pj<1>(cmul(cconj(twl[k]), csub(a, bc))));
+    }
+    fft_two_step<NC, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &area[r * GS + jj * (R1 + 1) + k1]; },
+                                TwiddleLDSHalf{}, SyncWave{});
+    SyncWave{}();
+    const int32_t oi = angle0 + o;
+#pragma unroll
+    for (int q = 0; q < R1; ++q) {
+      const float c0 = v[q].x, c1 = v[q].y;
+      if (c0 > bv[2 * q]) {
+        bv[2 * q] = c0;
+        bi[2 * q] = oi;
+      }
+      if (c1 > bv[2 * q + 1]) {
+        bv[2 * q + 1] = c1;
+        bi[2 * q + 1] = oi;
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R1; ++q) {
+    const int m = out_index<R1, R2>(j, q);
+    bp[m] = make_float2(bv[2 * q], bv[2 * q + 1]);
+    ip[m] = make_int2(bi[2 * q], bi[2 * q + 1]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The correlation of a small volume, zero-padded, with an image's spectrum
+// (the Picker): forward transforms that read only the small volume's lines, and
+// the z forward transform, the product with the image and the z inverse in one
+// kernel, which writes the spectrum once where the separate passes moved it
+// through memory seven times. Spectra of orientation o: the small volume's rows
+// [n0z][n0y][nh], after y [n0z][ny][nh], after the product [nz][ny][nh].
+// ---------------------------------------------------------------------------
+// The y transform of a padded axis: plane pl's n0 lines become n lines.
+template <int N>
+__global__ __launch_bounds__(fft_col_tx<N>() * ColShape<N>::R2) void k_cols_pad(
+    const float2* __restrict__ src, float2* __restrict__ dst, int width, int nplanes, PadMap pm,
+    const float2* __restrict__ tw) {
+  constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = fft_col_tx<N>();
+  __shared__ float2 xch[R2 > 1 ? TX * N : 1];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  const int col = blockIdx.x * TX + c;
+  const bool valid = col < width;
+  for (int pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
+    const float2* s = src + (size_t)pl * pm.n0 * width + col;
+    float2* d = dst + (size_t)pl * N * width + col;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1; ++m) {
+      const int q = pm.at(j + R2 * m, N);
+      v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    fft_two_step<N, R1, R2, -1>(v, j, tw, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; });
+    if (valid) {
+#pragma unroll
+      for (int q = 0; q < R1; ++q) d[(size_t)out_index<R1, R2>(j, q) * width] = v[q];
+    }
+  }
+}
+
+template <int M>
+__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols_pad(
+    const float2* __restrict__ src, float2* __restrict__ dst, int width, int nplanes, PadMap pm, int L,
+    const float2* __restrict__ chirp, const float2* __restrict__ B, const float2* __restrict__ tw) {
+  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
+  __shared__ float2 xch[TX * M];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
+  const int col = blockIdx.x * TX + c;
+  const bool valid = col < width;
+  for (int pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
+    const float2* s = src + (size_t)pl * pm.n0 * width + col;
+    float2* d = dst + (size_t)pl * L * width + col;
+    float2 v[R1];
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m, q = p < L ? pm.at(p, L) : -1;
+      v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      if (valid && p < L) d[(size_t)p * width] = cmul(v[m], cl[p]);
+    }
+  }
+}
+
+// E * conj((P - dc) / sd) at one bin: the padded volume's mean0/std1 in Fourier
+// space (norm[0] = mean * elements, taken off the DC bin alone, norm[1] = 1 / sd).
+__device__ __forceinline__ float2 image_times_ref(float2 e, float2 p, float dc, float inv_sd) {
+  p = make_float2((p.x - dc) * inv_sd, p.y * inv_sd);
+  return cmulc(e, p);
+}
+
+// Forward z of the padded axis, the product and the inverse z, for orientation
+// blockIdx.y: the forward transform ends with every k2 of a k1 in one thread,
+// where the inverse starts, as in blue_convolve.
+template <int N>
+__global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_cols_correlate(
+    const float2* __restrict__ src, const float2* __restrict__ E, float2* __restrict__ dst, int width, PadMap pm,
+    const float2* __restrict__ norm, const float2* __restrict__ tw) {
+  constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = ColShape<N>::TX, NT = TX * R2;
+  __shared__ float2 xch[R2 > 1 ? TX * N : 1];
+  __shared__ float2 twl[N];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  for (int i = t; i < N; i += NT) twl[i] = twiddle<-1, N>(tw, i);
+  const int col = blockIdx.x * TX + c, o = blockIdx.y;
+  const bool valid = col < width;
+  const float2* s = src + (size_t)o * pm.n0 * width + col;
+  const float2* e = E + col;
+  float2* d = dst + (size_t)o * N * width + col;
+  const float2 nm = norm[o];
+  float2 v[R1];
+#pragma unroll
+  for (int m = 0; m < R1; ++m) {
+    const int q = pm.at(j + R2 * m, N);
+    v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  dft<R1, -1>(v);
+  if constexpr (R2 == 1) {
+#pragma unroll
+    for (int k = 0; k < R1; ++k)
+      v[k] = image_times_ref(valid ? e[(size_t)k * width] : make_float2(0.f, 0.f), v[k], k == 0 && col == 0 ? nm.x : 0.f,
+                             nm.y);
+  } else {
+    auto at = [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; };
+#pragma unroll
+    for (int k1 = 0; k1 < R1; ++k1) *at(k1, j) = k1 == 0 ? v[k1] : cmul(v[k1], twl[j * k1 % N]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < R1 / R2; ++u) {
+      const int k1 = j * (R1 / R2) + u;
+      float2 z[R2];
+#pragma unroll
+      for (int jj = 0; jj < R2; ++jj) z[jj] = *at(k1, jj);
+      dft<R2, -1>(z);
+#pragma unroll
+      for (int k2 = 0; k2 < R2; ++k2) {
+        const int k = k1 + R1 * k2;
+        z[k2] = image_times_ref(valid ? e[(size_t)k * width] : make_float2(0.f, 0.f), z[k2],
+                                k == 0 && col == 0 ? nm.x : 0.f, nm.y);
+      }
+      dft<R2, 1>(z);
+#pragma unroll
+      for (int jj = 0; jj < R2; ++jj) *at(k1, jj) = jj == 0 ? z[jj] : cmulc(z[jj], twl[jj * k1 % N]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k1 = 0; k1 < R1; ++k1) v[k1] = *at(k1, j);
+  }
+  dft<R1, 1>(v);
+  if (valid) {
+#pragma unroll
+    for (int m = 0; m < R1; ++m) d[(size_t)(j + R2 * m) * width] = v[m];
+  }
+}
+
+template <int M>
+__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols_correlate(
+    const float2* __restrict__ src, const float2* __restrict__ E, float2* __restrict__ dst, int width, PadMap pm,
+    const float2* __restrict__ norm, int L, const float2* __restrict__ chirp, const float2* __restrict__ B,
+    const float2* __restrict__ tw) {
+  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
+  __shared__ float2 xch[TX * M];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
+  const int col = blockIdx.x * TX + c, o = blockIdx.y;
+  const bool valid = col < width;
+  const float2* s = src + (size_t)o * pm.n0 * width + col;
+  const float2* e = E + col;
+  float2* d = dst + (size_t)o * L * width + col;
+  const float2 nm = norm[o];
+  auto at = [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; };
+  float2 v[R1];
+#pragma unroll
+  for (int m = 0; m < R1 / 2; ++m) {
+    const int p = j + R2 * m, q = p < L ? pm.at(p, L) : -1;
+    v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
+#pragma unroll
+  for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+  blue_convolve<M>(v, j, twl, bl, at, SyncGroup{});
+#pragma unroll
+  for (int m = 0; m < R1 / 2; ++m) {
+    const int p = j + R2 * m;
+    const float2 ch = cl[p];  // 0 past the line
+    const float2 q = image_times_ref(valid && p < L ? e[(size_t)p * width] : make_float2(0.f, 0.f), cmul(v[m], ch),
+                                     p == 0 && col == 0 ? nm.x : 0.f, nm.y);
+    v[m] = cmulc(q, ch);
+  }
+#pragma unroll
+  for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+  __syncthreads();  // the first convolution's exchange is read
+  blue_convolve<M, true>(v, j, twl, bl, at, SyncGroup{});
+  if (valid) {
+#pragma unroll
+    for (int m = 0; m < R1 / 2; ++m) {
+      const int p = j + R2 * m;
+      if (p < L) d[(size_t)p * width] = cmulc(v[m], cl[p]);
     }
   }
 }
@@ -1523,15 +1774,7 @@ __global__ __launch_bounds__(256) void k_blue_store_rows(const float2* __restric
   }
 }
 
-// Chirp and kernel spectra of one length, per device, computed once in long
-// double: chirp[j] = exp(-i pi (j^2 mod 2L) / L), bf / bi = the M-point DFTs
-// of the forward / inverse convolution kernels, divided by M.
-struct BlueTables {
-  int M = 0;
-  float2* chirp = nullptr;
-  float2* bf = nullptr;
-  float2* bi = nullptr;
-};
+// The tables (BlueTables) of one length, per device, computed once in long double.
 std::mutex g_blue_mu;
 std::map<std::pair<int, int>, BlueTables> g_blue;
 
@@ -1614,22 +1857,10 @@ int blue_tables(int L, BlueTables* out) {
 
 unsigned blue_grid(long long n) { return (unsigned)std::max<long long>(1, std::min<long long>((n + 255) / 256, 65536)); }
 
-// f(integral_constant M) for the fused form's length M.
-template <class F> int with_blue_len(int M, F f) {
-  switch (M) {
-#define GX_CASE(N) \
-  case N:          \
-    return f(std::integral_constant<int, N>{});
-    GX_FOR_BLUE(GX_CASE)
-#undef GX_CASE
-    default: return fail(GTOMX_ERR_INTERNAL, "chirp-z length not instantiated");
-  }
-}
-
 // The fused form on a strided axis, from src into dst (which may be src).
 template <int DIR>
 int blue_cols(int L, const float2* src, float2* dst, int width, long long as, long long nplanes, long long P1,
-              long long S0, long long S1, hipStream_t s) {
+              long long S0, long long S1, hipStream_t s, int half = 0) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   BlueTables t;
@@ -1641,14 +1872,14 @@ int blue_cols(int L, const float2* src, float2* dst, int width, long long as, lo
     // enough workgroups to fill the device several times over, and several planes each to share the staged tables
     const long long gy = std::min<long long>(nplanes, std::max<long long>(1, 8192 / gx));
     hipLaunchKernelGGL((k_blue_cols<M, DIR>), dim3(gx, (unsigned)gy), dim3(S::TX * S::R2), 0, s, src, dst, width, as,
-                       nplanes, P1, S0, S1, L, t.chirp, DIR < 0 ? t.bf : t.bi, tw);
+                       nplanes, P1, S0, S1, L, t.chirp, DIR < 0 ? t.bf : t.bi, tw, half);
     GX_LAUNCHED("k_blue_cols");
     return GTOMX_OK;
   });
 }
 
 // The fused form on nrows contiguous rows of L reals / L/2 + 1 bins.
-int blue_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s) {
+int blue_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s, PadMap pm = PadMap{}) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   BlueTables t;
@@ -1657,7 +1888,7 @@ int blue_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStrea
     constexpr int M = decltype(MC)::value;
     const long long wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
     hipLaunchKernelGGL(k_blue_rows_r2c<M>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), 0, s, in, out,
-                       nrows, L, t.chirp, t.bf, tw);
+                       nrows, L, t.chirp, t.bf, tw, pm);
     GX_LAUNCHED("k_blue_rows_r2c");
     return GTOMX_OK;
   });
@@ -1679,40 +1910,165 @@ int blue_rows_c2r(int L, const float2* in, float* out, long long nrows, float sc
 
 bool rows_max_any_fused(int n) { return n <= BLUE_FUSED_MAX; }
 
-int rows_max_any_groups(int n, unsigned batch, int cus) {
-  const int M = blue_fused_len(n);
-  int wgs = 0, per_cu = 1;
-  const int st = with_blue_len(M, [&](auto MC) -> int {
-    constexpr int N = decltype(MC)::value;
-    wgs = (n * n + 2 * BlueRows<N>::TP - 1) / (2 * BlueRows<N>::TP);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_blue_rows_max<N, true>, 256, 0) != hipSuccess ||
-        per_cu < 1)
-      per_cu = 1;
-    return GTOMX_OK;
-  });
-  if (st != GTOMX_OK || wgs < 1) return 1;
-  return std::max(1, std::min((int)batch, per_cu * cus / wgs));
-}
-
-int rows_max_any(int n, const float2* G, long long H, int nb, int angle0, const float* scale, float* best,
+int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
                  int32_t* idx, int og, hipStream_t s) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
+  const int groups = og > 0 ? (nb + og - 1) / og : 1;
+  if (nb > 0xffff) return fail(GTOMX_ERR_INTERNAL, "row pass over more than 65535 orientations");
+  if (!sn && fft_len_ok(n)) {
+    switch (n) {
+#define GX_CASE(N)                                                                                              \
+  case N: {                                                                                                     \
+    const unsigned wgs = (unsigned)((nrows + rows_per_block<N>() - 1) / rows_per_block<N>());                   \
+    if (groups == 1)                                                                                            \
+      hipLaunchKernelGGL((k_rows_max<N, false>), dim3(wgs, 1), dim3(256), 0, s, G, H, nb, nrows, angle0, best,  \
+                         idx, og, tw);                                                                          \
+    else                                                                                                        \
+      hipLaunchKernelGGL((k_rows_max<N, true>), dim3(wgs, groups), dim3(256), 0, s, G, H, nb, nrows, angle0,    \
+                         best, idx, og, tw);                                                                    \
+    GX_LAUNCHED("k_rows_max");                                                                                  \
+    return GTOMX_OK;                                                                                            \
+  }
+      GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+    }
+  }
   BlueTables t;
   GX_TRY(blue_tables(n, &t));
   return with_blue_len(t.M, [&](auto MC) -> int {
     constexpr int M = decltype(MC)::value;
-    const int nrows = n * n, wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
-    const int groups = og > 0 ? (nb + og - 1) / og : 1;
-    if (groups == 1)
-      hipLaunchKernelGGL((k_blue_rows_max<M, false>), dim3(wgs, 1), dim3(256), 0, s, G, H, nb, n, nrows, angle0, scale,
-                         best, idx, og, t.chirp, t.bi, tw);
-    else
-      hipLaunchKernelGGL((k_blue_rows_max<M, true>), dim3(wgs, groups), dim3(256), 0, s, G, H, nb, n, nrows, angle0,
-                         scale, best, idx, og, t.chirp, t.bi, tw);
-    GX_LAUNCHED("k_blue_rows_max");
-    return GTOMX_OK;
+    const int wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
+    auto go = [&](auto kernel) -> int {
+      hipLaunchKernelGGL(kernel, dim3(wgs, groups), dim3(256), 0, s, G, H, nb, n, nrows, angle0, sn, best, idx, og,
+                         t.chirp, t.bi, tw);
+      GX_LAUNCHED("k_blue_rows_max");
+      return GTOMX_OK;
+    };
+    if (sn) return groups == 1 ? go(k_blue_rows_max<M, false, true>) : go(k_blue_rows_max<M, true, true>);
+    return groups == 1 ? go(k_blue_rows_max<M, false, false>) : go(k_blue_rows_max<M, true, false>);
   });
+}
+
+int blue_search_y(int n, float2* G, int nb, hipStream_t s) {
+  const int nc = (n + 1) / 2;
+  return blue_cols<1>(n, G, G, nc, nc, (long long)n * nb, 1LL << 62, (long long)nc * n, 0, s, n / 2);
+}
+
+// Two workgroups of 256 threads per CU fill the device; more groups cost more merging.
+int rows_max_any_groups(int n, int nrows, unsigned batch, int cus) {
+  int wgs = 1;
+  if (fft_len_ok(n)) {
+    const int rw = rows_per_workgroup(n);
+    wgs = (nrows + rw - 1) / rw;
+  } else {
+    const int st = with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
+      constexpr int per = 2 * BlueRows<decltype(MC)::value>::TP;
+      wgs = (nrows + per - 1) / per;
+      return GTOMX_OK;
+    });
+    if (st != GTOMX_OK) return 1;
+  }
+  return std::max(1, std::min((int)batch, 2 * cus / std::max(1, wgs)));
+}
+
+namespace {
+// d_FFTFullPad's placement of n0 points in FFT order within n (src/FFT/FFTResize.cu:212-238).
+PadMap pad_map(int n0, int n) {
+  PadMap pm;
+  pm.n0 = n0;
+  pm.c = n0 - (n / 2 + (n0 - n - ((n0 & (1 - (n & 1))) % 2)) / 2);
+  return pm;
+}
+bool padded_axis_ok(int n) { return fft_len_ok(n) || (n >= 2 && n <= BLUE_FUSED_MAX); }
+}  // namespace
+
+bool correlate_padded_ok(gtomx_int3 dr, gtomx_int3 di) {
+  auto ok = [](int n0, int n) {
+    const PadMap pm = pad_map(n0, n);
+    return padded_axis_ok(n) && n0 >= 1 && n0 <= n && pm.c >= 1 && pm.c <= n0;
+  };
+  return di.z > 1 && ok(dr.x, di.x) && ok(dr.y, di.y) && ok(dr.z, di.z);
+}
+
+int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, const float2* E, float2* out,
+                     gtomx_int3 di, unsigned nb, const float2* norm, hipStream_t s) {
+  const float2* tw = nullptr;
+  GX_TRY(twiddles(&tw));
+  const int nh = di.x / 2 + 1;
+  // x: the small volume's rows
+  const long long nrows = (long long)dr.y * dr.z * nb;
+  const PadMap px = pad_map(dr.x, di.x), py = pad_map(dr.y, di.y), pz = pad_map(dr.z, di.z);
+  if (fft_len_ok(di.x)) {
+    switch (di.x) {
+#define GX_CASE(N)                                                                                              \
+  case N:                                                                                                       \
+    hipLaunchKernelGGL((k_rows_r2c<N, true>), dim3((unsigned)((nrows + rows_per_block<N>() - 1) /               \
+                                                              rows_per_block<N>())),                            \
+                       dim3(256), 0, s, r, rows, nrows, tw, RowBand{}, px);                                     \
+    break;
+      GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+    }
+    GX_LAUNCHED("k_rows_r2c");
+  } else {
+    GX_TRY(blue_rows_r2c(di.x, r, rows, nrows, s, px));
+  }
+  // y: every plane of the small volume
+  const int planes = (int)(dr.z * nb);
+  if (fft_len_ok(di.y)) {
+    switch (di.y) {
+#define GX_CASE(N)                                                                                                \
+  case N:                                                                                                         \
+    hipLaunchKernelGGL(k_cols_pad<N>, dim3((nh + fft_col_tx<N>() - 1) / fft_col_tx<N>(), std::min(planes, 65535)), \
+                       dim3(fft_col_tx<N>() * ColShape<N>::R2), 0, s, rows, cols, nh, planes, py, tw);            \
+    break;
+      GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+    }
+    GX_LAUNCHED("k_cols_pad");
+  } else {
+    BlueTables t;
+    GX_TRY(blue_tables(di.y, &t));
+    GX_TRY(with_blue_len(t.M, [&](auto MC) -> int {
+      constexpr int M = decltype(MC)::value;
+      using S = BlueShape<M>;
+      const int gx = (nh + S::TX - 1) / S::TX;
+      hipLaunchKernelGGL(k_blue_cols_pad<M>, dim3(gx, std::min(planes, std::max(1, 8192 / gx))), dim3(S::TX * S::R2), 0,
+                         s, rows, cols, nh, planes, py, di.y, t.chirp, t.bf, tw);
+      GX_LAUNCHED("k_blue_cols_pad");
+      return GTOMX_OK;
+    }));
+  }
+  // z, the product, z back
+  const int width = nh * di.y;
+  if (fft_len_ok(di.z)) {
+    switch (di.z) {
+#define GX_CASE(N)                                                                                         \
+  case N:                                                                                                  \
+    hipLaunchKernelGGL(k_cols_correlate<N>, dim3((width + ColShape<N>::TX - 1) / ColShape<N>::TX, nb),     \
+                       dim3(ColShape<N>::TX * ColShape<N>::R2), 0, s, cols, E, out, width, pz, norm, tw);  \
+    break;
+      GX_FOR_SIZES(GX_CASE)
+#undef GX_CASE
+    }
+    GX_LAUNCHED("k_cols_correlate");
+  } else {
+    BlueTables t;
+    GX_TRY(blue_tables(di.z, &t));
+    GX_TRY(with_blue_len(t.M, [&](auto MC) -> int {
+      constexpr int M = decltype(MC)::value;
+      using S = BlueShape<M>;
+      hipLaunchKernelGGL(k_blue_cols_correlate<M>, dim3((width + S::TX - 1) / S::TX, nb), dim3(S::TX * S::R2), 0, s,
+                         cols, E, out, width, pz, norm, di.z, t.chirp, t.bf, tw);
+      GX_LAUNCHED("k_blue_cols_correlate");
+      return GTOMX_OK;
+    }));
+  }
+  // y back
+  if (fft_len_ok(di.y))
+    return launch_cols_n<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, tw, s);
+  return blue_cols<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, s);
 }
 
 // One axis of nlines lines of length L by the chirp-z form: IN / OUT are the

@@ -27,6 +27,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "dev_blue.hpp"
 #include "dev_fft.hpp"
 #include "dev_project.hpp"
 #include "pick_plan.hpp"
@@ -654,37 +655,43 @@ __global__ __launch_bounds__(PlaneShape<N>::T * PlaneShape<N>::PL) void k_pick_p
   const int gbase = ((z * N + j) * L::PITCH + c) * 8;
   for (int o = o0; o < o1; ++o) {
     const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + (size_t)o * L::STRIDE, (unsigned)(L::STRIDE * 8));
+    // with 24 points a thread opaque per orientation: what follows from them alone (disc tests, LDS
+    // addresses) is recomputed rather than held in registers (96: 255 instead of 276, two waves a SIMD
+    // instead of one, 8 volumes x 288 orientations 12.4 -> 10.1 ms); with fewer points it only costs
+    // (128: 2.26 -> 2.49 ms per 288 orientations, 64: 0.69 -> 0.71 per 588)
+    int jo = j, jxo = jx;
+    if constexpr (R1 > 16) asm volatile("" : "+v"(jo), "+v"(jxo));
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1; ++m) {
       // bins of columns outside the disc were not written by pass 1 and are zero
-      const int voff = column_in_disc<N>(c, signed_freq(j + R2 * m, N)) ? gbase : OUT_OF_RANGE;
+      const int voff = column_in_disc<N>(c, signed_freq(jo + R2 * m, N)) ? gbase : OUT_OF_RANGE;
       v[m] = buf_load2(rG, voff, m * R2 * L::PITCH * 8);
     }
     const float sc = sn[o].x, xn = sn[o].y;
     __syncthreads();  // the last orientation's rows are done (and, the first time, the twiddles staged)
-    fft_two_step<N, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * NC + c]; },
+    fft_two_step<N, R1, R2, 1>(v, jo, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * NC + c]; },
                                TwiddleLDS{});
     __syncthreads();
 #pragma unroll
-    for (int s = 0; s < R1; ++s) xch[out_index<R1, R2>(j, s) * NCP + c] = v[s];
+    for (int s = 0; s < R1; ++s) xch[out_index<R1, R2>(jo, s) * NCP + c] = v[s];
     __syncthreads();
     // row C2R as in k_pick_x_max; from here on a row belongs to XR2 lanes of one wave
 #pragma unroll
     for (int m = 0; m < R1; ++m) {
-      const int k = jx + XR2 * m;
+      const int k = jxo + XR2 * m;
       const float2 a = xch[r * NCP + k];
-      float2 b = xch[r * NCP + (m == 0 && jx == 0 ? 0 : NC - k)];
+      float2 b = xch[r * NCP + (m == 0 && jxo == 0 ? 0 : NC - k)];
       if (m == 0) {  // X[n/2] for k = 0, without a branch around the load
-        b.x = __builtin_unpredictable(jx == 0) ? xn : b.x;
-        b.y = __builtin_unpredictable(jx == 0) ? 0.f : b.y;
+        b.x = __builtin_unpredictable(jxo == 0) ? xn : b.x;
+        b.y = __builtin_unpredictable(jxo == 0) ? 0.f : b.y;
       }
       const float2 a0 = k == 0 ? make_float2(a.x, 0.f) : a;
       const float2 bc = cconj(b);
       v[m] = cadd(cadd(a0, bc), mul_pj<1>(cmul(cconj(twl[k]), csub(a0, bc))));
     }
     SyncWave{}();
-    fft_two_step<NC, R1, XR2, 1>(v, jx, twl, [&](int k1, int jj) { return &xch[r * NCP + jj * (R1 + 1) + k1]; },
+    fft_two_step<NC, R1, XR2, 1>(v, jxo, twl, [&](int k1, int jj) { return &xch[r * NCP + jj * (R1 + 1) + k1]; },
                                  TwiddleLDSHalf{}, SyncWave{});
     const int32_t oi = angle0 + o;
 #pragma unroll
@@ -913,11 +920,11 @@ __global__ __launch_bounds__(256) void k_pick2d_norm(Projector P, const float* _
   if (t == 0) sn[slot].x = (float)(1.0 / fmax(sqrt((red[0] + red[1] + red[2] + red[3]) / (double)H), 1e-20));
 }
 
-// scale[o] = 1/max(sqrt((sum of partial sums + corrections)/H), 1e-20) in double
+// scale[o * step] = 1/max(sqrt((sum of partial sums + corrections)/H), 1e-20) in double
 // (src/ImageManipulation/Norm.cu:476-509).
 __global__ __launch_bounds__(256) void k_pick_scale(const float* __restrict__ partial, int nparts,
                                                    const float* __restrict__ corr, int ncorr, double h,
-                                                   float* __restrict__ scale) {
+                                                   float* __restrict__ scale, int step = 1) {
   __shared__ double red[256];
   const int o = blockIdx.x, t = threadIdx.x;
   double sum = 0;
@@ -929,7 +936,7 @@ __global__ __launch_bounds__(256) void k_pick_scale(const float* __restrict__ pa
     if (t < w) red[t] += red[t + w];
     __syncthreads();
   }
-  if (t == 0) scale[o] = (float)(1.0 / fmax(sqrt(red[0] / h), 1e-20));
+  if (t == 0) scale[o * step] = (float)(1.0 / fmax(sqrt(red[0] / h), 1e-20));
 }
 
 // ---------------------------------------------------------------------------
@@ -1058,11 +1065,121 @@ __global__ __launch_bounds__(256) void k_pick3d_project_any(PJ P, const float* _
   }
 }
 
+// ---------------------------------------------------------------------------
+// Pass 1 of the sides up to 512 without a native transform: k_pick_project_z with
+// the z inverse by the chirp-z form. Columns (x, y), x < (n + 1) / 2, are numbered
+// y * nc + x, as G's planes hold them; a tile is TX consecutive ones, tiles[] those
+// with a column inside the disc. (The x = n/2 column of even n is one bin, as in
+// GLayout.) Projecting into a whole half spectrum first and transforming it in
+// place moved it through memory twice more (200^3: 0.41 ms each per 32
+// orientations).
+// ---------------------------------------------------------------------------
+template <int M> constexpr int blue_threads() { return BlueShape<M>::TX * BlueShape<M>::R2; }
+
+template <int M, class PJ>
+__global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
+    PJ P, const float* __restrict__ mats, int nb, const float2* __restrict__ E, const float* __restrict__ ctf,
+    float2* __restrict__ G, float* __restrict__ partial, int n, const int* __restrict__ tiles, int ntiles,
+    const float2* __restrict__ chirp, const float2* __restrict__ B, const float2* __restrict__ tw) {
+  using S = BlueShape<M>;
+  constexpr int R1 = S::R1, R2 = S::R2, TX = S::TX, NT = TX * R2, HP = R1 / 2, WAVES = (NT + 63) / 64;
+  __shared__ float2 xch[TX * M];
+  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  blue_stage<M, 1>(t, NT, n, tw, B, chirp, twl, bl, cl);
+  const int nh = n / 2 + 1, half = n / 2, nc = (n + 1) / 2;
+  const long long stride = (long long)nc * n * n;
+  const __amdgpu_buffer_rsrc_t rs = sampler_rsrc(P);
+  const unsigned HB = (unsigned)nh * n * n;
+  const __amdgpu_buffer_rsrc_t rE = make_rsrc(E, HB * 8u);
+  const __amdgpu_buffer_rsrc_t rC = make_rsrc(ctf, ctf ? HB * 4u : 0u);
+  const long long items = (long long)ntiles * nb;
+  const long long i1 = items * (blockIdx.x + 1) / gridDim.x;
+  for (long long it = items * blockIdx.x / gridDim.x; it < i1;) {
+    const int ti = (int)(it / nb);
+    const int o0 = (int)(it % nb);
+    const int o1 = (int)min((long long)nb, o0 + (i1 - it));
+    it += o1 - o0;
+    const int col = tiles[ti] * TX + c;
+    const int ix = col % nc, iy = col / nc;
+    const int y = signed_freq(iy, n);
+    const bool valid = iy < n && ix * ix + y * y <= half * half;
+    float2 e[HP];
+    float cf[HP];
+    // element (x, y, p) at (p * n + y) * nh + x: points p >= n lie past the buffers' ends, where loads give
+    // 0 and stores are dropped, as the out-of-range lanes of invalid columns
+    const int bin = (j * n + iy) * nh + ix;
+    auto load_bin = [&](int m) {
+      e[m] = buf_load2(rE, valid ? bin * 8 : OUT_OF_RANGE, m * R2 * n * nh * 8);
+      cf[m] = ctf ? buf_load1(rC, valid ? bin * 4 : OUT_OF_RANGE, m * R2 * n * nh * 4) : 1.f;
+    };
+    const int gout = valid ? (j * nc * n + col) * 8 : OUT_OF_RANGE;
+#pragma unroll
+    for (int m = 0; m < HP; ++m) load_bin(m);
+    const bool dc = col == 0 && j == 0;
+    for (int o = o0; o < o1; ++o) {
+      float Mo[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) Mo[k] = mats[9 * o + k];
+      const float qx = Mo[0] * ix + Mo[1] * y, qy = Mo[3] * ix + Mo[4] * y, qz = Mo[6] * ix + Mo[7] * y;
+      float acc = 0.f;
+      float2 v[R1];
+      // opaque per orientation: what follows from it alone is recomputed rather than held in registers
+      int jo = j;
+      asm volatile("" : "+v"(jo));
+      // samples two at a time, as in k_pick_project_z: the barrier keeps later gathers from being hoisted
+#pragma unroll
+      for (int m0 = 0; m0 < HP; m0 += 2) {
+#pragma unroll
+        for (int m = m0; m < m0 + 2; ++m) {
+          const int p = jo + R2 * m, z = signed_freq(p, n);
+          const bool in = valid && p < n && ix * ix + y * y + z * z <= half * half;
+          if (__any(in)) {
+            const float fz = (float)z;
+            const float2 r =
+                cscale(sample(rs, P, fmaf(Mo[2], fz, qx), fmaf(Mo[5], fz, qy), fmaf(Mo[8], fz, qz), in), cf[m]);
+            acc += r.x * r.x + r.y * r.y;
+            v[m] = cmulc(e[m], r);
+          } else {
+            v[m] = make_float2(0.f, 0.f);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (dc) v[0] = make_float2(0.f, 0.f);  // its |R|^2 is removed by k_pick_herm_norm
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[jo + R2 * m]);
+#pragma unroll
+      for (int m = HP; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
+      blue_convolve<M>(v, jo, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
+      const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + o * stride, (unsigned)stride * 8u);
+#pragma unroll
+      for (int m = 0; m < HP; ++m) {
+        const u32x2 w = __builtin_bit_cast(u32x2, cmul(v[m], cl[jo + R2 * m]));
+        __builtin_amdgcn_raw_buffer_store_b64(w, rG, gout, m * R2 * nc * n * 8, CPOL_NT);
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+      if ((t & 63) == 0) partial[((size_t)o * ntiles + ti) * WAVES + (t >> 6)] = acc;
+    }
+  }
+}
+
 }  // namespace gx
 
 // The plan (struct gtomx_pick_plan) is declared in pick_plan.hpp.
 
 namespace gx {
+
+int merge_group_maxima(const float* gbest, const int32_t* gidx, int groups, size_t v, float* best, int32_t* idx,
+                       unsigned items, hipStream_t s) {
+  hipLaunchKernelGGL(k_pick_merge, dim3((unsigned)((v + 63) / 64), items), dim3(256), 0, s, gbest, gidx, groups, v,
+                     best, idx);
+  GX_LAUNCHED("k_pick_merge");
+  return GTOMX_OK;
+}
+
 namespace {
 
 // Images of one launch of the fused 2D passes: with 4 the samples cost a quarter,
@@ -1214,10 +1331,7 @@ int plane_groups_for(int n, unsigned batch, int cus) {
 }
 
 int merge_groups(gtomx_pick_plan* pl, int groups, float* best, int32_t* idx, hipStream_t s, unsigned items = 1) {
-  hipLaunchKernelGGL(k_pick_merge, dim3((unsigned)((pl->V + 63) / 64), items), dim3(256), 0, s, pl->gbest, pl->gidx, groups,
-                     pl->V, best, idx);
-  GX_LAUNCHED("k_pick_merge");
-  return GTOMX_OK;
+  return merge_group_maxima(pl->gbest, pl->gidx, groups, pl->V, best, idx, items, s);
 }
 
 template <int N, class PJ>
@@ -1323,6 +1437,78 @@ __global__ __launch_bounds__(256) void k_pick_max_maps(const float* __restrict__
   }
 }
 
+// Column tiles of k_pick_project_blue that hold a column inside the disc.
+std::vector<int> blue_tiles(int n) {
+  std::vector<int> out;
+  const int nc = (n + 1) / 2, half = n / 2;
+  (void)with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
+    constexpr int TX = BlueShape<decltype(MC)::value>::TX;
+    for (int w = 0; w * TX < nc * n; ++w) {
+      bool in = false;
+      for (int col = w * TX; col < std::min((w + 1) * TX, nc * n); ++col) {
+        const int x = col % nc, iy = col / nc, y = iy <= half ? iy : iy - n;
+        in |= x * x + y * y <= half * half;
+      }
+      if (in) out.push_back(w);
+    }
+    return GTOMX_OK;
+  });
+  return out;
+}
+
+// Resident workgroups of k_pick_project_blue on the whole device.
+int blue_grid1(int n, bool centred, int cus) {
+  int per_cu = 1;
+  (void)with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
+    constexpr int M = decltype(MC)::value, NT = blue_threads<M>();
+    const hipError_t e =
+        centred ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_blue<M, CentredProjector>, NT, 0)
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_blue<M, Projector>, NT, 0);
+    if (e != hipSuccess || per_cu < 1) per_cu = 1;
+    return GTOMX_OK;
+  });
+  return per_cu * cus;
+}
+
+// Sides up to 512 without a native transform: project + chirp-z along z, the
+// correction and the scale, chirp-z along y in place, then the row pass per
+// orientation group and the in-order merge.
+template <class PJ>
+int run_batch_blue(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, const float2* E,
+                   const float* ctf, float* best, int32_t* idx, int angle0, const float2* tw, hipStream_t s) {
+  const int n = pl->n;
+  BlueTables t;
+  GX_TRY(blue_tables(n, &t));
+  GX_TRY(timed(pl, 0, s, [&]() -> int {
+    return with_blue_len(t.M, [&](auto MC) -> int {
+      constexpr int M = decltype(MC)::value;
+      hipLaunchKernelGGL((k_pick_project_blue<M, PJ>),
+                         dim3(pl->grid1[std::is_same<PJ, CentredProjector>::value ? 1 : 0]),
+                         dim3(blue_threads<M>()), 0, s, PS, mats, nb, E, ctf, pl->G, pl->partial, n,
+                         pl->tiles, pl->ntiles, t.chirp, t.bi, tw);
+      GX_LAUNCHED("k_pick_project_blue");
+      return GTOMX_OK;
+    });
+  }));
+  GX_TRY(timed(pl, 1, s, [&]() -> int {
+    hipLaunchKernelGGL(k_pick_herm_norm<0>, dim3(HERM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, pl->corr, n, E,
+                       pl->sn);
+    GX_LAUNCHED("k_pick_herm_norm");
+    hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, pl->nparts, pl->corr, HERM_BLOCKS,
+                       (double)pl->H, reinterpret_cast<float*>(pl->sn), 2);
+    GX_LAUNCHED("k_pick_scale");
+    return blue_search_y(n, pl->G, nb, s);
+  }));
+  return timed(pl, 2, s, [&]() -> int {
+    const long long stride = (long long)((n + 1) / 2) * n * n;
+    const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
+    const bool fresh = groups > 1;
+    GX_TRY(rows_max_any(n, n * n, pl->G, stride, nb, angle0, pl->sn, fresh ? pl->gbest : best, fresh ? pl->gidx : idx,
+                        og, s));
+    return fresh ? merge_groups(pl, groups, best, idx, s) : GTOMX_OK;
+  });
+}
+
 template <class PJ>
 int run_batch3d_any(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb,
                     const float2* E, const float* ctf, float* best, int32_t* idx, int angle0, hipStream_t s) {
@@ -1337,18 +1523,12 @@ int run_batch3d_any(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const
   GX_TRY(herm_norm3_any(n, P, mats, ctf, pl->corr, nb, s));
   GX_TRY(timed(pl, 1, s, [&]() -> int {
     hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, pl->nparts, pl->corr, HERM_BLOCKS,
-                       (double)pl->H, pl->scale);
+                       (double)pl->H, pl->scale, 1);
     GX_LAUNCHED("k_pick_scale");
     if (pl->gen3d) return yz_axes_any(pl->G, gtomx_int3{n, n, n}, (unsigned)nb, 1, s);
     return fft_c2r_cols_inplace(pl->G, gtomx_int3{n, n, n}, (unsigned)nb, s);
   }));
   return timed(pl, 2, s, [&]() -> int {
-    if (pl->gen3d && rows_max_any_fused(n)) {
-      const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
-      if (groups == 1) return rows_max_any(n, pl->G, H, nb, angle0, pl->scale, best, idx, nb, s);
-      GX_TRY(rows_max_any(n, pl->G, H, nb, angle0, pl->scale, pl->gbest, pl->gidx, og, s));
-      return merge_groups(pl, groups, best, idx, s);
-    }
     if (pl->gen3d) {
       // the rows' C2R into the first n^3 floats of each spectrum's slot, then the in-order update
       GX_TRY(rows_c2r_any_inplace(pl->G, n, nb, H, s));
@@ -1370,6 +1550,9 @@ int run_batch_n(gtomx_pick_plan* pl, const CentredProjector* C, const Projector&
                 hipStream_t s, const uint8_t* tmask = nullptr) {
   if (pl->n > 256 || pl->gen3d) {
     if (tmask) return fail(GTOMX_ERR_UNSUPPORTED, "tile masks need volumes of side 2^a or 3*2^a, at most 256");
+    if (pl->gen3d && rows_max_any_fused(pl->n))
+      return C ? run_batch_blue(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, tw, s)
+               : run_batch_blue(pl, P, P, mats, nb, E, ctf, best, idx, angle0, tw, s);
     return C ? run_batch3d_any(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, s)
              : run_batch3d_any(pl, P, P, mats, nb, E, ctf, best, idx, angle0, s);
   }
@@ -1484,7 +1667,7 @@ int run_batch2d_any(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const
   GX_TRY(herm_norm_any(n, P, mats, ctf, pl->corr, nb, s));
   GX_TRY(timed(pl, 1, s, [&]() -> int {
     hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, tiles * L2, pl->corr, 1, (double)pl->H,
-                       pl->scale);
+                       pl->scale, 1);
     GX_LAUNCHED("k_pick_scale");
     return GTOMX_OK;
   }));
@@ -1751,7 +1934,7 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   const bool big2d = is2d && dv.x > 256;  // micrographs: the generic-transform form of the 2D branch
   // volumes above 256: the generic-transform form (sides with a long-row pass)
   const bool big3d = !is2d && (dv.x == 512 || dv.x == 768 || dv.x == 1024);
-  // every other volume side from 8 to 1024: the same form on the chirp-z transforms
+  // every other volume side from 8 to 1024: chirp-z lines, in passes of their own up to 512
   const bool gen3d = !is2d && !big3d && !fft_len_ok(dv.x) && dv.x >= 8 && dv.x <= 1024;
   const bool any3d = big3d || gen3d;
   if (big2d ? !row_len_native(dv.x) : (!any3d && !fft_len_ok(dv.x)))
@@ -1778,6 +1961,11 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   // orientations of 64^3 at 256 against 2.68 ms at 16)
   pl->B = batch ? batch : (is2d ? (big2d ? big_b : 240u) : (any3d ? big3_b : (dv.x >= 128 ? 128u : 256u)));
   pl->gen3d = gen3d;
+  const bool blue = gen3d && rows_max_any_fused(dv.x);  // chirp-z lines inside the search's own passes
+  // small ones: as many as the native sides take while their spectra stay near 512 MB (75^3: 29 per pass
+  // left half the device idle)
+  if (blue && !batch)
+    pl->B = (unsigned)std::max<size_t>(pl->B, std::min<size_t>(256, (512ull << 20) / (pl->H * sizeof(float2))));
   int L1 = 0, L2 = 0;
   if (big2d && fft_len_split(dv.x, &L1, &L2) != GTOMX_OK) {
     delete pl;
@@ -1785,8 +1973,15 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   }
   pl->nparts = big2d ? (dv.x / 2 + 1 + 63) / 64 * L2
                      : (any3d ? (int)((pl->H + 256 * P3_BINS - 1) / (256 * P3_BINS)) : 0);
-  const std::vector<int> tiles = (is2d || any3d) ? std::vector<int>{0} : tiles_for(pl->n);
-  pl->ntiles = (big2d || any3d) ? 1 : (is2d ? g2_tiles_for(pl->n) : (int)tiles.size());
+  const std::vector<int> tiles =
+      blue ? blue_tiles(pl->n) : ((is2d || any3d) ? std::vector<int>{0} : tiles_for(pl->n));
+  pl->ntiles = blue ? (int)tiles.size() : ((big2d || any3d) ? 1 : (is2d ? g2_tiles_for(pl->n) : (int)tiles.size()));
+  if (blue)
+    GX_TRY(with_blue_len(blue_fused_len(pl->n), [&](auto MC) -> int {
+      using S = BlueShape<decltype(MC)::value>;
+      pl->nparts = pl->ntiles * ((S::TX * S::R2 + 63) / 64);
+      return GTOMX_OK;
+    }));
   int s = GTOMX_OK;
   hipError_t he = hipGetDevice(&pl->device);
   if (he != hipSuccess) {
@@ -1801,7 +1996,7 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   }
   if (is2d && !big2d) pl->pairs2 = pairs2_for(pl->n, pl->B, cus);
   if (!is2d && !any3d) pl->groups3 = plane_groups_for(pl->n, pl->B, cus);
-  if (gen3d && rows_max_any_fused(pl->n)) pl->groups3 = rows_max_any_groups(pl->n, pl->B, cus);
+  if (gen3d && rows_max_any_fused(pl->n)) pl->groups3 = rows_max_any_groups(pl->n, pl->n * pl->n, pl->B, cus);
   void* d = nullptr;
   auto alloc = [&](void** dst, size_t bytes) {
     if (s != GTOMX_OK) return;
@@ -1862,8 +2057,8 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
     plan_release(pl);
     return hip_fail(he, "plan set-up");
   }
-  pl->grid1[0] = resident_grid_for(pl->n, false, cus);
-  pl->grid1[1] = resident_grid_for(pl->n, true, cus);
+  pl->grid1[0] = blue ? blue_grid1(pl->n, false, cus) : resident_grid_for(pl->n, false, cus);
+  pl->grid1[1] = blue ? blue_grid1(pl->n, true, cus) : resident_grid_for(pl->n, true, cus);
   he = hipEventCreateWithFlags(&pl->mats_ev, hipEventDisableTiming);
   if (he != hipSuccess) {
     plan_release(pl);
