@@ -1129,7 +1129,7 @@ __global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_co
     const float2* __restrict__ tw, int half) {
   constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
   __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, c = t % TX, j = t / TX;
   blue_stage<M, DIR>(t, NT, L, tw, B, chirp, twl, bl, cl);
   const int col = blockIdx.x * TX + c;
@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_c2r(const
   using S = BlueRows<M>;
   constexpr int R1 = S::R1, R2 = S::R2;
   __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, j = t % R2;
   float2* xch = area + (t / R2) * S::AREA;
   blue_stage<M, 1>(t, 256, L, tw, B, chirp, twl, bl, cl);
@@ -1229,7 +1229,7 @@ __global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__
   using S = BlueRows<M>;
   constexpr int R1 = S::R1, R2 = S::R2;
   __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, j = t % R2;
   float2* xch = area + (t / R2) * S::AREA;
   blue_stage<M, -1>(t, 256, L, tw, B, chirp, twl, bl, cl);
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(
   constexpr int R1 = S::R1, R2 = S::R2, HP = R1 / 2;
   constexpr unsigned NONE = 0xffffu;
   __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, j = t % R2;
   float2* xch = area + (t / R2) * S::AREA;
   blue_stage<M, 1>(t, 256, n, tw, B, chirp, twl, bl, cl);
@@ -1484,7 +1484,7 @@ __global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_co
     const float2* __restrict__ chirp, const float2* __restrict__ B, const float2* __restrict__ tw) {
   constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
   __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, c = t % TX, j = t / TX;
   blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
   const int col = blockIdx.x * TX + c;
@@ -1590,7 +1590,7 @@ __global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_co
     const float2* __restrict__ tw) {
   constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
   __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, c = t % TX, j = t / TX;
   blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
   const int col = blockIdx.x * TX + c, o = blockIdx.y;

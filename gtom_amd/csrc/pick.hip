@@ -1084,7 +1084,7 @@ __global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
   using S = BlueShape<M>;
   constexpr int R1 = S::R1, R2 = S::R2, TX = S::TX, NT = TX * R2, HP = R1 / 2, WAVES = (NT + 63) / 64;
   __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[M], bl[M], cl[M / 2];
+  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
   const int t = threadIdx.x, c = t % TX, j = t / TX;
   blue_stage<M, 1>(t, NT, n, tw, B, chirp, twl, bl, cl);
   const int nh = n / 2 + 1, half = n / 2, nc = (n + 1) / 2;
