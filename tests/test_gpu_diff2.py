@@ -65,3 +65,32 @@ def test_diff2_planted_shift_found(gx, orc, cuda):
     assert np.unravel_index(np.argmin(best), rel) == (vz, vy, vx)
     assert ang[vz, vy, vx] == k
     assert best[vz, vy, vx] < 1e-4 * np.sum(np.abs(Ev) ** 2)
+
+
+@pytest.mark.parametrize("n,rel,nvol,nang", [(24, (3, 4, 5), 1, 5), (24, (13, 9, 12), 3, 300), (34, (17, 16, 18), 2, 37),
+                                             (32, (32, 1, 31), 2, 33), (2, (2, 1, 2), 1, 4)])
+def test_diff2_shift_ranges(gx, orc, cuda, n, rel, nvol, nang):
+    """Every count of shift pairs per axis (one chunk and several), odd and even ranges, one
+    orientation and four to a lane, more than one batch: against the same sum in 64 bits, by a
+    complex FFT of the half spectrum, from the float projections. 32-bit sums over the bins: 1e-5
+    of the largest score, as above."""
+    import torch
+    box = 2 if n == 2 else 12
+    projft, p, E, ctf = _setup(gx, orc, cuda, n, box, nvol, seed=n + sum(rel))
+    rng = np.random.default_rng(nang)
+    angles = rng.uniform(0, TAU, (nang, 3)).astype(np.float32)
+    best, ang = gx.d_PickSubTomogramsDiff2(projft, p, p / n, E, ctf, rel, angles)
+    best, ang = to_np(best), to_np(ang)
+    R = gx.d_rlnProject(projft, p, n, angles=angles, oversample=p / n).to(torch.complex128)
+    sh = [[(j - r // 2) % n for j in range(r)] for r in rel]  # z, y, x
+    for v in range(nvol):
+        Y = R * ctf[v].double()
+        full = torch.zeros((nang, n, n, n), dtype=torch.complex128, device=cuda)
+        full[..., :n // 2 + 1] = Y * E[v].to(torch.complex128).conj()
+        X = torch.fft.fftn(full, dim=(1, 2, 3)).real[:, sh[0]][:, :, sh[1]][:, :, :, sh[2]]
+        ref = (Y.abs() ** 2).sum((1, 2, 3))[:, None, None, None] + (E[v].to(torch.complex128).abs() ** 2).sum() - 2 * X
+        two = torch.topk(ref, 2, dim=0, largest=False)
+        rb, ri = two.values[0].cpu().numpy(), two.indices[0].cpu().numpy()
+        assert rel_linf(best[v], rb) <= 1e-5
+        sure = (two.values[1] - two.values[0]).cpu().numpy() > 1e-5 * np.abs(rb).max()
+        assert np.array_equal(ang[v][sure], ri[sure].astype(np.float32))
