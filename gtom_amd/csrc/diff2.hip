@@ -94,14 +94,16 @@ template <int PD> struct ShiftSums {
 };
 
 // T[(v nb + a) rz + dz][c] = sum over kz of Q_a, and the partial sums of |R_a ctf|^2
-// per (v, a) and wave. A lane is one column c = ky nh + kx of NA orientations, which
-// share the loads of E and ctf; a wave runs to the largest |kz| inside the sphere of
-// radius n/2 on any of its columns (R is zero beyond, half of the half spectrum).
-// Bound by its loads from the caches, (8 + 12 / NA) bytes per bin, orientation and
-// volume. Grid: x = waves / 4, y = volume x chunk of PD shift pairs, z = orientations
-// / NA, so that the volumes read the same R one after the other.
-template <int PD, int NA>
-__global__ __launch_bounds__(256, 2) void k_diff2_z(const float2* __restrict__ R, const float2* __restrict__ E,
+// per (v, a) and wave. A lane is one column c = ky nh + kx; a wave runs to the largest
+// |kz| inside the sphere of radius n/2 on any of its columns (R is zero beyond, half
+// of the half spectrum). Bound by its loads from the caches, 20 bytes per bin,
+// orientation and volume, and the waves in flight to hide them: several orientations
+// to a lane share E and ctf but cost registers (64^3 x 8 volumes x 250 orientations,
+// the whole search: 0.73 ms with one, 0.89 with two, 1.06 with four). Grid: x = waves
+// / 4, y = volume x chunk of PD shift pairs, z = orientation, so that the volumes
+// read the same R one after the other.
+template <int PD>
+__global__ __launch_bounds__(256) void k_diff2_z(const float2* __restrict__ R, const float2* __restrict__ E,
                                                     const float* __restrict__ ctf, const float2* __restrict__ W,
                                                     int wd, int chunks, int n, int r, int nb,
                                                     float2* __restrict__ T, double* __restrict__ parts) {
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void k_diff2_z(const float2* __restrict__ R
   const size_t C = (size_t)n * nh, h = C * n;
   const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / 64);
   const int nwaves = gridDim.x * 4;
-  const int v = blockIdx.y / chunks, d0 = (blockIdx.y % chunks) * PD, a0 = blockIdx.z * NA;
+  const int v = blockIdx.y / chunks, d0 = (blockIdx.y % chunks) * PD, a = blockIdx.z;
   const size_t col = (size_t)wave * 64 + threadIdx.x % 64;
   const bool ok = col < C;
   const size_t c = ok ? col : C - 1;
@@ -125,53 +127,31 @@ __global__ __launch_bounds__(256, 2) void k_diff2_z(const float2* __restrict__ R
   const int zmax = __builtin_amdgcn_readfirstlane(zl);
   E += v * h;
   ctf += v * h;
-  const float2* Ra[NA];
-#pragma unroll
-  for (int i = 0; i < NA; ++i) Ra[i] = R + (size_t)min(a0 + i, nb - 1) * h;
-  ShiftSums<PD> S[NA];
-  double norm[NA] = {};
-  auto product = [&](int i, float2 x, float ct, float2 e) {
+  R += a * h;
+  ShiftSums<PD> S;
+  double norm = 0;
+  auto product = [&](float2 x, float ct, float2 e) {
     const float2 y = make_float2(x.x * ct, x.y * ct);
-    norm[i] += (double)y.x * y.x + (double)y.y * y.y;
+    norm += (double)y.x * y.x + (double)y.y * y.y;
     return make_float2(y.x * e.x + y.y * e.y, y.y * e.x - y.x * e.y);
   };
   const float2 zero = make_float2(0.f, 0.f);
   auto single = [&](int k) {  // kz = 0 and, on the column (0, 0) only, kz = n/2
     const size_t p = k * C + c;
-    const float2 e = E[p];
-    const float ct = ctf[p];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) S[i].add(product(i, Ra[i][p], ct, e), zero, W + (size_t)k * wd + d0);
+    S.add(product(R[p], ctf[p], E[p]), zero, W + (size_t)k * wd + d0);
   };
   if (zmax >= 0) single(0);
   const int zpair = min(zmax, n / 2 - 1);
   for (int k = 1; k <= zpair; ++k) {
     const size_t p = k * C + c, m = (n - k) * C + c;
-    const float2 ep = E[p], em = E[m];
-    const float cp = ctf[p], cm = ctf[m];
-    float2 xp[NA], xm[NA];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      xp[i] = Ra[i][p];
-      xm[i] = Ra[i][m];
-    }
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const float2 qp = product(i, xp[i], cp, ep);
-      const float2 qm = product(i, xm[i], cm, em);
-      S[i].add(qp, qm, W + (size_t)k * wd + d0);
-    }
+    const float2 qp = product(R[p], ctf[p], E[p]), qm = product(R[m], ctf[m], E[m]);
+    S.add(qp, qm, W + (size_t)k * wd + d0);
   }
   if (zmax == n / 2) single(n / 2);
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    const int a = a0 + i;
-    if (a >= nb) break;
-    double t = ok ? norm[i] : 0.0;
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o);
-    if (d0 == 0 && threadIdx.x % 64 == 0) parts[((size_t)v * nb + a) * nwaves + wave] = t;
-    if (ok) S[i].store(T + ((size_t)v * nb + a) * r * C + c, C, r, d0);
-  }
+  double t = ok ? norm : 0.0;
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o);
+  if (d0 == 0 && threadIdx.x % 64 == 0) parts[((size_t)v * nb + a) * nwaves + wave] = t;
+  if (ok) S.store(T + ((size_t)v * nb + a) * r * C + c, C, r, d0);
 }
 
 // out[item][j][kx] = sum over ky of in[item][ky][kx], the columns of all items in a
@@ -371,16 +351,10 @@ extern "C" int gtomx_pick_subtomograms_diff2(const gtomx_complex* d_projectorft,
       GX_TRY(with_pairs(rz, [&](auto pd) {
         constexpr int PD = decltype(pd)::value;
         const unsigned chunks = (unsigned)std::max(1, (rz / 2 + PD - 1) / PD);
-        // Four orientations to a lane where that leaves a wave per SIMD.
-        const bool four = (size_t)gz * 4 * nv * chunks * (nb / 4) >= 1024;
-        auto go = [&](auto na) {
-          constexpr int NA = decltype(na)::value;
-          hipLaunchKernelGGL((k_diff2_z<PD, NA>), dim3(gz, nv * chunks, (nb + NA - 1) / NA), dim3(256), 0, s, R.p, Ev,
-                             cv, W.p + 1, wd, (int)chunks, n, rz, (int)nb, T1.p, parts);
-          GX_LAUNCHED("k_diff2_z");
-          return (int)GTOMX_OK;
-        };
-        return four ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
+        hipLaunchKernelGGL((k_diff2_z<PD>), dim3(gz, nv * chunks, nb), dim3(256), 0, s, R.p, Ev, cv, W.p + 1, wd,
+                           (int)chunks, n, rz, (int)nb, T1.p, parts);
+        GX_LAUNCHED("k_diff2_z");
+        return (int)GTOMX_OK;
       }));
       hipLaunchKernelGGL(k_diff2_sum, dim3(nv * nb), dim3(256), 0, s, parts, (int)gz * 4, asum);
       GX_LAUNCHED("k_diff2_sum");
