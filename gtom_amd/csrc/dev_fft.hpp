@@ -177,6 +177,101 @@ template <int A, int B, int DIR> __device__ __forceinline__ void dft_mixed(float
   }
 }
 
+// Odd prime length P: a[k] e^{i t k} + a[P-k] e^{-i t k} share their products.
+template <int P, int DIR> __device__ __forceinline__ void dft_prime(float2* a) {
+  static_assert(P == 5 || P == 7, "cosines of 2 pi k / 5 and 2 pi k / 7");
+  constexpr float C5[5] = {1.f, 0.30901699437494742410f, -0.80901699437494742410f, -0.80901699437494742410f,
+                           0.30901699437494742410f};
+  constexpr float S5[5] = {0.f, 0.95105651629515357212f, 0.58778525229247312917f, -0.58778525229247312917f,
+                           -0.95105651629515357212f};
+  constexpr float C7[7] = {1.f,
+                           0.62348980185873353053f,
+                           -0.22252093395631440429f,
+                           -0.90096886790241912624f,
+                           -0.90096886790241912624f,
+                           -0.22252093395631440429f,
+                           0.62348980185873353053f};
+  constexpr float S7[7] = {0.f,
+                           0.78183148246802980871f,
+                           0.97492791218182360702f,
+                           0.43388373911755812048f,
+                           -0.43388373911755812048f,
+                           -0.97492791218182360702f,
+                           -0.78183148246802980871f};
+  constexpr int H = P / 2;
+  float2 s[H], d[H], x0 = a[0];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    s[k] = cadd(a[k + 1], a[P - 1 - k]);
+    d[k] = csub(a[k + 1], a[P - 1 - k]);
+    x0 = cadd(x0, s[k]);
+  }
+  const float2 z = a[0];
+#pragma unroll
+  for (int q = 1; q <= H; ++q) {
+    float2 e = z, o = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      const float cc = P == 5 ? C5[q * k % 5] : C7[q * k % 7], ss = P == 5 ? S5[q * k % 5] : S7[q * k % 7];
+      e.x = fmaf(cc, s[k - 1].x, e.x);
+      e.y = fmaf(cc, s[k - 1].y, e.y);
+      o.x = k == 1 ? ss * d[0].x : fmaf(ss, d[k - 1].x, o.x);
+      o.y = k == 1 ? ss * d[0].y : fmaf(ss, d[k - 1].y, o.y);
+    }
+    o = mul_pj<DIR>(o);
+    a[q] = cadd(e, o);
+    a[P - q] = csub(e, o);
+  }
+  a[0] = x0;
+}
+
+// Length 9 as 3 x 3.
+template <int DIR> __device__ __forceinline__ void dft9(float2* x) {
+  constexpr float C[5] = {1.f, 0.76604444311897803520f, 0.17364817766693034885f, -0.5f, -0.93969262078590838405f};
+  constexpr float S[5] = {0.f, 0.64278760968653932632f, 0.98480775301220805937f, 0.86602540378443864676f,
+                          0.34202014332566873304f};
+  float2 y[3][3];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    float2 t[3] = {x[b], x[b + 3], x[b + 6]};
+    dft3<DIR>(t[0], t[1], t[2]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) y[b][k] = b * k == 0 ? t[k] : cmul(t[k], make_float2(C[b * k], DIR * S[b * k]));
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    dft3<DIR>(y[0][k], y[1][k], y[2][k]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) x[k + 3 * q] = y[q][k];
+  }
+}
+
+// Length A * B of coprime A and B (Good-Thomas: n = B a + A b, k by its remainders; no twiddles).
+template <int A, int B, int DIR> __device__ __forceinline__ void dft_coprime(float2* x) {
+  constexpr int N = A * B;
+  float2 y[B][A];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+#pragma unroll
+    for (int a = 0; a < A; ++a) y[b][a] = x[(B * a + A * b) % N];
+    dft<A, DIR>(y[b]);
+  }
+#pragma unroll
+  for (int a = 0; a < A; ++a) {
+    float2 t[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) t[b] = y[b][a];
+    dft<B, DIR>(t);
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      int k = a;  // k % A == a, k % B == b
+      for (int i = 0; i < B; ++i)
+        if (k % B != b) k += A;
+      x[k] = t[b];
+    }
+  }
+}
+
 template <int R, int DIR> __device__ __forceinline__ void dft(float2* a) {
   if constexpr (R == 1) {
   } else if constexpr (R == 2) {
@@ -185,6 +280,16 @@ template <int R, int DIR> __device__ __forceinline__ void dft(float2* a) {
     dft3<DIR>(a[0], a[1], a[2]);
   } else if constexpr (R == 4) {
     dft4<DIR>(a[0], a[1], a[2], a[3]);
+  } else if constexpr (R == 5 || R == 7) {
+    dft_prime<R, DIR>(a);
+  } else if constexpr (R == 9) {
+    dft9<DIR>(a);
+  } else if constexpr (R == 10) {
+    dft_coprime<2, 5, DIR>(a);
+  } else if constexpr (R == 15) {
+    dft_coprime<3, 5, DIR>(a);
+  } else if constexpr (R == 20) {
+    dft_coprime<4, 5, DIR>(a);
   } else if constexpr (R == 6) {
     dft_mixed<2, 3, DIR>(a);
   } else if constexpr (R == 8) {

@@ -14,6 +14,7 @@
 #include <complex>
 #include <cstdint>
 #include <map>
+#include <tuple>
 #include <mutex>
 #include <vector>
 #include <type_traits>
@@ -1122,50 +1123,39 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
 // A strided axis, from src into dst (which may be src), addressed as k_cols. With
 // half > 0 the axis is y of a search's planes, whose entries outside the disc
 // x^2 + y^2 <= half^2 (x the column) were not written and read as zero.
-template <int M, int DIR>
-__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols(
-    const float2* src, float2* dst, int width, long long axis_stride, long long nplanes, long long P1, long long S0,
-    long long S1, int L, const float2* __restrict__ chirp, const float2* __restrict__ B,
-    const float2* __restrict__ tw, int half) {
-  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
-  __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  blue_stage<M, DIR>(t, NT, L, tw, B, chirp, twl, bl, cl);
-  const int col = blockIdx.x * TX + c;
+template <class LN, int DIR>
+__global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols(const float2* src, float2* dst, int width,
+                                                               long long axis_stride, long long nplanes, long long P1,
+                                                               long long S0, long long S1, LineArgs A, int half) {
+  float2* lds = line_lds<LN::COL_LDS>();
+  float2* xch = lds + LN::tables(A);
+  const int lanes = LN::lanes(A), txlog = LN::txlog(A), L = A.L;
+  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
+  LN::stage(lds, t, lanes << txlog, A);
+  const int col = ((int)blockIdx.x << txlog) + c;
   const bool valid = col < width;
   for (long long pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
     const long long base = (pl / P1) * S1 + (pl % P1) * S0 + col;
-    float2 v[R1];
+    float2 v[LN::REGS];
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m, y = p <= L / 2 ? p : p - L;
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m, y = p <= L / 2 ? p : p - L;
       const bool in = half == 0 || col * col + y * y <= half * half;
       v[m] = valid && p < L && in ? src[base + (long long)p * axis_stride] : make_float2(0.f, 0.f);
     }
     __syncthreads();  // the tables are staged, the last plane's exchange is read
+    LN::template run<DIR>(v, j, A, lds, [&](int k, int i) { return &xch[((k * lanes + i) << txlog) + c]; },
+                          SyncGroup{});
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
-#pragma unroll
-    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
-#pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
-      if (valid && p < L) dst[base + (long long)p * axis_stride] = cmul(v[m], cl[p]);
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m;
+      if (valid && p < L) dst[base + (long long)p * axis_stride] = v[m];
     }
   }
 }
 
 // Rows, two to a transform: one as the real, one as the imaginary part. A pair's
-// R2 threads are lanes of one wave, so the exchanges need no barrier. Pairs per
-// workgroup of 256 threads, and their LDS area (R1 values of padding spread the
-// reads of a k1 over the banks).
-template <int M> struct BlueRows {
-  static constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2;
-  static constexpr int TP = 256 / R2, AREA = M + R1;
-};
-
+// threads are lanes of one wave, so the exchanges need no barrier.
 // z[p] = A[p] + i B[p] of two half-spectrum rows completed as X[L - q] = conj X[q],
 // without the imaginary parts of X[0] and X[L/2] (the real part of the inverse).
 __device__ __forceinline__ float2 row_pair_bin(const float2* __restrict__ a, const float2* __restrict__ b, bool va,
@@ -1178,84 +1168,72 @@ __device__ __forceinline__ float2 row_pair_bin(const float2* __restrict__ a, con
   return mirror ? make_float2(x.x + y.y, y.x - x.y) : make_float2(x.x - y.y, x.y + y.x);
 }
 
-template <int M>
-__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_c2r(const float2* __restrict__ in, float* __restrict__ out,
-                                                       long long nrows, int L, float scale,
-                                                       const float2* __restrict__ chirp,
-                                                       const float2* __restrict__ B, const float2* __restrict__ tw) {
-  using S = BlueRows<M>;
-  constexpr int R1 = S::R1, R2 = S::R2;
-  __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, j = t % R2;
-  float2* xch = area + (t / R2) * S::AREA;
-  blue_stage<M, 1>(t, 256, L, tw, B, chirp, twl, bl, cl);
+template <class LN>
+__global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_c2r(const float2* __restrict__ in,
+                                                                      float* __restrict__ out, long long nrows,
+                                                                      float scale, LineArgs A) {
+  float2* lds = line_lds<LN::ROW_LDS>();
+  const int t = threadIdx.x, L = A.L, lanes = LN::lanes(A), pitch = LN::row_pitch(A), pairs = row_pairs<LN>(A);
+  int j;
+  const int slot = row_slot<LN>(t, A, &j);
+  LN::stage(lds, t, 256, A);
   __syncthreads();
-  const long long step = 2LL * S::TP * gridDim.x;
-  for (long long row = 2 * ((long long)blockIdx.x * S::TP + t / R2); row < nrows; row += step) {
+  if (slot < 0) return;  // no barrier below
+  float2* xch = lds + LN::tables(A) + slot * LN::row_area(A);
+  const long long step = 2LL * pairs * gridDim.x;
+  for (long long row = 2 * ((long long)blockIdx.x * pairs + slot); row < nrows; row += step) {
     const int nh = L / 2 + 1;
     const bool two = row + 1 < nrows;
     const float2* a = in + row * nh;
-    float2 v[R1];
+    float2 v[LN::REGS];
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m;
       v[m] = row_pair_bin(a, a + nh, p < L, p < L && two, p < L ? p : 0, L);
     }
-#pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
-#pragma unroll
-    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    LN::template run<1>(v, j, A, lds, [&](int k, int i) { return &xch[k * pitch + i]; }, SyncWave{});
     SyncWave{}();
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m;
       if (p >= L) continue;
-      const float2 r = cmul(v[m], cl[p]);
-      out[row * L + p] = r.x * scale;
-      if (two) out[(row + 1) * L + p] = r.y * scale;
+      out[row * L + p] = v[m].x * scale;
+      if (two) out[(row + 1) * L + p] = v[m].y * scale;
     }
   }
 }
 
 // A[k] = (Z[k] + conj Z[L - k]) / 2, B[k] = (Z[k] - conj Z[L - k]) / 2i of Z = DFT(a + i b).
 // With pm.n0 the rows hold that many reals, padded to L on load.
-template <int M>
-__global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                       long long nrows, int L, const float2* __restrict__ chirp,
-                                                       const float2* __restrict__ B, const float2* __restrict__ tw,
-                                                       PadMap pm) {
-  using S = BlueRows<M>;
-  constexpr int R1 = S::R1, R2 = S::R2;
-  __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, j = t % R2;
-  float2* xch = area + (t / R2) * S::AREA;
-  blue_stage<M, -1>(t, 256, L, tw, B, chirp, twl, bl, cl);
+template <class LN>
+__global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
+                                                       long long nrows, LineArgs A, PadMap pm) {
+  float2* lds = line_lds<LN::ROW_LDS>();
+  const int t = threadIdx.x, L = A.L, lanes = LN::lanes(A), pitch = LN::row_pitch(A), pairs = row_pairs<LN>(A);
+  int j;
+  const int slot = row_slot<LN>(t, A, &j);
+  LN::stage(lds, t, 256, A);
   __syncthreads();
-  const long long step = 2LL * S::TP * gridDim.x;
-  for (long long row = 2 * ((long long)blockIdx.x * S::TP + t / R2); row < nrows; row += step) {
+  if (slot < 0) return;  // no barrier below
+  float2* xch = lds + LN::tables(A) + slot * LN::row_area(A);
+  const long long step = 2LL * pairs * gridDim.x;
+  for (long long row = 2 * ((long long)blockIdx.x * pairs + slot); row < nrows; row += step) {
     const int nh = L / 2 + 1;
     const bool two = row + 1 < nrows;
     const int len = pm.n0 ? pm.n0 : L;
     const float* a = in + row * len;
-    float2 v[R1];
+    float2 v[LN::REGS];
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m, q = p >= L ? -1 : (pm.n0 ? pm.at(p, L) : p);
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m, q = p >= L ? -1 : (pm.n0 ? pm.at(p, L) : p);
       v[m] = make_float2(q >= 0 ? a[q] : 0.f, q >= 0 && two ? a[len + q] : 0.f);
     }
-#pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
-#pragma unroll
-    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    LN::template run<-1>(v, j, A, lds, [&](int k, int i) { return &xch[k * pitch + i]; }, SyncWave{});
     SyncWave{}();
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) xch[j + R2 * m] = cmul(v[m], cl[j + R2 * m]);
+    for (int m = 0; m < LN::PTS; ++m) xch[j + lanes * m] = v[m];
     SyncWave{}();
-    for (int k = j; k < nh; k += R2) {
+    for (int k = j; k < nh; k += lanes) {
       const float2 z = xch[k], w = cconj(xch[k == 0 ? 0 : L - k]);
       const float2 s = cadd(z, w), d = csub(z, w);
       out[row * nh + k] = make_float2(0.5f * s.x, 0.5f * s.y);
@@ -1273,22 +1251,21 @@ __global__ __launch_bounds__(256) void k_blue_rows_r2c(const float* __restrict__
 // A pair of voxels keeps its two orientations as 16-bit offsets in the group in
 // one register (NONE: unchanged): with 32-bit indices the 512-point form spills
 // (200^3: 1.38 ms per 32 orientations).
-template <int M, bool FRESH, bool SEARCH>
-__global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(
-    const float2* __restrict__ G, long long H, int nb, int n, int nrows, int angle0, const float2* __restrict__ sn,
-    float* __restrict__ best, int32_t* __restrict__ bidx, int og, const float2* __restrict__ chirp,
-    const float2* __restrict__ B, const float2* __restrict__ tw) {
-  using S = BlueRows<M>;
-  constexpr int R1 = S::R1, R2 = S::R2, HP = R1 / 2;
+template <class LN, bool FRESH, bool SEARCH>
+__global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
+    const float2* __restrict__ G, long long H, int nb, int nrows, int angle0, const float2* __restrict__ sn,
+    float* __restrict__ best, int32_t* __restrict__ bidx, int og, LineArgs A) {
+  constexpr int HP = LN::PTS;
   constexpr unsigned NONE = 0xffffu;
-  __shared__ float2 area[S::TP * S::AREA];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, j = t % R2;
-  float2* xch = area + (t / R2) * S::AREA;
-  blue_stage<M, 1>(t, 256, n, tw, B, chirp, twl, bl, cl);
+  float2* lds = line_lds<LN::ROW_LDS>();
+  const int t = threadIdx.x, n = A.L, R2 = LN::lanes(A), xp = LN::row_pitch(A);
+  int j;
+  const int slot = row_slot<LN>(t, A, &j);
+  LN::stage(lds, t, 256, A);
   __syncthreads();
-  const int row = 2 * (blockIdx.x * S::TP + t / R2);
-  if (row >= nrows) return;  // no barrier below
+  const int row = 2 * ((int)blockIdx.x * row_pairs<LN>(A) + slot);
+  if (slot < 0 || row >= nrows) return;  // no barrier below
+  float2* xch = lds + LN::tables(A) + slot * LN::row_area(A);
   const bool two = row + 1 < nrows;
   int o0 = 0, o1 = nb;
   if (FRESH) {
@@ -1316,7 +1293,7 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(
     // in registers, which would spill
     int jo = j;
     asm volatile("" : "+v"(jo));
-    float2 v[R1];
+    float2 v[LN::REGS];
 #pragma unroll
     for (int m = 0; m < HP; ++m) {
       // z[p] of row_pair_bin; a last row without a partner reads past the buffer's end, which gives 0
@@ -1332,17 +1309,12 @@ __global__ __launch_bounds__(256, (M <= 512 ? 2 : 1)) void k_blue_rows_max(
       if (mid || p == 0) x.y = y.y = 0.f;
       v[m] = mirror ? make_float2(x.x + y.y, y.x - x.y) : make_float2(x.x - y.y, x.y + y.x);
     }
-#pragma unroll
-    for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[jo + R2 * m]);
-#pragma unroll
-    for (int m = HP; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, jo, twl, bl, [&](int k1, int jj) { return &xch[k1 * (R2 + 1) + jj]; }, SyncWave{});
+    LN::template run<1>(v, jo, A, lds, [&](int k, int i) { return &xch[k * xp + i]; }, SyncWave{});
     SyncWave{}();
     const unsigned lo = (unsigned)(o - o0);
 #pragma unroll
     for (int m = 0; m < HP; ++m) {
-      const float2 r = cmul(v[m], cl[jo + R2 * m]);
-      const float c0 = r.x * so.x, c1 = r.y * so.x;
+      const float c0 = v[m].x * so.x, c1 = v[m].y * so.x;
       if (c0 > bv[0][m]) {
         bv[0][m] = c0;
         bi[m] = (bi[m] & 0xffff0000u) | lo;
@@ -1478,36 +1450,33 @@ __global__ __launch_bounds__(fft_col_tx<N>() * ColShape<N>::R2) void k_cols_pad(
   }
 }
 
-template <int M>
-__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols_pad(
-    const float2* __restrict__ src, float2* __restrict__ dst, int width, int nplanes, PadMap pm, int L,
-    const float2* __restrict__ chirp, const float2* __restrict__ B, const float2* __restrict__ tw) {
-  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
-  __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
-  const int col = blockIdx.x * TX + c;
+template <class LN>
+__global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols_pad(const float2* __restrict__ src,
+                                                                   float2* __restrict__ dst, int width, int nplanes,
+                                                                   PadMap pm, LineArgs A) {
+  float2* lds = line_lds<LN::COL_LDS>();
+  float2* xch = lds + LN::tables(A);
+  const int lanes = LN::lanes(A), txlog = LN::txlog(A), L = A.L;
+  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
+  LN::stage(lds, t, lanes << txlog, A);
+  const int col = ((int)blockIdx.x << txlog) + c;
   const bool valid = col < width;
   for (int pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
     const float2* s = src + (size_t)pl * pm.n0 * width + col;
     float2* d = dst + (size_t)pl * L * width + col;
-    float2 v[R1];
+    float2 v[LN::REGS];
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m, q = p < L ? pm.at(p, L) : -1;
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m, q = p < L ? pm.at(p, L) : -1;
       v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
     }
     __syncthreads();
+    LN::template run<-1>(v, j, A, lds, [&](int k, int i) { return &xch[((k * lanes + i) << txlog) + c]; },
+                         SyncGroup{});
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
-#pragma unroll
-    for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-    blue_convolve<M>(v, j, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
-#pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
-      if (valid && p < L) d[(size_t)p * width] = cmul(v[m], cl[p]);
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m;
+      if (valid && p < L) d[(size_t)p * width] = v[m];
     }
   }
 }
@@ -1583,52 +1552,46 @@ __global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_cols_corr
   }
 }
 
-template <int M>
-__global__ __launch_bounds__(BlueShape<M>::TX * BlueShape<M>::R2) void k_blue_cols_correlate(
-    const float2* __restrict__ src, const float2* __restrict__ E, float2* __restrict__ dst, int width, PadMap pm,
-    const float2* __restrict__ norm, int L, const float2* __restrict__ chirp, const float2* __restrict__ B,
-    const float2* __restrict__ tw) {
-  constexpr int R1 = BlueShape<M>::R1, R2 = BlueShape<M>::R2, TX = BlueShape<M>::TX, NT = TX * R2;
-  __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  blue_stage<M, -1>(t, NT, L, tw, B, chirp, twl, bl, cl);
-  const int col = blockIdx.x * TX + c, o = blockIdx.y;
+template <class LN>
+__global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols_correlate(const float2* __restrict__ src,
+                                                                         const float2* __restrict__ E,
+                                                                         float2* __restrict__ dst, int width,
+                                                                         PadMap pm, const float2* __restrict__ norm,
+                                                                         LineArgs A) {
+  float2* lds = line_lds<LN::COL_LDS>();
+  float2* xch = lds + LN::tables(A);
+  const int lanes = LN::lanes(A), txlog = LN::txlog(A), L = A.L;
+  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
+  LN::stage(lds, t, lanes << txlog, A);
+  const int col = ((int)blockIdx.x << txlog) + c, o = blockIdx.y;
   const bool valid = col < width;
   const float2* s = src + (size_t)o * pm.n0 * width + col;
   const float2* e = E + col;
   float2* d = dst + (size_t)o * L * width + col;
   const float2 nm = norm[o];
-  auto at = [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; };
-  float2 v[R1];
+  auto at = [&](int k, int i) { return &xch[((k * lanes + i) << txlog) + c]; };
+  float2 v[LN::REGS];
 #pragma unroll
-  for (int m = 0; m < R1 / 2; ++m) {
-    const int p = j + R2 * m, q = p < L ? pm.at(p, L) : -1;
+  for (int m = 0; m < LN::PTS; ++m) {
+    const int p = j + lanes * m, q = p < L ? pm.at(p, L) : -1;
     v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
   }
   __syncthreads();
+  LN::template run<-1>(v, j, A, lds, at, SyncGroup{});
 #pragma unroll
-  for (int m = 0; m < R1 / 2; ++m) v[m] = cmul(v[m], cl[j + R2 * m]);
-#pragma unroll
-  for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-  blue_convolve<M>(v, j, twl, bl, at, SyncGroup{});
-#pragma unroll
-  for (int m = 0; m < R1 / 2; ++m) {
-    const int p = j + R2 * m;
-    const float2 ch = cl[p];  // 0 past the line
-    const float2 q = image_times_ref(valid && p < L ? e[(size_t)p * width] : make_float2(0.f, 0.f), cmul(v[m], ch),
+  for (int m = 0; m < LN::PTS; ++m) {
+    const int p = j + lanes * m;
+    const float2 q = image_times_ref(valid && p < L ? e[(size_t)p * width] : make_float2(0.f, 0.f), v[m],
                                      p == 0 && col == 0 ? nm.x : 0.f, nm.y);
-    v[m] = cmulc(q, ch);
+    v[m] = p < L ? q : make_float2(0.f, 0.f);
   }
-#pragma unroll
-  for (int m = R1 / 2; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-  __syncthreads();  // the first convolution's exchange is read
-  blue_convolve<M, true>(v, j, twl, bl, at, SyncGroup{});
+  __syncthreads();  // the first transform's exchange is read
+  LN::template run<1>(v, j, A, lds, at, SyncGroup{});
   if (valid) {
 #pragma unroll
-    for (int m = 0; m < R1 / 2; ++m) {
-      const int p = j + R2 * m;
-      if (p < L) d[(size_t)p * width] = cmulc(v[m], cl[p]);
+    for (int m = 0; m < LN::PTS; ++m) {
+      const int p = j + lanes * m;
+      if (p < L) d[(size_t)p * width] = v[m];
     }
   }
 }
@@ -1857,53 +1820,132 @@ int blue_tables(int L, BlueTables* out) {
 
 unsigned blue_grid(long long n) { return (unsigned)std::max<long long>(1, std::min<long long>((n + 255) / 256, 65536)); }
 
+// L = RL * lanes with DFT-RL in registers and lanes, at most 32, in one stage of up to 10 or two of {2, 3, 4, 5} x
+// {4 .. 9}; RL = 0 when there is no such form. Columns: one stage before two (200^3 x 32 orientations, y: 168 us a
+// launch as 20 x 10, 211 as 10 x (4 x 5)), then the smallest RL, which leaves the most threads to a line. Rows, whose
+// running maxima take registers by RL (763 us as 20 x 10, 386 as 10 x (4 x 5)): the smallest RL from 8 up (75: 139 us
+// as 15 x 5, 196 as 5 x (3 x 5)). Before that, lanes that fill 54 or more of a wave's 64 with whole row pairs.
+LineArgs line_shape(int L, bool rows) {
+  LineArgs A;
+  A.L = L;
+  int best = 0;
+  for (int RL : {5, 6, 7, 8, 9, 10, 12, 15, 16, 20}) {
+    if (L % RL) continue;
+    const int Q = L / RL;
+    if (Q < 3 || Q > 32) continue;
+    int r1 = 0, r2 = 1;
+    if (Q <= 10) {
+      r1 = Q;
+    } else {
+      for (int a : {5, 4, 3, 2})
+        if (!r1 && Q % a == 0 && Q / a >= 4 && Q / a <= 9) {
+          r1 = a;
+          r2 = Q / a;
+        }
+    }
+    if (!r1) continue;
+    const int score = ((rows ? RL >= 8 : r2 == 1) ? 1000 : 0) + (64 / Q * Q >= 54 ? 500 : 0) + 100 - RL;
+    if (score <= best) continue;
+    best = score;
+    A.RL = RL;
+    A.lanes = Q;
+    A.r1 = r1;
+    A.r2 = r2;
+    // 16 columns are whole 128-byte lines; more where a line has few threads, fewer where it is long (64 KB of LDS)
+    A.txlog = L > 400 ? 3 : Q <= 5 ? 5 : 4;
+    A.inv1 = 65536 / (Q / r1) + 1;
+    A.inv2 = 65536 / r1 + 1;
+  }
+  if (!best) A.M = blue_fused_len(L);
+  return A;
+}
+
+// Tables of the mixed-radix lengths, per device, computed once in long double.
+std::mutex g_smooth_mu;
+std::map<std::tuple<int, int, int>, const float2*> g_smooth;  // by device, L, RL
+
+int line_args(int L, bool rows, LineArgs* out) {
+  LineArgs A = line_shape(L, rows);
+  if (!A.RL) {
+    BlueTables t;
+    GX_TRY(twiddles(&A.tw));
+    GX_TRY(blue_tables(L, &t));
+    A.t0 = t.chirp;
+    A.t1 = t.bf;
+    *out = A;
+    return GTOMX_OK;
+  }
+  int dev = 0;
+  GX_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(g_smooth_mu);
+  const float2*& d = g_smooth[{dev, L, A.RL}];
+  if (!d) {
+    const int Q = A.lanes;
+    const long double two_pi = 6.283185307179586476925286766559005768L;
+    auto root = [&](int k, int n) {
+      const long double ph = -two_pi * (long double)(k % n) / (long double)n;
+      return make_float2((float)std::cos(ph), (float)std::sin(ph));
+    };
+    std::vector<float2> h((size_t)L + Q);
+    for (int k = 0; k < A.RL; ++k)
+      for (int j = 0; j < Q; ++j) h[k * Q + j] = root(j * k, L);
+    for (int k = 0; k < A.r1; ++k)
+      for (int b = 0; b < A.r2; ++b) h[L + k * A.r2 + b] = root(b * k, Q);
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, h.size() * sizeof(float2));
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc(line tables)");
+    e = hipMemcpy(p, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      return hip_fail(e, "hipMemcpy(line tables)");
+    }
+    d = static_cast<const float2*>(p);
+  }
+  A.t0 = d;
+  *out = A;
+  return GTOMX_OK;
+}
+
 // The fused form on a strided axis, from src into dst (which may be src).
 template <int DIR>
-int blue_cols(int L, const float2* src, float2* dst, int width, long long as, long long nplanes, long long P1,
+int line_cols(int L, const float2* src, float2* dst, int width, long long as, long long nplanes, long long P1,
               long long S0, long long S1, hipStream_t s, int half = 0) {
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
-  BlueTables t;
-  GX_TRY(blue_tables(L, &t));
-  return with_blue_len(t.M, [&](auto MC) -> int {
-    constexpr int M = decltype(MC)::value;
-    using S = BlueShape<M>;
-    const int gx = (width + S::TX - 1) / S::TX;
+  LineArgs A;
+  GX_TRY(line_args(L, false, &A));
+  return with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const int tx = 1 << LN::txlog(A), gx = (width + tx - 1) / tx;
     // enough workgroups to fill the device several times over, and several planes each to share the staged tables
     const long long gy = std::min<long long>(nplanes, std::max<long long>(1, 8192 / gx));
-    hipLaunchKernelGGL((k_blue_cols<M, DIR>), dim3(gx, (unsigned)gy), dim3(S::TX * S::R2), 0, s, src, dst, width, as,
-                       nplanes, P1, S0, S1, L, t.chirp, DIR < 0 ? t.bf : t.bi, tw, half);
-    GX_LAUNCHED("k_blue_cols");
+    hipLaunchKernelGGL((k_line_cols<LN, DIR>), dim3(gx, (unsigned)gy), dim3(col_threads<LN>(A)), col_lds<LN>(A), s, src,
+                       dst, width, as, nplanes, P1, S0, S1, A, half);
+    GX_LAUNCHED("k_line_cols");
     return GTOMX_OK;
   });
 }
 
 // The fused form on nrows contiguous rows of L reals / L/2 + 1 bins.
-int blue_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s, PadMap pm = PadMap{}) {
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
-  BlueTables t;
-  GX_TRY(blue_tables(L, &t));
-  return with_blue_len(t.M, [&](auto MC) -> int {
-    constexpr int M = decltype(MC)::value;
-    const long long wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
-    hipLaunchKernelGGL(k_blue_rows_r2c<M>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), 0, s, in, out,
-                       nrows, L, t.chirp, t.bf, tw, pm);
-    GX_LAUNCHED("k_blue_rows_r2c");
+int line_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s, PadMap pm = PadMap{}) {
+  LineArgs A;
+  GX_TRY(line_args(L, true, &A));
+  return with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const long long per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
+    hipLaunchKernelGGL(k_line_rows_r2c<LN>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), row_lds<LN>(A), s,
+                       in, out, nrows, A, pm);
+    GX_LAUNCHED("k_line_rows_r2c");
     return GTOMX_OK;
   });
 }
-int blue_rows_c2r(int L, const float2* in, float* out, long long nrows, float scale, hipStream_t s) {
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
-  BlueTables t;
-  GX_TRY(blue_tables(L, &t));
-  return with_blue_len(t.M, [&](auto MC) -> int {
-    constexpr int M = decltype(MC)::value;
-    const long long wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
-    hipLaunchKernelGGL(k_blue_rows_c2r<M>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), 0, s, in, out,
-                       nrows, L, scale, t.chirp, t.bi, tw);
-    GX_LAUNCHED("k_blue_rows_c2r");
+int line_rows_c2r(int L, const float2* in, float* out, long long nrows, float scale, hipStream_t s) {
+  LineArgs A;
+  GX_TRY(line_args(L, true, &A));
+  return with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const long long per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
+    hipLaunchKernelGGL(k_line_rows_c2r<LN>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), row_lds<LN>(A), s,
+                       in, out, nrows, scale, A);
+    GX_LAUNCHED("k_line_rows_c2r");
     return GTOMX_OK;
   });
 }
@@ -1934,25 +1976,25 @@ int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int ang
 #undef GX_CASE
     }
   }
-  BlueTables t;
-  GX_TRY(blue_tables(n, &t));
-  return with_blue_len(t.M, [&](auto MC) -> int {
-    constexpr int M = decltype(MC)::value;
-    const int wgs = (nrows + 2 * BlueRows<M>::TP - 1) / (2 * BlueRows<M>::TP);
+  LineArgs A;
+  GX_TRY(line_args(n, true, &A));
+  return with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const int per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
     auto go = [&](auto kernel) -> int {
-      hipLaunchKernelGGL(kernel, dim3(wgs, groups), dim3(256), 0, s, G, H, nb, n, nrows, angle0, sn, best, idx, og,
-                         t.chirp, t.bi, tw);
-      GX_LAUNCHED("k_blue_rows_max");
+      hipLaunchKernelGGL(kernel, dim3(wgs, groups), dim3(256), row_lds<LN>(A), s, G, H, nb, nrows, angle0, sn, best, idx,
+                         og, A);
+      GX_LAUNCHED("k_line_rows_max");
       return GTOMX_OK;
     };
-    if (sn) return groups == 1 ? go(k_blue_rows_max<M, false, true>) : go(k_blue_rows_max<M, true, true>);
-    return groups == 1 ? go(k_blue_rows_max<M, false, false>) : go(k_blue_rows_max<M, true, false>);
+    if (sn) return groups == 1 ? go(k_line_rows_max<LN, false, true>) : go(k_line_rows_max<LN, true, true>);
+    return groups == 1 ? go(k_line_rows_max<LN, false, false>) : go(k_line_rows_max<LN, true, false>);
   });
 }
 
-int blue_search_y(int n, float2* G, int nb, hipStream_t s) {
+int line_search_y(int n, float2* G, int nb, hipStream_t s) {
   const int nc = (n + 1) / 2;
-  return blue_cols<1>(n, G, G, nc, nc, (long long)n * nb, 1LL << 62, (long long)nc * n, 0, s, n / 2);
+  return line_cols<1>(n, G, G, nc, nc, (long long)n * nb, 1LL << 62, (long long)nc * n, 0, s, n / 2);
 }
 
 // Two workgroups of 256 threads per CU fill the device; more groups cost more merging.
@@ -1962,8 +2004,9 @@ int rows_max_any_groups(int n, int nrows, unsigned batch, int cus) {
     const int rw = rows_per_workgroup(n);
     wgs = (nrows + rw - 1) / rw;
   } else {
-    const int st = with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
-      constexpr int per = 2 * BlueRows<decltype(MC)::value>::TP;
+    const LineArgs A = line_shape(n, true);
+    const int st = with_line(A, [&](auto ln) -> int {
+      const int per = 2 * row_pairs<decltype(ln)>(A);
       wgs = (nrows + per - 1) / per;
       return GTOMX_OK;
     });
@@ -2012,7 +2055,7 @@ int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, 
     }
     GX_LAUNCHED("k_rows_r2c");
   } else {
-    GX_TRY(blue_rows_r2c(di.x, r, rows, nrows, s, px));
+    GX_TRY(line_rows_r2c(di.x, r, rows, nrows, s, px));
   }
   // y: every plane of the small volume
   const int planes = (int)(dr.z * nb);
@@ -2028,15 +2071,14 @@ int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, 
     }
     GX_LAUNCHED("k_cols_pad");
   } else {
-    BlueTables t;
-    GX_TRY(blue_tables(di.y, &t));
-    GX_TRY(with_blue_len(t.M, [&](auto MC) -> int {
-      constexpr int M = decltype(MC)::value;
-      using S = BlueShape<M>;
-      const int gx = (nh + S::TX - 1) / S::TX;
-      hipLaunchKernelGGL(k_blue_cols_pad<M>, dim3(gx, std::min(planes, std::max(1, 8192 / gx))), dim3(S::TX * S::R2), 0,
-                         s, rows, cols, nh, planes, py, di.y, t.chirp, t.bf, tw);
-      GX_LAUNCHED("k_blue_cols_pad");
+    LineArgs A;
+    GX_TRY(line_args(di.y, false, &A));
+    GX_TRY(with_line(A, [&](auto ln) -> int {
+      using LN = decltype(ln);
+      const int tx = 1 << LN::txlog(A), gx = (nh + tx - 1) / tx;
+      hipLaunchKernelGGL(k_line_cols_pad<LN>, dim3(gx, std::min(planes, std::max(1, 8192 / gx))),
+                         dim3(col_threads<LN>(A)), col_lds<LN>(A), s, rows, cols, nh, planes, py, A);
+      GX_LAUNCHED("k_line_cols_pad");
       return GTOMX_OK;
     }));
   }
@@ -2054,21 +2096,21 @@ int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, 
     }
     GX_LAUNCHED("k_cols_correlate");
   } else {
-    BlueTables t;
-    GX_TRY(blue_tables(di.z, &t));
-    GX_TRY(with_blue_len(t.M, [&](auto MC) -> int {
-      constexpr int M = decltype(MC)::value;
-      using S = BlueShape<M>;
-      hipLaunchKernelGGL(k_blue_cols_correlate<M>, dim3((width + S::TX - 1) / S::TX, nb), dim3(S::TX * S::R2), 0, s,
-                         cols, E, out, width, pz, norm, di.z, t.chirp, t.bf, tw);
-      GX_LAUNCHED("k_blue_cols_correlate");
+    LineArgs A;
+    GX_TRY(line_args(di.z, false, &A));
+    GX_TRY(with_line(A, [&](auto ln) -> int {
+      using LN = decltype(ln);
+      const int tx = 1 << LN::txlog(A);
+      hipLaunchKernelGGL(k_line_cols_correlate<LN>, dim3((width + tx - 1) / tx, nb), dim3(col_threads<LN>(A)),
+                         col_lds<LN>(A), s, cols, E, out, width, pz, norm, A);
+      GX_LAUNCHED("k_line_cols_correlate");
       return GTOMX_OK;
     }));
   }
   // y back
   if (fft_len_ok(di.y))
     return launch_cols_n<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, tw, s);
-  return blue_cols<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, s);
+  return line_cols<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, s);
 }
 
 // One axis of nlines lines of length L by the chirp-z form: IN / OUT are the
@@ -2135,7 +2177,7 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
     if (fft_len_ok_any(d.y))
       return cols_axis<D>(d.y, data, data, scr.p, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, tw, s);
     if (d.y <= BLUE_FUSED_MAX)
-      return blue_cols<D>(d.y, data, data, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, s);
+      return line_cols<D>(d.y, data, data, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, s);
     const AxisLines a{nh, 1, nh * d.y, nh};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.z * batch, d.y, 0, 1.f, s);
   };
@@ -2145,7 +2187,7 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
       return cols_axis<D>(d.z, data, data, scr.p, (int)nh, nh * d.y, (long long)d.y * batch, d.y, nh, nh * d.y * d.z, tw,
                           s);
     if (d.z <= BLUE_FUSED_MAX && nh * d.y < (1LL << 30))  // the columns of a volume are one contiguous row
-      return blue_cols<D>(d.z, data, data, (int)(nh * d.y), nh * d.y, batch, 1LL << 62, nh * d.y * d.z, 0, s);
+      return line_cols<D>(d.z, data, data, (int)(nh * d.y), nh * d.y, batch, 1LL << 62, nh * d.y * d.z, 0, s);
     const AxisLines a{nh * d.y, 1, nh * d.y * d.z, nh * d.y};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.y * batch, d.z, 0, 1.f, s);
   };
@@ -2176,7 +2218,7 @@ int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipS
     else
       GX_TRY(launch_rows_r2c(d.x, in, out, rows, tw, s));
   } else if (d.x <= BLUE_FUSED_MAX) {
-    GX_TRY(blue_rows_r2c(d.x, in, out, rows, s));
+    GX_TRY(line_rows_r2c(d.x, in, out, rows, s));
   } else {
     GX_TRY((blue_axis<1, 1, -1>(in, AxisLines{1LL << 62, d.x, 0, 1}, out, AxisLines{1LL << 62, nh, 0, 1}, rows, d.x,
                                 (int)nh, 1.f, s)));
@@ -2194,7 +2236,7 @@ int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float sc
     if (d.x > 256) return launch_rows_long<false>(d.x, work, out, rows, scale, tw, s);
     return launch_rows_c2r(d.x, work, out, rows, scale, tw, s);
   }
-  if (d.x <= BLUE_FUSED_MAX) return blue_rows_c2r(d.x, work, out, rows, scale, s);
+  if (d.x <= BLUE_FUSED_MAX) return line_rows_c2r(d.x, work, out, rows, scale, s);
   return blue_axis<2, 2, 1>(work, AxisLines{1LL << 62, nh, 0, 1}, out, AxisLines{1LL << 62, d.x, 0, 1}, rows, d.x,
                             (int)nh, scale, s);
 }

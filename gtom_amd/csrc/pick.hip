@@ -1067,26 +1067,24 @@ __global__ __launch_bounds__(256) void k_pick3d_project_any(PJ P, const float* _
 
 // ---------------------------------------------------------------------------
 // Pass 1 of the sides up to 512 without a native transform: k_pick_project_z with
-// the z inverse by the chirp-z form. Columns (x, y), x < (n + 1) / 2, are numbered
+// the z inverse of dev_blue.hpp's lines. Columns (x, y), x < (n + 1) / 2, are numbered
 // y * nc + x, as G's planes hold them; a tile is TX consecutive ones, tiles[] those
 // with a column inside the disc. (The x = n/2 column of even n is one bin, as in
 // GLayout.) Projecting into a whole half spectrum first and transforming it in
 // place moved it through memory twice more: 200^3 x 32 orientations 0.82 ms in one
 // pass, 0.41 before for the projection alone.
 // ---------------------------------------------------------------------------
-template <int M> constexpr int blue_threads() { return BlueShape<M>::TX * BlueShape<M>::R2; }
-
-template <int M, class PJ>
-__global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
+template <class LN, class PJ>
+__global__ __launch_bounds__(LN::COL_THREADS, 2) void k_pick_project_line(
     PJ P, const float* __restrict__ mats, int nb, const float2* __restrict__ E, const float* __restrict__ ctf,
-    float2* __restrict__ G, float* __restrict__ partial, int n, const int* __restrict__ tiles, int ntiles,
-    const float2* __restrict__ chirp, const float2* __restrict__ B, const float2* __restrict__ tw) {
-  using S = BlueShape<M>;
-  constexpr int R1 = S::R1, R2 = S::R2, TX = S::TX, NT = TX * R2, HP = R1 / 2, WAVES = (NT + 63) / 64;
-  __shared__ float2 xch[TX * M];
-  __shared__ float2 twl[blue_tw_len<M>()], bl[M], cl[M / 2];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  blue_stage<M, 1>(t, NT, n, tw, B, chirp, twl, bl, cl);
+    float2* __restrict__ G, float* __restrict__ partial, const int* __restrict__ tiles, int ntiles, LineArgs A) {
+  constexpr int HP = LN::PTS;
+  float2* lds = line_lds<LN::COL_LDS>();
+  float2* xch = lds + LN::tables(A);
+  const int n = A.L, R2 = LN::lanes(A), txlog = LN::txlog(A), NT = R2 << txlog, WAVES = (NT + 63) / 64;
+  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
+  const int wave_lanes = min(64, NT - (t & ~63));
+  LN::stage(lds, t, NT, A);
   const int nh = n / 2 + 1, half = n / 2, nc = (n + 1) / 2;
   const long long stride = (long long)nc * n * n;
   const __amdgpu_buffer_rsrc_t rs = sampler_rsrc(P);
@@ -1100,7 +1098,7 @@ __global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
     const int o0 = (int)(it % nb);
     const int o1 = (int)min((long long)nb, o0 + (i1 - it));
     it += o1 - o0;
-    const int col = tiles[ti] * TX + c;
+    const int col = (tiles[ti] << txlog) + c;
     const int ix = col % nc, iy = col / nc;
     const int y = signed_freq(iy, n);
     const bool valid = iy < n && ix * ix + y * y <= half * half;
@@ -1123,7 +1121,7 @@ __global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
       for (int k = 0; k < 9; ++k) Mo[k] = mats[9 * o + k];
       const float qx = Mo[0] * ix + Mo[1] * y, qy = Mo[3] * ix + Mo[4] * y, qz = Mo[6] * ix + Mo[7] * y;
       float acc = 0.f;
-      float2 v[R1];
+      float2 v[LN::REGS];
       // opaque per orientation: what follows from it alone is recomputed rather than held in registers
       int jo = j;
       asm volatile("" : "+v"(jo));
@@ -1131,7 +1129,7 @@ __global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
 #pragma unroll
       for (int m0 = 0; m0 < HP; m0 += 2) {
 #pragma unroll
-        for (int m = m0; m < m0 + 2; ++m) {
+        for (int m = m0; m < (m0 + 2 < HP ? m0 + 2 : HP); ++m) {
           const int p = jo + R2 * m, z = signed_freq(p, n);
           const bool in = valid && p < n && ix * ix + y * y + z * z <= half * half;
           if (__any(in)) {
@@ -1148,19 +1146,18 @@ __global__ __launch_bounds__(blue_threads<M>(), 2) void k_pick_project_blue(
       }
       if (dc) v[0] = make_float2(0.f, 0.f);  // its |R|^2 is removed by k_pick_herm_norm
       __syncthreads();
-#pragma unroll
-      for (int m = 0; m < HP; ++m) v[m] = cmul(v[m], cl[jo + R2 * m]);
-#pragma unroll
-      for (int m = HP; m < R1; ++m) v[m] = make_float2(0.f, 0.f);
-      blue_convolve<M>(v, jo, twl, bl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; }, SyncGroup{});
+      LN::template run<1>(v, jo, A, lds, [&](int k, int i) { return &xch[((k * R2 + i) << txlog) + c]; }, SyncGroup{});
       const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + o * stride, (unsigned)stride * 8u);
 #pragma unroll
       for (int m = 0; m < HP; ++m) {
-        const u32x2 w = __builtin_bit_cast(u32x2, cmul(v[m], cl[jo + R2 * m]));
+        const u32x2 w = __builtin_bit_cast(u32x2, v[m]);
         __builtin_amdgcn_raw_buffer_store_b64(w, rG, gout, m * R2 * nc * n * 8, CPOL_NT);
       }
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+      for (int off = 32; off > 0; off >>= 1) {
+        const float other = __shfl_down(acc, off, 64);
+        if ((t & 63) + off < wave_lanes) acc += other;
+      }
       if ((t & 63) == 0) partial[((size_t)o * ntiles + ti) * WAVES + (t >> 6)] = acc;
     }
   }
@@ -1437,12 +1434,15 @@ __global__ __launch_bounds__(256) void k_pick_max_maps(const float* __restrict__
   }
 }
 
-// Column tiles of k_pick_project_blue that hold a column inside the disc.
-std::vector<int> blue_tiles(int n) {
+// Column tiles of k_pick_project_line that hold a column inside the disc, and waves of a tile.
+std::vector<int> line_tiles(int n, int* waves) {
   std::vector<int> out;
   const int nc = (n + 1) / 2, half = n / 2;
-  (void)with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
-    constexpr int TX = BlueShape<decltype(MC)::value>::TX;
+  const LineArgs A = line_shape(n, false);
+  (void)with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const int TX = 1 << LN::txlog(A);
+    *waves = (int)(col_threads<LN>(A) + 63) / 64;
     for (int w = 0; w * TX < nc * n; ++w) {
       bool in = false;
       for (int col = w * TX; col < std::min((w + 1) * TX, nc * n); ++col) {
@@ -1456,37 +1456,41 @@ std::vector<int> blue_tiles(int n) {
   return out;
 }
 
-// Resident workgroups of k_pick_project_blue on the whole device.
-int blue_grid1(int n, bool centred, int cus) {
+// Resident workgroups of k_pick_project_line on the whole device.
+int line_grid1(int n, bool centred, int cus) {
   int per_cu = 1;
-  (void)with_blue_len(blue_fused_len(n), [&](auto MC) -> int {
-    constexpr int M = decltype(MC)::value, NT = blue_threads<M>();
+  const LineArgs A = line_shape(n, false);
+  (void)with_line(A, [&](auto ln) -> int {
+    using LN = decltype(ln);
+    const int nt = (int)col_threads<LN>(A);
     const hipError_t e =
-        centred ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_blue<M, CentredProjector>, NT, 0)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_blue<M, Projector>, NT, 0);
+        centred ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_line<LN, CentredProjector>, nt,
+                                                               col_lds<LN>(A))
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pick_project_line<LN, Projector>, nt,
+                                                               col_lds<LN>(A));
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     return GTOMX_OK;
   });
   return per_cu * cus;
 }
 
-// Sides up to 512 without a native transform: project + chirp-z along z, the
-// correction and the scale, chirp-z along y in place, then the row pass per
+// Sides up to 512 without a native transform: project + z inverse, the
+// correction and the scale, the y inverse in place, then the row pass per
 // orientation group and the in-order merge.
 template <class PJ>
-int run_batch_blue(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, const float2* E,
-                   const float* ctf, float* best, int32_t* idx, int angle0, const float2* tw, hipStream_t s) {
+int run_batch_line(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float* mats, int nb, const float2* E,
+                   const float* ctf, float* best, int32_t* idx, int angle0, hipStream_t s) {
   const int n = pl->n;
-  BlueTables t;
-  GX_TRY(blue_tables(n, &t));
+  LineArgs A;
+  GX_TRY(line_args(n, false, &A));
   GX_TRY(timed(pl, 0, s, [&]() -> int {
-    return with_blue_len(t.M, [&](auto MC) -> int {
-      constexpr int M = decltype(MC)::value;
-      hipLaunchKernelGGL((k_pick_project_blue<M, PJ>),
+    return with_line(A, [&](auto ln) -> int {
+      using LN = decltype(ln);
+      hipLaunchKernelGGL((k_pick_project_line<LN, PJ>),
                          dim3(pl->grid1[std::is_same<PJ, CentredProjector>::value ? 1 : 0]),
-                         dim3(blue_threads<M>()), 0, s, PS, mats, nb, E, ctf, pl->G, pl->partial, n,
-                         pl->tiles, pl->ntiles, t.chirp, t.bi, tw);
-      GX_LAUNCHED("k_pick_project_blue");
+                         dim3(col_threads<LN>(A)), col_lds<LN>(A), s, PS, mats, nb, E, ctf, pl->G, pl->partial,
+                         pl->tiles, pl->ntiles, A);
+      GX_LAUNCHED("k_pick_project_line");
       return GTOMX_OK;
     });
   }));
@@ -1497,7 +1501,7 @@ int run_batch_blue(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const 
     hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, pl->nparts, pl->corr, HERM_BLOCKS,
                        (double)pl->H, reinterpret_cast<float*>(pl->sn), 2);
     GX_LAUNCHED("k_pick_scale");
-    return blue_search_y(n, pl->G, nb, s);
+    return line_search_y(n, pl->G, nb, s);
   }));
   return timed(pl, 2, s, [&]() -> int {
     const long long stride = (long long)((n + 1) / 2) * n * n;
@@ -1551,8 +1555,8 @@ int run_batch_n(gtomx_pick_plan* pl, const CentredProjector* C, const Projector&
   if (pl->n > 256 || pl->gen3d) {
     if (tmask) return fail(GTOMX_ERR_UNSUPPORTED, "tile masks need volumes of side 2^a or 3*2^a, at most 256");
     if (pl->gen3d && rows_max_any_fused(pl->n))
-      return C ? run_batch_blue(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, tw, s)
-               : run_batch_blue(pl, P, P, mats, nb, E, ctf, best, idx, angle0, tw, s);
+      return C ? run_batch_line(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, s)
+               : run_batch_line(pl, P, P, mats, nb, E, ctf, best, idx, angle0, s);
     return C ? run_batch3d_any(pl, *C, P, mats, nb, E, ctf, best, idx, angle0, s)
              : run_batch3d_any(pl, P, P, mats, nb, E, ctf, best, idx, angle0, s);
   }
@@ -1961,10 +1965,10 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   // orientations of 64^3 at 256 against 2.68 ms at 16)
   pl->B = batch ? batch : (is2d ? (big2d ? big_b : 240u) : (any3d ? big3_b : (dv.x >= 128 ? 128u : 256u)));
   pl->gen3d = gen3d;
-  const bool blue = gen3d && rows_max_any_fused(dv.x);  // chirp-z lines inside the search's own passes
+  const bool line = gen3d && rows_max_any_fused(dv.x);  // lines inside the search's own passes
   // small ones: as many as the native sides take while their spectra stay near 512 MB (75^3: 29 per pass
   // left half the device idle)
-  if (blue && !batch)
+  if (line && !batch)
     pl->B = (unsigned)std::max<size_t>(pl->B, std::min<size_t>(256, (512ull << 20) / (pl->H * sizeof(float2))));
   int L1 = 0, L2 = 0;
   if (big2d && fft_len_split(dv.x, &L1, &L2) != GTOMX_OK) {
@@ -1973,15 +1977,11 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   }
   pl->nparts = big2d ? (dv.x / 2 + 1 + 63) / 64 * L2
                      : (any3d ? (int)((pl->H + 256 * P3_BINS - 1) / (256 * P3_BINS)) : 0);
+  int waves = 0;
   const std::vector<int> tiles =
-      blue ? blue_tiles(pl->n) : ((is2d || any3d) ? std::vector<int>{0} : tiles_for(pl->n));
-  pl->ntiles = blue ? (int)tiles.size() : ((big2d || any3d) ? 1 : (is2d ? g2_tiles_for(pl->n) : (int)tiles.size()));
-  if (blue)
-    GX_TRY(with_blue_len(blue_fused_len(pl->n), [&](auto MC) -> int {
-      using S = BlueShape<decltype(MC)::value>;
-      pl->nparts = pl->ntiles * ((S::TX * S::R2 + 63) / 64);
-      return GTOMX_OK;
-    }));
+      line ? line_tiles(pl->n, &waves) : ((is2d || any3d) ? std::vector<int>{0} : tiles_for(pl->n));
+  pl->ntiles = line ? (int)tiles.size() : ((big2d || any3d) ? 1 : (is2d ? g2_tiles_for(pl->n) : (int)tiles.size()));
+  if (line) pl->nparts = pl->ntiles * waves;
   int s = GTOMX_OK;
   hipError_t he = hipGetDevice(&pl->device);
   if (he != hipSuccess) {
@@ -2010,8 +2010,8 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   alloc(&d, (size_t)pl->B * gstride * sizeof(float2));
   pl->G = static_cast<float2*>(d);
   d = nullptr;
-  // up to 4 pass-1 waves per tile; above 256, one sum per pass-1 workgroup
-  alloc(&d, (size_t)pl->B * ((big2d || any3d) ? (size_t)pl->nparts : (size_t)pl->ntiles * 4) * sizeof(float));
+  // up to 4 pass-1 waves per tile; one sum per wave of the generic sides, per pass-1 workgroup above 256
+  alloc(&d, (size_t)pl->B * ((big2d || any3d || line) ? (size_t)pl->nparts : (size_t)pl->ntiles * 4) * sizeof(float));
   pl->partial = static_cast<float*>(d);
   d = nullptr;
   alloc(&d, (size_t)pl->ntiles * sizeof(int));
@@ -2057,8 +2057,8 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
     plan_release(pl);
     return hip_fail(he, "plan set-up");
   }
-  pl->grid1[0] = blue ? blue_grid1(pl->n, false, cus) : resident_grid_for(pl->n, false, cus);
-  pl->grid1[1] = blue ? blue_grid1(pl->n, true, cus) : resident_grid_for(pl->n, true, cus);
+  pl->grid1[0] = line ? line_grid1(pl->n, false, cus) : resident_grid_for(pl->n, false, cus);
+  pl->grid1[1] = line ? line_grid1(pl->n, true, cus) : resident_grid_for(pl->n, true, cus);
   he = hipEventCreateWithFlags(&pl->mats_ev, hipEventDisableTiming);
   if (he != hipSuccess) {
     plan_release(pl);

@@ -219,7 +219,7 @@ int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int ang
                  int32_t* idx, int og, hipStream_t s);
 // The y inverse, in place, of nb n^3 search spectra (planes z of n rows of (n + 1) / 2
 // bins) whose bins outside the disc x^2 + y^2 <= (n/2)^2 read as zero; n at most 512.
-int blue_search_y(int n, float2* G, int nb, hipStream_t s);
+int line_search_y(int n, float2* G, int nb, hipStream_t s);
 // Folds `groups` maxima of v values each (gbest, gidx) into best / idx in group
 // order (strict >), for each of `items` (pick.hip).
 int merge_group_maxima(const float* gbest, const int32_t* gidx, int groups, size_t v, float* best, int32_t* idx,

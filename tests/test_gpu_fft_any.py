@@ -1,5 +1,5 @@
 """R2C / C2R transforms with extents that have no native kernel (odd lengths,
-other prime factors, up to 2048) by the chirp-z form, alone and mixed with
+other prime factors, up to 2048) by mixed-radix lines or the chirp-z form, alone and mixed with
 native axes, against numpy's FP64 pocketfft (R2C, and C2R of Hermitian
 spectra) and the oracle's real-part C2R (non-Hermitian half spectra). cuFFT
 behind d_FFTR2C / d_IFFTC2R (src/FFT/FFT.cu:17-42, src/FFT/IFFT.cu:8-56) plans
@@ -118,6 +118,28 @@ def test_fft_any_edges_of_the_fused_lengths(gx, cuda, n):
     import torch
     rng = np.random.default_rng(n)
     for shape in ((3, 5, n), (3, n, 6), (n, 3, 10)):  # the length along x, y and z
+        x = rng.standard_normal(shape).astype(np.float32)
+        X = gx.d_FFTR2C(torch.from_numpy(x[None]).to(cuda))
+        assert rel_linf(to_np(X)[0], np.fft.rfftn(x.astype(np.float64))) < TOL, shape
+        back = gx.d_IFFTC2R(X, shape[2])
+        assert rel_linf(to_np(back)[0], x) < TOL, shape
+
+
+def _smooth(n):
+    for p in (2, 3, 5, 7):
+        while n % p == 0:
+            n //= p
+    return n == 1
+
+
+@pytest.mark.parametrize("axis", ["x", "y", "z"])
+def test_fft_any_small_factors(gx, cuda, axis):
+    """Every length up to 512 of the factors 2, 3, 5, 7: the mixed-radix lines (each split of rows
+    and of columns, one and two inner stages), the native and the chirp-z lengths among them."""
+    import torch
+    rng = np.random.default_rng(7)
+    for n in [n for n in range(12, 513) if _smooth(n)]:
+        shape = {"x": (3, 5, n), "y": (2, n, 38), "z": (n, 3, 6)}[axis]
         x = rng.standard_normal(shape).astype(np.float32)
         X = gx.d_FFTR2C(torch.from_numpy(x[None]).to(cuda))
         assert rel_linf(to_np(X)[0], np.fft.rfftn(x.astype(np.float64))) < TOL, shape
