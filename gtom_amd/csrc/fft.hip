@@ -1155,7 +1155,19 @@ __global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols(const float2* src
 }
 
 // Rows, two to a transform: one as the real, one as the imaginary part. A pair's
-// threads are lanes of one wave, so the exchanges need no barrier.
+// threads are lanes of one wave, so the exchanges need no barrier. The `per` rows of a
+// batch item pair among themselves, an odd last one alone: what one item holds (another
+// scale, a NaN) does not reach the next.
+struct RowPairs {
+  unsigned pairs, per, ppi;  // pairs in all, rows and pairs of an item
+  RowPairs(long long nrows, long long per_)
+      : pairs((unsigned)(nrows / per_ * ((per_ + 1) / 2))), per((unsigned)per_), ppi((unsigned)((per_ + 1) / 2)) {}
+  __device__ long long row(unsigned pair, bool* two) const {
+    const unsigned item = pair / ppi, r = 2 * (pair - item * ppi);
+    *two = r + 1 < per;
+    return (long long)item * per + r;
+  }
+};
 // z[p] = A[p] + i B[p] of two half-spectrum rows completed as X[L - q] = conj X[q],
 // without the imaginary parts of X[0] and X[L/2] (the real part of the inverse).
 __device__ __forceinline__ float2 row_pair_bin(const float2* __restrict__ a, const float2* __restrict__ b, bool va,
@@ -1170,7 +1182,7 @@ __device__ __forceinline__ float2 row_pair_bin(const float2* __restrict__ a, con
 
 template <class LN>
 __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_c2r(const float2* __restrict__ in,
-                                                                      float* __restrict__ out, long long nrows,
+                                                                      float* __restrict__ out, RowPairs rp,
                                                                       float scale, LineArgs A) {
   float2* lds = line_lds<LN::ROW_LDS>();
   const int t = threadIdx.x, L = A.L, lanes = LN::lanes(A), pitch = LN::row_pitch(A), pairs = row_pairs<LN>(A);
@@ -1180,10 +1192,11 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_c2r(const floa
   __syncthreads();
   if (slot < 0) return;  // no barrier below
   float2* xch = lds + LN::tables(A) + slot * LN::row_area(A);
-  const long long step = 2LL * pairs * gridDim.x;
-  for (long long row = 2 * ((long long)blockIdx.x * pairs + slot); row < nrows; row += step) {
+  const unsigned step = pairs * gridDim.x;
+  for (unsigned pair = blockIdx.x * pairs + slot; pair < rp.pairs; pair += step) {
     const int nh = L / 2 + 1;
-    const bool two = row + 1 < nrows;
+    bool two;
+    const long long row = rp.row(pair, &two);
     const float2* a = in + row * nh;
     float2 v[LN::REGS];
 #pragma unroll
@@ -1207,7 +1220,7 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_c2r(const floa
 // With pm.n0 the rows hold that many reals, padded to L on load.
 template <class LN>
 __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                       long long nrows, LineArgs A, PadMap pm) {
+                                                       RowPairs rp, LineArgs A, PadMap pm) {
   float2* lds = line_lds<LN::ROW_LDS>();
   const int t = threadIdx.x, L = A.L, lanes = LN::lanes(A), pitch = LN::row_pitch(A), pairs = row_pairs<LN>(A);
   int j;
@@ -1216,10 +1229,11 @@ __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__
   __syncthreads();
   if (slot < 0) return;  // no barrier below
   float2* xch = lds + LN::tables(A) + slot * LN::row_area(A);
-  const long long step = 2LL * pairs * gridDim.x;
-  for (long long row = 2 * ((long long)blockIdx.x * pairs + slot); row < nrows; row += step) {
+  const unsigned step = pairs * gridDim.x;
+  for (unsigned pair = blockIdx.x * pairs + slot; pair < rp.pairs; pair += step) {
     const int nh = L / 2 + 1;
-    const bool two = row + 1 < nrows;
+    bool two;
+    const long long row = rp.row(pair, &two);
     const int len = pm.n0 ? pm.n0 : L;
     const float* a = in + row * len;
     float2 v[LN::REGS];
@@ -1924,27 +1938,28 @@ int line_cols(int L, const float2* src, float2* dst, int width, long long as, lo
   });
 }
 
-// The fused form on nrows contiguous rows of L reals / L/2 + 1 bins.
-int line_rows_r2c(int L, const float* in, float2* out, long long nrows, hipStream_t s, PadMap pm = PadMap{}) {
+// The fused form on nrows contiguous rows of L reals / L/2 + 1 bins, `per` to a batch item.
+int line_rows_r2c(int L, const float* in, float2* out, long long nrows, long long per, hipStream_t s,
+                  PadMap pm = PadMap{}) {
+  const RowPairs rp(nrows, per);
   LineArgs A;
   GX_TRY(line_args(L, true, &A));
   return with_line(A, [&](auto ln) -> int {
     using LN = decltype(ln);
-    const long long per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
-    hipLaunchKernelGGL(k_line_rows_r2c<LN>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), row_lds<LN>(A), s,
-                       in, out, nrows, A, pm);
+    const unsigned n = row_pairs<LN>(A), wgs = (unsigned)(((long long)rp.pairs + n - 1) / n);
+    hipLaunchKernelGGL(k_line_rows_r2c<LN>, dim3(std::min(wgs, 4096u)), dim3(256), row_lds<LN>(A), s, in, out, rp, A, pm);
     GX_LAUNCHED("k_line_rows_r2c");
     return GTOMX_OK;
   });
 }
-int line_rows_c2r(int L, const float2* in, float* out, long long nrows, float scale, hipStream_t s) {
+int line_rows_c2r(int L, const float2* in, float* out, long long nrows, long long per, float scale, hipStream_t s) {
+  const RowPairs rp(nrows, per);
   LineArgs A;
   GX_TRY(line_args(L, true, &A));
   return with_line(A, [&](auto ln) -> int {
     using LN = decltype(ln);
-    const long long per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
-    hipLaunchKernelGGL(k_line_rows_c2r<LN>, dim3((unsigned)std::min<long long>(wgs, 4096)), dim3(256), row_lds<LN>(A), s,
-                       in, out, nrows, scale, A);
+    const unsigned n = row_pairs<LN>(A), wgs = (unsigned)(((long long)rp.pairs + n - 1) / n);
+    hipLaunchKernelGGL(k_line_rows_c2r<LN>, dim3(std::min(wgs, 4096u)), dim3(256), row_lds<LN>(A), s, in, out, rp, scale, A);
     GX_LAUNCHED("k_line_rows_c2r");
     return GTOMX_OK;
   });
@@ -2055,7 +2070,7 @@ int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, 
     }
     GX_LAUNCHED("k_rows_r2c");
   } else {
-    GX_TRY(line_rows_r2c(di.x, r, rows, nrows, s, px));
+    GX_TRY(line_rows_r2c(di.x, r, rows, nrows, (long long)dr.y * dr.z, s, px));
   }
   // y: every plane of the small volume
   const int planes = (int)(dr.z * nb);
@@ -2218,7 +2233,7 @@ int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipS
     else
       GX_TRY(launch_rows_r2c(d.x, in, out, rows, tw, s));
   } else if (d.x <= BLUE_FUSED_MAX) {
-    GX_TRY(line_rows_r2c(d.x, in, out, rows, s));
+    GX_TRY(line_rows_r2c(d.x, in, out, rows, (long long)d.y * d.z, s));
   } else {
     GX_TRY((blue_axis<1, 1, -1>(in, AxisLines{1LL << 62, d.x, 0, 1}, out, AxisLines{1LL << 62, nh, 0, 1}, rows, d.x,
                                 (int)nh, 1.f, s)));
@@ -2236,7 +2251,7 @@ int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float sc
     if (d.x > 256) return launch_rows_long<false>(d.x, work, out, rows, scale, tw, s);
     return launch_rows_c2r(d.x, work, out, rows, scale, tw, s);
   }
-  if (d.x <= BLUE_FUSED_MAX) return line_rows_c2r(d.x, work, out, rows, scale, s);
+  if (d.x <= BLUE_FUSED_MAX) return line_rows_c2r(d.x, work, out, rows, (long long)d.y * d.z, scale, s);
   return blue_axis<2, 2, 1>(work, AxisLines{1LL << 62, nh, 0, 1}, out, AxisLines{1LL << 62, d.x, 0, 1}, rows, d.x,
                             (int)nh, scale, s);
 }

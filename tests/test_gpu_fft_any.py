@@ -145,3 +145,20 @@ def test_fft_any_small_factors(gx, cuda, axis):
         assert rel_linf(to_np(X)[0], np.fft.rfftn(x.astype(np.float64))) < TOL, shape
         back = gx.d_IFFTC2R(X, shape[2])
         assert rel_linf(to_np(back)[0], x) < TOL, shape
+
+
+@pytest.mark.parametrize("ndims,shape", [(1, (5, 75)), (1, (4, 97)), (2, (3, 75, 50)), (2, (2, 31, 33)), (3, (2, 3, 5, 75))])
+def test_fft_any_batch_items_are_independent(gx, cuda, ndims, shape):
+    """Rows are transformed in pairs; an item of a batch that is not finite, or of another scale,
+    leaves the others as they are alone, bit for bit."""
+    import torch
+    rng = np.random.default_rng(shape[-1])
+    x = torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(cuda)
+    x[0] = float("nan")
+    x[-1] *= 1e6
+    X = gx.d_FFTR2C(x, ndims=ndims)
+    back = gx.d_IFFTC2R(X, shape[-1], ndims=ndims)
+    for i in range(1, shape[0]):
+        Xi = gx.d_FFTR2C(x[i:i + 1].contiguous(), ndims=ndims)
+        assert torch.equal(X[i:i + 1], Xi) and torch.isfinite(torch.view_as_real(Xi)).all()
+        assert torch.equal(back[i:i + 1], gx.d_IFFTC2R(Xi, shape[-1], ndims=ndims))
