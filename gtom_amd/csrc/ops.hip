@@ -23,6 +23,12 @@ inline unsigned grid_for(size_t n, unsigned cap = 1u << 20) {
 __global__ void k_fill_f32(float* d, size_t n, float v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = v;
 }
+__global__ void k_fill_search(float* best, int32_t* idx, size_t n) {
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+    best[i] = -1e30f;
+    idx[i] = 0;
+  }
+}
 __global__ void k_fill_i32(int32_t* d, size_t n, int32_t v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = v;
 }
@@ -150,14 +156,27 @@ __global__ void k_sphere_mask_ex(const float* in, float* out, int3 d, double rad
 // The soft sphere already moved to the origin: value at index i is the mask at
 // the position r with ifftshift(r) = i (d_SphereMask then d_RemapFull2FullFFT,
 // src/Generics/LocalStd.cu:24-26).
-__global__ void k_sphere_mask_ifftshift(float* out, int3 d, double radius, double sigma) {
-  size_t total = (size_t)d.x * d.y * d.z;
+// Its sum goes to one partial per block.
+__global__ __launch_bounds__(TPB) void k_sphere_mask_sum(float* out, int3 d, double radius, double sigma,
+                                                         double* partial) {
+  __shared__ double red[TPB];
+  const size_t total = (size_t)d.x * d.y * d.z;
+  double s = 0;
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    int x = (int)(i % d.x), y = (int)((i / d.x) % d.y), z = (int)(i / ((size_t)d.x * d.y));
-    int sx = (x + d.x - (d.x + 1) / 2) % d.x, sy = (y + d.y - (d.y + 1) / 2) % d.y,
-        sz = (z + d.z - (d.z + 1) / 2) % d.z;
-    out[i] = sphere_value(sx, sy, sz, d, radius, sigma);
+    const int x = (int)(i % d.x), y = (int)((i / d.x) % d.y), z = (int)(i / ((size_t)d.x * d.y));
+    const int sx = (x + d.x - (d.x + 1) / 2) % d.x, sy = (y + d.y - (d.y + 1) / 2) % d.y,
+              sz = (z + d.z - (d.z + 1) / 2) % d.z;
+    const float m = sphere_value(sx, sy, sz, d, radius, sigma);
+    out[i] = m;
+    s += m;
   }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = TPB / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
 // Two-stage deterministic double sum: stage 1 writes one partial per block.
@@ -215,6 +234,14 @@ __global__ void k_mask_fourier(float2* mft, const float* fm, size_t n, double* m
 __global__ void k_local_std_combine(const float* c1, const float* c2, const double* masksum, size_t n,
                                     double invN, const double* mapsum, float* std_out, float* mean_out, float* best,
                                     const int32_t* idx, float* angle_out) {
+  const size_t o = blockIdx.y * n;  // volume of a batch
+  c1 += o;
+  c2 += o;
+  if (best) best += o;
+  if (angle_out) {
+    idx += o;
+    angle_out += o;
+  }
   const double M = *masksum;
   const double mu = mapsum ? *mapsum * invN : 0.0;
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
@@ -225,6 +252,44 @@ __global__ void k_local_std_combine(const float* c1, const float* c2, const doub
     if (mean_out) mean_out[i] = (float)(a / M + mu);
     if (best) best[i] = fabsf(sd) > 1e-15f ? best[i] / sd : 0.f;
     if (angle_out) angle_out[i] = (float)idx[i];
+  }
+}
+
+// r = (r - mean)^2 of the maps r = C2R_u(E): their mean is E's DC bin.
+__global__ void k_square_centred(float* __restrict__ r, const float2* __restrict__ E, size_t V, size_t H) {
+  const float mu = E[blockIdx.y * H].x;
+  r += blockIdx.y * V;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < V; i += (size_t)gridDim.x * blockDim.x) {
+    const float t = r[i] - mu;
+    r[i] = t * t;
+  }
+}
+
+// A = the spectrum of the map C2R_u(E) without its mean, times conj(M); B *= conj(M).
+// The map sees the Hermitian part of E, which differs from E on the columns x = 0 and
+// x = d.x / 2 only: V (E[k] + conj E[-k]) / 2 there, V E[k] elsewhere.
+__global__ void k_local_std_product(const float2* __restrict__ E, const float2* __restrict__ M, int3 d,
+                                    float2* __restrict__ A, float2* __restrict__ B, size_t H) {
+  E += blockIdx.y * H;
+  A += blockIdx.y * H;
+  B += blockIdx.y * H;
+  const unsigned nh = d.x / 2 + 1;
+  const float V = (float)((double)d.x * d.y * d.z);
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < H; i += (size_t)gridDim.x * blockDim.x) {
+    const size_t row = i / nh;
+    const unsigned x = (unsigned)(i - row * nh);
+    float2 e = E[i];
+    if (x == 0 || 2 * x == (unsigned)d.x) {
+      const unsigned y = (unsigned)(row % d.y), z = (unsigned)(row / d.y);
+      const size_t my = y == 0 ? 0 : d.y - y, mz = z == 0 ? 0 : d.z - z;
+      const float2 f = E[(mz * d.y + my) * nh + x];
+      e = make_float2(0.5f * (e.x + f.x), 0.5f * (e.y - f.y));
+    }
+    const float v = i == 0 ? 0.f : V;
+    const float2 m = M[i], b = B[i];
+    const float2 a = make_float2(v * e.x, v * e.y);
+    A[i] = make_float2(a.x * m.x + a.y * m.y, a.y * m.x - a.x * m.y);
+    B[i] = make_float2(b.x * m.x + b.y * m.y, b.y * m.x - b.x * m.y);
   }
 }
 
@@ -360,6 +425,11 @@ int fill_f32(float* d, size_t n, float v, hipStream_t s) {
   GX_LAUNCHED("k_fill_f32");
   return GTOMX_OK;
 }
+int fill_search(float* best, int32_t* idx, size_t n, hipStream_t s) {
+  hipLaunchKernelGGL(k_fill_search, dim3(grid_for(n)), dim3(TPB), 0, s, best, idx, n);
+  GX_LAUNCHED("k_fill_search");
+  return GTOMX_OK;
+}
 int fill_i32(int32_t* d, size_t n, int32_t v, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n)), dim3(TPB), 0, s, d, n, v);
   GX_LAUNCHED("k_fill_i32");
@@ -375,13 +445,6 @@ int mul_conj_inplace(float2* a, const float2* b, size_t n, hipStream_t s) {
   GX_LAUNCHED("k_mul_conj_inplace");
   return GTOMX_OK;
 }
-int sphere_mask_ifftshift(float* out, gtomx_int3 d, float radius, float sigma, hipStream_t s) {
-  size_t n = elements(d);
-  hipLaunchKernelGGL(k_sphere_mask_ifftshift, dim3(grid_for(n)), dim3(TPB), 0, s, out, make_int3(d.x, d.y, d.z),
-                     (double)radius, (double)sigma);
-  GX_LAUNCHED("k_sphere_mask_ifftshift");
-  return GTOMX_OK;
-}
 // scratch must hold 257 doubles; the sum lands in scratch[256].
 int sum_f64(const float* d, size_t n, double* scratch, hipStream_t s) {
   hipLaunchKernelGGL(k_sum_stage1, dim3(256), dim3(TPB), 0, s, d, n, scratch);
@@ -392,8 +455,8 @@ int sum_f64(const float* d, size_t n, double* scratch, hipStream_t s) {
 }
 int local_std_combine(const float* c1, const float* c2, const double* d_masksum, size_t n, float* std_out,
                       float* mean_out, float* best, const int32_t* idx, float* angle_out, hipStream_t s,
-                      const double* d_mapsum) {
-  hipLaunchKernelGGL(k_local_std_combine, dim3(grid_for(n)), dim3(TPB), 0, s, c1, c2, d_masksum, n,
+                      const double* d_mapsum, unsigned nvolumes) {
+  hipLaunchKernelGGL(k_local_std_combine, dim3(grid_for(n), nvolumes), dim3(TPB), 0, s, c1, c2, d_masksum, n,
                      1.0 / (double)n, d_mapsum, std_out, mean_out, best, idx, angle_out);
   GX_LAUNCHED("k_local_std_combine");
   return GTOMX_OK;
@@ -401,7 +464,7 @@ int local_std_combine(const float* c1, const float* c2, const double* d_masksum,
 
 // Local standard deviation (d_LocalStd, src/Generics/LocalStd.cu:10-118).
 // Scratch layout: maskft, aft, bft (H complex each), rbuf (mask, then map^2),
-// c1, c2 (V floats each), then 257 doubles.
+// c1, c2 (V floats each), then LS_DOUBLES doubles.
 
 size_t local_std_scratch_bytes(gtomx_int3 d) {
   size_t H = elements_ft(d), V = elements(d);
@@ -427,8 +490,12 @@ LocalStdScratch local_std_carve(void* base, gtomx_int3 d) {
 // Mask FT and mask sum for a radius (once per call), optionally under a Fourier mask.
 int local_std_prepare(const LocalStdScratch& sc, gtomx_int3 d, float radius, hipStream_t s,
                       const float* fouriermask) {
-  GX_TRY(sphere_mask_ifftshift(sc.rbuf, d, radius, 1.0f, s));
-  GX_TRY(sum_f64(sc.rbuf, elements(d), sc.dsum, s));
+  const unsigned parts = grid_for(elements(d), LS_MASKPARTS);
+  hipLaunchKernelGGL(k_sphere_mask_sum, dim3(parts), dim3(TPB), 0, s, sc.rbuf, make_int3(d.x, d.y, d.z),
+                     (double)radius, 1.0, sc.dsum + LS_MAPSUM + 1);
+  GX_LAUNCHED("k_sphere_mask_sum");
+  hipLaunchKernelGGL(k_sum_stage2, dim3(1), dim3(TPB), 0, s, sc.dsum + LS_MAPSUM + 1, (int)parts, sc.dsum + 256);
+  GX_LAUNCHED("k_sum_stage2");
   GX_TRY(fft_r2c(sc.rbuf, sc.maskft, d, 1, s));
   if (fouriermask) {
     const size_t H = elements_ft(d);
@@ -439,10 +506,10 @@ int local_std_prepare(const LocalStdScratch& sc, gtomx_int3 d, float radius, hip
   return GTOMX_OK;
 }
 
-// sigma (and optional mean) of one map; with best != nullptr the best map is divided in place.
-// The map's global mean (double sum) is subtracted before the convolutions.
+// sigma (and optional mean) of one map. The map's global mean (double sum) is
+// subtracted before the convolutions.
 int local_std_apply(const LocalStdScratch& sc, const float* map, gtomx_int3 d, float* std_out, float* mean_out,
-                    float* best, const int32_t* idx, float* angle_out, hipStream_t s) {
+                    hipStream_t s) {
   size_t V = elements(d), H = elements_ft(d);
   double* mapsum = sc.dsum + LS_MAPSUM;
   GX_TRY(sum_f64(map, V, mapsum - 256, s));
@@ -455,8 +522,26 @@ int local_std_apply(const LocalStdScratch& sc, const float* map, gtomx_int3 d, f
   GX_TRY(mul_conj_inplace(sc.bft, sc.maskft, H, s));
   GX_TRY(fft_c2r(sc.aft, sc.aft, sc.c1, d, 1, 1.0f, s));
   GX_TRY(fft_c2r(sc.bft, sc.bft, sc.c2, d, 1, 1.0f, s));
-  GX_TRY(local_std_combine(sc.c1, sc.c2, sc.dsum + 256, V, std_out, mean_out, best, idx, angle_out, s, mapsum));
-  return GTOMX_OK;
+  return local_std_combine(sc.c1, sc.c2, sc.dsum + 256, V, std_out, mean_out, nullptr, nullptr, nullptr, s, mapsum);
+}
+
+// The maps come as spectra: their mean is the DC bin and their spectrum is at hand, so
+// the sum and one of the two R2C fall away, and a batch shares its launches (32^3: 18
+// launches of 3 to 5 us a search instead of 28, and 22 fewer for each further volume).
+int local_std_divide(const LocalStdScratch& sc, float2* spectra, float* maps, const float2* E, gtomx_int3 d,
+                     unsigned nv, float* best, const int32_t* idx, float* angle_out, hipStream_t s) {
+  const size_t V = elements(d), H = elements_ft(d);
+  float2 *A = spectra, *B = spectra + nv * H;
+  GX_TRY(fft_c2r(E, B, maps, d, nv, 1.0f, s));
+  hipLaunchKernelGGL(k_square_centred, dim3(grid_for(V), nv), dim3(TPB), 0, s, maps, E, V, H);
+  GX_LAUNCHED("k_square_centred");
+  GX_TRY(fft_r2c(maps, B, d, nv, s));
+  hipLaunchKernelGGL(k_local_std_product, dim3(grid_for(H), nv), dim3(TPB), 0, s, E, sc.maskft,
+                     make_int3(d.x, d.y, d.z), A, B, H);
+  GX_LAUNCHED("k_local_std_product");
+  GX_TRY(fft_c2r(spectra, spectra, maps, d, 2 * nv, 1.0f, s));
+  return local_std_combine(maps, maps + nv * V, sc.dsum + 256, V, nullptr, nullptr, best, idx, angle_out, s, nullptr,
+                           nv);
 }
 
 int project_launch(const float2* vol, int p, float2* out, int n, unsigned rmax, const float* d_mats,
@@ -721,7 +806,7 @@ int gtomx_local_std(const float* d_map, gtomx_int3 dims, const float* d_fourierm
   LocalStdScratch sc = local_std_carve(sb.p, dims);
   hipStream_t s = as_stream(stream);
   GX_TRY(local_std_prepare(sc, dims, localradius, s, d_fouriermask));
-  GX_TRY(local_std_apply(sc, d_map, dims, d_std, d_mean, nullptr, nullptr, nullptr, s));
+  GX_TRY(local_std_apply(sc, d_map, dims, d_std, d_mean, s));
   GX_HIP(hipStreamSynchronize(s));
   return GTOMX_OK;
 }

@@ -2003,7 +2003,7 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
     s = dev_alloc(dst, bytes);
     if (s == GTOMX_OK) pl->device_bytes += bytes;
   };
-  // The batch buffer also serves as the C2R workspace in pick_finish (H elements)
+  // The batch buffer also serves as workspace in pick_finish (whole half spectra)
   // and holds whole half spectra in the split-precision search.
   const size_t gstride =
       std::max(pl->H, (big2d || any3d) ? pl->H : (is2d ? g2_stride_for(pl->n) : g_stride_for(pl->n)));
@@ -2135,8 +2135,7 @@ int gtomx_pick_begin(gtomx_pick_plan* plan, gtomx_int3 dimsvolume, unsigned nvol
   hipStream_t s = as_stream(stream);
   GX_TRY(plan->fence.enter(s));
   // d_ValueFill best = -1e30, angle = 0 (src/Correlation/SubTomograms.cu:41-42)
-  GX_TRY(fill_f32(d_best, plan->V * nvolumes, -1e30f, s));
-  GX_TRY(fill_i32(d_idx, plan->V * nvolumes, 0, s));
+  GX_TRY(fill_search(d_best, d_idx, plan->V * nvolumes, s));
   return plan->fence.leave(s);
 }
 
@@ -2180,13 +2179,18 @@ int gtomx_pick_finish(gtomx_pick_plan* plan, const gtomx_complex* d_expft, gtomx
   hipStream_t s = as_stream(stream);
   GX_TRY(plan->fence.enter(s));
   GX_TRY(local_std_prepare(plan->ls, dimsvolume, maskradius, s));
-  for (unsigned v = 0; v < nvolumes; ++v) {
-    const float2* Ev = reinterpret_cast<const float2*>(d_expft) + (size_t)v * plan->H;
-    // e = C2R_u(E_v) (src/Correlation/SubTomograms.cu:105); the batch buffer is the workspace.
-    GX_TRY(fft_c2r(Ev, plan->G, plan->ebuf, dimsvolume, 1, 1.0f, s));
-    GX_TRY(local_std_apply(plan->ls, plan->ebuf, dimsvolume, nullptr, nullptr, d_best + (size_t)v * plan->V,
-                           d_idx + (size_t)v * plan->V, d_bestangle ? d_bestangle + (size_t)v * plan->V : nullptr,
-                           s));
+  // e = C2R_u(E_v) (src/Correlation/SubTomograms.cu:105) and its sigma, as many volumes at a time as the batch buffer
+  // has room for; one in the plan's own scratch.
+  const size_t per = 2 * (plan->H + (plan->V + 1) / 2);
+  const unsigned most = (unsigned)std::min<size_t>({nvolumes, 64, (size_t)plan->B * plan->H / per});
+  for (unsigned v = 0; v < nvolumes;) {
+    const unsigned nv = most > 1 ? std::min(most, nvolumes - v) : 1;
+    float2* spectra = most > 1 ? plan->G : plan->ls.aft;
+    float* maps = most > 1 ? reinterpret_cast<float*>(plan->G + 2 * nv * plan->H) : plan->ls.c1;
+    GX_TRY(local_std_divide(plan->ls, spectra, maps, reinterpret_cast<const float2*>(d_expft) + (size_t)v * plan->H,
+                            dimsvolume, nv, d_best + (size_t)v * plan->V, d_idx + (size_t)v * plan->V,
+                            d_bestangle ? d_bestangle + (size_t)v * plan->V : nullptr, s));
+    v += nv;
   }
   return plan->fence.leave(s);
 }

@@ -263,8 +263,8 @@ int image_times_conj(const float2* E, float2* P, size_t h, unsigned batch, hipSt
 
 // Element-wise helpers (ops.hip).
 int fill_f32(float* d, size_t n, float v, hipStream_t s);
+int fill_search(float* best, int32_t* idx, size_t n, hipStream_t s);  // -1e30, 0
 int fill_i32(int32_t* d, size_t n, int32_t v, hipStream_t s);
-int sphere_mask_ifftshift(float* out, gtomx_int3 dims, float radius, float sigma, hipStream_t s);
 int sum_f64(const float* d, size_t n, double* d_result, hipStream_t s);
 int mul_conj_inplace(float2* a, const float2* b, size_t n, hipStream_t s);
 int square_f32(const float* in, float* out, size_t n, hipStream_t s);
@@ -273,7 +273,7 @@ int square_f32(const float* in, float* out, size_t n, hipStream_t s);
 // d_mapsum (or nullptr): the map's sum; its mean was subtracted before the convolutions and is added back to the mean.
 int local_std_combine(const float* c1, const float* c2, const double* d_masksum, size_t n,
                       float* std_out, float* mean_out, float* best, const int32_t* idx,
-                      float* angle_out, hipStream_t s, const double* d_mapsum = nullptr);
+                      float* angle_out, hipStream_t s, const double* d_mapsum = nullptr, unsigned nvolumes = 1);
 
 // Local standard deviation chain (ops.hip). The scratch holds the mask FT,
 // two spectra, three real volumes and a few doubles.
@@ -287,14 +287,19 @@ struct LocalStdScratch {
   double* dsum;  // LS_DOUBLES doubles; the mask sum is dsum[256], the map sum dsum[LS_MAPSUM]
 };
 constexpr int LS_MAPSUM = 520;  // its 256 partials precede it
-constexpr int LS_DOUBLES = LS_MAPSUM + 1;
+constexpr int LS_MASKPARTS = 1024;  // partials of the mask sum, after the map sum
+constexpr int LS_DOUBLES = LS_MAPSUM + 1 + LS_MASKPARTS;
 size_t local_std_scratch_bytes(gtomx_int3 d);
 LocalStdScratch local_std_carve(void* base, gtomx_int3 d);
 // fouriermask: NULL, or a real half spectrum (FFT order) that scales the mask spectrum.
 int local_std_prepare(const LocalStdScratch& sc, gtomx_int3 d, float radius, hipStream_t s,
                       const float* fouriermask = nullptr);
 int local_std_apply(const LocalStdScratch& sc, const float* map, gtomx_int3 d, float* std_out, float* mean_out,
-                    float* best, const int32_t* idx, float* angle_out, hipStream_t s);
+                    hipStream_t s);
+// best /= sigma of the nv maps C2R_u(E) (0 where sigma is 0), and idx as floats into angle_out (or NULL). spectra:
+// 2 nv half spectra, maps: 2 nv real volumes of scratch (sc.aft and sc.c1 hold those of one).
+int local_std_divide(const LocalStdScratch& sc, float2* spectra, float* maps, const float2* E, gtomx_int3 d,
+                     unsigned nv, float* best, const int32_t* idx, float* angle_out, hipStream_t s);
 
 // Standalone projector launch (ops.hip).
 // nz = n: n^3 projections; nz = 1: n x n central sections (2D). volz: the
