@@ -379,6 +379,9 @@ __device__ __forceinline__ float2 twiddle_from(const float2* tw, int m, TwiddleL
   return DIR > 0 ? make_float2(w.x, -w.y) : w;
 }
 
+// Or an LDS copy for one split and direction: exp(DIR 2 pi i j k1 / N) at k1 R2 + j.
+template <int R2> struct TwiddleStage {};
+
 // What separates the writes of the exchange from its reads: the workgroup's
 // barrier, or, where the R2 threads of a transform are lanes of one wave and
 // nobody else touches their exchange area, the wave's own order (LDS accesses
@@ -393,26 +396,14 @@ struct SyncWave {
   }
 };
 
-// Or twiddles the thread holds in registers: w[k1] = exp(DIR 2 pi i j k1 / N)
-// for its j (w[0] unused), loaded once by load_two_step_twiddles.
-template <int R1> struct TwiddleRegs {
-  const float2 (&w)[R1];
-};
-template <int N, int R1, int DIR>
-__device__ __forceinline__ void load_two_step_twiddles(float2 (&w)[R1], int j, const float2* __restrict__ tw) {
-  w[0] = make_float2(1.f, 0.f);
-#pragma unroll
-  for (int k1 = 1; k1 < R1; ++k1) w[k1] = twiddle<DIR, N>(tw, j * k1);
-}
 template <int DIR, int N, class Src>
 __device__ __forceinline__ float2 stage_twiddle(const float2* tw, int j, int k1, Src src) {
   return twiddle_from<DIR, N>(tw, j * k1, src);
 }
-template <int DIR, int N, int R1>
-__device__ __forceinline__ float2 stage_twiddle(const float2*, int, int k1, TwiddleRegs<R1> src) {
-  return src.w[k1];
+template <int DIR, int N, int R2>
+__device__ __forceinline__ float2 stage_twiddle(const float2* tw, int j, int k1, TwiddleStage<R2>) {
+  return tw[k1 * R2 + j];
 }
-
 template <int N, int R1, int R2, int DIR, class Xch, class Src = TwiddleGlobal, class Sync = SyncGroup>
 __device__ __forceinline__ void fft_two_step(float2 (&v)[R1], int j, const float2* __restrict__ tw, Xch xch,
                                              Src src = Src{}, Sync sync = Sync{}) {

@@ -479,7 +479,16 @@ __global__ __launch_bounds__(Pass2Tile<N>::TX * ColShape<N>::R2) void k_pick_y(
 // best/bidx: orientation group blockIdx.y (og orientations from og*blockIdx.y)
 // of image blockIdx.z (whose nb spectra follow those of the images before it)
 // then writes its own maximum to best/bidx + (image * groups + group) * ROWS * N,
-// and k_pick_merge combines the groups in order.
+// and k_pick_merge combines the groups in order. nb is below 65,535.
+//
+// Bound by the reads of the batch, which need waves in flight: with the twiddles in
+// registers (64 of them at N = 256, 96 at 192) and an orientation per voxel one wave
+// fitted a SIMD at 192, two at 256. Both in LDS and packed: 192^3 x 288 orientations
+// 11.95 -> 9.2 ms, the whole search. More workgroups than three to a CU read too many
+// places of the batch at once: 256^3 x 128 orientations 2.03 ms with three, 2.16 with
+// two, 2.72 with four. Images take two: each group of orientations more is
+// another image to merge (16 images of 256^2 x 1,000 orientations: 3.8 ms with two, 4.6
+// with four).
 template <int N, class L = GLayout<N>, bool FRESH = false>
 __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G, int nb, int angle0,
                                                     const float2* __restrict__ sn, float* __restrict__ best,
@@ -488,9 +497,19 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
   constexpr int NC = N / 2;
   constexpr int R1 = RowShape<NC>::R1, R2 = RowShape<NC>::R2, RW = 256 / R2;
   constexpr int GS = R2 * (R1 + 2);  // two float2 of padding per thread slot (fewer bank conflicts than one)
-  __shared__ float2 xch[R2 > 1 ? RW * GS : 1];
+  constexpr unsigned NONE = 0xffffu;
+  // at most two workgroups to a CU for images, three for volumes, see above: 56 and 46 KB
+  constexpr int XCH = R2 > 1 ? RW * GS : 1, LEAST = FRESH ? 7168 : 5888;
+  __shared__ float2 xch[XCH > LEAST ? XCH : LEAST];
+  // W_N^k, and the stage twiddles W_NC^{j k1} at k1 R2 + j: a row's R2 lanes read neighbours
+  __shared__ float2 twp[NC], twh[R2 > 1 ? NC : 1];
   const int t = threadIdx.x, r = t / R2, j = t % R2;
   const int row = blockIdx.x * RW + r;  // row = z*N + y (volumes) or y (images)
+  for (int i = t; i < NC; i += 256) {
+    twp[i] = twiddle<1, N>(tw, i);
+    if (R2 > 1) twh[i] = twiddle<1, NC>(tw, i / R2 * (i % R2));
+  }
+  __syncthreads();
   // tile bits of this row (volumes with a mask): bit k covers x in [32k, 32k + 32)
   unsigned xbits = 0xffffffffu;
   if (!FRESH && tmask) {
@@ -510,27 +529,19 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
     bidx += ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * L::ROWS * N;
   }
 
+  // Two voxels' orientations in one register, 16-bit offsets (NONE: unchanged).
   float bv[2 * R1];
-  int32_t bi[2 * R1];
+  unsigned bi[R1];
   float2* bp = reinterpret_cast<float2*>(best + (size_t)row * N);
   int2* ip = reinterpret_cast<int2*>(bidx + (size_t)row * N);
 #pragma unroll
   for (int s = 0; s < R1; ++s) {
     const int m = out_index<R1, R2>(j, s);
     float2 b = valid && !FRESH ? bp[m] : make_float2(-__builtin_inff(), -__builtin_inff());
-    int2 a = valid && !FRESH ? ip[m] : make_int2(0, 0);
     bv[2 * s] = b.x;
     bv[2 * s + 1] = b.y;
-    bi[2 * s] = a.x;
-    bi[2 * s + 1] = a.y;
+    bi[s] = NONE | NONE << 16;
   }
-  // This thread's twiddles, the same for every orientation, held in
-  // registers: exp(2 pi i k/N) for its pre-processing bins k = j + R2*m and
-  // the stage twiddles of the half-length transform.
-  float2 twp[R1], twh[R1];
-#pragma unroll
-  for (int m = 0; m < R1; ++m) twp[m] = twiddle<1, N>(tw, j + R2 * m);
-  load_two_step_twiddles<NC, R1, 1>(twh, j, tw);
   const int xrow = valid ? row * L::PITCH : (int)L::STRIDE;  // invalid rows read nothing (0)
 
   for (int o = 0; o < nb; ++o) {
@@ -548,23 +559,23 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
       // the imaginary parts of X[0] and X[n/2] do not enter the real inverse
       const float2 a0 = k == 0 ? make_float2(a.x, 0.f) : a;
       const float2 bc = make_float2(m == 0 ? b.x + (j == 0 ? xn : 0.f) : b.x, -b.y);
-      v[m] = cadd(cadd(a0, bc), mul_pj<1>(cmul(twp[m], csub(a0, bc))));
+      v[m] = cadd(cadd(a0, bc), mul_pj<1>(cmul(twp[k], csub(a0, bc))));
     }
-    __syncthreads();
-    fft_two_step<NC, R1, R2, 1>(v, j, tw, [&](int k1, int jj) { return &xch[r * GS + jj * (R1 + 2) + k1]; },
-                                TwiddleRegs<R1>{twh});
-    const int32_t oi = angle0 + o;
+    SyncWave{}();  // a row's R2 threads are lanes of one wave
+    fft_two_step<NC, R1, R2, 1>(v, j, twh, [&](int k1, int jj) { return &xch[r * GS + jj * (R1 + 2) + k1]; },
+                                TwiddleStage<R2>{}, SyncWave{});
+    const unsigned oi = (unsigned)o;
 #pragma unroll
     for (int s = 0; s < R1; ++s) {
       const float c0 = v[s].x * sc, c1 = v[s].y * sc;
       if (tmask && !FRESH && !((xbits >> (out_index<R1, R2>(j, s) >> 4)) & 1u)) continue;  // x = 2m, 2m + 1
       if (c0 > bv[2 * s]) {
         bv[2 * s] = c0;
-        bi[2 * s] = oi;
+        bi[s] = (bi[s] & 0xffff0000u) | oi;
       }
       if (c1 > bv[2 * s + 1]) {
         bv[2 * s + 1] = c1;
-        bi[2 * s + 1] = oi;
+        bi[s] = (bi[s] & NONE) | oi << 16;
       }
     }
   }
@@ -572,8 +583,11 @@ __global__ __launch_bounds__(256) void k_pick_x_max(const float2* __restrict__ G
 #pragma unroll
     for (int s = 0; s < R1; ++s) {
       const int m = out_index<R1, R2>(j, s);
+      const unsigned a = bi[s] & NONE, b = bi[s] >> 16;
+      if (!FRESH && a == NONE && b == NONE) continue;
+      const int2 old = FRESH ? make_int2(0, 0) : ip[m];
       bp[m] = make_float2(bv[2 * s], bv[2 * s + 1]);
-      ip[m] = make_int2(bi[2 * s], bi[2 * s + 1]);
+      ip[m] = make_int2(a == NONE ? old.x : angle0 + (int)a, b == NONE ? old.y : angle0 + (int)b);
     }
   }
 }
@@ -805,9 +819,10 @@ __global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_pick2d_pr
   constexpr int NT = TX * R2;
   __shared__ float2 xch[R2 > 1 ? TX * N : 1];
   __shared__ float red[(NT + 63) / 64];
-  __shared__ float2 twl[N];
+  __shared__ float2 twl[R2 > 1 ? N : 1];  // the stage twiddles
   const int t = threadIdx.x, c = t % TX, j = t / TX;
-  for (int i = t; i < N; i += NT) twl[i] = twiddle<-1, N>(tw, i);
+  if (R2 > 1)
+    for (int i = t; i < N; i += NT) twl[i] = twiddle<1, N>(tw, i / R2 * (i % R2));
   const int tile = blockIdx.x, o = blockIdx.y, nb = gridDim.y;
   const int ix = tile * TX + c;
   const bool valid = ix < HALF;
@@ -815,23 +830,31 @@ __global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_pick2d_pr
 #pragma unroll
   for (int k = 0; k < 9; ++k) M[k] = mats[9 * o + k];
   const __amdgpu_buffer_rsrc_t rs = sampler_rsrc(P);
+  // two at a time: with every gather in flight at once one wave fits a SIMD (4 images of 256^2 x
+  // 60 orientations: 28 us, 40 before)
   float2 r[R1];
 #pragma unroll
-  for (int m = 0; m < R1; ++m) {
-    const int y = signed_freq(j + R2 * m, N);
-    const bool ins = valid && ix * ix + y * y <= RMAX2;
-    r[m] = sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins);
+  for (int m0 = 0; m0 < R1; m0 += 2) {
+#pragma unroll
+    for (int m = m0; m < m0 + 2; ++m) {
+      const int y = signed_freq(j + R2 * m, N);
+      const bool ins = valid && ix * ix + y * y <= RMAX2;
+      r[m] = make_float2(0.f, 0.f);
+      if (__any(ins)) r[m] = sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  const size_t bin = valid ? (size_t)j * NH + ix : 0;
+  const int bin = valid ? j * NH + ix : OUT_OF_RANGE / 8;
+  const int gout = (out_index<R1, R2>(j, 0) * (int)L::PITCH + ix) * 8;
   for (int w = 0; w < vb; ++w) {
-    const float2* Ew = E + w * H + bin;
-    const float* cw = ctf ? ctf + w * ctf_stride + bin : nullptr;
+    const __amdgpu_buffer_rsrc_t rE = make_rsrc(E + w * H, (unsigned)(H * 8));
+    const __amdgpu_buffer_rsrc_t rC = make_rsrc(ctf ? ctf + w * ctf_stride : nullptr, ctf ? (unsigned)(H * 4) : 0u);
     float acc = 0.f;
     float2 v[R1];
 #pragma unroll
     for (int m = 0; m < R1; ++m) {
-      const float2 e = valid ? Ew[m * R2 * NH] : make_float2(0.f, 0.f);
-      const float cf = valid ? (cw ? cw[m * R2 * NH] : 1.f) : 0.f;
+      const float2 e = buf_load2(rE, bin * 8, m * R2 * NH * 8);
+      const float cf = ctf ? buf_load1(rC, bin * 4, m * R2 * NH * 4) : 1.f;
       const float2 rc = cscale(r[m], cf);
       acc += rc.x * rc.x + rc.y * rc.y;
       v[m] = cmulc(e, rc);
@@ -839,10 +862,11 @@ __global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_pick2d_pr
     if (ix == 0 && j == 0) v[0] = make_float2(0.f, 0.f);  // DC
     __syncthreads();
     fft_two_step<N, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; },
-                               TwiddleLDS{});
-    float2* g = G + (size_t)(w * nb + o) * L::STRIDE;
+                               TwiddleStage<R2>{});
+    const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + (size_t)(w * nb + o) * L::STRIDE, (unsigned)(L::STRIDE * 8));
 #pragma unroll
-    for (int s = 0; s < R1; ++s) g[(size_t)out_index<R1, R2>(j, s) * L::PITCH + ix] = v[s];
+    for (int s = 0; s < R1; ++s)
+      buf_store2(v[s], rG, gout, (R2 > 1 ? s / R2 + R1 * (s % R2) : s) * (int)L::PITCH * 8);
     const float tot = block_sum(acc, red);
     if (t == 0) partial[(size_t)(w * nb + o) * L::FT + tile] = tot;
   }
@@ -962,7 +986,9 @@ __global__ __launch_bounds__(TX * LineShape<L1>::R2) void k_pick2d_project_cols(
   __shared__ float2 xch[R2 > 1 ? TX * L1 : 1];
   __shared__ float red[(NT + 63) / 64];
   const int NH = n / 2 + 1, HALF = n / 2;
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
+  // whole waves share j with 64 columns, so that rows and twiddles are wave-uniform (with that, no reads of E
+  // outside the disc and whole 8-byte stores 4096^2 x 15 orientations take 0.82 ms, 0.95 before)
+  const int t = threadIdx.x, c = t % TX, j = TX % 64 == 0 ? __builtin_amdgcn_readfirstlane(t / TX) : t / TX;
   const int o = blockIdx.y / L2, n2 = blockIdx.y % L2;
   const int ix = blockIdx.x * TX + c;
   const bool valid = ix < NH;
@@ -973,16 +999,22 @@ __global__ __launch_bounds__(TX * LineShape<L1>::R2) void k_pick2d_project_cols(
   float acc = 0.f;
   float2 v[R1];
 #pragma unroll
-  for (int m = 0; m < R1; ++m) {
-    const int iy = n2 + L2 * (j + R2 * m), y = signed_freq(iy, n);
-    const bool ins = valid && ix * ix + y * y <= HALF * HALF;
-    const size_t b = (size_t)iy * NH + ix;
-    const float2 e = valid ? E[b] : make_float2(0.f, 0.f);
-    const float cf = valid ? (ctf ? ctf[b] : 1.f) : 0.f;
-    const float2 r =
-        cscale(sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins), cf);
-    acc += r.x * r.x + r.y * r.y;
-    v[m] = ix == 0 && iy == 0 ? make_float2(0.f, 0.f) : cmulc(e, r);
+  for (int m0 = 0; m0 < R1; m0 += 2) {
+#pragma unroll
+    for (int m = m0; m < m0 + 2; ++m) {
+      const int iy = n2 + L2 * (j + R2 * m), y = signed_freq(iy, n);
+      const bool ins = valid && ix * ix + y * y <= HALF * HALF;
+      v[m] = make_float2(0.f, 0.f);
+      if (!__any(ins)) continue;  // E is not read outside the disc
+      const size_t b = (size_t)iy * NH + ix;
+      const float2 e = valid ? E[b] : make_float2(0.f, 0.f);
+      const float cf = valid ? (ctf ? ctf[b] : 1.f) : 0.f;
+      const float2 r =
+          cscale(sample(rs, P, M[0] * ix + M[1] * y, M[3] * ix + M[4] * y, M[6] * ix + M[7] * y, ins), cf);
+      acc += r.x * r.x + r.y * r.y;
+      v[m] = ix == 0 && iy == 0 ? make_float2(0.f, 0.f) : cmulc(e, r);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   fft_two_step<L1, R1, R2, 1>(v, j, tw, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; });
   if (valid) {
@@ -992,9 +1024,8 @@ __global__ __launch_bounds__(TX * LineShape<L1>::R2) void k_pick2d_project_cols(
       const int k1 = out_index<R1, R2>(j, s);
       // streaming stores: the spectra are read once, by the second pass
       const float2 w = cmul(v[s], twiddle_rt<1>(tw, n, n2 * k1));
-      float* dst = reinterpret_cast<float*>(So + (size_t)(n2 + L2 * k1) * NH + ix);
-      __builtin_nontemporal_store(w.x, dst);
-      __builtin_nontemporal_store(w.y, dst + 1);
+      __builtin_nontemporal_store(__builtin_bit_cast(u32x2, w),
+                                  reinterpret_cast<u32x2*>(So + (size_t)(n2 + L2 * k1) * NH + ix));
     }
   }
   const float tot = block_sum(acc, red);
@@ -1825,7 +1856,8 @@ int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const Centred
   const unsigned images = pl->nz == 1 && pl->n <= 256 ? std::min({nvol, (unsigned)MAX_IMAGES2, pl->B}) : 1u;
   for (unsigned v = 0; v < nvol; v += images) {
     const unsigned vb = std::min(images, nvol - v);
-    const unsigned B = even_batch(pl->B / vb, nangles);
+    // at most 65,534: the row passes keep an orientation's place in its batch in 16 bits
+    const unsigned B = even_batch(std::min(pl->B / vb, 65534u), nangles);
     const float2* Ev = E + (size_t)v * pl->H;
     const float* cv = ctf ? ctf + (size_t)v * ctf_stride : nullptr;
     float* bv = best + (size_t)v * pl->V;
