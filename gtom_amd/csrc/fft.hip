@@ -128,21 +128,9 @@ __global__ __launch_bounds__(256) void k_rows_c2r(const float2* __restrict__ in,
 // Row R2C: N reals -> N/2+1 bins. z[m] = x[2m] + i x[2m+1], Z = DFT_{N/2}(z),
 // X[k] = ((Z[k] + conj Z[N/2-k]) - i w^k (Z[k] - conj Z[N/2-k])) / 2, w = e^{-2 pi i/N}.
 // ---------------------------------------------------------------------------
-// A line of n0 points in FFT order (origin first, c of them at non-negative
-// positions) inside a longer one: the index of the n-point line's point p in the
-// short one, -1 where the long line is zero. n0 = 0: the line itself.
-struct PadMap {
-  int n0 = 0, c = 0;
-  __device__ __forceinline__ int at(int p, int n) const {
-    return p < c ? p : (p >= n - (n0 - c) ? p - (n - n0) : -1);
-  }
-};
-
-// PAD: the rows hold pm.n0 reals, padded to N on load.
-template <int N, bool PAD = false>
+template <int N>
 __global__ __launch_bounds__(256) void k_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                  long long nrows, const float2* __restrict__ tw, RowBand rb,
-                                                  PadMap pm = PadMap{}) {
+                                                  long long nrows, const float2* __restrict__ tw, RowBand rb) {
   constexpr int NC = N / 2, NH = N / 2 + 1;
   constexpr int R1 = RowShape<NC>::R1, R2 = RowShape<NC>::R2, RW = 256 / R2;
   constexpr int GS = R2 * (R1 + 1);
@@ -153,18 +141,9 @@ __global__ __launch_bounds__(256) void k_rows_r2c(const float* __restrict__ in, 
   const bool valid = (long long)blockIdx.x * RW + r < nrows;
   const long long row = band_row((long long)blockIdx.x * RW, rb) + r;
   float2 v[R1];
-  if constexpr (PAD) {
-    const float* x = in + row * pm.n0;
+  const float2* x = reinterpret_cast<const float2*>(in + row * N);
 #pragma unroll
-    for (int m = 0; m < R1; ++m) {
-      const int a = pm.at(2 * (j + R2 * m), N), b = pm.at(2 * (j + R2 * m) + 1, N);
-      v[m] = make_float2(valid && a >= 0 ? x[a] : 0.f, valid && b >= 0 ? x[b] : 0.f);
-    }
-  } else {
-    const float2* x = reinterpret_cast<const float2*>(in + row * N);
-#pragma unroll
-    for (int m = 0; m < R1; ++m) v[m] = valid ? x[j + R2 * m] : make_float2(0.f, 0.f);
-  }
+  for (int m = 0; m < R1; ++m) v[m] = valid ? x[j + R2 * m] : make_float2(0.f, 0.f);
   fft_two_step<NC, R1, R2, -1>(v, j, tw, [&](int k1, int jj) { return &xch[r * GS + jj * (R1 + 1) + k1]; });
 #pragma unroll
   for (int s = 0; s < R1; ++s) zrow[r * ZS + out_index<R1, R2>(j, s)] = v[s];
@@ -733,7 +712,7 @@ int launch_rows_r2c(int n, const float* in, float2* out, long long nrows, const 
   auto go = [&](auto kernel, int rw) -> int {
     if (rb.by % rw) return fail(GTOMX_ERR_INTERNAL, "row band not a multiple of the rows per workgroup");
     dim3 grid((unsigned)((nrows + rw - 1) / rw));
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, out, nrows, tw, rb, PadMap{});
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, out, nrows, tw, rb);
     GX_LAUNCHED("k_rows_r2c");
     return GTOMX_OK;
   };
@@ -1217,10 +1196,9 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_c2r(const floa
 }
 
 // A[k] = (Z[k] + conj Z[L - k]) / 2, B[k] = (Z[k] - conj Z[L - k]) / 2i of Z = DFT(a + i b).
-// With pm.n0 the rows hold that many reals, padded to L on load.
 template <class LN>
 __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__ in, float2* __restrict__ out,
-                                                       RowPairs rp, LineArgs A, PadMap pm) {
+                                                       RowPairs rp, LineArgs A) {
   float2* lds = line_lds<LN::ROW_LDS>();
   const int t = threadIdx.x, L = A.L, lanes = LN::lanes(A), pitch = LN::row_pitch(A), pairs = row_pairs<LN>(A);
   int j;
@@ -1234,13 +1212,12 @@ __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__
     const int nh = L / 2 + 1;
     bool two;
     const long long row = rp.row(pair, &two);
-    const int len = pm.n0 ? pm.n0 : L;
-    const float* a = in + row * len;
+    const float* a = in + row * L;
     float2 v[LN::REGS];
 #pragma unroll
     for (int m = 0; m < LN::PTS; ++m) {
-      const int p = j + lanes * m, q = p >= L ? -1 : (pm.n0 ? pm.at(p, L) : p);
-      v[m] = make_float2(q >= 0 ? a[q] : 0.f, q >= 0 && two ? a[len + q] : 0.f);
+      const int p = j + lanes * m;
+      v[m] = make_float2(p < L ? a[p] : 0.f, p < L && two ? a[L + p] : 0.f);
     }
     LN::template run<-1>(v, j, A, lds, [&](int k, int i) { return &xch[k * pitch + i]; }, SyncWave{});
     SyncWave{}();
@@ -1260,12 +1237,12 @@ __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__
 // A search's row pass: the C2R of every row of the orientations o in group
 // blockIdx.y (og of them), folded into a running maximum in registers (strict >,
 // increasing o). With FRESH the maximum starts at -infinity / -1 and goes to the
-// group's own nrows * n values. SEARCH: rows of (n + 1) / 2 bins without X[n/2],
-// which is sn[o].y, times sn[o].x; otherwise rows of n/2 + 1 bins, not scaled.
+// group's own nrows * n values. Rows of (n + 1) / 2 bins without X[n/2], which is
+// sn[o].y, times sn[o].x.
 // A pair of voxels keeps its two orientations as 16-bit offsets in the group in
 // one register (NONE: unchanged): with 32-bit indices the 512-point form spills
 // (200^3: 1.38 ms per 32 orientations).
-template <class LN, bool FRESH, bool SEARCH>
+template <class LN, bool FRESH>
 __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
     const float2* __restrict__ G, long long H, int nb, int nrows, int angle0, const float2* __restrict__ sn,
     float* __restrict__ best, int32_t* __restrict__ bidx, int og, LineArgs A) {
@@ -1288,7 +1265,7 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
     best += (size_t)blockIdx.y * nrows * n;
     bidx += (size_t)blockIdx.y * nrows * n;
   }
-  const int pitch = SEARCH ? (n + 1) / 2 : n / 2 + 1;
+  const int pitch = (n + 1) / 2;
   float bv[2][HP];
   unsigned bi[HP];
 #pragma unroll
@@ -1302,7 +1279,7 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
   }
   for (int o = o0; o < o1; ++o) {
     const __amdgpu_buffer_rsrc_t rG = make_rsrc(G + o * H, (unsigned)(H * 8));
-    const float2 so = SEARCH ? sn[o] : make_float2(1.f, 0.f);
+    const float2 so = sn[o];
     // opaque per orientation: what follows from it alone (addresses, bounds) is recomputed rather than held
     // in registers, which would spill
     int jo = j;
@@ -1314,12 +1291,10 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
       const int p = jo + R2 * m;
       const bool mirror = p > n / 2, mid = 2 * p == n;
       const int q = mirror ? n - p : p;
-      const int off = p < n && !(SEARCH && mid) ? (row * pitch + q) * 8 : OUT_OF_RANGE;
+      const int off = p < n && !mid ? (row * pitch + q) * 8 : OUT_OF_RANGE;
       float2 x = buf_load2(rG, off, 0), y = buf_load2(rG, off, pitch * 8);
-      if (SEARCH) {
-        x.x += mid ? so.y : 0.f;
-        y.x += mid ? so.y : 0.f;
-      }
+      x.x += mid ? so.y : 0.f;
+      y.x += mid ? so.y : 0.f;
       if (mid || p == 0) x.y = y.y = 0.f;
       v[m] = mirror ? make_float2(x.x + y.y, y.x - x.y) : make_float2(x.x - y.y, x.y + y.x);
     }
@@ -1352,260 +1327,6 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
     if (two && (FRESH || b != NONE)) {
       best[i + n] = bv[1][m];
       bidx[i + n] = b == NONE ? -1 : angle0 + o0 + (int)b;
-    }
-  }
-}
-
-// The same, not scaled, on rows with a native transform.
-template <int N, bool FRESH>
-__global__ __launch_bounds__(256) void k_rows_max(const float2* __restrict__ G, long long H, int nb, int nrows,
-                                                  int angle0, float* __restrict__ best, int32_t* __restrict__ bidx,
-                                                  int og, const float2* __restrict__ tw) {
-  constexpr int NC = N / 2, NH = NC + 1;
-  constexpr int R1 = RowShape<NC>::R1, R2 = RowShape<NC>::R2, RW = 256 / R2;
-  constexpr int GS = R2 * (R1 + 1);
-  __shared__ float2 area[R2 > 1 ? RW * GS : 1];
-  __shared__ float2 twl[N];
-  const int t = threadIdx.x, r = t / R2, j = t % R2;
-  for (int i = t; i < N; i += 256) twl[i] = twiddle<-1, N>(tw, i);
-  __syncthreads();
-  const int row = blockIdx.x * RW + r;
-  if (row >= nrows) return;  // no barrier below: a row's R2 threads are lanes of one wave
-  int o0 = 0, o1 = nb;
-  if (FRESH) {
-    o0 = og * (int)blockIdx.y;
-    o1 = min(nb, o0 + og);
-    best += (size_t)blockIdx.y * nrows * N;
-    bidx += (size_t)blockIdx.y * nrows * N;
-  }
-  float2* bp = reinterpret_cast<float2*>(best + (size_t)row * N);
-  int2* ip = reinterpret_cast<int2*>(bidx + (size_t)row * N);
-  float bv[2 * R1];
-  int32_t bi[2 * R1];
-#pragma unroll
-  for (int q = 0; q < R1; ++q) {
-    const int m = out_index<R1, R2>(j, q);
-    const float2 b = FRESH ? make_float2(-__builtin_inff(), -__builtin_inff()) : bp[m];
-    const int2 a = FRESH ? make_int2(-1, -1) : ip[m];
-    bv[2 * q] = b.x;
-    bv[2 * q + 1] = b.y;
-    bi[2 * q] = a.x;
-    bi[2 * q + 1] = a.y;
-  }
-  for (int o = o0; o < o1; ++o) {
-    const float2* X = G + o * H + (long long)row * NH;
-    float2 v[R1];
-#pragma unroll
-    for (int m = 0; m < R1; ++m) {
-      const int k = j + R2 * m;
-      float2 a = X[k], b = X[NC - k];
-      if (k == 0) a.y = b.y = 0.f;
-      const float2 bc = cconj(b);
-      v[m] = cadd(cadd(a, bc), mul_pj<1>(cmul(cconj(twl[k]), csub(a, bc))));
-    }
-    fft_two_step<NC, R1, R2, 1>(v, j, twl, [&](int k1, int jj) { return &area[r * GS + jj * (R1 + 1) + k1]; },
-                                TwiddleLDSHalf{}, SyncWave{});
-    SyncWave{}();
-    const int32_t oi = angle0 + o;
-#pragma unroll
-    for (int q = 0; q < R1; ++q) {
-      const float c0 = v[q].x, c1 = v[q].y;
-      if (c0 > bv[2 * q]) {
-        bv[2 * q] = c0;
-        bi[2 * q] = oi;
-      }
-      if (c1 > bv[2 * q + 1]) {
-        bv[2 * q + 1] = c1;
-        bi[2 * q + 1] = oi;
-      }
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < R1; ++q) {
-    const int m = out_index<R1, R2>(j, q);
-    bp[m] = make_float2(bv[2 * q], bv[2 * q + 1]);
-    ip[m] = make_int2(bi[2 * q], bi[2 * q + 1]);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The correlation of a small volume, zero-padded, with an image's spectrum
-// (the Picker): forward transforms that read only the small volume's lines, and
-// the z forward transform, the product with the image and the z inverse in one
-// kernel, which writes the spectrum once where the separate passes moved it
-// through memory seven times. Spectra of orientation o: the small volume's rows
-// [n0z][n0y][nh], after y [n0z][ny][nh], after the product [nz][ny][nh].
-// ---------------------------------------------------------------------------
-// The y transform of a padded axis: plane pl's n0 lines become n lines.
-template <int N>
-__global__ __launch_bounds__(fft_col_tx<N>() * ColShape<N>::R2) void k_cols_pad(
-    const float2* __restrict__ src, float2* __restrict__ dst, int width, int nplanes, PadMap pm,
-    const float2* __restrict__ tw) {
-  constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = fft_col_tx<N>();
-  __shared__ float2 xch[R2 > 1 ? TX * N : 1];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  const int col = blockIdx.x * TX + c;
-  const bool valid = col < width;
-  for (int pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
-    const float2* s = src + (size_t)pl * pm.n0 * width + col;
-    float2* d = dst + (size_t)pl * N * width + col;
-    float2 v[R1];
-#pragma unroll
-    for (int m = 0; m < R1; ++m) {
-      const int q = pm.at(j + R2 * m, N);
-      v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    fft_two_step<N, R1, R2, -1>(v, j, tw, [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; });
-    if (valid) {
-#pragma unroll
-      for (int q = 0; q < R1; ++q) d[(size_t)out_index<R1, R2>(j, q) * width] = v[q];
-    }
-  }
-}
-
-template <class LN>
-__global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols_pad(const float2* __restrict__ src,
-                                                                   float2* __restrict__ dst, int width, int nplanes,
-                                                                   PadMap pm, LineArgs A) {
-  float2* lds = line_lds<LN::COL_LDS>();
-  float2* xch = lds + LN::tables(A);
-  const int lanes = LN::lanes(A), txlog = LN::txlog(A), L = A.L;
-  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
-  LN::stage(lds, t, lanes << txlog, A);
-  const int col = ((int)blockIdx.x << txlog) + c;
-  const bool valid = col < width;
-  for (int pl = blockIdx.y; pl < nplanes; pl += gridDim.y) {
-    const float2* s = src + (size_t)pl * pm.n0 * width + col;
-    float2* d = dst + (size_t)pl * L * width + col;
-    float2 v[LN::REGS];
-#pragma unroll
-    for (int m = 0; m < LN::PTS; ++m) {
-      const int p = j + lanes * m, q = p < L ? pm.at(p, L) : -1;
-      v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    LN::template run<-1>(v, j, A, lds, [&](int k, int i) { return &xch[((k * lanes + i) << txlog) + c]; },
-                         SyncGroup{});
-#pragma unroll
-    for (int m = 0; m < LN::PTS; ++m) {
-      const int p = j + lanes * m;
-      if (valid && p < L) d[(size_t)p * width] = v[m];
-    }
-  }
-}
-
-// E * conj((P - dc) / sd) at one bin: the padded volume's mean0/std1 in Fourier
-// space (norm[0] = mean * elements, taken off the DC bin alone, norm[1] = 1 / sd).
-__device__ __forceinline__ float2 image_times_ref(float2 e, float2 p, float dc, float inv_sd) {
-  p = make_float2((p.x - dc) * inv_sd, p.y * inv_sd);
-  return cmulc(e, p);
-}
-
-// Forward z of the padded axis, the product and the inverse z, for orientation
-// blockIdx.y: the forward transform ends with every k2 of a k1 in one thread,
-// where the inverse starts, as in blue_convolve.
-template <int N>
-__global__ __launch_bounds__(ColShape<N>::TX * ColShape<N>::R2) void k_cols_correlate(
-    const float2* __restrict__ src, const float2* __restrict__ E, float2* __restrict__ dst, int width, PadMap pm,
-    const float2* __restrict__ norm, const float2* __restrict__ tw) {
-  constexpr int R1 = ColShape<N>::R1, R2 = ColShape<N>::R2, TX = ColShape<N>::TX, NT = TX * R2;
-  __shared__ float2 xch[R2 > 1 ? TX * N : 1];
-  __shared__ float2 twl[N];
-  const int t = threadIdx.x, c = t % TX, j = t / TX;
-  for (int i = t; i < N; i += NT) twl[i] = twiddle<-1, N>(tw, i);
-  const int col = blockIdx.x * TX + c, o = blockIdx.y;
-  const bool valid = col < width;
-  const float2* s = src + (size_t)o * pm.n0 * width + col;
-  const float2* e = E + col;
-  float2* d = dst + (size_t)o * N * width + col;
-  const float2 nm = norm[o];
-  float2 v[R1];
-#pragma unroll
-  for (int m = 0; m < R1; ++m) {
-    const int q = pm.at(j + R2 * m, N);
-    v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  dft<R1, -1>(v);
-  if constexpr (R2 == 1) {
-#pragma unroll
-    for (int k = 0; k < R1; ++k)
-      v[k] = image_times_ref(valid ? e[(size_t)k * width] : make_float2(0.f, 0.f), v[k], k == 0 && col == 0 ? nm.x : 0.f,
-                             nm.y);
-  } else {
-    auto at = [&](int k1, int jj) { return &xch[(k1 * R2 + jj) * TX + c]; };
-#pragma unroll
-    for (int k1 = 0; k1 < R1; ++k1) *at(k1, j) = k1 == 0 ? v[k1] : cmul(v[k1], twl[j * k1 % N]);
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < R1 / R2; ++u) {
-      const int k1 = j * (R1 / R2) + u;
-      float2 z[R2];
-#pragma unroll
-      for (int jj = 0; jj < R2; ++jj) z[jj] = *at(k1, jj);
-      dft<R2, -1>(z);
-#pragma unroll
-      for (int k2 = 0; k2 < R2; ++k2) {
-        const int k = k1 + R1 * k2;
-        z[k2] = image_times_ref(valid ? e[(size_t)k * width] : make_float2(0.f, 0.f), z[k2],
-                                k == 0 && col == 0 ? nm.x : 0.f, nm.y);
-      }
-      dft<R2, 1>(z);
-#pragma unroll
-      for (int jj = 0; jj < R2; ++jj) *at(k1, jj) = jj == 0 ? z[jj] : cmulc(z[jj], twl[jj * k1 % N]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k1 = 0; k1 < R1; ++k1) v[k1] = *at(k1, j);
-  }
-  dft<R1, 1>(v);
-  if (valid) {
-#pragma unroll
-    for (int m = 0; m < R1; ++m) d[(size_t)(j + R2 * m) * width] = v[m];
-  }
-}
-
-template <class LN>
-__global__ __launch_bounds__(LN::COL_THREADS) void k_line_cols_correlate(const float2* __restrict__ src,
-                                                                         const float2* __restrict__ E,
-                                                                         float2* __restrict__ dst, int width,
-                                                                         PadMap pm, const float2* __restrict__ norm,
-                                                                         LineArgs A) {
-  float2* lds = line_lds<LN::COL_LDS>();
-  float2* xch = lds + LN::tables(A);
-  const int lanes = LN::lanes(A), txlog = LN::txlog(A), L = A.L;
-  const int t = threadIdx.x, c = t & ((1 << txlog) - 1), j = t >> txlog;
-  LN::stage(lds, t, lanes << txlog, A);
-  const int col = ((int)blockIdx.x << txlog) + c, o = blockIdx.y;
-  const bool valid = col < width;
-  const float2* s = src + (size_t)o * pm.n0 * width + col;
-  const float2* e = E + col;
-  float2* d = dst + (size_t)o * L * width + col;
-  const float2 nm = norm[o];
-  auto at = [&](int k, int i) { return &xch[((k * lanes + i) << txlog) + c]; };
-  float2 v[LN::REGS];
-#pragma unroll
-  for (int m = 0; m < LN::PTS; ++m) {
-    const int p = j + lanes * m, q = p < L ? pm.at(p, L) : -1;
-    v[m] = valid && q >= 0 ? s[(size_t)q * width] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  LN::template run<-1>(v, j, A, lds, at, SyncGroup{});
-#pragma unroll
-  for (int m = 0; m < LN::PTS; ++m) {
-    const int p = j + lanes * m;
-    const float2 q = image_times_ref(valid && p < L ? e[(size_t)p * width] : make_float2(0.f, 0.f), v[m],
-                                     p == 0 && col == 0 ? nm.x : 0.f, nm.y);
-    v[m] = p < L ? q : make_float2(0.f, 0.f);
-  }
-  __syncthreads();  // the first transform's exchange is read
-  LN::template run<1>(v, j, A, lds, at, SyncGroup{});
-  if (valid) {
-#pragma unroll
-    for (int m = 0; m < LN::PTS; ++m) {
-      const int p = j + lanes * m;
-      if (p < L) d[(size_t)p * width] = v[m];
     }
   }
 }
@@ -1939,15 +1660,14 @@ int line_cols(int L, const float2* src, float2* dst, int width, long long as, lo
 }
 
 // The fused form on nrows contiguous rows of L reals / L/2 + 1 bins, `per` to a batch item.
-int line_rows_r2c(int L, const float* in, float2* out, long long nrows, long long per, hipStream_t s,
-                  PadMap pm = PadMap{}) {
+int line_rows_r2c(int L, const float* in, float2* out, long long nrows, long long per, hipStream_t s) {
   const RowPairs rp(nrows, per);
   LineArgs A;
   GX_TRY(line_args(L, true, &A));
   return with_line(A, [&](auto ln) -> int {
     using LN = decltype(ln);
     const unsigned n = row_pairs<LN>(A), wgs = (unsigned)(((long long)rp.pairs + n - 1) / n);
-    hipLaunchKernelGGL(k_line_rows_r2c<LN>, dim3(std::min(wgs, 4096u)), dim3(256), row_lds<LN>(A), s, in, out, rp, A, pm);
+    hipLaunchKernelGGL(k_line_rows_r2c<LN>, dim3(std::min(wgs, 4096u)), dim3(256), row_lds<LN>(A), s, in, out, rp, A);
     GX_LAUNCHED("k_line_rows_r2c");
     return GTOMX_OK;
   });
@@ -1969,28 +1689,8 @@ bool rows_max_any_fused(int n) { return n <= BLUE_FUSED_MAX; }
 
 int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
                  int32_t* idx, int og, hipStream_t s) {
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
   const int groups = og > 0 ? (nb + og - 1) / og : 1;
   if (nb > 0xffff) return fail(GTOMX_ERR_INTERNAL, "row pass over more than 65535 orientations");
-  if (!sn && fft_len_ok(n)) {
-    switch (n) {
-#define GX_CASE(N)                                                                                              \
-  case N: {                                                                                                     \
-    const unsigned wgs = (unsigned)((nrows + rows_per_block<N>() - 1) / rows_per_block<N>());                   \
-    if (groups == 1)                                                                                            \
-      hipLaunchKernelGGL((k_rows_max<N, false>), dim3(wgs, 1), dim3(256), 0, s, G, H, nb, nrows, angle0, best,  \
-                         idx, og, tw);                                                                          \
-    else                                                                                                        \
-      hipLaunchKernelGGL((k_rows_max<N, true>), dim3(wgs, groups), dim3(256), 0, s, G, H, nb, nrows, angle0,    \
-                         best, idx, og, tw);                                                                    \
-    GX_LAUNCHED("k_rows_max");                                                                                  \
-    return GTOMX_OK;                                                                                            \
-  }
-      GX_FOR_SIZES(GX_CASE)
-#undef GX_CASE
-    }
-  }
   LineArgs A;
   GX_TRY(line_args(n, true, &A));
   return with_line(A, [&](auto ln) -> int {
@@ -2002,8 +1702,7 @@ int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int ang
       GX_LAUNCHED("k_line_rows_max");
       return GTOMX_OK;
     };
-    if (sn) return groups == 1 ? go(k_line_rows_max<LN, false, true>) : go(k_line_rows_max<LN, true, true>);
-    return groups == 1 ? go(k_line_rows_max<LN, false, false>) : go(k_line_rows_max<LN, true, false>);
+    return groups == 1 ? go(k_line_rows_max<LN, false>) : go(k_line_rows_max<LN, true>);
   });
 }
 
@@ -2015,117 +1714,14 @@ int line_search_y(int n, float2* G, int nb, hipStream_t s) {
 // Two workgroups of 256 threads per CU fill the device; more groups cost more merging.
 int rows_max_any_groups(int n, int nrows, unsigned batch, int cus) {
   int wgs = 1;
-  if (fft_len_ok(n)) {
-    const int rw = rows_per_workgroup(n);
-    wgs = (nrows + rw - 1) / rw;
-  } else {
-    const LineArgs A = line_shape(n, true);
-    const int st = with_line(A, [&](auto ln) -> int {
-      const int per = 2 * row_pairs<decltype(ln)>(A);
-      wgs = (nrows + per - 1) / per;
-      return GTOMX_OK;
-    });
-    if (st != GTOMX_OK) return 1;
-  }
+  const LineArgs A = line_shape(n, true);
+  const int st = with_line(A, [&](auto ln) -> int {
+    const int per = 2 * row_pairs<decltype(ln)>(A);
+    wgs = (nrows + per - 1) / per;
+    return GTOMX_OK;
+  });
+  if (st != GTOMX_OK) return 1;
   return std::max(1, std::min((int)batch, 2 * cus / std::max(1, wgs)));
-}
-
-namespace {
-// d_FFTFullPad's placement of n0 points in FFT order within n (src/FFT/FFTResize.cu:212-238).
-PadMap pad_map(int n0, int n) {
-  PadMap pm;
-  pm.n0 = n0;
-  pm.c = n0 - (n / 2 + (n0 - n - ((n0 & (1 - (n & 1))) % 2)) / 2);
-  return pm;
-}
-bool padded_axis_ok(int n) { return fft_len_ok(n) || (n >= 2 && n <= BLUE_FUSED_MAX); }
-}  // namespace
-
-bool correlate_padded_ok(gtomx_int3 dr, gtomx_int3 di) {
-  auto ok = [](int n0, int n) {
-    const PadMap pm = pad_map(n0, n);
-    return padded_axis_ok(n) && n0 >= 1 && n0 <= n && pm.c >= 1 && pm.c <= n0;
-  };
-  return di.z > 1 && ok(dr.x, di.x) && ok(dr.y, di.y) && ok(dr.z, di.z);
-}
-
-int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, const float2* E, float2* out,
-                     gtomx_int3 di, unsigned nb, const float2* norm, hipStream_t s) {
-  const float2* tw = nullptr;
-  GX_TRY(twiddles(&tw));
-  const int nh = di.x / 2 + 1;
-  // x: the small volume's rows
-  const long long nrows = (long long)dr.y * dr.z * nb;
-  const PadMap px = pad_map(dr.x, di.x), py = pad_map(dr.y, di.y), pz = pad_map(dr.z, di.z);
-  if (fft_len_ok(di.x)) {
-    switch (di.x) {
-#define GX_CASE(N)                                                                                              \
-  case N:                                                                                                       \
-    hipLaunchKernelGGL((k_rows_r2c<N, true>), dim3((unsigned)((nrows + rows_per_block<N>() - 1) /               \
-                                                              rows_per_block<N>())),                            \
-                       dim3(256), 0, s, r, rows, nrows, tw, RowBand{}, px);                                     \
-    break;
-      GX_FOR_SIZES(GX_CASE)
-#undef GX_CASE
-    }
-    GX_LAUNCHED("k_rows_r2c");
-  } else {
-    GX_TRY(line_rows_r2c(di.x, r, rows, nrows, (long long)dr.y * dr.z, s, px));
-  }
-  // y: every plane of the small volume
-  const int planes = (int)(dr.z * nb);
-  if (fft_len_ok(di.y)) {
-    switch (di.y) {
-#define GX_CASE(N)                                                                                                \
-  case N:                                                                                                         \
-    hipLaunchKernelGGL(k_cols_pad<N>, dim3((nh + fft_col_tx<N>() - 1) / fft_col_tx<N>(), std::min(planes, 65535)), \
-                       dim3(fft_col_tx<N>() * ColShape<N>::R2), 0, s, rows, cols, nh, planes, py, tw);            \
-    break;
-      GX_FOR_SIZES(GX_CASE)
-#undef GX_CASE
-    }
-    GX_LAUNCHED("k_cols_pad");
-  } else {
-    LineArgs A;
-    GX_TRY(line_args(di.y, false, &A));
-    GX_TRY(with_line(A, [&](auto ln) -> int {
-      using LN = decltype(ln);
-      const int tx = 1 << LN::txlog(A), gx = (nh + tx - 1) / tx;
-      hipLaunchKernelGGL(k_line_cols_pad<LN>, dim3(gx, std::min(planes, std::max(1, 8192 / gx))),
-                         dim3(col_threads<LN>(A)), col_lds<LN>(A), s, rows, cols, nh, planes, py, A);
-      GX_LAUNCHED("k_line_cols_pad");
-      return GTOMX_OK;
-    }));
-  }
-  // z, the product, z back
-  const int width = nh * di.y;
-  if (fft_len_ok(di.z)) {
-    switch (di.z) {
-#define GX_CASE(N)                                                                                         \
-  case N:                                                                                                  \
-    hipLaunchKernelGGL(k_cols_correlate<N>, dim3((width + ColShape<N>::TX - 1) / ColShape<N>::TX, nb),     \
-                       dim3(ColShape<N>::TX * ColShape<N>::R2), 0, s, cols, E, out, width, pz, norm, tw);  \
-    break;
-      GX_FOR_SIZES(GX_CASE)
-#undef GX_CASE
-    }
-    GX_LAUNCHED("k_cols_correlate");
-  } else {
-    LineArgs A;
-    GX_TRY(line_args(di.z, false, &A));
-    GX_TRY(with_line(A, [&](auto ln) -> int {
-      using LN = decltype(ln);
-      const int tx = 1 << LN::txlog(A);
-      hipLaunchKernelGGL(k_line_cols_correlate<LN>, dim3((width + tx - 1) / tx, nb), dim3(col_threads<LN>(A)),
-                         col_lds<LN>(A), s, cols, E, out, width, pz, norm, A);
-      GX_LAUNCHED("k_line_cols_correlate");
-      return GTOMX_OK;
-    }));
-  }
-  // y back
-  if (fft_len_ok(di.y))
-    return launch_cols_n<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, tw, s);
-  return line_cols<1>(di.y, out, out, nh, nh, (long long)di.z * nb, 1LL << 62, (long long)nh * di.y, 0, s);
 }
 
 // One axis of nlines lines of length L by the chirp-z form: IN / OUT are the

@@ -39,7 +39,7 @@ struct gtomx_pick_plan {
   float* gbest = nullptr;   // per-orientation-group maxima (groups x V)
   int32_t* gidx = nullptr;
   int pairs2 = 0;           // fused 2D passes: most (image, group) pairs of a launch
-  int groups3 = 0;          // 3D sides of k_pick_plane_max and k_blue_rows_max: most groups of a batch
+  int groups3 = 0;          // 3D sides of k_pick_plane_max and k_line_rows_max: most groups of a batch
   bool gen3d = false;       // 3D volumes whose side has no fused or long-row search: chirp-z transforms
   int nparts = 0;           // 2D above 256: pass-1 workgroups per orientation
   float2* scr = nullptr;    // 2D above 256: pass-1 output (B spectra)

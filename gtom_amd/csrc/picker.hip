@@ -14,9 +14,7 @@
 // Orientations are processed B at a time: the projection, C2R, padding,
 // normalisation, R2C, product and C2R are each one batched launch (or a few),
 // and the running maximum takes the B maps in increasing orientation order,
-// which keeps the reference's per-orientation strict '>' rule. 3D references and
-// images with axes up to 256 (native) or 512 never form the padded volume
-// (correlate_padded) and fold the maximum into the last row transform.
+// which keeps the reference's per-orientation strict '>' rule.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -125,6 +123,29 @@ __global__ __launch_bounds__(256) void k_image_times_conj(const float2* __restri
   }
 }
 
+// The same product with P the R2C of the un-normalised padded reference: the
+// normalisation (x - mean) / sd of k_norm_apply applied in Fourier space,
+// P' = (P - mean * n at the DC bin) / sd (sd = 0: no division), since the
+// transform is linear. Lets the R2C skip the rows the padding leaves zero.
+__global__ __launch_bounds__(256) void k_image_times_conj_norm(const float2* __restrict__ E, float2* __restrict__ P,
+                                                               size_t h, unsigned batch,
+                                                               const double* __restrict__ stats, size_t n) {
+  const size_t total = h * batch;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
+    const size_t b = i / h;
+    const double mean = stats[2 * b], sd = stats[2 * b + 1];
+    const float2 e = E[i % h], q = P[i];
+    double px = q.x, py = q.y;
+    if (i % h == 0) px -= mean * (double)n;
+    if (sd != 0.0) {
+      px /= sd;
+      py /= sd;
+    }
+    const float2 p = make_float2((float)px, (float)py);
+    P[i] = make_float2(e.x * p.x + e.y * p.y, e.y * p.x - e.x * p.y);
+  }
+}
+
 // PickingUpdateKernel (src/Correlation/Picker.cu:249-276) over B maps in order.
 __global__ __launch_bounds__(256) void k_update_max_angle(const float* __restrict__ C, size_t v, unsigned batch,
                                                           const float3* __restrict__ angles, float* __restrict__ best,
@@ -144,46 +165,6 @@ __global__ __launch_bounds__(256) void k_update_max_angle(const float* __restric
       bestangle[i] = angles[k];
     }
   }
-}
-
-// norm[o] = (mean * v, 1 / sd) of volume o's n0 values padded with zeros to v
-// elements (sd = 0: 1), sums in double; one workgroup per volume.
-__global__ __launch_bounds__(1024) void k_padded_norm(const float* __restrict__ r, size_t n0, double v,
-                                                      float2* __restrict__ norm) {
-  __shared__ double red[2][16];
-  const float* x = r + (size_t)blockIdx.x * n0;
-  double s1 = 0, s2 = 0;
-  for (size_t i = threadIdx.x; i < n0; i += 1024) {
-    const double d = (double)x[i];
-    s1 += d;
-    s2 += d * d;
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    s1 += __shfl_down(s1, o);
-    s2 += __shfl_down(s2, o);
-  }
-  if (threadIdx.x % 64 == 0) {
-    red[0][threadIdx.x / 64] = s1;
-    red[1][threadIdx.x / 64] = s2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    s1 = s2 = 0;
-    for (int w = 0; w < 16; ++w) {
-      s1 += red[0][w];
-      s2 += red[1][w];
-    }
-    const double var = fmax(0.0, (s2 - s1 * s1 / v) / v), sd = sqrt(var);
-    norm[blockIdx.x] = make_float2((float)s1, (float)(sd == 0.0 ? 1.0 : 1.0 / sd));
-  }
-}
-
-// The angle triples of the voxels whose maximum rose in this call.
-__global__ __launch_bounds__(256) void k_write_angles(const int32_t* __restrict__ idx, size_t v,
-                                                      const float3* __restrict__ angles,
-                                                      float3* __restrict__ bestangle) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < v; i += (size_t)gridDim.x * 256)
-    if (idx[i] >= 0) bestangle[i] = angles[idx[i]];
 }
 
 }  // namespace
@@ -215,19 +196,9 @@ struct gtomx_picker {
   float* padded = nullptr;     // B x V, then the correlation maps
   float2* pft = nullptr;       // B x H, also the C2R workspace at the image size
   double* nscr = nullptr;      // normalisation scratch
-  // the padded form (3D, axes of correlate_padded_ok), which needs neither `padded` nor `nscr` past SetImage
-  bool compact = false;
-  float2* rows = nullptr;      // B x nr x nr x (nx/2 + 1)
-  float2* cols = nullptr;      // B x nr x ny x (nx/2 + 1)
-  float2* norm = nullptr;      // B
-  int32_t* bidx = nullptr;     // V: orientation of the maxima that rose in the call
-  float* gbest = nullptr;      // groups x V
-  int32_t* gidx = nullptr;
-  int groups = 1;
-  size_t cap = 0;              // orientations that mats, dang and h_mats hold
-  float* mats = nullptr;       // cap x 9
-  float3* dang = nullptr;      // cap angles
-  float* h_mats = nullptr;     // pinned staging: cap x 9 matrices, then cap x 3 angles
+  float* mats = nullptr;       // B x 9
+  float3* dang = nullptr;      // B angles
+  float* h_mats = nullptr;     // pinned staging: B x 9 matrices, then B x 3 angles
   hipEvent_t staged = nullptr;
   bool staged_recorded = false;
   bool have_image = false;
@@ -241,8 +212,7 @@ void picker_release(gtomx_picker* pk) {
   if (!pk) return;
   pk->fence.release();
   for (void* p : {(void*)pk->refft, (void*)pk->imageft, (void*)pk->proj, (void*)pk->realref, (void*)pk->padded,
-                  (void*)pk->pft, (void*)pk->nscr, (void*)pk->mats, (void*)pk->dang, (void*)pk->rows, (void*)pk->cols,
-                  (void*)pk->norm, (void*)pk->bidx, (void*)pk->gbest, (void*)pk->gidx})
+                  (void*)pk->pft, (void*)pk->nscr, (void*)pk->mats, (void*)pk->dang})
     dev_free(p);
   if (pk->h_mats) (void)hipHostFree(pk->h_mats);
   if (pk->staged) (void)hipEventDestroy(pk->staged);
@@ -254,40 +224,6 @@ int picker_check(const gtomx_picker* pk) {
   int dev = 0;
   GX_HIP(hipGetDevice(&dev));
   if (dev != pk->device) return fail(GTOMX_ERR_INVALID_ARGUMENT, "picker was created on another device");
-  return GTOMX_OK;
-}
-
-// Matrices transpose(Euler) (no scale) and angles of nangles orientations to the
-// device through pinned staging. The last copy out of the staging is waited for.
-int picker_upload(gtomx_picker* pk, const gtomx_float3* h_angles, unsigned nangles, hipStream_t s) {
-  if (pk->staged_recorded) GX_HIP(hipEventSynchronize(pk->staged));
-  pk->staged_recorded = false;
-  if (pk->cap < nangles) {
-    pk->fence.drain();  // the last call's kernels read the old buffers
-    dev_free(pk->mats);
-    dev_free(pk->dang);
-    if (pk->h_mats) (void)hipHostFree(pk->h_mats);
-    pk->mats = nullptr;
-    pk->dang = nullptr;
-    pk->h_mats = nullptr;
-    pk->cap = 0;
-    GX_TRY(dev_alloc((void**)&pk->mats, (size_t)nangles * 9 * sizeof(float)));
-    GX_TRY(dev_alloc((void**)&pk->dang, (size_t)nangles * sizeof(float3)));
-    hipError_t e = hipHostMalloc((void**)&pk->h_mats, (size_t)nangles * 12 * sizeof(float), hipHostMallocDefault);
-    if (e != hipSuccess) return hip_fail(e, "hipHostMalloc(picker staging)");
-    pk->cap = nangles;
-  }
-  GX_TRY(gtomx_projector_matrices(h_angles, nangles, 1.0f, pk->h_mats));
-  float* ha = pk->h_mats + 9 * (size_t)nangles;
-  for (unsigned k = 0; k < nangles; ++k) {
-    ha[3 * k] = h_angles[k].x;
-    ha[3 * k + 1] = h_angles[k].y;
-    ha[3 * k + 2] = h_angles[k].z;
-  }
-  GX_HIP(hipMemcpyAsync(pk->mats, pk->h_mats, (size_t)nangles * 9 * sizeof(float), hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(pk->dang, ha, (size_t)nangles * 3 * sizeof(float), hipMemcpyHostToDevice, s));
-  GX_HIP(hipEventRecord(pk->staged, s));
-  pk->staged_recorded = true;
   return GTOMX_OK;
 }
 
@@ -333,13 +269,7 @@ int gtomx_picker_create(gtomx_picker** out, const float* d_ref, gtomx_int3 dimsr
   pk->nr = dimsref.x;
   pk->nrz = dimsref.z;
   pk->di = dimsimage;
-  pk->compact = !is2d && correlate_padded_ok(dimsref, dimsimage);
-  // without a batch: 8 orientations per pass, up to 32 in the padded form while their spectra stay within
-  // 256 MB (its passes over one orientation of 128^3 take 2 us each)
-  pk->B = batch ? batch
-                : (pk->compact ? (unsigned)std::max<size_t>(
-                                     8, std::min<size_t>(32, (256u << 20) / (elements_ft(dimsimage) * sizeof(float2))))
-                               : 8u);
+  pk->B = batch ? batch : 8u;
   pk->Hr = elements_ft(dimsref);
   pk->Vr = elements(dimsref);
   pk->H = elements_ft(dimsimage);
@@ -358,28 +288,15 @@ int gtomx_picker_create(gtomx_picker** out, const float* d_ref, gtomx_int3 dimsr
   alloc((void**)&pk->imageft, pk->H * sizeof(float2));
   alloc((void**)&pk->proj, B * pk->Hr * sizeof(float2));
   alloc((void**)&pk->realref, B * pk->Vr * sizeof(float));
+  alloc((void**)&pk->padded, B * pk->V * sizeof(float));
   alloc((void**)&pk->pft, B * pk->H * sizeof(float2));
   alloc((void**)&pk->nscr, norm_scratch_doubles((unsigned)B) * sizeof(double));
-  if (pk->compact) {
-    int cus = 0;
-    he = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pk->device);
-    if (he != hipSuccess && st == GTOMX_OK) st = hip_fail(he, "hipDeviceGetAttribute");
-    const size_t nh = dimsimage.x / 2 + 1;
-    pk->groups = rows_max_any_groups(dimsimage.x, dimsimage.y * dimsimage.z, (unsigned)B, cus);
-    alloc((void**)&pk->rows, B * dimsref.z * dimsref.y * nh * sizeof(float2));
-    alloc((void**)&pk->cols, B * dimsref.z * dimsimage.y * nh * sizeof(float2));
-    alloc((void**)&pk->norm, B * sizeof(float2));
-    alloc((void**)&pk->bidx, pk->V * sizeof(int32_t));
-    if (pk->groups > 1) {
-      alloc((void**)&pk->gbest, pk->groups * pk->V * sizeof(float));
-      alloc((void**)&pk->gidx, pk->groups * pk->V * sizeof(int32_t));
-    }
-  } else {
-    alloc((void**)&pk->padded, B * pk->V * sizeof(float));
-  }
+  alloc((void**)&pk->mats, B * 9 * sizeof(float));
+  alloc((void**)&pk->dang, B * sizeof(float3));
   if (st == GTOMX_OK) {
-    he = hipEventCreateWithFlags(&pk->staged, hipEventDisableTiming);
-    if (he != hipSuccess) st = hip_fail(he, "picker staging event");
+    he = hipHostMalloc((void**)&pk->h_mats, B * 12 * sizeof(float), hipHostMallocDefault);
+    if (he == hipSuccess) he = hipEventCreateWithFlags(&pk->staged, hipEventDisableTiming);
+    if (he != hipSuccess) st = hip_fail(he, "picker host staging");
   }
   if (st == GTOMX_OK) {
     // Initialize: refft = R2C(ifftshift(ref)) at the reference size (src/Correlation/Picker.cu:92-94, 112-114);
@@ -424,56 +341,61 @@ int gtomx_picker_correlate_angles(gtomx_picker* pk, const gtomx_float3* h_angles
   if (!pk->have_image) return fail(GTOMX_ERR_INVALID_ARGUMENT, "SetImage has not been called");
   if (!d_bestccf || !d_bestangle) return fail(GTOMX_ERR_INVALID_ARGUMENT, "NULL output buffer");
   if (nangles > 0 && !h_angles) return fail(GTOMX_ERR_INVALID_ARGUMENT, "h_angles is NULL");
-  if (nangles > 0x7fffffffu) return fail(GTOMX_ERR_INVALID_ARGUMENT, "orientation index exceeds int32");
   hipStream_t s = as_stream(stream);
   const gtomx_int3 dr{pk->nr, pk->nr, pk->nrz};
   const unsigned grid_i = (unsigned)std::min<size_t>((pk->H * pk->B + 255) / 256, 65536);
   const unsigned grid_v = (unsigned)std::min<size_t>((pk->V + 255) / 256, 65536);
-  if (nangles == 0) return GTOMX_OK;
   GX_TRY(pk->fence.enter(s));
-  GX_TRY(picker_upload(pk, h_angles, nangles, s));
-  if (pk->compact) GX_TRY(fill_i32(pk->bidx, pk->V, -1, s));
-  const unsigned passes = (nangles + pk->B - 1) / pk->B, B = (nangles + passes - 1) / passes;
-  for (unsigned b0 = 0; b0 < nangles; b0 += B) {
-    const unsigned nb = std::min(B, nangles - b0);
+  for (unsigned b0 = 0; b0 < nangles; b0 += pk->B) {
+    const unsigned nb = std::min(pk->B, nangles - b0);
+    // stage the matrices transpose(Euler) (no scale) and the angles for this batch
+    if (pk->staged_recorded) GX_HIP(hipEventSynchronize(pk->staged));
+    GX_TRY(gtomx_projector_matrices(h_angles + b0, nb, 1.0f, pk->h_mats));
+    for (unsigned k = 0; k < nb; ++k) {
+      pk->h_mats[9 * pk->B + 3 * k] = h_angles[b0 + k].x;
+      pk->h_mats[9 * pk->B + 3 * k + 1] = h_angles[b0 + k].y;
+      pk->h_mats[9 * pk->B + 3 * k + 2] = h_angles[b0 + k].z;
+    }
+    GX_HIP(hipMemcpyAsync(pk->mats, pk->h_mats, nb * 9 * sizeof(float), hipMemcpyHostToDevice, s));
+    GX_HIP(hipMemcpyAsync(pk->dang, pk->h_mats + 9 * pk->B, nb * 3 * sizeof(float), hipMemcpyHostToDevice, s));
+    GX_HIP(hipEventRecord(pk->staged, s));
+    pk->staged_recorded = true;
     // R = project(refft) * ctf; r = C2R_n(R)   (src/Correlation/Picker.cu:185-190)
-    GX_TRY(project_launch(pk->refft, pk->nr, pk->proj, pk->nr, (unsigned)(pk->nr / 2), pk->mats + 9 * (size_t)b0, nb,
-                          s, pk->nrz, pk->nrz));
+    GX_TRY(project_launch(pk->refft, pk->nr, pk->proj, pk->nr, (unsigned)(pk->nr / 2), pk->mats, nb, s, pk->nrz,
+                          pk->nrz));
     GX_TRY(gtomx_complex_multiply_by_vector(reinterpret_cast<const gtomx_complex*>(pk->proj), pk->ctf,
                                             reinterpret_cast<gtomx_complex*>(pk->proj), pk->Hr, nb, stream));
     GX_TRY(fft_c2r(pk->proj, pk->proj, pk->realref, dr, nb, 1.0f / (float)pk->Vr, s));
-    if (pk->compact) {
-      // FullPad, mean0/std1, R2C, C = C2R_u(imageft * conj(P)) (:225-229) without the padded volume: it is
-      // zero outside the reference, so its transforms read the reference's lines, its mean and deviation
-      // are sums over the reference, and the normalisation, linear, goes into the product
-      hipLaunchKernelGGL(k_padded_norm, dim3(nb), dim3(1024), 0, s, pk->realref, pk->Vr, (double)pk->V, pk->norm);
-      GX_LAUNCHED("k_padded_norm");
-      GX_TRY(correlate_padded(pk->realref, dr, pk->rows, pk->cols, pk->imageft, pk->pft, pk->di, nb, pk->norm, s));
-      // the rows' C2R and best / orientation where C > best   (:233-241)
-      const int og = ((int)nb + pk->groups - 1) / pk->groups, groups = ((int)nb + og - 1) / og;
-      const bool fresh = groups > 1;
-      GX_TRY(rows_max_any(pk->di.x, pk->di.y * pk->di.z, pk->pft, (long long)pk->H, (int)nb, (int)b0, nullptr,
-                          fresh ? pk->gbest : d_bestccf, fresh ? pk->gidx : pk->bidx, og, s));
-      if (fresh) GX_TRY(merge_group_maxima(pk->gbest, pk->gidx, groups, pk->V, d_bestccf, pk->bidx, 1, s));
-      continue;
-    }
     // FullPad, mean0/std1, R2C   (:225-227)
     GX_TRY(fft_resize(FFT_FULL_PAD, false, pk->realref, pk->padded, dr, pk->di, nb, s));
-    GX_TRY(norm_mean01std(pk->padded, pk->padded, pk->V, nb, pk->nscr, s));
-    GX_TRY(fft_r2c(pk->padded, pk->pft, pk->di, nb, s));
-    // C = C2R_u(imageft * conj(P))   (:228-229)
-    hipLaunchKernelGGL(k_image_times_conj, dim3(grid_i), dim3(256), 0, s, pk->imageft, pk->pft, pk->H, nb);
-    GX_LAUNCHED("k_image_times_conj");
+    // The padded reference is zero outside the z x y box of the reference
+    // (FFT order); where the row kernels allow, the R2C runs over that band
+    // of rows and the normalisation moves into the product (same values up
+    // to rounding).
+    const int rw = dims_native(pk->di) ? rows_per_workgroup(pk->di.x) : 0;
+    const int vby = rw > 0 ? (dr.y / 2 + 1 + rw - 1) / rw * rw : 0;
+    const int vbz = 2 * (dr.z / 2 + 1) <= pk->di.z ? dr.z / 2 + 1 : 0;
+    const bool vbanded = pk->nrz > 1 && pk->di.x <= 256 && pk->di.y <= 256 && pk->di.z <= 256 && vby > 0 &&
+                         2 * vby <= pk->di.y;
+    if (vbanded) {
+      GX_TRY(norm_stats(pk->padded, pk->V, nb, pk->nscr, s));
+      GX_TRY(volume_r2c_banded(pk->padded, pk->pft, pk->di, nb, vby, vbz, s));
+      // C = C2R_u(imageft * conj(P))   (:228-229)
+      hipLaunchKernelGGL(k_image_times_conj_norm, dim3(grid_i), dim3(256), 0, s, pk->imageft, pk->pft, pk->H, nb,
+                         pk->nscr + (size_t)NB * nb, pk->V);
+      GX_LAUNCHED("k_image_times_conj_norm");
+    } else {
+      GX_TRY(norm_mean01std(pk->padded, pk->padded, pk->V, nb, pk->nscr, s));
+      GX_TRY(fft_r2c(pk->padded, pk->pft, pk->di, nb, s));
+      // C = C2R_u(imageft * conj(P))   (:228-229)
+      hipLaunchKernelGGL(k_image_times_conj, dim3(grid_i), dim3(256), 0, s, pk->imageft, pk->pft, pk->H, nb);
+      GX_LAUNCHED("k_image_times_conj");
+    }
     GX_TRY(fft_c2r(pk->pft, pk->pft, pk->padded, pk->di, nb, 1.0f, s));
     // best/angle where C > best   (:233-241)
-    hipLaunchKernelGGL(k_update_max_angle, dim3(grid_v), dim3(256), 0, s, pk->padded, pk->V, nb, pk->dang + b0,
+    hipLaunchKernelGGL(k_update_max_angle, dim3(grid_v), dim3(256), 0, s, pk->padded, pk->V, nb, pk->dang,
                        d_bestccf, reinterpret_cast<float3*>(d_bestangle));
     GX_LAUNCHED("k_update_max_angle");
-  }
-  if (pk->compact) {
-    hipLaunchKernelGGL(k_write_angles, dim3(grid_v), dim3(256), 0, s, pk->bidx, pk->V, pk->dang,
-                       reinterpret_cast<float3*>(d_bestangle));
-    GX_LAUNCHED("k_write_angles");
   }
   return pk->fence.leave(s);
 }

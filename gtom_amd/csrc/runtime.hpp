@@ -208,9 +208,8 @@ int yz_axes_any(float2* data, gtomx_int3 dims, unsigned batch, int dir, hipStrea
 // the rows it overwrites are written). n at most 2048.
 int rows_c2r_any_inplace(float2* G, int n, int nb, long long H, hipStream_t s);
 // A search's row pass on rows of n <= 512 reals (rows_max_any_fused): the C2R of
-// the nrows rows of nb half spectra H apart in G (with sn rows of (n + 1) / 2 bins
-// without X[n/2] = sn[o].y, times sn[o].x; without, n/2 + 1 bins, not scaled),
-// folded into best / idx in orientation order from angle0 (strict >). og > 0 and
+// the nrows rows of nb half spectra H apart in G (rows of (n + 1) / 2 bins without
+// X[n/2] = sn[o].y, times sn[o].x), folded into best / idx in orientation order from angle0 (strict >). og > 0 and
 // below nb: group g of og orientations starts afresh (-infinity, -1) and writes at
 // g * nrows * n of best / idx, for merge_group_maxima.
 bool rows_max_any_fused(int n);
@@ -224,14 +223,6 @@ int line_search_y(int n, float2* G, int nb, hipStream_t s);
 // order (strict >), for each of `items` (pick.hip).
 int merge_group_maxima(const float* gbest, const int32_t* gidx, int groups, size_t v, float* best, int32_t* idx,
                        unsigned items, hipStream_t s);
-// Spectra of nb volumes r of dr (FFT order), zero-padded to di as d_FFTFullPad
-// places them, in E * conj((P - dc) / sd) with (dc, 1 / sd) = norm[o], transformed
-// back along z and y: out holds nb half spectra ready for the row pass. rows:
-// nb * dr.z * dr.y * (di.x / 2 + 1) values, cols: nb * dr.z * di.y * (di.x / 2 + 1).
-bool correlate_padded_ok(gtomx_int3 dr, gtomx_int3 di);
-int correlate_padded(const float* r, gtomx_int3 dr, float2* rows, float2* cols, const float2* E, float2* out,
-                     gtomx_int3 di, unsigned nb, const float2* norm, hipStream_t s);
-
 // Fourier-space resizing (resize.hip): op is one of the GTOMX_FFT_* values.
 constexpr int FFT_CROP = GTOMX_FFT_CROP, FFT_PAD = GTOMX_FFT_PAD, FFT_FULL_CROP = GTOMX_FFT_FULL_CROP,
               FFT_FULL_PAD = GTOMX_FFT_FULL_PAD;

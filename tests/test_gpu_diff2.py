@@ -70,8 +70,7 @@ def test_diff2_planted_shift_found(gx, orc, cuda):
 @pytest.mark.parametrize("n,rel,nvol,nang", [(24, (3, 4, 5), 1, 5), (24, (13, 9, 12), 3, 300), (34, (17, 16, 18), 2, 37),
                                              (32, (32, 1, 31), 2, 33), (2, (2, 1, 2), 1, 4)])
 def test_diff2_shift_ranges(gx, orc, cuda, n, rel, nvol, nang):
-    """Every count of shift pairs per axis (one chunk and several), odd and even ranges,
-    more than one batch: against the same sum in 64 bits, by a
+    """Odd and even ranges, one volume and several, more than one batch: against the same sum in 64 bits, by a
     complex FFT of the half spectrum, from the float projections. 32-bit sums over the bins: 1e-5
     of the largest score, as above."""
     import torch
