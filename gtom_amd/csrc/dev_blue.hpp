@@ -197,7 +197,7 @@ template <int RL_> struct SmoothLine {
 };
 #define GX_FOR_SMOOTH(X) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(15) X(16) X(20)
 
-// Chirp and kernel spectra of one length (fft.hip): chirp[j] = exp(-i pi (j^2 mod
+// Chirp and kernel spectra of one length L and convolution length M (fft.hip): chirp[j] = exp(-i pi (j^2 mod
 // 2L) / L), bf / bi the M-point DFTs of the forward / inverse kernels over M.
 struct BlueTables {
   int M = 0;
@@ -205,7 +205,7 @@ struct BlueTables {
   float2* bf = nullptr;
   float2* bi = nullptr;
 };
-int blue_tables(int L, BlueTables* out);
+int blue_tables(int L, int M, BlueTables* out);
 // The form of lines of L points, 2 <= L <= BLUE_FUSED_MAX, without and with its device tables.
 // Rows and columns may be split differently.
 LineArgs line_shape(int L, bool rows);

@@ -856,8 +856,8 @@ int yz_axes(const float2* src, float2* data, float2* scr, gtomx_int3 d, unsigned
   return GTOMX_OK;
 }
 
-int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s);
-int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s);
+int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s, LineForm form);
+int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s, LineForm form);
 
 // Items of a batch that go through the two-pass axes together (0: no axis needs
 // them): scratch of about 128 MB, which the 256 MB last-level cache holds beside
@@ -868,8 +868,8 @@ unsigned two_pass_items(gtomx_int3 d, unsigned batch) {
   return (unsigned)std::max<size_t>(1, std::min<size_t>(batch, (128u << 20) / (elements_ft(d) * sizeof(float2))));
 }
 
-int fft_r2c(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s) {
-  if (!dims_native(d)) return fft_r2c_any(in, out, d, batch, s);
+int fft_r2c(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s, LineForm form) {
+  if (!dims_native(d)) return fft_r2c_any(in, out, d, batch, s, form);
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   StreamScratch scr;
@@ -890,14 +890,14 @@ int fft_r2c(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStrea
 }
 
 int fft_c2r(const float2* in, float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s,
-            int cols) {
+            int cols, LineForm form) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   const size_t H = elements_ft(d) * batch;
   if (cols < 0 || cols > d.x / 2 + 1) return fail(GTOMX_ERR_INTERNAL, "column count outside the half spectrum");
   if (!dims_native(d)) {
     if (work != in) GX_HIP(hipMemcpyAsync(work, in, H * sizeof(float2), hipMemcpyDeviceToDevice, s));
-    return fft_c2r_any(work, out, d, batch, scale, s);
+    return fft_c2r_any(work, out, d, batch, scale, s, form);
   }
   const bool axes = d.y > 1 || d.z > 1;
   // with a column limit the first axis leaves the other columns as they are
@@ -1086,7 +1086,7 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
 // convolution of a line inside one kernel (below); above, the lines of one axis
 // are gathered into an M x (lines) block (line index fastest, the layout the
 // column kernels take), in chunks that keep the block within 2^31 elements
-// and 256 MB.
+// and 256 MB. The Picker takes the gathered form at every length (LineForm).
 
 // ---------------------------------------------------------------------------
 // Lengths up to 512: load, both M-point transforms and the store in one kernel,
@@ -1332,7 +1332,7 @@ __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
 }
 
 // ---------------------------------------------------------------------------
-// Lengths above 512.
+// The gathered form: lengths above 512, and any length for LineForm::Gathered.
 // ---------------------------------------------------------------------------
 
 // Line l of an axis: its first point at (l / P) * S1 + (l % P) * S0, its
@@ -1472,9 +1472,9 @@ __global__ __launch_bounds__(256) void k_blue_store_rows(const float2* __restric
   }
 }
 
-// The tables (BlueTables) of one length, per device, computed once in long double.
+// The tables (BlueTables) of one length and convolution length, per device, computed once in long double.
 std::mutex g_blue_mu;
-std::map<std::pair<int, int>, BlueTables> g_blue;
+std::map<std::tuple<int, int, int>, BlueTables> g_blue;  // by device, L, M
 
 int blue_fused_len(int L) {
 #define GX_CASE(M) \
@@ -1484,23 +1484,21 @@ int blue_fused_len(int L) {
   return 0;
 }
 
-int blue_tables(int L, BlueTables* out) {
+// The gathered form's: the shortest native length (2^a or 3 * 2^a, at least 8) that holds the linear convolution.
+int blue_gathered_len(int L) {
+  int M = 8;
+  while (M < 2 * L - 1 || !fft_len_ok_any(M)) ++M;
+  return M;
+}
+
+int blue_tables(int L, int M, BlueTables* out) {
   int dev = 0;
   GX_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_blue_mu);
-  auto it = g_blue.find({dev, L});
+  auto it = g_blue.find({dev, L, M});
   if (it != g_blue.end()) {
     *out = it->second;
     return GTOMX_OK;
-  }
-  // the shortest native length (2^a or 3 * 2^a, at least 8) that holds the linear convolution
-  if (L > 2048) return fail(GTOMX_ERR_UNSUPPORTED, "lengths without a native transform must be at most 2048");
-  int M = 8;
-  if (L <= BLUE_FUSED_MAX) {
-    // the shortest the fused form has (384 and 768 points need three steps there)
-    M = blue_fused_len(L);
-  } else {
-    while (M < 2 * L - 1 || !fft_len_ok_any(M)) ++M;
   }
   const long double pi = 3.141592653589793238462643383279502884L;
   std::vector<std::complex<long double>> c(L), bf(M), bi(M);
@@ -1548,7 +1546,7 @@ int blue_tables(int L, BlueTables* out) {
   t.chirp = static_cast<float2*>(d);
   t.bf = t.chirp + L;
   t.bi = t.bf + M;
-  g_blue[{dev, L}] = t;
+  g_blue[{dev, L, M}] = t;
   *out = t;
   return GTOMX_OK;
 }
@@ -1604,7 +1602,7 @@ int line_args(int L, bool rows, LineArgs* out) {
   if (!A.RL) {
     BlueTables t;
     GX_TRY(twiddles(&A.tw));
-    GX_TRY(blue_tables(L, &t));
+    GX_TRY(blue_tables(L, A.M, &t));
     A.t0 = t.chirp;
     A.t1 = t.bf;
     *out = A;
@@ -1733,8 +1731,9 @@ int blue_axis(const void* src, AxisLines as, void* dst, AxisLines ad, long long 
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   BlueTables t;
-  GX_TRY(blue_tables(L, &t));
-  const int M = t.M;
+  if (L > 2048) return fail(GTOMX_ERR_UNSUPPORTED, "lengths without a native transform must be at most 2048");
+  const int M = blue_gathered_len(L);
+  GX_TRY(blue_tables(L, M, &t));
   // chunks within 2^31 elements, 256 MB and 65535 tiles of 64 lines
   const long long cap =
       std::max<long long>(1, std::min({((1LL << 31) - 1) / M, (32LL << 20) / M, 65535LL * 64}));
@@ -1776,7 +1775,7 @@ int blue_axis(const void* src, AxisLines as, void* dst, AxisLines ad, long long 
 }
 
 // The y and z axes of half spectra, each native or by the chirp-z form.
-int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t s) {
+int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t s, LineForm form) {
   const float2* tw = nullptr;
   GX_TRY(twiddles(&tw));
   const long long nh = d.x / 2 + 1;
@@ -1787,7 +1786,7 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
     constexpr int D = decltype(DIRC)::value;
     if (fft_len_ok_any(d.y))
       return cols_axis<D>(d.y, data, data, scr.p, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, tw, s);
-    if (d.y <= BLUE_FUSED_MAX)
+    if (d.y <= BLUE_FUSED_MAX && form == LineForm::Fused)
       return line_cols<D>(d.y, data, data, (int)nh, nh, (long long)d.z * batch, 1LL << 62, nh * d.y, 0, s);
     const AxisLines a{nh, 1, nh * d.y, nh};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.z * batch, d.y, 0, 1.f, s);
@@ -1797,7 +1796,8 @@ int yz_axes_any(float2* data, gtomx_int3 d, unsigned batch, int dir, hipStream_t
     if (fft_len_ok_any(d.z))
       return cols_axis<D>(d.z, data, data, scr.p, (int)nh, nh * d.y, (long long)d.y * batch, d.y, nh, nh * d.y * d.z, tw,
                           s);
-    if (d.z <= BLUE_FUSED_MAX && nh * d.y < (1LL << 30))  // the columns of a volume are one contiguous row
+    // the columns of a volume are one contiguous row
+    if (d.z <= BLUE_FUSED_MAX && form == LineForm::Fused && nh * d.y < (1LL << 30))
       return line_cols<D>(d.z, data, data, (int)(nh * d.y), nh * d.y, batch, 1LL << 62, nh * d.y * d.z, 0, s);
     const AxisLines a{nh * d.y, 1, nh * d.y * d.z, nh * d.y};
     return blue_axis<0, 0, D>(data, a, data, a, nh * d.y * batch, d.z, 0, 1.f, s);
@@ -1818,7 +1818,7 @@ bool dims_native(gtomx_int3 d) {
   return row_len_native(d.x) && (d.y == 1 || fft_len_ok_any(d.y)) && (d.z == 1 || fft_len_ok_any(d.z));
 }
 
-int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s) {
+int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipStream_t s, LineForm form) {
   if (dims_native(d)) return fft_r2c(in, out, d, batch, s);
   const long long rows = (long long)d.y * d.z * batch, nh = d.x / 2 + 1;
   if (row_len_native(d.x)) {
@@ -1828,18 +1828,18 @@ int fft_r2c_any(const float* in, float2* out, gtomx_int3 d, unsigned batch, hipS
       GX_TRY(launch_rows_long<true>(d.x, in, out, rows, 1.f, tw, s));
     else
       GX_TRY(launch_rows_r2c(d.x, in, out, rows, tw, s));
-  } else if (d.x <= BLUE_FUSED_MAX) {
+  } else if (d.x <= BLUE_FUSED_MAX && form == LineForm::Fused) {
     GX_TRY(line_rows_r2c(d.x, in, out, rows, (long long)d.y * d.z, s));
   } else {
     GX_TRY((blue_axis<1, 1, -1>(in, AxisLines{1LL << 62, d.x, 0, 1}, out, AxisLines{1LL << 62, nh, 0, 1}, rows, d.x,
                                 (int)nh, 1.f, s)));
   }
-  return yz_axes_any(out, d, batch, -1, s);
+  return yz_axes_any(out, d, batch, -1, s, form);
 }
 
 // work holds a copy of the half spectra (it is transformed in place).
-int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s) {
-  GX_TRY(yz_axes_any(work, d, batch, 1, s));
+int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float scale, hipStream_t s, LineForm form) {
+  GX_TRY(yz_axes_any(work, d, batch, 1, s, form));
   const long long rows = (long long)d.y * d.z * batch, nh = d.x / 2 + 1;
   if (row_len_native(d.x)) {
     const float2* tw = nullptr;
@@ -1847,7 +1847,8 @@ int fft_c2r_any(float2* work, float* out, gtomx_int3 d, unsigned batch, float sc
     if (d.x > 256) return launch_rows_long<false>(d.x, work, out, rows, scale, tw, s);
     return launch_rows_c2r(d.x, work, out, rows, scale, tw, s);
   }
-  if (d.x <= BLUE_FUSED_MAX) return line_rows_c2r(d.x, work, out, rows, (long long)d.y * d.z, scale, s);
+  if (d.x <= BLUE_FUSED_MAX && form == LineForm::Fused)
+    return line_rows_c2r(d.x, work, out, rows, (long long)d.y * d.z, scale, s);
   return blue_axis<2, 2, 1>(work, AxisLines{1LL << 62, nh, 0, 1}, out, AxisLines{1LL << 62, d.x, 0, 1}, rows, d.x,
                             (int)nh, scale, s);
 }

@@ -159,12 +159,18 @@ struct StreamScratch {
 // Batched 3D/2D transforms (dims with dims.z == 1 for 2D). `work` must hold
 // elements_ft(dims) * batch complex values for c2r (the input is copied
 // there first so it is left unmodified); r2c needs no workspace.
-// Extents without a native transform (at most 2048) go through the chirp-z form.
-int fft_r2c(const float* in, float2* out, gtomx_int3 dims, unsigned batch, hipStream_t s);
+// Axes of up to 512 points without a native transform: Fused runs each line inside one
+// kernel (mixed radix or chirp-z), Gathered takes the chirp-z form over gathered lines
+// that every longer one (at most 2048) takes. The two agree to rounding only. A caller
+// whose result is a choice between maps keeps the one it has, or another orientation
+// wins where two tie within rounding: the Picker is Gathered.
+enum class LineForm { Fused, Gathered };
+int fft_r2c(const float* in, float2* out, gtomx_int3 dims, unsigned batch, hipStream_t s,
+            LineForm form = LineForm::Fused);
 // cols > 0 declares the columns x >= cols of every half spectrum zero: the y
 // and z inverses skip them (the result is the same).
 int fft_c2r(const float2* in, float2* work, float* out, gtomx_int3 dims, unsigned batch,
-            float scale, hipStream_t s, int cols = 0);
+            float scale, hipStream_t s, int cols = 0, LineForm form = LineForm::Fused);
 // Axes above 256 go through two passes with a scratch copy of the data
 // (StreamScratch).
 // L = L1 * L2 as the two-pass transforms split it (L above 256).
@@ -200,8 +206,9 @@ int pick_rows_max_long(int n, const float2* G, int nb, long long H, int nrows, i
 // True when every axis of dims has a native transform.
 bool dims_native(gtomx_int3 dims);
 // The inverse along z then y of nb half spectra in place, each axis native or
-// by the chirp-z form (dir -1 forward, +1 inverse).
-int yz_axes_any(float2* data, gtomx_int3 dims, unsigned batch, int dir, hipStream_t s);
+// by a LineForm (dir -1 forward, +1 inverse).
+int yz_axes_any(float2* data, gtomx_int3 dims, unsigned batch, int dir, hipStream_t s,
+                LineForm form = LineForm::Fused);
 // The x C2R (real part, unscaled) of the nb * n * n rows of nb n^3 half spectra
 // H apart in G, by the chirp-z form, written in place: the real map of
 // spectrum o fills the first n^3 floats of its slot (every row is read before

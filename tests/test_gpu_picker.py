@@ -6,6 +6,8 @@ result; the Picker's best-CC map within 1e-4 normwise of the FP64 oracle
 (max|gpu - fp64| / max|fp64|), and the orientation triple identical wherever
 the oracle's top-2 margin exceeds 1e-4 * max|best|.
 """
+import os
+
 import numpy as np
 import pytest
 
@@ -187,3 +189,41 @@ def test_picker_non_native_sizes_match_oracle(gx, orc, cuda):
     sure = ref64["best"] - ref64["top2"] > 1e-4 * np.max(np.abs(ref64["best"]))
     assert sure.sum() > 0.9 * sure.size
     assert np.array_equal(ang[sure], angles[ref64["idx"][sure]])
+
+
+# image (z, y, x), reference: no extent native; native y and z; the reference alone not native; 2D
+LINE_CASES = [((20, 25, 30), 10), ((12, 16, 75), 12), ((32, 16, 16), 14), ((45, 50), 15)]
+
+
+def picker_lines_case(gx, cuda, shape, nr):
+    """(best, winning orientation) of a noise image and reference over 24 orientations (in-plane steps in 2D)."""
+    import torch
+    rng = np.random.default_rng(nr + sum(shape))
+    ref = rng.standard_normal((nr,) * len(shape)).astype(np.float32)
+    image = rng.standard_normal(shape).astype(np.float32)
+    ctf = rng.uniform(-1, 1, ref.shape[:-1] + (nr // 2 + 1,)).astype(np.float32)
+    angles = np.zeros((24, 3), np.float32)
+    angles[:, 2] = np.arange(24) / np.float32(4)
+    if len(shape) == 3:
+        angles[:, :2] = rng.uniform(0, np.pi, (24, 2))
+    pk = gx.Picker(torch.from_numpy(ref).to(cuda), shape)
+    pk.set_image(torch.from_numpy(image).to(cuda), torch.from_numpy(ctf).to(cuda))
+    best = torch.full(shape, -1e30, device=cuda)
+    ang = torch.full(shape + (3,), -1.0, device=cuda)
+    pk.perform_correlation(best, ang, angles=angles)
+    torch.cuda.synchronize()
+    pk.close()
+    same = (to_np(ang)[..., None, :] == angles).all(-1)
+    assert (same.sum(-1) == 1).all()
+    return to_np(best), same.argmax(-1).astype(np.uint8)
+
+
+@pytest.mark.parametrize("shape,nr", LINE_CASES)
+def test_picker_extents_without_native_transform_round_as_recorded(gx, cuda, shape, nr):
+    """golden/picker_lines.npz holds what the class gave before lines of up to 512 points had kernels of their own
+    (commit 899c80c). The winning orientation follows the last bit of the maps where two tie, so the maps keep
+    every bit, whatever the other transforms of these lengths do."""
+    golden = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "picker_lines.npz"))
+    best, index = picker_lines_case(gx, cuda, shape, nr)
+    key = "x".join(map(str, shape))
+    assert np.array_equal(best, golden["best_" + key]) and np.array_equal(index, golden["index_" + key])
