@@ -6,7 +6,7 @@
 //
 // Both are a "line" type LN of the kernels: LN::lanes threads hold a line, thread j
 // the points j + lanes * m, m < LN::PTS, in natural order before and after
-// LN::run. A workgroup stages LN::tables values, then has LN::col_area (strided
+// LN::run (LN::WHOLE: all of them below the line's length). A workgroup stages LN::tables values, then has LN::col_area (strided
 // axes: lanes over adjacent columns) or LN::row_area (contiguous rows: a line's
 // threads are lanes of one wave) values of exchange per line.
 #pragma once
@@ -88,6 +88,7 @@ struct LineArgs {
 template <int M> struct BlueLine {
   using S = BlueShape<M>;
   static constexpr int R1 = S::R1, R2 = S::R2, PTS = R1 / 2, REGS = R1;
+  static constexpr bool WHOLE = false;
   static constexpr int COL_THREADS = S::TX * R2, ROW_WAVES = M <= 512 ? 2 : 1;
   static constexpr int TWL = R1 * (R2 + 1), TABLES = TWL + M + M / 2;
   // LDS of a workgroup, in float2; a constant here, so that it is a static array
@@ -130,6 +131,7 @@ template <int M> struct BlueLine {
 // Tables: W_L^{j k0} at k0 lanes + j, W_lanes^{b k1} at k1 r2 + b.
 template <int RL_> struct SmoothLine {
   static constexpr int RL = RL_, PTS = RL, REGS = RL;
+  static constexpr bool WHOLE = true;
   static constexpr int COL_THREADS = 512, ROW_WAVES = 2;
   static constexpr int COL_LDS = 0, ROW_LDS = 0;  // sized by the length: dynamic
   __host__ __device__ static int lanes(const LineArgs& A) { return A.lanes; }

@@ -1135,14 +1135,20 @@ __global__ __launch_bounds__(LN::COL_THREADS, 2) void k_pick_project_line(
     const bool valid = iy < n && ix * ix + y * y <= half * half;
     float2 e[HP];
     float cf[HP];
-    // element (x, y, p) at (p * n + y) * nh + x: points p >= n lie past the buffers' ends, where loads give
-    // 0 and stores are dropped, as the out-of-range lanes of invalid columns
-    const int bin = (j * n + iy) * nh + ix;
-    auto load_bin = [&](int m) {
-      e[m] = buf_load2(rE, valid ? bin * 8 : OUT_OF_RANGE, m * R2 * n * nh * 8);
-      cf[m] = ctf ? buf_load1(rC, valid ? bin * 4 : OUT_OF_RANGE, m * R2 * n * nh * 4) : 1.f;
+    // element (x, y, p) at (p * n + y) * nh + x. Points p >= n of a chirp-z line (up to its M / 2) load 0 and store
+    // nothing, as the lanes of invalid columns. They say so in the lane's offset: the range check is against the
+    // buffer's size less the scalar offset, which must not pass it, so the scalar offset steps through whole lines only.
+    auto lane_at = [&](int m, int base, int step) {
+      const bool in = valid && (LN::WHOLE || j + R2 * m < n);
+      return in ? base + (LN::WHOLE ? 0 : m * step) : OUT_OF_RANGE;
     };
-    const int gout = valid ? (j * nc * n + col) * 8 : OUT_OF_RANGE;
+    auto scalar_at = [&](int m, int step) { return LN::WHOLE ? m * step : 0; };
+    const int bin = (j * n + iy) * nh + ix, bstep = R2 * n * nh;
+    auto load_bin = [&](int m) {
+      e[m] = buf_load2(rE, lane_at(m, bin * 8, bstep * 8), scalar_at(m, bstep * 8));
+      cf[m] = ctf ? buf_load1(rC, lane_at(m, bin * 4, bstep * 4), scalar_at(m, bstep * 4)) : 1.f;
+    };
+    const int gout = (j * nc * n + col) * 8, gstep = R2 * nc * n * 8;
 #pragma unroll
     for (int m = 0; m < HP; ++m) load_bin(m);
     const bool dc = col == 0 && j == 0;
@@ -1182,7 +1188,7 @@ __global__ __launch_bounds__(LN::COL_THREADS, 2) void k_pick_project_line(
 #pragma unroll
       for (int m = 0; m < HP; ++m) {
         const u32x2 w = __builtin_bit_cast(u32x2, v[m]);
-        __builtin_amdgcn_raw_buffer_store_b64(w, rG, gout, m * R2 * nc * n * 8, CPOL_NT);
+        __builtin_amdgcn_raw_buffer_store_b64(w, rG, lane_at(m, gout, gstep), scalar_at(m, gstep), CPOL_NT);
       }
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) {

@@ -27,8 +27,10 @@ def _inputs(gx, cuda, n, box, nvol, nd, seed):
 
 
 # k_pick_plane_max: 16 .. 128 (several planes per workgroup up to 48); 8, 12, 192: the passes above and
-# below it; chirp-z lines: the edges of the convolution lengths 48 .. 1024, odd and even
-@pytest.mark.parametrize("n", [8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 21, 25, 49, 50, 97, 129, 150, 258])
+# below it; chirp-z lines: the edges of the convolution lengths 48 .. 1024, odd and even; 37, 67, 131, 191: chirp-z
+# lines whose threads hold whole rows of points past the side
+@pytest.mark.parametrize("n", [8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 21, 25, 49, 50, 97, 129, 150, 258, 37, 67, 131,
+                               191])
 def test_passes_match_oracle_and_each_other(gx, orc, cuda, n):
     import torch
     box = 2 * max(2, min(8, n // 4))
