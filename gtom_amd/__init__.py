@@ -78,6 +78,8 @@ _SIGS = {
     "gtomx_status_string": [_I],
     "gtomx_last_error": [],
     "gtomx_debug_fail_alloc_after": [_I],
+    "gtomx_scratch_held": [ctypes.POINTER(_SZ)],
+    "gtomx_scratch_release": [],
     "gtomx_equal_angular_spacing": [_F, _F, _F, _F, _F, _F, _F, _P, _I, ctypes.POINTER(_I)],
     "gtomx_fibonacci_angles": [_I, _I, _P],
     "gtomx_projector_matrices": [_P, _U, _F, _P],
@@ -209,6 +211,18 @@ def exported_symbols():
 
 def last_error():
     return lib().gtomx_last_error().decode()
+
+
+def scratch_held():
+    """Bytes of scratch the library keeps between calls on the current device."""
+    n = _SZ()
+    check(lib().gtomx_scratch_held(ctypes.byref(n)), "gtomx_scratch_held")
+    return n.value
+
+
+def scratch_release():
+    """Returns the kept scratch of the current device to the runtime."""
+    check(lib().gtomx_scratch_release(), "gtomx_scratch_release")
 
 
 def check(status, where):

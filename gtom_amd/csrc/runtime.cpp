@@ -57,10 +57,10 @@ int alloc_hook() {
 // runtime's own pool. Each block carries the event of its last use, which the
 // next taker's stream waits for, so a block is never written while an earlier
 // user still reads it, whatever became of that user's stream. Unused blocks hold
-// at most SCRATCH_CAP bytes per device: the least recently used go back to the
-// runtime when a new block would pass that, those not taken for SCRATCH_IDLE
-// takes at the next new block, and all of them when an allocation of this
-// library fails. Blocks come from hipMallocAsync and go back through
+// at most SCRATCH_CAP bytes per device: whenever a block is given back or a new one
+// made, the least recently used beyond that go back to the runtime, and those not
+// taken for SCRATCH_IDLE takes with them. All of them go when an allocation of this
+// library fails, and when the program asks (gtomx_scratch_release). Blocks come from hipMallocAsync and go back through
 // hipFreeAsync, which other threads' stream captures allow.
 struct ScratchBlock {
   void* p = nullptr;  // nullptr: a free slot
@@ -110,14 +110,15 @@ void trim_locked(ScratchPool& pool, int dev, size_t keep, hipStream_t s) {
   }
 }
 
-// Gives every unused block of the current device back (an allocation has failed).
-void trim_all() {
+// Gives every unused block of the current device back (an allocation has failed, or the program asks).
+hipError_t trim_all() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
   ScratchPool& pool = scratch_pool();
   std::lock_guard<std::mutex> lk(pool.mu);
   trim_locked(pool, dev, 0, nullptr);
-  (void)hipStreamSynchronize(nullptr);  // the runtime's pool releases what is free at a wait
+  return hipStreamSynchronize(nullptr);  // the runtime's pool releases what is free at a wait
 }
 
 // hipMalloc, once more without the kept scratch if it fails.
@@ -125,7 +126,7 @@ hipError_t malloc_or_trim(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  trim_all();
+  (void)trim_all();
   return hipMalloc(p, bytes);
 }
 
@@ -224,6 +225,7 @@ StreamScratch::~StreamScratch() {
   ScratchPool& pool = scratch_pool();
   std::lock_guard<std::mutex> lk(pool.mu);
   ScratchBlock& b = pool.blocks[block];
+  const int dev = b.dev;
   b.busy = false;
   b.last = s;
   if (hipEventRecord(b.ev, s) != hipSuccess) {  // the end of its use is not known: not kept
@@ -232,6 +234,8 @@ StreamScratch::~StreamScratch() {
     (void)hipEventDestroy(b.ev);
     b = ScratchBlock{};
   }
+  // a call with several blocks may have taken more than the cap together
+  trim_locked(pool, dev, SCRATCH_CAP, s);
 }
 
 int twiddles(const float2** table) {
@@ -314,6 +318,23 @@ const char* gtomx_status_string(int s) {
 }
 
 const char* gtomx_last_error(void) { return g_last_error.c_str(); }
+
+int gtomx_scratch_release(void) {
+  GX_HIP(trim_all());
+  return GTOMX_OK;
+}
+
+int gtomx_scratch_held(size_t* bytes) {
+  if (!bytes) return fail(GTOMX_ERR_INVALID_ARGUMENT, "bytes is NULL");
+  *bytes = 0;
+  int dev = 0;
+  GX_HIP(hipGetDevice(&dev));
+  ScratchPool& pool = scratch_pool();
+  std::lock_guard<std::mutex> lk(pool.mu);
+  for (const auto& b : pool.blocks)
+    if (b.p && b.dev == dev && !b.busy) *bytes += b.bytes;
+  return GTOMX_OK;
+}
 
 void gtomx_debug_fail_alloc_after(int n) { g_fail_alloc_after.store(n < 0 ? 0 : n); }
 

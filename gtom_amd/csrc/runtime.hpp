@@ -140,7 +140,7 @@ struct DevBuf {
 
 // Stream-ordered scratch of one call: taken on stream s, given back on s when
 // the object goes away, so the caller does not synchronise. Blocks are kept
-// for the next call of any thread or stream (scratch_take in runtime.cpp).
+// for the next call of any thread or stream (the pool in runtime.cpp).
 struct StreamScratch {
   float2* p = nullptr;
   StreamScratch() = default;

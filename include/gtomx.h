@@ -59,6 +59,14 @@ const char* gtomx_last_error(void);
  * library fail with GTOMX_ERR_OUT_OF_MEMORY (n = 0 disables). */
 void gtomx_debug_fail_alloc_after(int n);
 
+/* Scratch that calls keep for the next ones, at most 4 GiB per device between
+ * calls (no reference counterpart): gtomx_scratch_held gives the bytes held on
+ * the current device, gtomx_scratch_release returns them to the runtime, for a
+ * program that needs the memory elsewhere, once their last uses are over. Any
+ * thread may call it, but none while a stream captures in global mode. */
+int gtomx_scratch_held(size_t* bytes);
+int gtomx_scratch_release(void);
+
 /* ------------------------------------------------------------------------ */
 /* Angles and rotation matrices (host)                                       */
 /* ------------------------------------------------------------------------ */

@@ -70,3 +70,33 @@ def test_scratch_from_threads(gx, cuda):
     for t in threads:
         t.join()
     assert not bad
+
+
+CAP = 4 << 30  # include/gtomx.h
+
+
+def test_kept_scratch_is_bounded_and_released(gx, cuda):
+    """Two blocks of 2.02 GiB and three small ones of one call pass the cap together: what is held afterwards does
+    not, on the default stream and on another, and a release gives all of it back to the device."""
+    import torch
+    n, p, nang = 256, 32, 32
+    rng = np.random.default_rng(8)
+    projft = gx.prepare_projector(torch.from_numpy(rng.standard_normal((16, 16, 16)).astype(np.float32)).to(cuda), p)
+    E = gx.d_FFTR2C(torch.from_numpy(rng.standard_normal((2, n, n, n)).astype(np.float32)).to(cuda))
+    ctf = torch.ones((2, n, n, n // 2 + 1), device=cuda)
+    angles = rng.uniform(0, 6, (nang, 3)).astype(np.float32)
+    assert 2 * nang * (n // 2 + 1) * n * n * 8 > CAP
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            gx.d_PickSubTomogramsDiff2(projft, p, p / n, E, ctf, (2, 2, 2), angles)
+        stream.synchronize()
+        held = gx.scratch_held()
+        assert 0 < held <= CAP, held
+    free = torch.cuda.mem_get_info()[0]
+    gx.scratch_release()
+    assert gx.scratch_held() == 0
+    assert torch.cuda.mem_get_info()[0] >= free + held // 2
+    X = gx.d_IFFTC2R(E, n)  # and the next call takes blocks again
+    torch.cuda.synchronize()
+    assert gx.scratch_held() > 0 and torch.isfinite(X).all()
