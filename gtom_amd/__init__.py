@@ -78,6 +78,7 @@ _SIGS = {
     "gtomx_status_string": [_I],
     "gtomx_last_error": [],
     "gtomx_debug_fail_alloc_after": [_I],
+    "gtomx_debug_out_of_memory": [_I],
     "gtomx_scratch_held": [ctypes.POINTER(_SZ)],
     "gtomx_scratch_release": [],
     "gtomx_equal_angular_spacing": [_F, _F, _F, _F, _F, _F, _F, _P, _I, ctypes.POINTER(_I)],
@@ -175,7 +176,8 @@ _SIGS = {
     "gtomx_pnet_debug_gemm": [_P, _P, _P, _I, _I, _I, _P],
 }
 _RESTYPES = {"gtomx_version": ctypes.c_char_p, "gtomx_status_string": ctypes.c_char_p,
-             "gtomx_last_error": ctypes.c_char_p, "gtomx_debug_fail_alloc_after": None}
+             "gtomx_last_error": ctypes.c_char_p, "gtomx_debug_fail_alloc_after": None,
+             "gtomx_debug_out_of_memory": None}
 
 
 def _load_torch_runtime_first():

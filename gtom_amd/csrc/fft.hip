@@ -1534,7 +1534,7 @@ int blue_tables(int L, int M, BlueTables* out) {
     h[L + M + k] = make_float2((float)bi[k].real(), (float)bi[k].imag());
   }
   void* d = nullptr;
-  hipError_t e = hipMalloc(&d, h.size() * sizeof(float2));
+  hipError_t e = malloc_or_trim(&d, h.size() * sizeof(float2));
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(chirp tables)");
   e = hipMemcpy(d, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -1625,7 +1625,7 @@ int line_args(int L, bool rows, LineArgs* out) {
     for (int k = 0; k < A.r1; ++k)
       for (int b = 0; b < A.r2; ++b) h[L + k * A.r2 + b] = root(b * k, Q);
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, h.size() * sizeof(float2));
+    hipError_t e = malloc_or_trim(&p, h.size() * sizeof(float2));
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(line tables)");
     e = hipMemcpy(p, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice);
     if (e != hipSuccess) {

@@ -14,6 +14,7 @@ namespace gx {
 namespace {
 thread_local std::string g_last_error;
 std::atomic<int> g_fail_alloc_after{0};
+std::atomic<int> g_oom_tries{0};
 
 struct DeviceTables {
   float2* tw = nullptr;
@@ -121,16 +122,35 @@ hipError_t trim_all() {
   return hipStreamSynchronize(nullptr);  // the runtime's pool releases what is free at a wait
 }
 
-// hipMalloc, once more without the kept scratch if it fails.
-hipError_t malloc_or_trim(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipErrorOutOfMemory) return e;
+// One try of an allocation (on stream s: hipMallocAsync), or the out-of-memory hook's answer.
+hipError_t try_malloc(void** p, size_t bytes, bool ordered, hipStream_t s) {
+  int n = g_oom_tries.load();
+  while (n > 0)
+    if (g_oom_tries.compare_exchange_weak(n, n - 1)) return hipErrorOutOfMemory;
+  return ordered ? hipMallocAsync(p, bytes, s) : hipMalloc(p, bytes);
+}
+
+// hipMallocAsync, once more without the kept scratch if it fails. The pool is locked.
+hipError_t malloc_async_or_trim(ScratchPool& pool, int dev, void** p, size_t bytes, hipStream_t s) {
+  hipError_t e = try_malloc(p, bytes, true, s);
+  if (e == hipSuccess) return e;
   (void)hipGetLastError();
-  (void)trim_all();
-  return hipMalloc(p, bytes);
+  trim_locked(pool, dev, 0, s);
+  (void)hipStreamSynchronize(s);
+  e = try_malloc(p, bytes, true, s);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 }  // namespace
+
+hipError_t malloc_or_trim(void** p, size_t bytes) {
+  hipError_t e = try_malloc(p, bytes, false, nullptr);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  (void)trim_all();
+  return try_malloc(p, bytes, false, nullptr);
+}
 
 int dev_alloc(void** p, size_t bytes) {
   *p = nullptr;
@@ -156,11 +176,9 @@ int StreamScratch::take(size_t n, hipStream_t st, bool counted) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   const bool plain = hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
   if (!plain) (void)hipGetLastError();
-  if (!plain || bytes > SCRATCH_CAP) {
-    // a capture records the allocation as a node of its graph; larger requests are not kept
-    void* q = nullptr;
-    hipError_t e = hipMallocAsync(&q, bytes, st);
-    if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(FFT scratch)");
+  void* q = nullptr;
+  if (!plain) {  // a capture records the allocation as a node of its graph
+    GX_HIP(hipMallocAsync(&q, bytes, st));
     p = static_cast<float2*>(q);
     return GTOMX_OK;
   }
@@ -168,6 +186,12 @@ int StreamScratch::take(size_t n, hipStream_t st, bool counted) {
   GX_HIP(hipGetDevice(&dev));
   ScratchPool& pool = scratch_pool();
   std::lock_guard<std::mutex> lk(pool.mu);
+  if (bytes > SCRATCH_CAP) {  // not kept
+    hipError_t e = malloc_async_or_trim(pool, dev, &q, bytes, st);
+    if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(scratch)");
+    p = static_cast<float2*>(q);
+    return GTOMX_OK;
+  }
   ++pool.tick;
   // the smallest unused block of this stream that fits without wasting more than half of it; another
   // stream's only where the cap leaves no room for a block of this one's own (it would wait for the other)
@@ -190,14 +214,8 @@ int StreamScratch::take(size_t n, hipStream_t st, bool counted) {
     ScratchBlock b;
     b.bytes = (std::max<size_t>(bytes, 1) + 0xffff) & ~(size_t)0xffff;
     b.dev = dev;
-    hipError_t e = hipMallocAsync(&b.p, b.bytes, st);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      trim_locked(pool, dev, 0, st);
-      (void)hipStreamSynchronize(st);
-      e = hipMallocAsync(&b.p, b.bytes, st);
-    }
-    if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(FFT scratch)");
+    hipError_t e = malloc_async_or_trim(pool, dev, &b.p, b.bytes, st);
+    if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(scratch)");
     e = hipEventCreateWithFlags(&b.ev, hipEventDisableTiming);
     if (e != hipSuccess) {
       (void)hipFreeAsync(b.p, st);
@@ -256,7 +274,7 @@ int twiddles(const float2** table) {
       h[TW_LEN_HOST + m] = make_float2((float)std::cos(a), (float)std::sin(a));
     }
     void* d = nullptr;
-    hipError_t e = hipMalloc(&d, sizeof(float2) * total);
+    hipError_t e = malloc_or_trim(&d, sizeof(float2) * total);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(twiddles)");
     e = hipMemcpy(d, h.data(), sizeof(float2) * total, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -337,6 +355,7 @@ int gtomx_scratch_held(size_t* bytes) {
 }
 
 void gtomx_debug_fail_alloc_after(int n) { g_fail_alloc_after.store(n < 0 ? 0 : n); }
+void gtomx_debug_out_of_memory(int n) { g_oom_tries.store(n < 0 ? 0 : n); }
 
 // GetEqualAngularSpacing (src/Helpers/AngularSpacing.cu:46-67) with float32
 // loop counters so that the orientation count and order match the reference.

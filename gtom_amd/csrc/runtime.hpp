@@ -43,6 +43,9 @@ int hip_fail(hipError_t e, const char* what);
     if (gx_s_ != GTOMX_OK) return gx_s_; \
   } while (0)
 
+// hipMalloc, once more without the kept scratch (StreamScratch) if memory is out; for
+// tables that stay.
+hipError_t malloc_or_trim(void** p, size_t bytes);
 // Device allocation through the library's allocator (honours the test hook).
 int dev_alloc(void** p, size_t bytes);
 void dev_free(void* p);

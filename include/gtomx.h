@@ -58,6 +58,9 @@ const char* gtomx_last_error(void);
  * counterpart): makes the n-th following device allocation made by this
  * library fail with GTOMX_ERR_OUT_OF_MEMORY (n = 0 disables). */
 void gtomx_debug_fail_alloc_after(int n);
+/* The same one level down: the device answers "out of memory" to the next n tries
+ * of an allocation (an allocation gives the kept scratch back and tries twice). */
+void gtomx_debug_out_of_memory(int n);
 
 /* Scratch that calls keep for the next ones, at most 4 GiB per device between
  * calls (no reference counterpart): gtomx_scratch_held gives the bytes held on

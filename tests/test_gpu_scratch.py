@@ -100,3 +100,43 @@ def test_kept_scratch_is_bounded_and_released(gx, cuda):
     X = gx.d_IFFTC2R(E, n)  # and the next call takes blocks again
     torch.cuda.synchronize()
     assert gx.scratch_held() > 0 and torch.isfinite(X).all()
+
+
+@pytest.mark.parametrize("what", ["kept", "above the cap", "tables"])
+def test_out_of_memory_gives_the_kept_scratch_back_and_tries_again(gx, cuda, what):
+    """Every allocation behind a transform, told once that memory is out, is made at the second try with nothing kept;
+    told twice it is refused, and the next call is well again."""
+    import torch
+    x = torch.from_numpy(np.random.default_rng(9).standard_normal((1, 64, 64)).astype(np.float32)).to(cuda)
+    X = gx.d_FFTR2C(x, ndims=2)
+    if what == "above the cap":
+        X = X.expand(CAP // (8 * 64 * 33) + 1, 64, 33).contiguous()
+    for tries in (1, 2):
+        gx.scratch_release()
+        big = gx.d_IFFTC2R(gx.d_FFTR2C(torch.zeros((1, 512, 512), device=cuda), ndims=2), 512, ndims=2)
+        torch.cuda.synchronize()
+        kept = gx.scratch_held()
+        assert kept >= 8 * 512 * 257
+        lines = torch.ones((1, 3, 467 if tries == 1 else 461), device=cuda)  # chirp-z lengths no other test takes
+        gx.lib().gtomx_debug_out_of_memory(tries)
+        try:
+            if what == "tables":
+                call = lambda: gx.d_FFTR2C(lines, ndims=2)  # takes no scratch of its own
+            else:
+                call = lambda: gx.d_IFFTC2R(X, 64, ndims=2)
+            if tries == 2:
+                with pytest.raises(gx.GtomxError, match="(?i)memory"):
+                    call()
+            else:
+                y = call()
+        finally:
+            gx.lib().gtomx_debug_out_of_memory(0)
+        torch.cuda.synchronize()
+        assert gx.scratch_held() < kept
+        if tries == 1 and what == "tables":
+            assert abs(to_np(y)[0, 0, 0] - 3 * 467) <= 1e-2 and np.abs(to_np(y)[0].ravel()[1:]).max() <= 1e-2
+        elif tries == 1:
+            assert torch.equal(y[0], y[-1]) and (y[0] - x[0]).abs().max() <= 1e-5
+        y = call()
+        torch.cuda.synchronize()
+        del y, big
