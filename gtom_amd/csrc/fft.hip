@@ -1881,7 +1881,15 @@ extern "C" int gtomx_ifft_c2r(const gtomx_complex* d_input, float* d_output, int
   StreamScratch work;
   GX_TRY(work.take(elements_ft(dims) * batch, s, true));
   float scale = renormalize ? (float)(1.0 / (double)elements(dims)) : 1.0f;
-  GX_TRY(fft_c2r(reinterpret_cast<const float2*>(d_input), work.p, d_output, dims, batch, scale, s));
+  const float2* in = reinterpret_cast<const float2*>(d_input);
+  const size_t H = elements_ft(dims) * batch;
+  // an output over the input: rows and slices of the batch are written while others are still to be read
+  const uintptr_t i0 = (uintptr_t)in, o0 = (uintptr_t)d_output;
+  if (o0 < i0 + H * sizeof(float2) && i0 < o0 + elements(dims) * batch * sizeof(float)) {
+    GX_HIP(hipMemcpyAsync(work.p, in, H * sizeof(float2), hipMemcpyDeviceToDevice, s));
+    in = work.p;
+  }
+  GX_TRY(fft_c2r(in, work.p, d_output, dims, batch, scale, s));
   GX_HIP(hipStreamSynchronize(s));
   return GTOMX_OK;
 }

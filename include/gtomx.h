@@ -108,8 +108,8 @@ int gtomx_fft_r2c(const float* d_input, gtomx_complex* d_output, int ndims, gtom
 /* d_IFFTC2R, include/FFT.cuh:150 / src/FFT/IFFT.cu:8-56: inverse transform of
  * half spectra; renormalize != 0 multiplies by 1/N. The result is the real
  * part of the inverse DFT of the Hermitian-completed spectrum. The input is
- * not modified (the reference's cuFFT call may clobber it). Extents as for
- * gtomx_fft_r2c. */
+ * not modified (the reference's cuFFT call may clobber it) unless the output
+ * lies over it, which is allowed. Extents as for gtomx_fft_r2c. */
 int gtomx_ifft_c2r(const gtomx_complex* d_input, float* d_output, int ndims, gtomx_int3 dims,
                    unsigned batch, int renormalize, void* stream);
 

@@ -140,3 +140,24 @@ def test_out_of_memory_gives_the_kept_scratch_back_and_tries_again(gx, cuda, wha
         y = call()
         torch.cuda.synchronize()
         del y, big
+
+
+# rows alone (native up to 256 and above), rows without a native transform, and a batch of several slices
+@pytest.mark.parametrize("ndims,shape", [(1, (37, 64)), (1, (9, 4096)), (1, (6, 75)), (2, (20, 1024, 2048)),
+                                         (2, (3, 64, 48))])
+@pytest.mark.parametrize("at", ["start", "end"])
+def test_c2r_over_its_own_input(gx, cuda, ndims, shape, at):
+    """The output may lie over the spectra: at their start, and at the end of the same buffer."""
+    import torch
+    nx, batch = shape[-1], int(np.prod(shape[:-ndims]))
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(nx)
+    X = gx.d_FFTR2C(torch.randn(shape, device=cuda, generator=gen), ndims=ndims)
+    want = gx.d_IFFTC2R(X, nx, ndims=ndims)
+    buf = torch.view_as_real(X).reshape(-1).clone()
+    n = want.numel()
+    o = 0 if at == "start" else (buf.numel() - n) // 2 * 2
+    dims = (nx,) + tuple(reversed(shape[-ndims:-1])) + (1,) * (3 - ndims)
+    gx.check(gx.lib().gtomx_ifft_c2r(gx._ptr(buf), gx._ptr(buf[o:]), ndims, gx.int3(*dims), batch, 1, gx._stream()),
+             "gtomx_ifft_c2r")
+    assert torch.equal(buf[o:o + n].reshape(want.shape), want)
