@@ -161,3 +161,20 @@ def test_c2r_over_its_own_input(gx, cuda, ndims, shape, at):
     gx.check(gx.lib().gtomx_ifft_c2r(gx._ptr(buf), gx._ptr(buf[o:]), ndims, gx.int3(*dims), batch, 1, gx._stream()),
              "gtomx_ifft_c2r")
     assert torch.equal(buf[o:o + n].reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("ndims,shape", [(2, (20, 1024, 2048)), (3, (7, 768, 16, 512)), (2, (3, 4096, 4096))])
+def test_slices_of_a_batch_equal_items_alone(gx, cuda, ndims, shape):
+    """Axes of two passes go through the scratch in slices of about 128 MB (15 of 20 items, 5 of 7, one by one): every item bit for bit as transformed alone, and the C2R's input as it was."""
+    import torch
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(shape[0])
+    x = torch.randn(shape, device=cuda, generator=gen)
+    X = gx.d_FFTR2C(x, ndims=ndims)
+    keep = X.clone()
+    y = gx.d_IFFTC2R(X, shape[-1], ndims=ndims)
+    assert torch.equal(torch.view_as_real(X), torch.view_as_real(keep))
+    for i in range(shape[0]):
+        Xi = gx.d_FFTR2C(x[i:i + 1].contiguous(), ndims=ndims)
+        assert torch.equal(torch.view_as_real(X[i:i + 1]), torch.view_as_real(Xi)), i
+        assert torch.equal(y[i:i + 1], gx.d_IFFTC2R(Xi, shape[-1], ndims=ndims)), i
