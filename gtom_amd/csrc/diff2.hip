@@ -205,6 +205,11 @@ extern "C" int gtomx_pick_subtomograms_diff2(const gtomx_complex* d_projectorft,
   const unsigned B = std::min<unsigned>(nangles, 32);
   std::vector<float> h_mats(9 * (size_t)nangles);
   GX_TRY(gtomx_projector_matrices(h_angles, nangles, oversample, h_mats.data()));
+  // R_a: the projections at the volume size (d_rlnProject, :195), rmax = n/2, once for all volumes (each volume
+  // sampling every orientation anew was 64 of 256 launches and 1.5 of 7.1 ms for 8 volumes of 64^3 x 250), as long as
+  // their copy stays below 4 GiB (320^3 with 32 orientations). Above, each volume's in place: the copy would take as
+  // much again as the projections (137 GB at 1024^3), and sampling is a smaller part of the work there.
+  const bool share = nvolumes > 1 && (size_t)B * H * sizeof(float2) <= (4ull << 30);
   const std::vector<float2> wx = phases(nh, rx, n), wy = phases(n, ry, n), wz = phases(n, rz, n);
   StreamScratch mats, Wx, Wy, Wz, R, Q, T1, T2, T3, sums;
   GX_TRY(mats.take((h_mats.size() + 1) / 2, s, true));
@@ -212,12 +217,12 @@ extern "C" int gtomx_pick_subtomograms_diff2(const gtomx_complex* d_projectorft,
   GX_TRY(Wy.take(wy.size(), s, true));
   GX_TRY(Wz.take(wz.size(), s, true));
   GX_TRY(R.take((size_t)B * H, s, true));
-  if (nvolumes > 1) GX_TRY(Q.take((size_t)B * H, s, true));
+  if (share) GX_TRY(Q.take((size_t)B * H, s, true));
   GX_TRY(T1.take((size_t)B * n * n * rx, s, true));
   GX_TRY(T2.take((size_t)B * n * rx * ry, s, true));
   GX_TRY(T3.take((size_t)B * Vr, s, true));
   GX_TRY(sums.take((size_t)B * NBLK + B + NBLK + 1, s, true));
-  float2* q = nvolumes > 1 ? Q.p : R.p;  // one volume: in place
+  float2* q = share ? Q.p : R.p;
   float* d_mats = reinterpret_cast<float*>(mats.p);
   double *parts = reinterpret_cast<double*>(sums.p), *asum = parts + (size_t)B * NBLK, *eparts = asum + B,
          *esum = eparts + NBLK;
@@ -228,11 +233,10 @@ extern "C" int gtomx_pick_subtomograms_diff2(const gtomx_complex* d_projectorft,
 
   for (unsigned b0 = 0; b0 < nangles; b0 += B) {
     const unsigned nb = std::min(B, nangles - b0);
-    // R_a: the projection at the volume size (d_rlnProject, :195), rmax = n/2, once for all volumes (each volume
-    // sampling every orientation anew was 64 of 256 launches and 1.5 of 7.1 ms for 8 volumes of 64^3 x 250)
-    GX_TRY(project_launch(reinterpret_cast<const float2*>(d_projectorft), p, R.p, n, (unsigned)(n / 2),
-                          d_mats + 9 * (size_t)b0, nb, s));
     for (unsigned v = 0; v < nvolumes; ++v) {
+      if (v == 0 || !share)
+        GX_TRY(project_launch(reinterpret_cast<const float2*>(d_projectorft), p, R.p, n, (unsigned)(n / 2),
+                              d_mats + 9 * (size_t)b0, nb, s));
       const float2* Ev = reinterpret_cast<const float2*>(d_expft) + (size_t)v * H;
       const float* cv = d_ctf + (size_t)v * H;  // one CTF per volume (src/Correlation/SubTomograms.cu:199)
       hipLaunchKernelGGL(k_diff2_q, dim3(NBLK, nb), dim3(256), 0, s, R.p, q, cv, Ev, H, parts, eparts);
@@ -250,8 +254,8 @@ extern "C" int gtomx_pick_subtomograms_diff2(const gtomx_complex* d_projectorft,
       // z: T2 rows (a, dx*ry + dy) over kz -> T3[a][dx][dy][dz]
       GX_TRY(contract(T2.p, T3.p, Wz.p, (long long)nb, rx * ry, rz, n,
                       (long long)n * rx * ry, 1LL, (long long)rx * ry, (long long)Vr, (long long)rz, s));
-      hipLaunchKernelGGL(k_diff2_update, dim3((unsigned)((Vr + 255) / 256)), dim3(256), 0, s, T3.p, asum, esum, rx, ry, rz, (int)nb, (int)b0,
-                         d_bestdiff2 + (size_t)v * Vr, d_bestangle + (size_t)v * Vr);
+      hipLaunchKernelGGL(k_diff2_update, dim3((unsigned)((Vr + 255) / 256)), dim3(256), 0, s, T3.p, asum, esum, rx, ry,
+                         rz, (int)nb, (int)b0, d_bestdiff2 + (size_t)v * Vr, d_bestangle + (size_t)v * Vr);
       GX_LAUNCHED("k_diff2_update");
     }
   }

@@ -93,3 +93,31 @@ def test_diff2_shift_ranges(gx, orc, cuda, n, rel, nvol, nang):
         assert rel_linf(best[v], rb) <= 1e-5
         sure = (two.values[1] - two.values[0]).cpu().numpy() > 1e-5 * np.abs(rb).max()
         assert np.array_equal(ang[v][sure], ri[sure].astype(np.float32))
+
+
+@pytest.mark.parametrize("n,allocations", [(320, 10), (322, 9)])
+def test_diff2_large_volumes_take_no_copy_of_the_projections(gx, cuda, n, allocations):
+    """32 projections of 320^3 are just below 4 GiB, of 322^3 above: up to there the volumes of a call share them
+    (10 allocations), above each volume's are made in place (9). Either way a volume's result is that of a call
+    on its own, bit for bit."""
+    import torch
+    rng = np.random.default_rng(n)
+    p = 32
+    projft = gx.prepare_projector(torch.from_numpy(rng.standard_normal((16, 16, 16)).astype(np.float32)).to(cuda), p)
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(n)
+    E = torch.randn((2, n, n, n // 2 + 1), device=cuda, generator=gen, dtype=torch.complex64)
+    ctf = torch.rand((2, n, n, n // 2 + 1), device=cuda, generator=gen)
+    angles = rng.uniform(0, TAU, (33, 3)).astype(np.float32)
+    args = (projft, p, p / n, E, ctf, (3, 2, 4), angles)
+    try:
+        gx.lib().gtomx_debug_fail_alloc_after(allocations)
+        with pytest.raises(gx.GtomxError):
+            gx.d_PickSubTomogramsDiff2(*args)
+        gx.lib().gtomx_debug_fail_alloc_after(allocations + 1)
+        best, index = gx.d_PickSubTomogramsDiff2(*args)
+    finally:
+        gx.lib().gtomx_debug_fail_alloc_after(0)
+    for v in range(2):
+        b, i = gx.d_PickSubTomogramsDiff2(projft, p, p / n, E[v:v + 1], ctf[v:v + 1], (3, 2, 4), angles)
+        assert torch.equal(b[0], best[v]) and torch.equal(i[0], index[v])
