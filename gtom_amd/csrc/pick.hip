@@ -1231,7 +1231,6 @@ void plan_release(gtomx_pick_plan* pl) {
   dev_free(pl->sn);
   dev_free(pl->mats);
   dev_free(pl->ls_mem);
-  dev_free(pl->ebuf);
   dev_free(pl->cproj);
   dev_free(pl->gbest);
   dev_free(pl->gidx);
@@ -2065,9 +2064,6 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   pl->sn = static_cast<float2*>(d);
   d = nullptr;
   alloc(&pl->ls_mem, local_std_scratch_bytes(dv));
-  alloc(&d, pl->V * sizeof(float));
-  pl->ebuf = static_cast<float*>(d);
-  d = nullptr;
   alloc(&d, (size_t)centred_bytes(pl->p));
   pl->cproj = static_cast<float2*>(d);
   if (big2d) {
@@ -2308,10 +2304,11 @@ int gtomx_pick_subtomograms_learned(gtomx_pick_plan* plan, gtomx_pnet* net, cons
   std::vector<float> mass(ntl), pnp(ntl);
   gtomx_learned_stats st{};
   for (unsigned v = 0; v < nvolumes; ++v) {
-    // the network reads the block in real space: C2R_u(E_v) (its standardisation removes the scale)
+    // the network reads the block in real space: C2R_u(E_v) (its standardisation removes the scale), in a volume of
+    // the local deviation's scratch, which pick_finish fills later
     const float2* Ev = reinterpret_cast<const float2*>(d_expft) + (size_t)v * plan->H;
-    GX_TRY(fft_c2r(Ev, plan->G, plan->ebuf, dimsvolume, 1, 1.0f, s));
-    GX_TRY(gtomx_pnet_load_volume(net, plan->ebuf, dimsvolume, stream));
+    GX_TRY(fft_c2r(Ev, plan->G, plan->ls.c1, dimsvolume, 1, 1.0f, s));
+    GX_TRY(gtomx_pnet_load_volume(net, plan->ls.c1, dimsvolume, stream));
     GX_TRY(gtomx_pnet_forward(net, (unsigned)ntl, nullptr, stream));
     GX_TRY(gtomx_pnet_propose(net, topk, plan->ldirs, plan->ltop1, plan->lcls, plan->lmass, plan->lpnp, stream));
     GX_HIP(hipMemcpyAsync(dirs.data(), plan->ldirs, ntl * topk * sizeof(int32_t), hipMemcpyDeviceToHost, s));

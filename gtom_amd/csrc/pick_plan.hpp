@@ -34,7 +34,6 @@ struct gtomx_pick_plan {
   bool mats_ev_recorded = false;
   void* ls_mem = nullptr;
   gx::LocalStdScratch ls{};
-  float* ebuf = nullptr;
   float2* cproj = nullptr;  // centred projector layout
   float* gbest = nullptr;   // per-orientation-group maxima (groups x V)
   int32_t* gidx = nullptr;

@@ -70,3 +70,13 @@ def test_images_in_one_call_equal_images_alone(gx, cuda, n, batch):
             torch.cuda.synchronize()
             assert torch.equal(b[0], best[v]) and torch.equal(i[0], idx[v]), (shared, v)
         plan.close()
+
+
+def test_plan_holds_what_its_passes_use(gx, cuda):
+    """One orientation a pass of 300^3: the batch's spectrum, three spectra and three volumes of the local deviation,
+    and tables; no volume (108 MB) that only another form reads."""
+    n = 300
+    plan = gx.PickPlan(32, n, 1)
+    h, v = (n // 2 + 1) * n * n, n ** 3
+    assert 0 <= plan.device_bytes - (4 * 8 * h + 3 * 4 * v) <= 4 << 20
+    plan.close()
