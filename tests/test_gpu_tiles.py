@@ -5,8 +5,9 @@ on the tiles set in its mask. Checked bit for bit against the plain update
 maximum over the groups whose mask sets that tile, in increasing orientation
 order, with those groups' indices; tiles set in no mask keep the values begin
 wrote. The masks reach pass 2 (planes and rows skipped) and pass 3 (rows
-skipped, voxels of unset tiles untouched), so random masks at the benchmark's
-256^3 shape and at 64^3 cover both the skipping and the per-voxel masking."""
+skipped, voxels of unset tiles untouched), or the plane kernel up to 128, so
+random masks at the benchmark's 256^3 shape and at every smaller side a mask can
+have cover both the skipping and the per-voxel masking."""
 import numpy as np
 import pytest
 
@@ -28,7 +29,8 @@ def _setup(gx, cuda, n, box, seed):
     return rng, p, projft, exp_ft, ctf
 
 
-@pytest.mark.parametrize("n,box,ngroups,group", [(64, 16, 5, 6), (256, 48, 4, 18)])
+@pytest.mark.parametrize("n,box,ngroups,group", [(64, 16, 5, 6), (256, 48, 4, 18), (32, 16, 5, 6), (96, 24, 5, 7),
+                                                 (128, 24, 4, 9), (192, 24, 3, 6)])
 def test_grouped_update_equals_plain_update_per_tile(gx, cuda, n, box, ngroups, group):
     import torch
     rng, p, projft, exp_ft, ctf = _setup(gx, cuda, n, box, n)
@@ -37,7 +39,10 @@ def test_grouped_update_equals_plain_update_per_tile(gx, cuda, n, box, ngroups, 
     nt = n // 32
     masks = (rng.random((1, ngroups, nt, nt, nt)) < 0.4)
     masks[0, 1] = False  # an empty group is skipped
-    masks[0, :, nt - 1, 0, nt - 1] = False  # and one tile is set in no group
+    if nt > 1:
+        masks[0, :, nt - 1, 0, nt - 1] = False  # and one tile is set in no group
+    else:
+        masks[0, ::2] = True
     packed = np.zeros((1, ngroups, nt, nt), np.uint8)
     for tx in range(nt):
         packed |= (masks[..., tx].astype(np.uint8) << tx)
@@ -67,4 +72,4 @@ def test_grouped_update_equals_plain_update_per_tile(gx, cuda, n, box, ngroups, 
     assert np.array_equal(got_b, want_b)
     assert np.array_equal(got_i, want_i)
     untouched = ~masks[0].any(axis=0)[tz, ty, tx]
-    assert untouched.any() and (got_b[untouched] == -1e30).all()
+    assert (untouched.any() or nt == 1) and (got_b[untouched] == -1e30).all()
