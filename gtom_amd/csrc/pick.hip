@@ -358,9 +358,14 @@ __global__ __launch_bounds__(256) void k_pick_herm_norm(Projector P, const float
 }
 
 // The correction, the reduction of the pass-1 sums and the scale in one launch of
-// a workgroup per orientation, for the sides of k_pick_plane_max: their planes
-// are at most 128 x 65 pairs, and one launch less per batch counts (64^3, 196
-// orientations: 27 us for the 32-workgroup form above).
+// a workgroup per orientation, up to 64: one launch less per batch counts there (64^3,
+// 196 orientations: 27 us for the form above with 32 workgroups and k_pick_scale).
+// Above, the two launches: a plane of 128 x 65 pairs keeps one workgroup busy for 28 us
+// whether the batch holds one orientation or 128, which a batch of few cannot hide
+// (128^3, 64 orientations, 1 at a time: 3.6 ms, 2.3 with the two; 2.7 with the separate
+// y and x passes) and a full one need not pay (3 volumes x 288: 5.49 -> 5.39 ms).
+constexpr bool norm_one_launch(int n) { return n <= 64; }
+constexpr int NORM_BLOCKS = 16;
 template <int N>
 __global__ __launch_bounds__(512) void k_pick_norm(Projector P, const float* __restrict__ mats,
                                                    const float2* __restrict__ E, const float* __restrict__ ctf,
@@ -1352,6 +1357,11 @@ template <int N> int plane_groups(unsigned batch, int cus) {
     return std::max(1, std::min((int)batch, resident_planes<N>(cus) / (N / PlaneShape<N>::PL)));
   return 0;
 }
+// The fewest orientations of a group in a batch of nb: above 64 the merge reads more than a plane's chain of two or
+// three takes (128^3: 4 us a group), so up to three orientations stay one group and others make groups of two or
+// more (128^3, 64 orientations in batches of 2: 2.0 -> 1.6 ms, of 3: 1.65 -> 1.40; at least three or four to a group
+// is slower at 96^3 from batches of 5 on).
+constexpr int least_group(int n, int nb) { return n <= 64 ? 1 : (nb <= 3 ? nb : 2); }
 int plane_groups_for(int n, unsigned batch, int cus) {
   switch (n) {
 #define GX_CASE(N) \
@@ -1386,13 +1396,23 @@ int run_batch(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const float
   if constexpr (plane_side(N)) {
     using S = PlaneShape<N>;
     GX_TRY(timed(pl, 1, s, [&]() -> int {
-      hipLaunchKernelGGL(k_pick_norm<N>, dim3(nb), dim3(512), 0, s, P, mats, E, ctf, pl->partial,
-                         pl->ntiles * pass1_waves<N>(), pl->sn);
-      GX_LAUNCHED("k_pick_norm");
+      const int nparts = pl->ntiles * pass1_waves<N>();
+      if constexpr (norm_one_launch(N)) {
+        hipLaunchKernelGGL(k_pick_norm<N>, dim3(nb), dim3(512), 0, s, P, mats, E, ctf, pl->partial, nparts, pl->sn);
+        GX_LAUNCHED("k_pick_norm");
+      } else {
+        hipLaunchKernelGGL(k_pick_herm_norm<N>, dim3(NORM_BLOCKS, nb), dim3(256), 0, s, P, mats, ctf, pl->corr, N, E,
+                           pl->sn);
+        GX_LAUNCHED("k_pick_herm_norm");
+        hipLaunchKernelGGL(k_pick_scale, dim3(nb), dim3(256), 0, s, pl->partial, nparts, pl->corr, NORM_BLOCKS,
+                           (double)pl->H, reinterpret_cast<float*>(pl->sn), 2);
+        GX_LAUNCHED("k_pick_scale");
+      }
       return GTOMX_OK;
     }));
     return timed(pl, 2, s, [&]() -> int {
-      const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
+      const int og = std::max(least_group(N, nb), (nb + pl->groups3 - 1) / pl->groups3);
+      const int groups = (nb + og - 1) / og;
       const bool fresh = groups > 1;
       auto go = [&](auto kernel) -> int {
         hipLaunchKernelGGL(kernel, dim3(N / S::PL, groups), dim3(S::T * S::PL), 0, s, pl->G, nb, angle0, pl->sn,

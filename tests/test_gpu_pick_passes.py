@@ -1,7 +1,7 @@
 """The search's passes at every side class they are chosen for, against the FP64 oracle (max-CC 1e-4
 normwise, identical argmax where the oracle's top-2 margin exceeds 1e-4 * max|top1|, the search's own
 bar), and bit for bit against themselves: results must not depend on the batch (one orientation per
-pass runs ungrouped, a full batch in orientation groups that are merged) nor on how many images share
+pass runs ungrouped, three in one group or three, a full batch in orientation groups that are merged) nor on how many images share
 a launch."""
 import numpy as np
 import pytest
@@ -38,7 +38,7 @@ def test_passes_match_oracle_and_each_other(gx, orc, cuda, n):
     angles = gx.fibonacci_angles(5, 3)[:13]
     norc = 13 if n <= 64 else (4 if n <= 130 else 2)
     res = []
-    for batch, ang in ((0, angles[:norc]), (0, angles), (1, angles), (5, angles)):
+    for batch, ang in ((0, angles[:norc]), (0, angles), (1, angles), (3, angles), (5, angles)):
         plan = gx.PickPlan(p, n, batch)
         best, idx = gx.d_PickSubTomograms(plan, projft, p / n, exp_ft, ctf, ang, n / 8)
         torch.cuda.synchronize()
