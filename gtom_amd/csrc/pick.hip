@@ -1871,6 +1871,25 @@ unsigned even_batch(unsigned most, unsigned count) {
   return (count + passes - 1) / passes;
 }
 
+// Images of a launch of the fused 2D passes in batches of B spectra, which they divide among them. From 16 spectra
+// on four share the samples; below, where a launch costs more than its work, the number with the fewest launches in
+// all, and the fewest images of those (four images of 128^2, 64 orientations: batches of 4 1.77 ms with an orientation
+// of each of four, 1.31 with four of one; of 6 1.76 with one of each, 1.12; each image on its own before 1.71 and 1.29).
+unsigned images_for(unsigned B, unsigned nvol, unsigned nangles) {
+  const unsigned most = std::min({nvol, (unsigned)MAX_IMAGES2, B});
+  if (B >= 16) return most;
+  auto launches = [&](unsigned v) { return (nangles + B / v - 1) / (B / v); };
+  unsigned best = 1, fewest = ~0u;
+  for (unsigned k = 1; k <= most; ++k) {
+    const unsigned passes = nvol / k * launches(k) + (nvol % k ? launches(nvol % k) : 0);
+    if (passes < fewest) {
+      fewest = passes;
+      best = k;
+    }
+  }
+  return best;
+}
+
 int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const CentredProjector* C, const float* mats,
                           unsigned nangles, unsigned nvol, const float2* E, const float* ctf, size_t ctf_stride,
                           float* best, int32_t* idx, int angle0, hipStream_t s) {
@@ -1878,11 +1897,11 @@ int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const Centred
   GX_TRY(twiddles(&tw));
   if (nangles == 0) return GTOMX_OK;
   // images of the fused 2D passes share the samples of an orientation
-  const unsigned images = pl->nz == 1 && pl->n <= 256 ? std::min({nvol, (unsigned)MAX_IMAGES2, pl->B}) : 1u;
+  const unsigned images = pl->nz == 1 && pl->n <= 256 ? images_for(pl->B, nvol, nangles) : 1u;
   for (unsigned v = 0; v < nvol; v += images) {
     const unsigned vb = std::min(images, nvol - v);
-    // at most 65,534: the row passes keep an orientation's place in its batch in 16 bits
-    const unsigned B = even_batch(std::min(pl->B / vb, 65534u), nangles);
+    // (a plan's batch is at most 256: the row passes keep an orientation's place in it in 16 bits)
+    const unsigned B = even_batch(pl->B / vb, nangles);
     const float2* Ev = E + (size_t)v * pl->H;
     const float* cv = ctf ? ctf + (size_t)v * ctf_stride : nullptr;
     float* bv = best + (size_t)v * pl->V;

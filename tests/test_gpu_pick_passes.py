@@ -53,7 +53,7 @@ def test_passes_match_oracle_and_each_other(gx, orc, cuda, n):
     assert cnt > 0 and agree == 1.0
 
 
-@pytest.mark.parametrize("n,batch", [(8, 0), (24, 3), (32, 0), (96, 7), (128, 0), (256, 0)])
+@pytest.mark.parametrize("n,batch", [(8, 0), (24, 3), (32, 0), (96, 7), (128, 0), (256, 0), (48, 6), (64, 11)])
 def test_images_in_one_call_equal_images_alone(gx, cuda, n, batch):
     import torch
     box = 2 * max(2, min(8, n // 4))
