@@ -1237,19 +1237,19 @@ __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__
 // A search's row pass: the C2R of every row of the orientations o in group
 // blockIdx.y (og of them), folded into a running maximum in registers (strict >,
 // increasing o). With FRESH the maximum starts at -infinity / -1 and goes to the
-// group's own nrows * n values. Rows of (n + 1) / 2 bins without X[n/2], which is
+// group's own n^3 values. Rows of (n + 1) / 2 bins without X[n/2], which is
 // sn[o].y, times sn[o].x.
 // A pair of voxels keeps its two orientations as 16-bit offsets in the group in
 // one register (NONE: unchanged): with 32-bit indices the 512-point form spills
 // (200^3: 1.38 ms per 32 orientations).
 template <class LN, bool FRESH>
 __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
-    const float2* __restrict__ G, long long H, int nb, int nrows, int angle0, const float2* __restrict__ sn,
+    const float2* __restrict__ G, long long H, int nb, int angle0, const float2* __restrict__ sn,
     float* __restrict__ best, int32_t* __restrict__ bidx, int og, LineArgs A) {
   constexpr int HP = LN::PTS;
   constexpr unsigned NONE = 0xffffu;
   float2* lds = line_lds<LN::ROW_LDS>();
-  const int t = threadIdx.x, n = A.L, R2 = LN::lanes(A), xp = LN::row_pitch(A);
+  const int t = threadIdx.x, n = A.L, nrows = n * n, R2 = LN::lanes(A), xp = LN::row_pitch(A);
   int j;
   const int slot = row_slot<LN>(t, A, &j);
   LN::stage(lds, t, 256, A);
@@ -1685,7 +1685,7 @@ int line_rows_c2r(int L, const float2* in, float* out, long long nrows, long lon
 
 bool rows_max_any_fused(int n) { return n <= BLUE_FUSED_MAX; }
 
-int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
+int rows_max_any(int n, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
                  int32_t* idx, int og, hipStream_t s) {
   const int groups = og > 0 ? (nb + og - 1) / og : 1;
   if (nb > 0xffff) return fail(GTOMX_ERR_INTERNAL, "row pass over more than 65535 orientations");
@@ -1693,10 +1693,10 @@ int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int ang
   GX_TRY(line_args(n, true, &A));
   return with_line(A, [&](auto ln) -> int {
     using LN = decltype(ln);
-    const int per = 2 * row_pairs<LN>(A), wgs = (nrows + per - 1) / per;
+    const int per = 2 * row_pairs<LN>(A), wgs = (n * n + per - 1) / per;
     auto go = [&](auto kernel) -> int {
-      hipLaunchKernelGGL(kernel, dim3(wgs, groups), dim3(256), row_lds<LN>(A), s, G, H, nb, nrows, angle0, sn, best, idx,
-                         og, A);
+      hipLaunchKernelGGL(kernel, dim3(wgs, groups), dim3(256), row_lds<LN>(A), s, G, H, nb, angle0, sn, best, idx, og,
+                         A);
       GX_LAUNCHED("k_line_rows_max");
       return GTOMX_OK;
     };
@@ -1710,12 +1710,12 @@ int line_search_y(int n, float2* G, int nb, hipStream_t s) {
 }
 
 // Two workgroups of 256 threads per CU fill the device; more groups cost more merging.
-int rows_max_any_groups(int n, int nrows, unsigned batch, int cus) {
+int rows_max_any_groups(int n, unsigned batch, int cus) {
   int wgs = 1;
   const LineArgs A = line_shape(n, true);
   const int st = with_line(A, [&](auto ln) -> int {
     const int per = 2 * row_pairs<decltype(ln)>(A);
-    wgs = (nrows + per - 1) / per;
+    wgs = (n * n + per - 1) / per;
     return GTOMX_OK;
   });
   if (st != GTOMX_OK) return 1;

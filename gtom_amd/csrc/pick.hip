@@ -1211,14 +1211,6 @@ __global__ __launch_bounds__(LN::COL_THREADS, 2) void k_pick_project_line(
 
 namespace gx {
 
-int merge_group_maxima(const float* gbest, const int32_t* gidx, int groups, size_t v, float* best, int32_t* idx,
-                       unsigned items, hipStream_t s) {
-  hipLaunchKernelGGL(k_pick_merge, dim3((unsigned)((v + 63) / 64), items), dim3(256), 0, s, gbest, gidx, groups, v,
-                     best, idx);
-  GX_LAUNCHED("k_pick_merge");
-  return GTOMX_OK;
-}
-
 namespace {
 
 // Images of one launch of the fused 2D passes: with 4 the samples cost a quarter,
@@ -1373,8 +1365,12 @@ int plane_groups_for(int n, unsigned batch, int cus) {
   return 0;
 }
 
+// The plan's `groups` maxima folded into best / idx, for each of `items` volumes or images.
 int merge_groups(gtomx_pick_plan* pl, int groups, float* best, int32_t* idx, hipStream_t s, unsigned items = 1) {
-  return merge_group_maxima(pl->gbest, pl->gidx, groups, pl->V, best, idx, items, s);
+  hipLaunchKernelGGL(k_pick_merge, dim3((unsigned)((pl->V + 63) / 64), items), dim3(256), 0, s, pl->gbest, pl->gidx,
+                     groups, pl->V, best, idx);
+  GX_LAUNCHED("k_pick_merge");
+  return GTOMX_OK;
 }
 
 template <int N, class PJ>
@@ -1563,8 +1559,7 @@ int run_batch_line(gtomx_pick_plan* pl, const PJ& PS, const Projector& P, const 
     const long long stride = (long long)((n + 1) / 2) * n * n;
     const int og = (nb + pl->groups3 - 1) / pl->groups3, groups = (nb + og - 1) / og;
     const bool fresh = groups > 1;
-    GX_TRY(rows_max_any(n, n * n, pl->G, stride, nb, angle0, pl->sn, fresh ? pl->gbest : best, fresh ? pl->gidx : idx,
-                        og, s));
+    GX_TRY(rows_max_any(n, pl->G, stride, nb, angle0, pl->sn, fresh ? pl->gbest : best, fresh ? pl->gidx : idx, og, s));
     return fresh ? merge_groups(pl, groups, best, idx, s) : GTOMX_OK;
   });
 }
@@ -2072,7 +2067,7 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   }
   if (is2d && !big2d) pl->pairs2 = pairs2_for(pl->n, pl->B, cus);
   if (!is2d && !any3d) pl->groups3 = plane_groups_for(pl->n, pl->B, cus);
-  if (gen3d && rows_max_any_fused(pl->n)) pl->groups3 = rows_max_any_groups(pl->n, pl->n * pl->n, pl->B, cus);
+  if (gen3d && rows_max_any_fused(pl->n)) pl->groups3 = rows_max_any_groups(pl->n, pl->B, cus);
   void* d = nullptr;
   auto alloc = [&](void** dst, size_t bytes) {
     if (s != GTOMX_OK) return;

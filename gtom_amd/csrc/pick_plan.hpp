@@ -87,8 +87,10 @@ int check_update_args(const gtomx_pick_plan* plan, const gtomx_complex* d_projec
 // The orientation loop of nvol volumes or images (spectra H apart, CTFs
 // ctf_stride apart): batches of at most pl->B spectra over mats (nangles matrices
 // already on the device) through the search's kernels with indices angle0 + o.
-// Kernel launches only (no host synchronisation, no allocation), so it can be
-// captured in a graph.
+// Images and the sides with fused passes: kernel launches only (no host
+// synchronisation, no allocation), so it can be captured in a graph. Other sides
+// build the tables of their lines at the first call of a length, and above 512 take
+// stream-ordered scratch.
 int launch_update_batches(gtomx_pick_plan* pl, const Projector& P, const CentredProjector* C, const float* mats,
                           unsigned nangles, unsigned nvol, const float2* E, const float* ctf, size_t ctf_stride,
                           float* best, int32_t* idx, int angle0, hipStream_t s);

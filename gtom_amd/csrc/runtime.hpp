@@ -217,22 +217,18 @@ int yz_axes_any(float2* data, gtomx_int3 dims, unsigned batch, int dir, hipStrea
 // spectrum o fills the first n^3 floats of its slot (every row is read before
 // the rows it overwrites are written). n at most 2048.
 int rows_c2r_any_inplace(float2* G, int n, int nb, long long H, hipStream_t s);
-// A search's row pass on rows of n <= 512 reals (rows_max_any_fused): the C2R of
-// the nrows rows of nb half spectra H apart in G (rows of (n + 1) / 2 bins without
-// X[n/2] = sn[o].y, times sn[o].x), folded into best / idx in orientation order from angle0 (strict >). og > 0 and
-// below nb: group g of og orientations starts afresh (-infinity, -1) and writes at
-// g * nrows * n of best / idx, for merge_group_maxima.
+// A search's row pass on volumes of side n <= 512 (rows_max_any_fused): the C2R of
+// the n^2 rows of nb half spectra H apart in G (rows of (n + 1) / 2 bins without
+// X[n/2] = sn[o].y, times sn[o].x), folded into best / idx in orientation order from
+// angle0 (strict >). og > 0 and below nb: group g of og orientations starts afresh
+// (-infinity, -1) and writes at g * n^3 of best / idx, for the search's merge.
 bool rows_max_any_fused(int n);
-int rows_max_any_groups(int n, int nrows, unsigned batch, int cus);  // groups of a batch that fill the device
-int rows_max_any(int n, int nrows, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
+int rows_max_any_groups(int n, unsigned batch, int cus);  // groups of a batch that fill the device
+int rows_max_any(int n, const float2* G, long long H, int nb, int angle0, const float2* sn, float* best,
                  int32_t* idx, int og, hipStream_t s);
 // The y inverse, in place, of nb n^3 search spectra (planes z of n rows of (n + 1) / 2
 // bins) whose bins outside the disc x^2 + y^2 <= (n/2)^2 read as zero; n at most 512.
 int line_search_y(int n, float2* G, int nb, hipStream_t s);
-// Folds `groups` maxima of v values each (gbest, gidx) into best / idx in group
-// order (strict >), for each of `items` (pick.hip).
-int merge_group_maxima(const float* gbest, const int32_t* gidx, int groups, size_t v, float* best, int32_t* idx,
-                       unsigned items, hipStream_t s);
 // Fourier-space resizing (resize.hip): op is one of the GTOMX_FFT_* values.
 constexpr int FFT_CROP = GTOMX_FFT_CROP, FFT_PAD = GTOMX_FFT_PAD, FFT_FULL_CROP = GTOMX_FFT_FULL_CROP,
               FFT_FULL_PAD = GTOMX_FFT_FULL_PAD;
