@@ -1230,7 +1230,6 @@ void plan_release(gtomx_pick_plan* pl) {
   dev_free(pl->ls_mem);
   dev_free(pl->cproj);
   dev_free(pl->gbest);
-  dev_free(pl->gidx);
   dev_free(pl->scr);
   dev_free(pl->tmasks);
   dev_free(pl->ldirs);
@@ -2107,11 +2106,10 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   } else if (is2d || pl->groups3 > 1) {
     const size_t groups = is2d ? (size_t)pl->pairs2 : (size_t)pl->groups3;
     d = nullptr;
-    alloc(&d, groups * pl->V * sizeof(float));
+    // one block for both: each large one costs a plan's life 40 us (creating and destroying one for 16^3 117 -> 78 us)
+    alloc(&d, groups * pl->V * (sizeof(float) + sizeof(int32_t)));
     pl->gbest = static_cast<float*>(d);
-    d = nullptr;
-    alloc(&d, groups * pl->V * sizeof(int32_t));
-    pl->gidx = static_cast<int32_t*>(d);
+    pl->gidx = d ? reinterpret_cast<int32_t*>(pl->gbest + groups * pl->V) : nullptr;
   }
   if (s != GTOMX_OK) {
     std::string msg = gtomx_last_error();

@@ -35,7 +35,7 @@ struct gtomx_pick_plan {
   void* ls_mem = nullptr;
   gx::LocalStdScratch ls{};
   float2* cproj = nullptr;  // centred projector layout
-  float* gbest = nullptr;   // per-orientation-group maxima (groups x V)
+  float* gbest = nullptr;   // per-orientation-group maxima (groups x V), gidx behind them in the same block
   int32_t* gidx = nullptr;
   int pairs2 = 0;           // fused 2D passes: most (image, group) pairs of a launch
   int groups3 = 0;          // 3D sides of k_pick_plane_max and k_line_rows_max: most groups of a batch
