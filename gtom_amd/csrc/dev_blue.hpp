@@ -38,8 +38,8 @@ constexpr int BLUE_FUSED_MAX = 512;  // longest L of the fused form
 // M values with the 1/M in them), or with CONJ conj(B): the kernels of the two
 // directions are conjugate and even, so their spectra are conjugate too. v[m] in
 // and out: point j + R2 m, zero for m >= R1/2 on entry, meaningful for m < R1/2 on
-// exit. Bound by its instructions: 3.9e8 vector instructions per pass of 200^3 x 32
-// orientations are 0.65 ms of issue in passes of 0.8 to 1.2 ms.
+// exit. Bound by its instructions: 3.8e8 vector instructions in pass 1 and 3.9e8 in the row
+// pass of 197^3 x 32 orientations are 0.62 ms of issue each, in 0.87 and 1.19 ms.
 template <int M, bool CONJ = false, class Xch, class Sync>
 __device__ __forceinline__ void blue_convolve(float2 (&v)[BlueShape<M>::R1], int j, const float2* twl,
                                               const float2* B, Xch xch, Sync sync) {
@@ -84,7 +84,8 @@ struct LineArgs {
 // Chirp-z. Tables: the twiddles W_M^{j k1} at k1 (R2 + 1) + j, the kernel spectrum,
 // the chirp. (A table of W_M^i read at i = j k1 puts the 16 lanes of a row on up to 16
 // addresses of one bank; by k1 and j, with one value of padding, both transforms read
-// it without conflicts: rows of 200^3 x 32 orientations 1.17 ms, 1.23 before.)
+// it without conflicts: the row pass of a 200^3 search took 1.17 ms per 32 orientations in
+// this form, which that side had then, 1.23 before.)
 template <int M> struct BlueLine {
   using S = BlueShape<M>;
   static constexpr int R1 = S::R1, R2 = S::R2, PTS = R1 / 2, REGS = R1;

@@ -1089,15 +1089,18 @@ int fft_c2r_cols_inplace(float2* data, gtomx_int3 d, unsigned batch, hipStream_t
 // and 256 MB. The Picker takes the gathered form at every length (LineForm).
 
 // ---------------------------------------------------------------------------
-// Lengths up to 512: load, both M-point transforms and the store in one kernel,
-// one pass over memory instead of five over a block 2 to 4 times as long (a 200^3
-// search spent 64% of its time in the column transforms and k_blue_mul of that
-// block). R2 threads hold a line; thread j the points j + R2 m. L <= M/2, so only
-// m < R1/2 hold input and only those are wanted back: the compiler drops the
+// Lengths up to 512: load, transform and store of a line (dev_blue.hpp) in one
+// kernel, one pass over memory. A chirp-z line in five passes moves a block 2 to 4
+// times as long (a 200^3 search spent 64% of its time in the column transforms and
+// k_blue_mul of that block: 64.7 ms for 96 orientations, 10.9 as chirp-z lines, 4.9
+// as mixed-radix ones).
+//
+// Chirp-z lines: R2 threads hold a line; thread j the points j + R2 m. L <= M/2, so
+// only m < R1/2 hold input and only those are wanted back: the compiler drops the
 // rest of the first and last stages. The transform ends with every k2 of a k1 in
 // one thread (k = k1 + R1 k2), which is where the inverse can start, so the
 // product with B needs no exchange of its own: two exchanges in all, the second
-// through the addresses a thread read itself.
+// through the addresses a thread read itself. Mixed-radix lines: SmoothLine.
 // ---------------------------------------------------------------------------
 // A strided axis, from src into dst (which may be src), addressed as k_cols. With
 // half > 0 the axis is y of a search's planes, whose entries outside the disc
@@ -1240,8 +1243,8 @@ __global__ __launch_bounds__(256) void k_line_rows_r2c(const float* __restrict__
 // group's own n^3 values. Rows of (n + 1) / 2 bins without X[n/2], which is
 // sn[o].y, times sn[o].x.
 // A pair of voxels keeps its two orientations as 16-bit offsets in the group in
-// one register (NONE: unchanged): with 32-bit indices the 512-point form spills
-// (200^3: 1.38 ms per 32 orientations).
+// one register (NONE: unchanged): with 32-bit indices the chirp-z form of 512 points
+// spills (200^3, when it had that form: 1.38 ms per 32 orientations instead of 1.17).
 template <class LN, bool FRESH>
 __global__ __launch_bounds__(256, LN::ROW_WAVES) void k_line_rows_max(
     const float2* __restrict__ G, long long H, int nb, int angle0, const float2* __restrict__ sn,
@@ -1557,7 +1560,13 @@ unsigned blue_grid(long long n) { return (unsigned)std::max<long long>(1, std::m
 // {4 .. 9}; RL = 0 when there is no such form. Columns: one stage before two (200^3 x 32 orientations, y: 168 us a
 // launch as 20 x 10, 211 as 10 x (4 x 5)), then the smallest RL, which leaves the most threads to a line. Rows, whose
 // running maxima take registers by RL (763 us as 20 x 10, 386 as 10 x (4 x 5)): the smallest RL from 8 up (75: 139 us
-// as 15 x 5, 196 as 5 x (3 x 5)). Before that, lanes that fill 54 or more of a wave's 64 with whole row pairs.
+// as 15 x 5, 196 as 5 x (3 x 5)). Before that, lanes that fill 54 or more of a wave's 64 with whole row pairs, which
+// decides at three lengths only and is worth little either way (searches of 200^3 3% faster with it, of 225^3 and
+// 400^3 up to 3 and 4% slower).
+// In the standalone transforms, over the 73 lengths that take this form (16 Mi points): rows within 10% of the best
+// split at 65 of them, 1.3 times it at 75 and 105 (15 x 5 and 15 x 7, for the search's sake); columns within 10% at
+// 64, and 1.2 to 1.4 times it at 30 to 60, 80 and 100, where a larger RL leaves 5 lanes or fewer,
+// whose tiles are 32 columns wide.
 LineArgs line_shape(int L, bool rows) {
   LineArgs A;
   A.L = L;

@@ -992,7 +992,7 @@ __global__ __launch_bounds__(TX * LineShape<L1>::R2) void k_pick2d_project_cols(
   __shared__ float red[(NT + 63) / 64];
   const int NH = n / 2 + 1, HALF = n / 2;
   // whole waves share j with 64 columns, so that rows and twiddles are wave-uniform (with that, no reads of E
-  // outside the disc and whole 8-byte stores 4096^2 x 15 orientations take 0.82 ms, 0.95 before)
+  // outside the disc and whole 8-byte stores 4096^2 x 24 orientations take 0.81 ms, 0.95 before)
   const int t = threadIdx.x, c = t % TX, j = TX % 64 == 0 ? __builtin_amdgcn_readfirstlane(t / TX) : t / TX;
   const int o = blockIdx.y / L2, n2 = blockIdx.y % L2;
   const int ix = blockIdx.x * TX + c;
@@ -2031,8 +2031,8 @@ int gtomx_pick_plan_create(gtomx_pick_plan** out, gtomx_int3 dp, gtomx_int3 dv, 
   const unsigned big3_b = (unsigned)std::max<size_t>(1, std::min<size_t>(32, (8ull << 30) / (pl->H * sizeof(float2))));
   // volumes of 128 and more: 128 orientations per batch (the fixed costs of a batch -- E and the CTF
   // in pass 1, the running maxima in pass 3 -- spread over more orientations; 8.7 GB of spectra at 256^3);
-  // smaller volumes: 256 (their launches are short, so their number matters most: 1.89 ms for 588
-  // orientations of 64^3 at 256 against 2.68 ms at 16)
+  // smaller volumes: 256 (their launches are short, so their number matters most: 0.66 ms for 588
+  // orientations of 64^3 at 256, 0.76 at 128, 2.08 at 16)
   pl->B = batch ? batch : (is2d ? (big2d ? big_b : 240u) : (any3d ? big3_b : (dv.x >= 128 ? 128u : 256u)));
   pl->gen3d = gen3d;
   const bool line = gen3d && rows_max_any_fused(dv.x);  // lines inside the search's own passes

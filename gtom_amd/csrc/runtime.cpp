@@ -61,8 +61,9 @@ int alloc_hook() {
 // at most SCRATCH_CAP bytes per device: whenever a block is given back or a new one
 // made, the least recently used beyond that go back to the runtime, and those not
 // taken for SCRATCH_IDLE takes with them. All of them go when an allocation of this
-// library fails, and when the program asks (gtomx_scratch_release). Blocks come from hipMallocAsync and go back through
-// hipFreeAsync, which other threads' stream captures allow.
+// library fails, and when the program asks (gtomx_scratch_release). Blocks come
+// from hipMallocAsync and go back through hipFreeAsync, which other threads' stream
+// captures allow.
 struct ScratchBlock {
   void* p = nullptr;  // nullptr: a free slot
   size_t bytes = 0;
