@@ -1563,10 +1563,10 @@ unsigned blue_grid(long long n) { return (unsigned)std::max<long long>(1, std::m
 // as 15 x 5, 196 as 5 x (3 x 5)). Before that, lanes that fill 54 or more of a wave's 64 with whole row pairs, which
 // decides at three lengths only and is worth little either way (searches of 200^3 3% faster with it, of 225^3 and
 // 400^3 up to 3 and 4% slower).
-// In the standalone transforms, over the 73 lengths that take this form (16 Mi points): rows within 10% of the best
-// split at 65 of them, 1.3 times it at 75 and 105 (15 x 5 and 15 x 7, for the search's sake); columns within 10% at
-// 64, and 1.2 to 1.4 times it at 30 to 60, 80 and 100, where a larger RL leaves 5 lanes or fewer,
-// whose tiles are 32 columns wide.
+// In the standalone transforms (16 Mi points; 73 of the 74 lengths that take this form, without 384): rows within 10%
+// of the best split at 65, 1.3 times it at 75 and 105 (15 x 5 and 15 x 7, for the search's sake); columns within 10%
+// at 64, and 1.2 to 1.4 times it at 30 to 60, 80 and 100, where a larger RL leaves 5 lanes or fewer, whose tiles are 32
+// columns wide.
 LineArgs line_shape(int L, bool rows) {
   LineArgs A;
   A.L = L;
