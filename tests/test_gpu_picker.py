@@ -220,9 +220,9 @@ def picker_lines_case(gx, cuda, shape, nr):
 
 @pytest.mark.parametrize("shape,nr", LINE_CASES)
 def test_picker_extents_without_native_transform_round_as_recorded(gx, cuda, shape, nr):
-    """golden/picker_lines.npz holds what the class gave before lines of up to 512 points had kernels of their own
-    (commit 899c80c). The winning orientation follows the last bit of the maps where two tie, so the maps keep
-    every bit, whatever the other transforms of these lengths do."""
+    """golden/picker_lines.npz holds picker_lines_case of each case (best_SHAPE, index_SHAPE), recorded when every
+    transform of such extents took the gathered chirp-z form. The winning orientation follows the last bit of the
+    maps where two tie, so the maps keep every bit, whatever the other transforms of these lengths do."""
     golden = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "picker_lines.npz"))
     best, index = picker_lines_case(gx, cuda, shape, nr)
     key = "x".join(map(str, shape))
